@@ -51,6 +51,8 @@ enum : uint32_t {
   F_SCALE = 1u << 6,      // FieldScaling != 1
   F_THICK = 1u << 7,      // RF / corrector with non-zero length
   F_RFKICK = 1u << 8,     // RF with nv != 0
+  F_LEAN = 1u << 9,       // thick multipole without FieldScaling, quadrupole fringes, edges with
+                          // a tangent per particle and op table
 };
 
 // Edge-focusing modes (vertical term fy) chosen on the host from
@@ -115,11 +117,67 @@ struct DevElem {
 // then (code, length) pairs with code 0 = drift of that length, 1 = kick.
 static_assert(sizeof(DevElem) == 64, "DevElem must stay 64 bytes (dword fields: scalar loads)");
 
+// The tracking kernel's program of a lattice: one record per element that
+// does work, holding the markers and the plain drift before it, so that a
+// record costs one round of scalar loads and one dispatch. Elements of a
+// record, in order: markers (IdentityPass without attributes), a plain drift
+// (flag OPF_DRIFT), the element of `op` (other than OP_NONE); `last` is the
+// index of the last of them. The constants an op needs are in the record
+// itself, at fixed offsets, so that no address depends on an earlier load. A
+// terminal record follows the last one: the kernel reads the head (the first
+// 16 bytes) one record ahead.
+enum OpKind : int32_t {
+  OP_NONE = 0,      // no element after the markers and the drift
+  OP_GENERIC = 1,   // the element by its DevElem header
+  OP_APERTURE = 2,  // AperturePass: c[0..3] = limits
+  OP_CORR = 3,      // CorrectorPass without attributes: c[OC_*]
+  // thick multipoles without FieldScaling, quadrupole fringes, apertures and
+  // op table, of the orders that rings are made of: c[OM_*]
+  OP_STR1 = 4,
+  OP_STR2 = 5,
+  OP_STR3 = 6,
+  OP_BND1 = 7,
+  OP_STRRAD1 = 8,
+  OP_BNDRAD1 = 9,
+  // ThinMPolePass without attributes: c[OT_*], c[OM_POLY...]
+  OP_THIN2 = 10,
+  OP_THIN3 = 11,
+};
+enum : int32_t {
+  OPF_DRIFT = 1 << 8,  // a plain drift of length `len` before the element
+  OPF_THICK = 2 << 8,  // corrector of non-zero length
+  OPF_XF = 4 << 8,     // misaligned by transverse shifts and rolls: c[OM_XF...]
+  OPF_EDGE = 8 << 8,   // a bend's edges by its header (not of constant strength)
+};
+// constants of OP_CORR, the thin and the thick multipoles
+enum OpSlot : int32_t {
+  OC_XK = 0, OC_YK = 1, OC_LEN = 2, OC_Q0 = 3,
+  OT_BAX = 0, OT_BAY = 1,
+  OM_L1 = 0, OM_L2 = 1, OM_K1 = 2, OM_K2 = 3, OM_IRHO = 4, OM_RADC = 5, OM_RK1 = 6, OM_RK2 = 7,
+  OM_POLY = 8,  // A[0..order], then B[0..order]
+  OM_FX_IN = 12, OM_FY_IN = 13, OM_FX_OUT = 14, OM_FY_OUT = 15,  // bends (order 1)
+  // entry: x, px, y, py shifts, then cos and sin of the roll; exit: cos, sin, shifts
+  OM_XF = 16,
+};
+constexpr int kOpConsts = 28;
+struct LatOp {
+  int32_t op;      // OpKind | OPF_*
+  int32_t last;    // index of the record's last element
+  double len;      // the drift's length
+  int32_t first;   // index of its first element (the next record's: one past its last)
+  int32_t nslice;
+  int32_t pad[2];
+  double c[kOpConsts];
+};
+static_assert(sizeof(LatOp) == 256, "LatOp: four 64-byte lines");
+
 // One tracked lattice instance inside a launch. A single-lattice call has one
 // instance; batched error realisations have one per lattice.
 struct Instance {
   const DevElem* elems;
   const double* pool;
+  const LatOp* ops;         // program records
+  const int32_t* opof;      // record of each element
   const int32_t* slots;     // 2*(nelem+1): refpt copy rank per element, first turn then later turns
   double* r;                // particle state, updated in place
   double* rout;             // refpt copies (6, N, R, T) F-order

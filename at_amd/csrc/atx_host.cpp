@@ -113,6 +113,8 @@ struct HostElem {
 struct Compiled {
   std::vector<DevElem> elems;
   std::vector<double> pool;
+  std::vector<LatOp> ops;      // program of the tracking kernel (build_program)
+  std::vector<int32_t> opof;   // record of each element
   double T0 = 0.0;
   std::vector<int32_t> r1inv, r2inv;  // per element, pool offsets (-1: none)
   std::vector<std::string> adjerr;    // per element, why the adjoint cannot run it ("" = it can)
@@ -194,13 +196,14 @@ struct atx_lattice {
   std::vector<atx::HostElem> elems;
   // device copy of the compiled lattice, valid for (energy, rest, elempass)
   bool dev_valid = false;
-  bool has_ext = false;  // CavityPass or exact passes present: extended kernel variant
   double dev_energy = -1.0, dev_rest = -1.0;
   bool dev_elempass = false;
   int dev_device = -1;
+  char* d_lat = nullptr;  // one allocation: program records, elements, pool, records of elements
+  atx::LatOp* d_ops = nullptr;
   atx::DevElem* d_elems = nullptr;
   double* d_pool = nullptr;
-  size_t d_elems_n = 0, d_pool_n = 0;
+  int32_t* d_opof = nullptr;
   int64_t turn_counter = 0;
   int integrator = 4;
   atx_launch_shape shape{0, 0, 0, 0};  // atx_track / atx_elempass launches (0: default)
@@ -568,6 +571,12 @@ int compile_elem(const HostElem& e, int idx, double energy, double rest, double 
   }
   if (rd.err) return rd.err;
   h.sc = push(pool, sc, S_NSCALAR);
+  if (h.kind == K_STR || h.kind == K_BND || h.kind == K_STRRAD || h.kind == K_BNDRAD) {
+    auto flat = [](int m) { return m == E_CONST || m == E_DIVP || m == E_MULPN; };
+    if (!(h.flags & F_SCALE) && h.fringe == 0 && h.ops < 0 && flat(h.edge & 0xff) &&
+        flat((h.edge >> 8) & 0xff))
+      h.flags |= F_LEAN;
+  }
   // adjoint support: inverse misalignment matrices, and whether the reverse
   // kernel can invert this element in closed form
   int32_t r1i = -1, r2i = -1;
@@ -603,6 +612,114 @@ int compile_elem(const HostElem& e, int idx, double energy, double rest, double 
   return ATX_OK;
 }
 
+// Transverse shifts (T: no delta, no ct) and a roll about s (R: cos, sin of
+// one angle in both planes), the misalignments that records hold.
+bool plain_shift(const double* t) { return t[4] == 0.0 && t[5] == 0.0; }
+bool plain_roll(const double* m, double* c, double* s) {
+  *c = m[0];
+  *s = m[0 + 6 * 2];
+  for (int i = 0; i < 6; i++)
+    for (int j = 0; j < 6; j++) {
+      double want = 0.0;
+      if (i == j) want = i < 4 ? *c : 1.0;
+      if (j == i + 2 && i < 2) want = *s;
+      if (i == j + 2 && j < 2) want = -*s;
+      if (m[i + 6 * j] != want) return false;
+    }
+  return true;
+}
+
+// The op of an element with constants in its record, or OP_GENERIC.
+void fill_op(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
+  const double* sc = &pool[h.sc];
+  const int32_t drift = r.op;  // the flags so far
+  r.op = drift | OP_GENERIC;
+  if (h.kind == K_APERTURE) {
+    r.op = drift | OP_APERTURE;
+    for (int k = 0; k < 4; k++) r.c[k] = pool[h.rap + k];
+  } else if (h.kind == K_CORR && (h.flags & ~(uint32_t)F_THICK) == 0) {
+    r.op = drift | OP_CORR | ((h.flags & F_THICK) ? OPF_THICK : 0);
+    r.c[OC_XK] = sc[S_C_XK];
+    r.c[OC_YK] = sc[S_C_YK];
+    r.c[OC_LEN] = sc[S_C_LEN];
+    r.c[OC_Q0] = sc[S_C_Q0];
+  } else if (h.kind == K_THIN && h.flags == 0 && (h.order == 2 || h.order == 3)) {
+    r.op = drift | (h.order == 2 ? OP_THIN2 : OP_THIN3);
+    r.c[OT_BAX] = sc[S_BAX];
+    r.c[OT_BAY] = sc[S_BAY];
+    for (int k = 0; k < 2 * (h.order + 1); k++) r.c[OM_POLY + k] = pool[h.poly + k];
+  } else if ((h.kind == K_STR || h.kind == K_BND || h.kind == K_STRRAD || h.kind == K_BNDRAD) &&
+             !(h.flags & (F_RAP | F_EAP | F_SCALE)) && h.fringe == 0 && h.ops < 0) {
+    int op = OP_GENERIC;
+    if (h.kind == K_STR && h.order >= 1 && h.order <= 3) op = OP_STR1 + (h.order - 1);
+    if (h.order == 1) {
+      if (h.kind == K_BND) op = OP_BND1;
+      if (h.kind == K_STRRAD) op = OP_STRRAD1;
+      if (h.kind == K_BNDRAD) op = OP_BNDRAD1;
+    }
+    // a missing transform is the identity: + 0 and (1, 0) leave a coordinate as it is
+    double* xf = r.c + OM_XF;
+    const double* t1 = (h.flags & F_T1) ? &pool[h.t1] : nullptr;
+    const double* t2 = (h.flags & F_T2) ? &pool[h.t2] : nullptr;
+    for (int k = 0; k < 4; k++) {
+      xf[k] = t1 ? t1[k] : 0.0;
+      xf[8 + k] = t2 ? t2[k] : 0.0;
+    }
+    xf[4] = xf[6] = 1.0;
+    bool plain = (!t1 || plain_shift(t1)) && (!t2 || plain_shift(t2));
+    if (h.flags & F_R1) plain = plain && plain_roll(&pool[h.r1], &xf[4], &xf[5]);
+    if (h.flags & F_R2) plain = plain && plain_roll(&pool[h.r2], &xf[6], &xf[7]);
+    if (op == OP_GENERIC || !plain) return;
+    if (h.flags & (F_T1 | F_T2 | F_R1 | F_R2)) op |= OPF_XF;
+    if ((h.edge & 0xff) != E_CONST || ((h.edge >> 8) & 0xff) != E_CONST) op |= OPF_EDGE;
+    r.op = drift | op;
+    r.nslice = h.nslice;
+    static const int from[8] = {S_L1, S_L2, S_K1, S_K2, S_IRHO, S_RADC, S_RK1, S_RK2};
+    for (int k = 0; k < 8; k++) r.c[k] = sc[from[k]];
+    for (int k = 0; k < 2 * (h.order + 1); k++) r.c[OM_POLY + k] = pool[h.poly + k];
+    if (h.kind == K_BND || h.kind == K_BNDRAD) {
+      r.c[OM_FX_IN] = sc[S_FX_IN];
+      r.c[OM_FY_IN] = sc[S_FY_IN];
+      r.c[OM_FX_OUT] = sc[S_FX_OUT];
+      r.c[OM_FY_OUT] = sc[S_FY_OUT];
+    }
+  }
+}
+
+// The program of a compiled lattice (LatOp).
+void build_program(Compiled& out) {
+  const int n = (int)out.elems.size();
+  out.ops.clear();
+  out.opof.assign(n + 1, 0);
+  int e = 0;
+  while (e < n) {
+    LatOp r;
+    std::memset(&r, 0, sizeof(r));
+    r.first = e;
+    while (e < n && out.elems[e].kind == K_IDENTITY && out.elems[e].flags == 0) e++;
+    if (e < n && out.elems[e].kind == K_DRIFT && out.elems[e].flags == 0) {
+      r.op = OPF_DRIFT;
+      r.len = out.pool[out.elems[e].sc + S_D_LEN];
+      e++;
+    }
+    const bool plain = e < n && out.elems[e].flags == 0 &&
+                       (out.elems[e].kind == K_DRIFT || out.elems[e].kind == K_IDENTITY);
+    if (e < n && !plain) {
+      fill_op(out.elems[e], out.pool, r);
+      e++;
+    }
+    r.last = e - 1;
+    for (int k = r.first; k < e; k++) out.opof[k] = (int32_t)out.ops.size();
+    out.ops.push_back(r);
+  }
+  LatOp last;
+  std::memset(&last, 0, sizeof(last));
+  last.first = n;
+  last.last = n - 1;
+  out.opof[n] = (int32_t)out.ops.size();
+  out.ops.push_back(last);
+}
+
 int compile_lattice(const atx_lattice* lat, double energy, double rest, bool elempass,
                     Compiled& out) {
   double ring_length = 0.0;
@@ -618,6 +735,7 @@ int compile_lattice(const atx_lattice* lat, double energy, double rest, bool ele
     if (rc) return rc;
   }
   if (out.pool.empty()) out.pool.push_back(0.0);
+  build_program(out);
   return ATX_OK;
 }
 
@@ -654,29 +772,32 @@ int ensure_device_lattice(atx_lattice* lat, double energy, double rest, bool ele
   Compiled c;
   int rc = compile_lattice(lat, energy, rest, elempass, c);
   if (rc) return rc;
-  if (lat->d_elems) (void)hipFree(lat->d_elems);
-  if (lat->d_pool) (void)hipFree(lat->d_pool);
-  lat->d_elems = nullptr;
-  lat->d_pool = nullptr;
+  if (lat->d_lat) (void)hipFree(lat->d_lat);
+  lat->d_lat = nullptr;
   lat->dev_valid = false;
-  const size_t ne = c.elems.empty() ? 1 : c.elems.size();
-  HIPCHK(hipMalloc(&lat->d_elems, ne * sizeof(DevElem)));
-  HIPCHK(hipMalloc(&lat->d_pool, c.pool.size() * sizeof(double)));
-  if (!c.elems.empty())
-    HIPCHK(hipMemcpy(lat->d_elems, c.elems.data(), c.elems.size() * sizeof(DevElem), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(lat->d_pool, c.pool.data(), c.pool.size() * sizeof(double), hipMemcpyHostToDevice));
-  lat->d_elems_n = c.elems.size();
-  lat->d_pool_n = c.pool.size();
+  // one allocation and one copy; every part starts on a 64-byte line
+  const size_t part[4] = {c.ops.size() * sizeof(LatOp), c.elems.size() * sizeof(DevElem),
+                          c.pool.size() * sizeof(double), c.opof.size() * sizeof(int32_t)};
+  const void* src[4] = {c.ops.data(), c.elems.data(), c.pool.data(), c.opof.data()};
+  size_t off[5] = {0, 0, 0, 0, 0};
+  for (int k = 0; k < 4; k++) off[k + 1] = (off[k] + part[k] + 63) & ~(size_t)63;
+  std::vector<char> host(off[4]);
+  for (int k = 0; k < 4; k++)
+    if (part[k]) std::memcpy(host.data() + off[k], src[k], part[k]);
+  HIPCHK(hipMalloc((void**)&lat->d_lat, host.size()));
+  HIPCHK(hipMemcpy(lat->d_lat, host.data(), host.size(), hipMemcpyHostToDevice));
+  lat->d_ops = (LatOp*)(lat->d_lat + off[0]);
+  lat->d_elems = (DevElem*)(lat->d_lat + off[1]);
+  lat->d_pool = (double*)(lat->d_lat + off[2]);
+  lat->d_opof = (int32_t*)(lat->d_lat + off[3]);
   lat->h_r1inv = c.r1inv;
   lat->h_r2inv = c.r2inv;
   lat->h_adjerr = c.adjerr;
   lat->h_order.clear();
   lat->h_kind.clear();
-  lat->has_ext = false;
   for (const auto& h : c.elems) {
     lat->h_order.push_back(h.order);
     lat->h_kind.push_back(h.kind);
-    lat->has_ext |= h.kind >= K_CAVITY;
   }
   lat->dev_valid = true;
   lat->dev_energy = energy;
@@ -793,11 +914,13 @@ hipError_t upload_async(void* dst, const void* src, size_t bytes, hipStream_t st
 // slots[i] is the refpt slot table of instance i; instances that share a
 // table (same pointer) share its device copy.
 int launch_instances(std::vector<Instance>& insts, const std::vector<const std::vector<int32_t>*>& slots,
-                     const atx_launch_shape& shape, hipStream_t stream, bool strict, bool ext) {
+                     const atx_launch_shape& shape, hipStream_t stream, bool strict) {
   const int block = shape.block;
   const int per_wg = block * shape.ppt;  // particle slots per workgroup
   int nblocks = 0;
+  bool refs = false;  // some instance has refpt copies: the kernel with them
   for (auto& in : insts) {
+    refs |= (in.n_first | in.n_std) != 0;
     in.block_begin = nblocks;
     nblocks += (int)((in.npart + per_wg - 1) / per_wg);
   }
@@ -827,7 +950,7 @@ int launch_instances(std::vector<Instance>& insts, const std::vector<const std::
   hipError_t le = hipSuccess;
   if (ce == hipSuccess)
     le = track_launcher(strict, shape)((const Instance*)d_scratch, (int)insts.size(), nblocks, block,
-                                       ext ? 1 : 0, xcd_order(insts.data(), insts.size()) ? 1 : 0,
+                                       refs ? 1 : 0, xcd_order(insts.data(), insts.size()) ? 1 : 0,
                                        nullptr, stream);
   hipError_t fe = hipFreeAsync(d_scratch, stream);
   if (ce != hipSuccess) return fail(ATX_E_RUNTIME, std::string("upload: ") + hipGetErrorString(ce));
@@ -881,7 +1004,7 @@ std::vector<int> repack_bounds(int nturns) {
 // private stream into one graph, which runs on `stream`. Each particle's
 // arithmetic is unchanged, so results equal those of launch_instances.
 int launch_repacked(std::vector<Instance>& insts, const std::vector<const std::vector<int32_t>*>& slots,
-                    const atx_launch_shape& shape, hipStream_t stream, bool strict, bool ext) {
+                    const atx_launch_shape& shape, hipStream_t stream, bool strict) {
   const int block = shape.block, ppt = shape.ppt;
   const int per_wg = block * ppt;  // particle slots per workgroup
   const int fine = 64 * ppt;       // ... when the survivors run one wave per workgroup
@@ -974,8 +1097,7 @@ int launch_repacked(std::vector<Instance>& insts, const std::vector<const std::v
       if (le != hipSuccess) break;
       const int32_t* lb = k > 0 ? live : nullptr;
       const int grid = k > 0 ? nblocks_fine : nblocks;
-      le = track_launcher(strict, shape)(t, (int)ninst, grid, block, ext ? 1 : 0, xcd ? 1 : 0, lb,
-                                         cap);
+      le = track_launcher(strict, shape)(t, (int)ninst, grid, block, 0, xcd ? 1 : 0, lb, cap);
       if (le == hipSuccess && k + 1 < nblk)
         le = atx_launch_repack((const Instance*)(d + (size_t)(k + 1) * tab), (int)ninst, k == 0 ? 1 : 0, cap);
     }
@@ -1020,6 +1142,8 @@ int single_instance(atx_lattice* lat, double* d_r, int64_t pstride, int64_t cstr
   std::memset(&inst, 0, sizeof(inst));
   inst.elems = lat->d_elems;
   inst.pool = lat->d_pool;
+  inst.ops = lat->d_ops;
+  inst.opof = lat->d_opof;
   inst.r = d_r;
   inst.rout = d_rout;
   inst.lost_flag = d_lf;
@@ -1069,8 +1193,8 @@ int track_device(atx_lattice* lat, double* d_r, int64_t pstride, int64_t cstride
   // survivors repacked between turn blocks: only without refpts (lost
   // particles still fill their copies, at.c:622-626)
   if (repack && nref == 0 && nturns > 1)
-    return launch_repacked(insts, {&slots[0]}, shape, stream, strict, lat->has_ext);
-  return launch_instances(insts, {&slots[0]}, shape, stream, strict, lat->has_ext);
+    return launch_repacked(insts, {&slots[0]}, shape, stream, strict);
+  return launch_instances(insts, {&slots[0]}, shape, stream, strict);
 }
 
 int check_partial(int nelem, int nturns, int& start, int& end) {
@@ -1157,8 +1281,7 @@ int atx_lattice_create(atx_lattice** out) {
 
 int atx_lattice_destroy(atx_lattice* lat) {
   if (!lat) return ATX_OK;
-  if (lat->d_elems) (void)hipFree(lat->d_elems);
-  if (lat->d_pool) (void)hipFree(lat->d_pool);
+  if (lat->d_lat) (void)hipFree(lat->d_lat);
   delete lat;
   return ATX_OK;
 }
@@ -1375,7 +1498,6 @@ int atx_track_batch(const atx_batch_item* items, int32_t nitems, int32_t nturns,
     if (items[i].nturns >= 0 && items[i].turn < 0)
       return fail(ATX_E_VALUE, "item " + std::to_string(i) + ": turn must be >= 0");
   std::vector<Instance> insts;
-  bool ext = false;
   std::map<int, std::vector<int32_t>> empty_slots;  // refpts = [] table per ring length
   std::vector<const std::vector<int32_t>*> slots;
   for (int i = 0; i < nitems; i++) {
@@ -1400,12 +1522,13 @@ int atx_track_batch(const atx_batch_item* items, int32_t nitems, int32_t nturns,
     int rc = ensure_device_lattice(it.lattice, energy, rest_energy, false);
     if (rc) return fail(rc, "item " + std::to_string(i) + ": " + g_err);
     if (it.num_particles == 0) continue;
-    ext |= it.lattice->has_ext;
     const int nelem = (int)it.lattice->elems.size();
     Instance in;
     std::memset(&in, 0, sizeof(in));
     in.elems = it.lattice->d_elems;
     in.pool = it.lattice->d_pool;
+    in.ops = it.lattice->d_ops;
+    in.opof = it.lattice->d_opof;
     in.r = it.r;
     in.lost_flag = it.lost_flag;
     in.lost_turn = it.lost_turn;
@@ -1442,8 +1565,8 @@ int atx_track_batch(const atx_batch_item* items, int32_t nitems, int32_t nturns,
     sorted_slots.push_back(slots[i]);
   }
   if (flags & ATX_REPACK)
-    return launch_repacked(sorted_insts, sorted_slots, shape, stream, strict, ext);
-  return launch_instances(sorted_insts, sorted_slots, shape, stream, strict, ext);
+    return launch_repacked(sorted_insts, sorted_slots, shape, stream, strict);
+  return launch_instances(sorted_insts, sorted_slots, shape, stream, strict);
 }
 
 int atx_track_batch_noalloc(const atx_batch_item* items, int32_t nitems, int32_t nturns,
@@ -1494,7 +1617,6 @@ int atx_track_batch_noalloc(const atx_batch_item* items, int32_t nitems, int32_t
   Instance tab[kNoAllocItems];
   int64_t work[kNoAllocItems];
   int n = 0;
-  bool ext = false;
   for (int i = 0; i < nitems; i++) {
     const atx_batch_item& it = items[i];
     atx_lattice* lat = it.lattice;
@@ -1507,12 +1629,13 @@ int atx_track_batch_noalloc(const atx_batch_item* items, int32_t nitems, int32_t
                                    "with atx_track or atx_track_batch first)");
     const int nt = it.nturns >= 0 ? it.nturns : nturns;
     if (it.num_particles == 0 || nt == 0) continue;
-    ext |= lat->has_ext;
     Instance& in = tab[n];
     std::memset(&in, 0, sizeof(in));
     const int nelem = (int)lat->elems.size();
     in.elems = lat->d_elems;
     in.pool = lat->d_pool;
+    in.ops = lat->d_ops;
+    in.opof = lat->d_opof;
     in.slots = nullptr;  // no refpts: the kernel reads no slot table
     in.r = it.r;
     in.lost_flag = it.lost_flag;
@@ -1557,7 +1680,7 @@ int atx_track_batch_noalloc(const atx_batch_item* items, int32_t nitems, int32_t
     hipLaunchKernelGGL(put_instances, dim3(1), dim3(64), 0, stream, d_tab + c, chunk, m);
     HIPCHK(hipGetLastError());
   }
-  const hipError_t le = track_launcher(strict, shape)(d_tab, n, nblocks, shape.block, ext ? 1 : 0,
+  const hipError_t le = track_launcher(strict, shape)(d_tab, n, nblocks, shape.block, 0,
                                                       xcd_order(tab, (size_t)n) ? 1 : 0, nullptr,
                                                       stream);
   if (le != hipSuccess) return fail(ATX_E_RUNTIME, std::string("kernel launch: ") + hipGetErrorString(le));
@@ -1798,7 +1921,7 @@ int atx_element_matrices(atx_lattice* lat, const double* orbits, double step, do
   if (!rc && e == hipSuccess) e = atx_launch_element_probes(d_o, step, d_r, nelem, stream);
   if (!rc && e == hipSuccess)
     rc = launch_instances(insts, std::vector<const std::vector<int32_t>*>(nelem, &slots), shape,
-                          stream, strict, lat->has_ext);
+                          stream, strict);
   if (!rc && e == hipSuccess) e = atx_launch_element_diffs(d_r, step, d_m, nelem, stream);
   if (!rc && e == hipSuccess && !dev)
     e = hipMemcpyAsync(m66, d_m, nm * sizeof(double), hipMemcpyDeviceToHost, stream);

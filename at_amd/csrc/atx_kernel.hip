@@ -3,11 +3,12 @@
 // One lane tracks one particle through every element of every turn in a
 // single launch; the particle's 6-vector lives in registers from the first
 // load to the final store, and HBM is touched only at start, at refpt
-// copies, on a loss and at the end. Element parameters are compile-time
-// prepared by atx_host.cpp and read through the constant address space, so
-// the uniform per-element values land in SGPRs via scalar loads (every lane
-// of a workgroup walks the same element sequence; no divergence on the
-// element switch).
+// copies, on a loss and at the end. A lattice is a list of records (LatOp,
+// prepared by atx_host.cpp) read through the constant address space: every
+// lane of a wave is at the same record, so its constants land in SGPRs and
+// its branches are scalar. The loop over the records has no divergent branch
+// (losses, the only ones, are handled in a function that the whole wave
+// calls), and keeps the common elements inline and all others in functions.
 //
 // This file is compiled twice:
 //   ATX_STRICT=1, -ffp-contract=off: the reference operation order of
@@ -50,6 +51,7 @@ namespace ATX_NS {
 typedef __attribute__((address_space(4))) const double cdouble;
 typedef __attribute__((address_space(4))) const DevElem cDevElem;
 typedef __attribute__((address_space(4))) const Instance cInstance;
+typedef __attribute__((address_space(4))) const LatOp cLatOp;
 typedef __attribute__((address_space(4))) const int32_t cint;
 
 struct R6 {
@@ -75,7 +77,7 @@ __device__ __forceinline__ void add_t(R6& r, cdouble* t) {
 
 // r <- M r with M column-major (atlalib.c:17-32); the sum starts from 0.0 as
 // in the reference.
-__device__ __noinline__ R6 mul_r_v(R6 r, cdouble* m) {
+__device__ __forceinline__ R6 mul_r_inl(const R6& r, cdouble* m) {
   const double v[6] = {r.x, r.px, r.y, r.py, r.dp, r.ct};
   double o[6];
 #pragma unroll
@@ -87,6 +89,8 @@ __device__ __noinline__ R6 mul_r_v(R6 r, cdouble* m) {
   }
   return R6{o[0], o[1], o[2], o[3], o[4], o[5]};
 }
+
+__device__ __noinline__ R6 mul_r_v(R6 r, cdouble* m) { return mul_r_inl(r, m); }
 
 __device__ __forceinline__ void mul_r(R6& r, cdouble* m) { r = mul_r_v(r, m); }
 
@@ -104,10 +108,8 @@ __device__ __forceinline__ void change_pref(R6& r, double s) { r = change_pref_v
 // that the loss element is the reference's (atlalib.c:164-190).
 __device__ __forceinline__ void rect_ap(R6& r, cdouble* lim) {
 #pragma clang fp contract(off)
-  if (r.x < lim[0] || r.x > lim[1])
-    r.ct = __builtin_inf();
-  else if (r.y < lim[2] || r.y > lim[3])
-    r.ct = __builtin_inf();
+  const bool out = (r.x < lim[0]) | (r.x > lim[1]) | (r.y < lim[2]) | (r.y > lim[3]);
+  r.ct = out ? __builtin_inf() : r.ct;
 }
 
 __device__ __forceinline__ void ellip_ap(R6& r, cdouble* ax) {
@@ -275,9 +277,8 @@ __device__ __forceinline__ double rcp_after_kick(double opd2, double pn) {
   const double e = __builtin_fma(-opd2, pn, 1.0);
   double q = __builtin_fma(pn, __builtin_fma(e, e, e), pn);
   const bool far = __builtin_fabs(e) > 2e-6;
-  if (__builtin_expect(__ballot(far) != 0, 0)) {
-    if (far) q = fast_rcp(opd2);
-  }
+  // a select under the vote: no divergent branch in the slices
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) q = far ? fast_rcp(opd2) : q;
   return q;
 }
 
@@ -333,9 +334,8 @@ __device__ __forceinline__ void rad_str_kick(R6& r, cdouble* a, cdouble* b, int 
   // (angles up to 10 mrad); a wave with a wider angle divides.
   double g = __builtin_fma(-0.5 * s2, __builtin_fma(s2, s2, 1.0 - s2), 1.0);
   const bool wide = s2 > 1e-4;
-  if (__builtin_expect(__ballot(wide) != 0, 0)) {
-    if (wide) g = __builtin_fma(0.5, s2, 1.0) * rcp1(1.0 + s2);
-  }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(wide) != 0, 0))
+    g = wide ? __builtin_fma(0.5, s2, 1.0) * rcp1(1.0 + s2) : g;
   r.dp = __builtin_fma(-radk, (b2 * g) * (opd * opd), r.dp);
   const double opd2 = 1.0 + r.dp;
   r.px = __builtin_fma(xpr, opd2, -kl * re);
@@ -430,6 +430,7 @@ __device__ __noinline__ double edge_fy_tan(int mode, double dp, double px, doubl
   }
 }
 
+template <bool LEAN>
 __device__ __forceinline__ void edge(R6& r, int mode, double irho, double fx, double c0,
                                      double edge_angle, double corr, double sgn) {
   double fy;
@@ -437,7 +438,7 @@ __device__ __forceinline__ void edge(R6& r, int mode, double irho, double fx, do
     fy = c0;
   else if (mode == E_DIVP)
     fy = c0 / (1.0 + r.dp);
-  else if (mode == E_MULPN)
+  else if (LEAN || mode == E_MULPN)
     fy = c0 * (1.0 / (1.0 + r.dp));
   else
     fy = edge_fy_tan(mode, r.dp, r.px, irho, edge_angle, corr, sgn);
@@ -596,15 +597,17 @@ __device__ __forceinline__ void rad_str_kick_ang(R6& r, Ang& g, cdouble* a, cdou
   // one vote for both exceptions of the wave: a wide angle (the factor by
   // division) and a large radiated fraction (the reciprocal from fast_rcp)
   const bool wide = s2 > 1e-4;
-  if (__builtin_expect(__ballot(wide || __builtin_fabs(e) > 2e-6) != 0, 0)) {
-    if (wide) {
-      const double fw = __builtin_fma(0.5, s2, 1.0) * rcp1(1.0 + s2);
-      dp = __builtin_fma(-radk, (b2 * fw) * oo, d0);
-      opd2 = 1.0 + dp;
-      e = __builtin_fma(-opd2, g.pn, 1.0);
-      pn = __builtin_fma(g.pn, __builtin_fma(e, e, e), g.pn);
-    }
-    if (__builtin_fabs(e) > 2e-6) pn = fast_rcp(opd2);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(wide || __builtin_fabs(e) > 2e-6) != 0, 0)) {
+    const double fw = __builtin_fma(0.5, s2, 1.0) * rcp1(1.0 + s2);
+    const double dpw = __builtin_fma(-radk, (b2 * fw) * oo, d0);
+    const double opw = 1.0 + dpw;
+    const double ew = __builtin_fma(-opw, g.pn, 1.0);
+    const double pw = __builtin_fma(g.pn, __builtin_fma(ew, ew, ew), g.pn);
+    dp = wide ? dpw : dp;
+    opd2 = wide ? opw : opd2;
+    e = wide ? ew : e;
+    pn = wide ? pw : pn;
+    pn = __builtin_fabs(e) > 2e-6 ? fast_rcp(opd2) : pn;
   }
   r.dp = dp;
   const double klpn = kl * pn;
@@ -651,30 +654,214 @@ __device__ __forceinline__ void rad_bnd_kick_ang(R6& r, Ang& g, cdouble* a, cdou
 constexpr uint32_t F_ENTRY_ANY = F_T1 | F_R1 | F_RAP | F_EAP;
 constexpr uint32_t F_EXIT_ANY = F_R2 | F_T2 | F_RAP | F_EAP | F_SCALE;
 
-template <bool BEND>
+// LEAN: without the maps that are functions of their own (F_LEAN).
+template <bool BEND, bool LEAN>
 __device__ __forceinline__ void mpole_entry(R6& r, cDevElem& h, cdouble* pool, cdouble* s) {
   if (h.flags & F_ENTRY_ANY) {
-    entry_xform(r, h, pool);
+    if (LEAN) {
+      if (h.flags & F_T1) add_t(r, pool + h.t1);
+      if (h.flags & F_R1) r = mul_r_inl(r, pool + h.r1);
+    } else {
+      entry_xform(r, h, pool);
+    }
     apertures(r, h, pool);
   }
-  if (BEND) edge(r, h.edge & 0xff, s[S_IRHO], s[S_FX_IN], s[S_FY_IN], s[S_EDGE_IN], s[S_CORR_IN], 1.0);
-  if (h.fringe & 0xff) quad_fringe_in(r, h, pool, s[S_B2]);
+  if (BEND) edge<LEAN>(r, h.edge & 0xff, s[S_IRHO], s[S_FX_IN], s[S_FY_IN], s[S_EDGE_IN], s[S_CORR_IN], 1.0);
+  if (!LEAN && (h.fringe & 0xff)) quad_fringe_in(r, h, pool, s[S_B2]);
 }
 
-template <bool BEND>
+template <bool BEND, bool LEAN>
 __device__ __forceinline__ void mpole_exit(R6& r, cDevElem& h, cdouble* pool, cdouble* s) {
-  if (h.fringe & 0xff00) quad_fringe_out(r, h, pool, s[S_B2]);
-  if (BEND) edge(r, (h.edge >> 8) & 0xff, s[S_IRHO], s[S_FX_OUT], s[S_FY_OUT], s[S_EDGE_OUT], s[S_CORR_OUT], -1.0);
+  if (!LEAN && (h.fringe & 0xff00)) quad_fringe_out(r, h, pool, s[S_B2]);
+  if (BEND) edge<LEAN>(r, (h.edge >> 8) & 0xff, s[S_IRHO], s[S_FX_OUT], s[S_FY_OUT], s[S_EDGE_OUT], s[S_CORR_OUT], -1.0);
   if (h.flags & F_EXIT_ANY) {
     apertures(r, h, pool);
-    exit_xform(r, h, pool);
-    if (h.flags & F_SCALE) change_pref(r, s[S_INVSCALE]);
+    if (LEAN) {
+      if (h.flags & F_R2) r = mul_r_inl(r, pool + h.r2);
+      if (h.flags & F_T2) add_t(r, pool + h.t2);
+    } else {
+      exit_xform(r, h, pool);
+      if (h.flags & F_SCALE) change_pref(r, s[S_INVSCALE]);
+    }
   }
+}
+
+// Slices of StrMPoleSymplectic4Pass.c:79-93 and BndMPoleSymplectic4Pass.c:97-111
+// for the P particles of a lane; U slices per loop iteration. pn = 1/(1+delta)
+// at the entry, nl1, nl2 = the drift lengths times it.
+template <bool BEND, int N, int P, int U>
+__device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int n, int nslice,
+                                             const double* nl1, const double* nl2, double k1,
+                                             double k2, double irho) {
+  const double ki1 = k1 * irho, ki2 = k2 * irho;
+  double blo, alo;
+  horner_addends<N>(a, b, n, blo, alo);
+#if ATX_STRICT
+  // U slices per iteration: a constant-count inner loop, fully unrolled
+  // (the slices may hold wave-wide votes, which a runtime-count unroll
+  // cannot duplicate), then the remaining slices one by one
+  auto slice = [&]() {
+#pragma unroll
+    for (int q = 0; q < P; q++) fastdrift(r[q], nl1[q], 0.0);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) fastdrift(r[q], nl2[q], 0.0);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2); else str_kick<N>(r[q], a, b, n, blo, alo, k2);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) fastdrift(r[q], nl2[q], 0.0);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) fastdrift(r[q], nl1[q], 0.0);
+  };
+  int m = 0;
+  for (; m + U <= nslice; m += U) {
+#pragma unroll
+    for (int u = 0; u < U; u++) slice();
+  }
+  for (; m < nslice; m++) slice();
+#else
+  double nh1[P], nh2[P];  // delta is constant through the slices
+#pragma unroll
+  for (int q = 0; q < P; q++) {
+    const double h2 = 0.5 * fast_rcp(1.0 + r[q].dp);
+    nh1[q] = nl1[q] * h2;
+    nh2[q] = nl2[q] * h2;
+  }
+  // U slices per iteration: a constant-count inner loop, fully unrolled
+  // (the slices may hold wave-wide votes, which a runtime-count unroll
+  // cannot duplicate), then the remaining slices one by one
+  auto slice = [&]() {
+#pragma unroll
+    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl1[q], nh1[q]);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl2[q], nh2[q]);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2); else str_kick<N>(r[q], a, b, n, blo, alo, k2);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl2[q], nh2[q]);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl1[q], nh1[q]);
+  };
+  int m = 0;
+  for (; m + U <= nslice; m += U) {
+#pragma unroll
+    for (int u = 0; u < U; u++) slice();
+  }
+  for (; m < nslice; m++) slice();
+#endif
+}
+
+// Slices of StrMPoleSymplectic4RadPass.c:83-99 and
+// BndMPoleSymplectic4RadPass.c:98-112, likewise.
+template <bool BEND, int N, int P, int U>
+__device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, int n, int nslice,
+                                                 double l1, double l2, double k1, double k2,
+                                                 double irho, double radc, double rk1, double rk2) {
+  const double ki1 = k1 * irho, ki2 = k2 * irho;
+  double blo, alo;
+  horner_addends<N>(a, b, n, blo, alo);
+#if ATX_STRICT
+  double pn = 0.0;  // unused: the strict steps divide as the reference does
+  // U slices per iteration: a constant-count inner loop, fully unrolled
+  // (the slices may hold wave-wide votes, which a runtime-count unroll
+  // cannot duplicate), then the remaining slices one by one
+  auto slice = [&]() {
+#pragma unroll
+    for (int q = 0; q < P; q++) rad_drift(r[q], l1);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1, radc, 0.0, pn);
+      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k1, radc, 0.0, pn);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) rad_drift(r[q], l2);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2, radc, 0.0, pn);
+      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k2, radc, 0.0, pn);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) rad_drift(r[q], l2);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1, radc, 0.0, pn);
+      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k1, radc, 0.0, pn);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) rad_drift(r[q], l1);
+  };
+  int m = 0;
+  for (; m + U <= nslice; m += U) {
+#pragma unroll
+    for (int u = 0; u < U; u++) slice();
+  }
+  for (; m < nslice; m++) slice();
+#else
+  const double hl1 = 0.5 * l1, hl2 = 0.5 * l2;
+  Ang g[P];
+#pragma unroll
+  for (int q = 0; q < P; q++) g[q] = to_angles(r[q]);  // one reciprocal per magnet
+  // U slices per iteration: a constant-count inner loop, fully unrolled
+  // (the slices may hold wave-wide votes, which a runtime-count unroll
+  // cannot duplicate), then the remaining slices one by one
+  auto slice = [&]() {
+#pragma unroll
+    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l1, hl1);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, irho, ki1, rk1);
+      else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, rk1);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l2, hl2);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k2, irho, ki2, rk2);
+      else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k2, rk2);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l2, hl2);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, irho, ki1, rk1);
+      else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, rk1);
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l1, hl1);
+  };
+  int m = 0;
+  for (; m + U <= nslice; m += U) {
+#pragma unroll
+    for (int u = 0; u < U; u++) slice();
+  }
+  for (; m < nslice; m++) slice();
+#pragma unroll
+  for (int q = 0; q < P; q++) from_angles(r[q], g[q]);
+#endif
 }
 
 // StrMPoleSymplectic4Pass.c:57-104 and BndMPoleSymplectic4Pass.c:75-122 for
 // the P particles of a lane; U slices per loop iteration.
-template <bool BEND, int N, int P, int U>
+template <bool BEND, int N, int P, int U, bool LEAN>
 __device__ __forceinline__ void mpole(R6* r, cDevElem& h, cdouble* pool) {
   cdouble* s = pool + h.sc;
   cdouble* a = pool + h.poly;
@@ -683,7 +870,7 @@ __device__ __forceinline__ void mpole(R6* r, cDevElem& h, cdouble* pool) {
   double pn[P], nl1[P], nl2[P];
 #pragma unroll
   for (int q = 0; q < P; q++) {
-    if (h.flags & F_SCALE) change_pref(r[q], s[S_SCALE]);
+    if (!LEAN && (h.flags & F_SCALE)) change_pref(r[q], s[S_SCALE]);
 #if ATX_STRICT
     pn[q] = 1.0 / (1.0 + r[q].dp);  // before T1/R1, as the reference hoists it
 #else
@@ -691,98 +878,23 @@ __device__ __forceinline__ void mpole(R6* r, cDevElem& h, cdouble* pool) {
 #endif
     nl1[q] = s[S_L1] * pn[q];
     nl2[q] = s[S_L2] * pn[q];
-    mpole_entry<BEND>(r[q], h, pool, s);
+    mpole_entry<BEND, LEAN>(r[q], h, pool, s);
   }
   const double irho = s[S_IRHO];
-  if (h.ops >= 0) {
+  if (!LEAN && h.ops >= 0) {
 #pragma unroll
     for (int q = 0; q < P; q++)
       r[q] = slices_ops<BEND, false>(r[q], a, b, n, pool + h.ops, h.nslice, pn[q], irho, 0.0);
   } else {
-    const double k1 = s[S_K1], k2 = s[S_K2];
-    const double ki1 = k1 * irho, ki2 = k2 * irho;
-    double blo, alo;
-    horner_addends<N>(a, b, n, blo, alo);
-#if ATX_STRICT
-    // U slices per iteration: a constant-count inner loop, fully unrolled
-    // (the slices may hold wave-wide votes, which a runtime-count unroll
-    // cannot duplicate), then the remaining slices one by one
-    auto slice = [&]() {
-#pragma unroll
-      for (int q = 0; q < P; q++) fastdrift(r[q], nl1[q], 0.0);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) fastdrift(r[q], nl2[q], 0.0);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2); else str_kick<N>(r[q], a, b, n, blo, alo, k2);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) fastdrift(r[q], nl2[q], 0.0);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) fastdrift(r[q], nl1[q], 0.0);
-    };
-    int m = 0;
-    for (; m + U <= h.nslice; m += U) {
-#pragma unroll
-      for (int u = 0; u < U; u++) slice();
-    }
-    for (; m < h.nslice; m++) slice();
-#else
-    double nh1[P], nh2[P];  // delta is constant through the slices
-#pragma unroll
-    for (int q = 0; q < P; q++) {
-      const double h2 = 0.5 * fast_rcp(1.0 + r[q].dp);
-      nh1[q] = nl1[q] * h2;
-      nh2[q] = nl2[q] * h2;
-    }
-    // U slices per iteration: a constant-count inner loop, fully unrolled
-    // (the slices may hold wave-wide votes, which a runtime-count unroll
-    // cannot duplicate), then the remaining slices one by one
-    auto slice = [&]() {
-#pragma unroll
-      for (int q = 0; q < P; q++) fastdrift_h(r[q], nl1[q], nh1[q]);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) fastdrift_h(r[q], nl2[q], nh2[q]);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2); else str_kick<N>(r[q], a, b, n, blo, alo, k2);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) fastdrift_h(r[q], nl2[q], nh2[q]);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) fastdrift_h(r[q], nl1[q], nh1[q]);
-    };
-    int m = 0;
-    for (; m + U <= h.nslice; m += U) {
-#pragma unroll
-      for (int u = 0; u < U; u++) slice();
-    }
-    for (; m < h.nslice; m++) slice();
-#endif
+    mpole_slices<BEND, N, P, U>(r, a, b, n, h.nslice, nl1, nl2, s[S_K1], s[S_K2], irho);
   }
 #pragma unroll
-  for (int q = 0; q < P; q++) mpole_exit<BEND>(r[q], h, pool, s);
+  for (int q = 0; q < P; q++) mpole_exit<BEND, LEAN>(r[q], h, pool, s);
 }
 
 // StrMPoleSymplectic4RadPass.c:61-110 and BndMPoleSymplectic4RadPass.c:76-123
 // for the P particles of a lane; U slices per loop iteration.
-template <bool BEND, int N, int P, int U>
+template <bool BEND, int N, int P, int U, bool LEAN>
 __device__ __forceinline__ void mpole_rad(R6* r, cDevElem& h, cdouble* pool) {
   cdouble* s = pool + h.sc;
   cdouble* a = pool + h.poly;
@@ -790,112 +902,63 @@ __device__ __forceinline__ void mpole_rad(R6* r, cDevElem& h, cdouble* pool) {
   const int n = h.order;
 #pragma unroll
   for (int q = 0; q < P; q++) {
-    if (h.flags & F_SCALE) change_pref(r[q], s[S_SCALE]);
-    mpole_entry<BEND>(r[q], h, pool, s);
+    if (!LEAN && (h.flags & F_SCALE)) change_pref(r[q], s[S_SCALE]);
+    mpole_entry<BEND, LEAN>(r[q], h, pool, s);
   }
   const double irho = s[S_IRHO];
   const double radc = s[S_RADC];
-  if (h.ops >= 0) {
+  if (!LEAN && h.ops >= 0) {
 #pragma unroll
     for (int q = 0; q < P; q++)
       r[q] = slices_ops<BEND, true>(r[q], a, b, n, pool + h.ops, h.nslice, 0.0, irho, radc);
   } else {
-    const double l1 = s[S_L1], l2 = s[S_L2], k1 = s[S_K1], k2 = s[S_K2];
-    const double ki1 = k1 * irho, ki2 = k2 * irho;
-    double blo, alo;
-    horner_addends<N>(a, b, n, blo, alo);
-#if ATX_STRICT
-    double pn = 0.0;  // unused: the strict steps divide as the reference does
-    // U slices per iteration: a constant-count inner loop, fully unrolled
-    // (the slices may hold wave-wide votes, which a runtime-count unroll
-    // cannot duplicate), then the remaining slices one by one
-    auto slice = [&]() {
-#pragma unroll
-      for (int q = 0; q < P; q++) rad_drift(r[q], l1);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1, radc, 0.0, pn);
-        else rad_str_kick<N>(r[q], a, b, n, blo, alo, k1, radc, 0.0, pn);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) rad_drift(r[q], l2);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2, radc, 0.0, pn);
-        else rad_str_kick<N>(r[q], a, b, n, blo, alo, k2, radc, 0.0, pn);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) rad_drift(r[q], l2);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1, radc, 0.0, pn);
-        else rad_str_kick<N>(r[q], a, b, n, blo, alo, k1, radc, 0.0, pn);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) rad_drift(r[q], l1);
-    };
-    int m = 0;
-    for (; m + U <= h.nslice; m += U) {
-#pragma unroll
-      for (int u = 0; u < U; u++) slice();
-    }
-    for (; m < h.nslice; m++) slice();
-#else
-    const double rk1 = s[S_RK1], rk2 = s[S_RK2], hl1 = s[S_HL1], hl2 = s[S_HL2];
-    Ang g[P];
-#pragma unroll
-    for (int q = 0; q < P; q++) g[q] = to_angles(r[q]);  // one reciprocal per magnet
-    // U slices per iteration: a constant-count inner loop, fully unrolled
-    // (the slices may hold wave-wide votes, which a runtime-count unroll
-    // cannot duplicate), then the remaining slices one by one
-    auto slice = [&]() {
-#pragma unroll
-      for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l1, hl1);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, irho, ki1, rk1);
-        else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, rk1);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l2, hl2);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k2, irho, ki2, rk2);
-        else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k2, rk2);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l2, hl2);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, irho, ki1, rk1);
-        else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, rk1);
-      }
-#pragma unroll
-      for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l1, hl1);
-    };
-    int m = 0;
-    for (; m + U <= h.nslice; m += U) {
-#pragma unroll
-      for (int u = 0; u < U; u++) slice();
-    }
-    for (; m < h.nslice; m++) slice();
-#pragma unroll
-    for (int q = 0; q < P; q++) from_angles(r[q], g[q]);
-#endif
+    mpole_rad_slices<BEND, N, P, U>(r, a, b, n, h.nslice, s[S_L1], s[S_L2], s[S_K1], s[S_K2], irho,
+                                    radc, s[S_RK1], s[S_RK2]);
   }
 #pragma unroll
-  for (int q = 0; q < P; q++) mpole_exit<BEND>(r[q], h, pool, s);
+  for (int q = 0; q < P; q++) mpole_exit<BEND, LEAN>(r[q], h, pool, s);
 }
 
-template <bool BEND, bool RAD, int P, int U>
-__device__ __forceinline__ void mpole_dispatch(R6* r, cDevElem& h, cdouble* pool) {
+// Pointers that every lane of the wave holds alike, back in scalar registers
+// (arguments of a function that is not inlined arrive in vector registers).
+template <typename T>
+__device__ __forceinline__ T uniform(T p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (T)(((uint64_t)hi << 32) | lo);
+}
+
+// Elements by their headers run out of line, one function per kind and order:
+// the loop over the records then keeps its registers (and its code, which
+// has to stay in the instruction cache) for the common ops. A call costs about
+// 0.4 us with one wave per SIMD (the callee saves the scalar registers it
+// uses), so what rings are made of runs inline.
+template <bool BEND, bool RAD, int N, int U, bool LEAN>
+__device__ __noinline__ R6 mpole_call(R6 r, cDevElem* hp, cdouble* poolp) {
+  cDevElem& h = *uniform(hp);
+  cdouble* pool = uniform(poolp);
+  if (RAD) mpole_rad<BEND, N, 1, U, LEAN>(&r, h, pool); else mpole<BEND, N, 1, U, LEAN>(&r, h, pool);
+  return r;
+}
+
+template <bool BEND, bool RAD, int U, bool LEAN>
+__device__ __forceinline__ R6 mpole_order(const R6& r, cDevElem& h, cdouble* pool) {
   switch (h.order) {
-    case 0: RAD ? mpole_rad<BEND, 0, P, U>(r, h, pool) : mpole<BEND, 0, P, U>(r, h, pool); break;
-    case 1: RAD ? mpole_rad<BEND, 1, P, U>(r, h, pool) : mpole<BEND, 1, P, U>(r, h, pool); break;
-    case 2: RAD ? mpole_rad<BEND, 2, P, U>(r, h, pool) : mpole<BEND, 2, P, U>(r, h, pool); break;
-    case 3: RAD ? mpole_rad<BEND, 3, P, U>(r, h, pool) : mpole<BEND, 3, P, U>(r, h, pool); break;
-    default: RAD ? mpole_rad<BEND, -1, P, U>(r, h, pool) : mpole<BEND, -1, P, U>(r, h, pool); break;
+    case 0: return mpole_call<BEND, RAD, 0, U, LEAN>(r, &h, pool);
+    case 1: return mpole_call<BEND, RAD, 1, U, LEAN>(r, &h, pool);
+    case 2: return mpole_call<BEND, RAD, 2, U, LEAN>(r, &h, pool);
+    case 3: return mpole_call<BEND, RAD, 3, U, LEAN>(r, &h, pool);
+    default: return mpole_call<BEND, RAD, -1, U, LEAN>(r, &h, pool);
   }
+}
+
+// A function that calls others keeps its return address in scratch memory
+// over the calls, so the magnets without such maps have functions without.
+template <bool BEND, bool RAD, int U>
+__device__ __forceinline__ R6 mpole_dispatch(const R6& r, cDevElem& h, cdouble* pool) {
+  if (h.flags & F_LEAN) return mpole_order<BEND, RAD, U, true>(r, h, pool);
+  return mpole_order<BEND, RAD, U, false>(r, h, pool);
 }
 
 // ThinMPolePass.c:42-63
@@ -1082,6 +1145,25 @@ __device__ __forceinline__ void exact_mpole(R6& r, cDevElem& h, cdouble* pool, b
   if (h.flags & F_SCALE) change_pref(r, s[S_INVSCALE]);
 }
 
+// Thick corrector without misalignment (CorrectorPass.c:55-89); q0 = xk*xk/3
+// + yk*yk/3, the sum's first two terms; nl = L pn, pn = 1/(1+delta).
+__device__ __forceinline__ void corrector_map(R6& r, double xk, double yk, double q0, double nl,
+                                              double pn) {
+  r.ct += nl * pn * (q0 + r.px * r.px + r.py * r.py + r.px * xk + r.py * yk) / 2.0;
+  r.x += nl * (r.px + xk / 2.0);
+  r.px += xk;
+  r.y += nl * (r.py + yk / 2.0);
+  r.py += yk;
+}
+
+__device__ __forceinline__ double rcp_opd(const R6& r) {
+#if ATX_STRICT
+  return 1.0 / (1.0 + r.dp);
+#else
+  return fast_rcp(1.0 + r.dp);
+#endif
+}
+
 // CorrectorPass.c:25-90
 __device__ __forceinline__ void corrector(R6& r, cDevElem& h, cdouble* pool) {
   cdouble* s = pool + h.sc;
@@ -1093,20 +1175,11 @@ __device__ __forceinline__ void corrector(R6& r, cDevElem& h, cdouble* pool) {
     r.px += xk;
     r.py += yk;
   } else {
-#if ATX_STRICT
-    const double pn = 1.0 / (1.0 + r.dp);
-#else
-    const double pn = fast_rcp(1.0 + r.dp);
-#endif
+    const double pn = rcp_opd(r);
     const double nl = s[S_C_LEN] * pn;
     entry_xform(r, h, pool);
     apertures(r, h, pool);
-    // s[S_C_Q0] = xk*xk/3 + yk*yk/3, the sum's first two terms
-    r.ct += nl * pn * (s[S_C_Q0] + r.px * r.px + r.py * r.py + r.px * xk + r.py * yk) / 2.0;
-    r.x += nl * (r.px + xk / 2.0);
-    r.px += xk;
-    r.y += nl * (r.py + yk / 2.0);
-    r.py += yk;
+    corrector_map(r, xk, yk, s[S_C_Q0], nl, pn);
     apertures(r, h, pool);
   }
   exit_xform(r, h, pool);
@@ -1420,85 +1493,150 @@ __global__ void __launch_bounds__(64) diffusion_kernel(DiffArgs args) {
 
 #endif  // ATX_AUX
 
-// The kinds other than drifts and thick multipoles, for one particle. EXT:
-// the kernel variant that also runs CavityPass and the exact passes;
-// lattices without them use the variant without, whose element switch keeps
-// the register demand of the common passes only.
-template <bool EXT>
-__device__ __forceinline__ void element_misc(R6& r, cDevElem& h, cdouble* pool, int nturn) {
-  if (EXT) {
-    switch (h.kind) {
-      case K_CAVITY: r = cavity(r, pool + h.sc, (h.flags & F_THICK) != 0); return;
-      case K_EXDRIFT:  // ExactDriftPass.c:15-44
-        entry_xform(r, h, pool);
-        apertures(r, h, pool);
-        exact_drift(r, pool[h.sc + S_D_LEN]);
-        r.ct -= pool[h.sc + S_D_LEN];
-        apertures(r, h, pool);
-        exit_xform(r, h, pool);
-        return;
-      case K_EXMPOLE: exact_mpole(r, h, pool, false); return;
-      case K_EXMPOLERAD: exact_mpole(r, h, pool, true); return;
-      default: break;
+// The kinds other than thick multipoles, each out of line as well.
+template <int KIND>
+__device__ __noinline__ R6 misc_call(R6 r, cDevElem* hp, cdouble* poolp, int nturnp) {
+  cDevElem& h = *uniform(hp);
+  cdouble* pool = uniform(poolp);
+  if (KIND == K_IDENTITY || KIND == K_DRIFT || KIND == K_EXDRIFT) {
+    // IdentityPass.c:20-43, DriftPass.c:16-48, ExactDriftPass.c:15-44
+    entry_xform(r, h, pool);
+    apertures(r, h, pool);
+    if (KIND == K_DRIFT) drift6(r, pool[h.sc + S_D_LEN]);
+    if (KIND == K_EXDRIFT) {
+      exact_drift(r, pool[h.sc + S_D_LEN]);
+      r.ct -= pool[h.sc + S_D_LEN];
     }
+    if (KIND != K_IDENTITY) apertures(r, h, pool);
+    exit_xform(r, h, pool);
   }
+  if (KIND == K_THIN) thin(r, h, pool);
+  if (KIND == K_RF) rf_cavity(r, h, pool, __builtin_amdgcn_readfirstlane(nturnp));
+  if (KIND == K_CORR) corrector(r, h, pool);
+  if (KIND == K_CAVITY) r = cavity(r, pool + h.sc, (h.flags & F_THICK) != 0);
+  if (KIND == K_EXMPOLE || KIND == K_EXMPOLERAD) exact_mpole(r, h, pool, KIND == K_EXMPOLERAD);
+  return r;
+}
+
+// One particle through an element by its header.
+template <int U>
+__device__ __forceinline__ R6 generic_element(const R6& r, cDevElem& h, cdouble* pool, int nturn) {
   switch (h.kind) {
-    case K_IDENTITY:  // IdentityPass.c:20-43
-      entry_xform(r, h, pool);
-      apertures(r, h, pool);
-      exit_xform(r, h, pool);
-      break;
-    case K_THIN: thin(r, h, pool); break;
-    case K_RF: rf_cavity(r, h, pool, nturn); break;
-    case K_CORR: corrector(r, h, pool); break;
-    case K_APERTURE: rect_ap(r, pool + h.rap); break;  // AperturePass.c:9-26
-    default: break;
+    case K_STR: return mpole_dispatch<false, false, U>(r, h, pool);
+    case K_BND: return mpole_dispatch<true, false, U>(r, h, pool);
+    case K_STRRAD: return mpole_dispatch<false, true, U>(r, h, pool);
+    case K_BNDRAD: return mpole_dispatch<true, true, U>(r, h, pool);
+    case K_IDENTITY: return misc_call<K_IDENTITY>(r, &h, pool, nturn);
+    case K_DRIFT: return misc_call<K_DRIFT>(r, &h, pool, nturn);
+    case K_THIN: return misc_call<K_THIN>(r, &h, pool, nturn);
+    case K_RF: return misc_call<K_RF>(r, &h, pool, nturn);
+    case K_CORR: return misc_call<K_CORR>(r, &h, pool, nturn);
+    case K_APERTURE: {  // AperturePass.c:9-26
+      R6 v = r;
+      rect_ap(v, pool + h.rap);
+      return v;
+    }
+    case K_CAVITY: return misc_call<K_CAVITY>(r, &h, pool, nturn);
+    case K_EXDRIFT: return misc_call<K_EXDRIFT>(r, &h, pool, nturn);
+    case K_EXMPOLE: return misc_call<K_EXMPOLE>(r, &h, pool, nturn);
+    case K_EXMPOLERAD: return misc_call<K_EXMPOLERAD>(r, &h, pool, nturn);
+    default: return r;
   }
 }
 
-// The P particles of a lane through one element: drifts and thick
-// multipoles step all P together, the other kinds run per particle.
-// A drift's length, kept in the header words its kind does not use.
-__device__ __forceinline__ double drift_length(cDevElem& h) {
-  const uint64_t bits = ((uint64_t)(uint32_t)h.fringe << 32) | (uint32_t)h.edge;
-  return __builtin_bit_cast(double, bits);
+// An edge of a bend by its header.
+__device__ __noinline__ R6 edge_call(R6 r, cDevElem* hp, cdouble* poolp, int exit) {
+  cDevElem& h = *uniform(hp);
+  cdouble* s = uniform(poolp) + h.sc;
+  if (__builtin_amdgcn_readfirstlane(exit))
+    edge<false>(r, (h.edge >> 8) & 0xff, s[S_IRHO], s[S_FX_OUT], s[S_FY_OUT], s[S_EDGE_OUT],
+                s[S_CORR_OUT], -1.0);
+  else
+    edge<false>(r, h.edge & 0xff, s[S_IRHO], s[S_FX_IN], s[S_FY_IN], s[S_EDGE_IN], s[S_CORR_IN],
+                1.0);
+  return r;
 }
 
-template <bool EXT, int P, int U>
-__device__ __forceinline__ void element_lane(R6* r, cDevElem& h, cdouble* pool, int nturn) {
-  if (h.kind == K_DRIFT) {  // DriftPass.c:16-48 with misalignment or apertures
-    const double len = drift_length(h);
+// A thick multipole by its record; the misalignment is applied around it by
+// the caller.
+template <bool BEND, bool RAD, int N, int P, int U>
+__device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flags, cDevElem* h,
+                                         cdouble* pool) {
+  cdouble* a = c + OM_POLY;
+  cdouble* b = a + N + 1;
+  const double irho = BEND ? c[OM_IRHO] : 0.0;
+  if (BEND) {
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      entry_xform(r[q], h, pool);
-      apertures(r[q], h, pool);
+      if (flags & OPF_EDGE) {
+        r[q] = edge_call(r[q], h, pool, 0);
+      } else {
+        r[q].px += r[q].x * c[OM_FX_IN];
+        r[q].py -= r[q].y * c[OM_FY_IN];
+      }
     }
-#pragma unroll
-    for (int q = 0; q < P; q++) drift6(r[q], len);
+  }
+  if (RAD) {
+    mpole_rad_slices<BEND, N, P, U>(r, a, b, N, nslice, c[OM_L1], c[OM_L2], c[OM_K1], c[OM_K2],
+                                    irho, c[OM_RADC], c[OM_RK1], c[OM_RK2]);
+  } else {
+    double nl1[P], nl2[P];
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      apertures(r[q], h, pool);
-      exit_xform(r[q], h, pool);
+      const double pn = rcp_opd(r[q]);
+      nl1[q] = c[OM_L1] * pn;
+      nl2[q] = c[OM_L2] * pn;
     }
-    return;
+    mpole_slices<BEND, N, P, U>(r, a, b, N, nslice, nl1, nl2, c[OM_K1], c[OM_K2], irho);
   }
-  switch (h.kind) {
-    case K_STR: mpole_dispatch<false, false, P, U>(r, h, pool); break;
-    case K_BND: mpole_dispatch<true, false, P, U>(r, h, pool); break;
-    case K_STRRAD: mpole_dispatch<false, true, P, U>(r, h, pool); break;
-    case K_BNDRAD: mpole_dispatch<true, true, P, U>(r, h, pool); break;
-    default:
-      element_misc<EXT>(r[0], h, pool, nturn);
-      if constexpr (P > 1) element_misc<EXT>(r[1], h, pool, nturn);
-      break;
+  if (BEND) {
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (flags & OPF_EDGE) {
+        r[q] = edge_call(r[q], h, pool, 1);
+      } else {
+        r[q].px += r[q].x * c[OM_FX_OUT];
+        r[q].py -= r[q].y * c[OM_FY_OUT];
+      }
+    }
   }
+}
+
+// ThinMPolePass.c:42-63 by its record.
+template <int N>
+__device__ __forceinline__ void thin_op(R6& r, cdouble* c) {
+  cdouble* a = c + OM_POLY;
+  cdouble* b = a + N + 1;
+  str_kick<N>(r, a, b, N, b[N - 1], a[N - 1], 1.0);
+  const double bax = c[OT_BAX], bay = c[OT_BAY];
+  r.px += bax * r.dp;
+  r.py -= bay * r.dp;
+  r.ct -= bax * r.x - bay * r.y;
+}
+
+// The same out of line, for the few elements of a call that are not run by
+// records.
+template <int U>
+__device__ __noinline__ R6 header_call(R6 r, cDevElem* hp, cdouble* poolp, int nturnp) {
+  return generic_element<U>(r, *uniform(hp), uniform(poolp),
+                            __builtin_amdgcn_readfirstlane(nturnp));
 }
 
 // at.c:115-139 predicate: any coordinate not finite, or |r_n| > 1 for n < 5.
+// Without short circuits: six compares and mask logic, no branch.
 __device__ __forceinline__ bool is_lost(const R6& r) {
-  return !(__builtin_fabs(r.x) <= 1.0) || !(__builtin_fabs(r.px) <= 1.0) ||
-         !(__builtin_fabs(r.y) <= 1.0) || !(__builtin_fabs(r.py) <= 1.0) ||
-         !(__builtin_fabs(r.dp) <= 1.0) || !(__builtin_fabs(r.ct) < __builtin_inf());
+  const bool ok = (__builtin_fabs(r.x) <= 1.0) & (__builtin_fabs(r.px) <= 1.0) &
+                  (__builtin_fabs(r.y) <= 1.0) & (__builtin_fabs(r.py) <= 1.0) &
+                  (__builtin_fabs(r.dp) <= 1.0) & (__builtin_fabs(r.ct) < __builtin_inf());
+  return !ok;
+}
+
+// The same after a drift of a particle that passed the test before it:
+// px, py and delta are unchanged.
+__device__ __forceinline__ bool is_lost_drift(const R6& r) {
+  const bool ok = (__builtin_fabs(r.x) <= 1.0) & (__builtin_fabs(r.y) <= 1.0) &
+                  (__builtin_fabs(r.ct) < __builtin_inf());
+  return !ok;
 }
 
 __device__ __forceinline__ void store6(double* base, int64_t cs, const R6& r) {
@@ -1530,7 +1668,292 @@ __device__ __forceinline__ void store_state(cInstance& I, int p, const R6& r) {
   rp[5 * cs] = r.ct;
 }
 
+__device__ __forceinline__ R6 load_state(cInstance& I, int p) {
+  const double* rp = I.r + (int64_t)p * I.pstride;
+  const int64_t cs = I.cstride;
+  return R6{rp[0], rp[cs], rp[2 * cs], rp[3 * cs], rp[4 * cs], rp[5 * cs]};
+}
+
 __device__ __forceinline__ R6 lost_state() { return R6{__builtin_nan(""), 0.0, 0.0, 0.0, 0.0, 0.0}; }
+
+// What a lane without a live particle tracks: the origin.
+__device__ __forceinline__ R6 idle_state() { return R6{0.0, 0.0, 0.0, 0.0, 0.0, 0.0}; }
+
+// Head of a program record, read one record ahead: its flags and op, the
+// index of its last element, its drift's length.
+// It holds a word of each of the record's other lines, too: reading them
+// brings the lines into the scalar cache before the op asks for its
+// constants.
+struct OpHead {
+  int op, last;
+  double len;
+  int line1, line2;
+};
+
+__device__ __forceinline__ OpHead op_head(cLatOp* p) {
+  return OpHead{p->op, p->last, p->len, ((cint*)p)[16], ((cint*)p)[32]};
+}
+
+// Roll of both planes by the angle of (c, s): the 6x6 product of mul_r
+// without its zeros, in its order of summation.
+__device__ __forceinline__ void roll(R6& r, double c, double s) {
+  const double x = r.x, px = r.px;
+#if ATX_STRICT
+  r.x = c * x + s * r.y;
+  r.px = c * px + s * r.py;
+  r.y = -s * x + c * r.y;
+  r.py = -s * px + c * r.py;
+#else
+  r.x = __builtin_fma(s, r.y, c * x);
+  r.px = __builtin_fma(s, r.py, c * px);
+  r.y = __builtin_fma(c, r.y, -s * x);
+  r.py = __builtin_fma(c, r.py, -s * px);
+#endif
+}
+
+// A particle with its lane's state: what the loss handling changes.
+struct Lane {
+  R6 r;
+  int flags;
+};
+enum : int { L_HAS = 1, L_ALIVE = 2, L_LOST = 4 };
+
+// at.c:115-161 for the lanes with `fail` set: live particles that fail the
+// loss test after element e, or whose x is NaN. Rare, so out of line, and
+// called by the whole wave, so that the loop over the records has no
+// divergent branch; the lane's state goes through memory, so that the loop's
+// registers are not arranged around this call. A particle whose state is final is stored and its lane
+// idles from then on. elempass: a NaN input of a single element pass, which
+// leaves it in memory as it is.
+__device__ __noinline__ void loss_call(Lane* lp, const Instance* inst, int p, int fail, int nturn,
+                                       int e) {
+  cInstance& I = *uniform((cInstance*)inst);
+  Lane l = *lp;
+  if (fail) {
+    bool final = false;
+    R6 fin = l.r;
+    if (I.elempass) {
+      final = true;
+    } else if (I.losses) {
+      if (!(l.flags & L_LOST)) {
+        I.lost_flag[p] = 1;
+        I.lost_turn[p] = (uint32_t)nturn;
+        I.lost_elem[p] = (uint32_t)e;
+        store6(I.lost_coord + 6 * (int64_t)p, 1, l.r);
+        l.flags |= L_LOST;
+        fin = lost_state();
+        final = true;
+      } else {
+        final = __builtin_isnan(l.r.x);  // recorded by an earlier call: left as it is
+      }
+    } else if (__builtin_isfinite(l.r.x)) {
+      fin = lost_state();
+      final = true;
+    } else {
+      final = __builtin_isnan(l.r.x);
+    }
+    if (final) {
+      store_state(I, p, fin);
+      l.flags &= ~L_ALIVE;
+      l.r = idle_state();
+    }
+  }
+  *lp = l;
+}
+
+// Refpt copy: dst is the particle's six doubles in r_out; a particle whose
+// state is final is copied from memory.
+__device__ __noinline__ void copy_call(R6 r, const Instance* inst, double* dst, int p, int flags) {
+  cInstance& I = *uniform((cInstance*)inst);
+  if (flags & L_HAS) {
+    if (!(flags & L_ALIVE)) r = load_state(I, p);
+    store6(dst, 1, r);
+  }
+}
+
+// One turn (or the part of it from e0 to e1) of a wave's particles. A function
+// of its own, called once per turn: the loop over the records then has the
+// scalar registers to itself instead of sharing them with everything that
+// the kernel keeps for the turn boundaries.
+template <int P>
+struct Slots {
+  Lane l[P];
+};
+
+template <bool REFS, int P, int U>
+__device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Instance* instp, int tp) {
+  const Instance* inst = uniform(instp);
+  cInstance& I = *(cInstance*)inst;
+  const int t = __builtin_amdgcn_readfirstlane(tp);
+  cDevElem* elems = (cDevElem*)I.elems;
+  cdouble* pool = (cdouble*)I.pool;
+  cLatOp* ops = (cLatOp*)I.ops;
+  const int p[2] = {p0, p1};
+  R6 r[P];
+  int fl[P];
+#pragma unroll
+  for (int q = 0; q < P; q++) {
+    r[q] = S.l[q].r;
+    fl[q] = S.l[q].flags;
+  }
+  const bool check = !I.elempass;
+  const int nturn = I.turn0 + t;
+  const int e0 = (t == 0) ? I.start_elem : 0;
+  const int e1 = I.end_elem;
+  cint* slot = (cint*)I.slots + ((t == 0) ? 0 : I.nelem + 1);
+  const int64_t base = (t == 0) ? 0 : (int64_t)I.n_first + (int64_t)(t - 1) * I.n_std;
+  // Refpt copy of the state before element e (at.c:622-626).
+  auto copy_refs = [&](int e) {
+    const int sl = slot[e];
+    if (sl < 0) return;
+    double* dst = I.rout + (base + sl) * 6 * (int64_t)I.npart;
+#pragma unroll
+    for (int q = 0; q < P; q++)
+      copy_call(r[q], inst, dst + 6 * (int64_t)p[q], p[q], fl[q]);
+  };
+  // Live particles that fail the loss test after element e: `lost` is the
+  // test's result for every lane, and the lanes with a live particle are a
+  // scalar mask, so that the test ends in one scalar branch.
+  uint64_t alive[P];
+#pragma unroll
+  for (int q = 0; q < P; q++) alive[q] = __builtin_amdgcn_ballot_w64((fl[q] & L_ALIVE) != 0);
+  auto lose = [&](int q, bool lost, int e) {
+    const uint64_t bad = __builtin_amdgcn_ballot_w64(lost) & alive[q];
+    if (__builtin_expect(bad != 0, 0)) {
+      Lane l{r[q], fl[q]};
+      loss_call(&l, inst, p[q], (int)((bad >> (threadIdx.x & 63)) & 1), nturn, e);
+      r[q] = l.r;
+      fl[q] = l.flags;
+      alive[q] = __builtin_amdgcn_ballot_w64((fl[q] & L_ALIVE) != 0);
+    }
+  };
+  // One element by its header, with its refpt copy and loss test. A NaN
+  // input is skipped by the first element and lost at its test.
+  auto by_header = [&](int e, bool entry) {
+    if (REFS) copy_refs(e);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      if (entry) lose(q, __builtin_isnan(r[q].x), e);
+      r[q] = header_call<U>(r[q], &elems[e], pool, nturn);
+      if (check) lose(q, is_lost(r[q]), e);
+    }
+  };
+  // The loop over the records. With few waves per SIMD it is bound by the
+  // time around an element's arithmetic: scalar loads waited for one after
+  // the other (kind, then flags, then pool offsets, then constants), a tree of
+  // branches over 147 KB of code, and the state copied for lanes that skip
+  // an element. One record per drift-and-element pair, its head read one
+  // record ahead, its constants at fixed offsets, no skipping lanes and 35
+  // KB of code brought the large ring (10 slices per magnet) from 3.35 to
+  // 2.56 ms per turn for one wave, from 3.54 to 2.70 for 24,001 particles and
+  // from 8.32 to 7.70 for 262,144; without the slices (extrapolated from 4
+  // and 10 per magnet) one wave went from 1.33 to 0.58 ms.
+  // A turn runs the records o0..o1-1 whole. The first element of a call
+  // (whose input has not passed a loss test yet) and the elements of a
+  // record that a partial turn starts or ends in run by their headers,
+  // before and after the records.
+  cint* opof = (cint*)I.opof;
+  const int o1 = opof[e1];
+  int o0 = e0 < e1 ? 0 : o1;
+  int e = e0;
+  if (t == 0 && e0 < e1) {
+    o0 = opof[e0] + 1;
+    for (const int stop = min(ops[o0].first, e1); e < stop; e++) by_header(e, e == e0);
+  }
+  cLatOp* rec = ops + o0;
+  cLatOp* const end = ops + max(o0, o1);
+  OpHead nxt = op_head(rec);
+  for (; rec != end; rec++) {
+    const OpHead cur = nxt;
+    asm volatile("" ::"s"(cur.line1), "s"(cur.line2));
+    nxt = op_head(rec + 1);
+    const int kind = cur.op & 0xff;
+    if (REFS) {  // markers change nothing: only their copies
+      const int ndo = (kind != OP_NONE ? 1 : 0) + ((cur.op & OPF_DRIFT) ? 1 : 0);
+      for (int k = rec->first; k <= cur.last - ndo; k++) copy_refs(k);
+    }
+    if (cur.op & OPF_DRIFT) {
+      const int at = cur.last - (kind != OP_NONE ? 1 : 0);
+      if (REFS) copy_refs(at);
+#pragma unroll
+      for (int q = 0; q < P; q++) drift6(r[q], cur.len);
+#pragma unroll
+      for (int q = 0; q < P; q++) lose(q, is_lost_drift(r[q]), at);
+    }
+    if (kind == OP_NONE) continue;
+    if (REFS) copy_refs(cur.last);
+    cdouble* c = rec->c;
+    cDevElem* h = &elems[cur.last];
+    if (cur.op & OPF_XF) {
+#pragma unroll
+      for (int q = 0; q < P; q++) {
+        r[q].x += c[OM_XF];
+        r[q].px += c[OM_XF + 1];
+        r[q].y += c[OM_XF + 2];
+        r[q].py += c[OM_XF + 3];
+        roll(r[q], c[OM_XF + 4], c[OM_XF + 5]);
+      }
+    }
+    switch (kind) {
+      case OP_STR1: mpole_op<false, false, 1, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
+      case OP_STR2: mpole_op<false, false, 2, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
+      case OP_STR3: mpole_op<false, false, 3, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
+      case OP_BND1: mpole_op<true, false, 1, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
+      case OP_STRRAD1: mpole_op<false, true, 1, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
+      case OP_BNDRAD1: mpole_op<true, true, 1, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
+      case OP_THIN2:
+#pragma unroll
+        for (int q = 0; q < P; q++) thin_op<2>(r[q], c);
+        break;
+      case OP_THIN3:
+#pragma unroll
+        for (int q = 0; q < P; q++) thin_op<3>(r[q], c);
+        break;
+      case OP_APERTURE:  // AperturePass.c:9-26
+#pragma unroll
+        for (int q = 0; q < P; q++) rect_ap(r[q], c);
+        break;
+      case OP_CORR:
+#pragma unroll
+        for (int q = 0; q < P; q++) {
+          if (cur.op & OPF_THICK) {
+            const double pn = rcp_opd(r[q]);
+            corrector_map(r[q], c[OC_XK], c[OC_YK], c[OC_Q0], c[OC_LEN] * pn, pn);
+          } else {
+            r[q].px += c[OC_XK];
+            r[q].py += c[OC_YK];
+          }
+        }
+        break;
+      default:
+#pragma unroll
+        for (int q = 0; q < P; q++) r[q] = generic_element<U>(r[q], *h, pool, nturn);
+        break;
+    }
+    if (cur.op & OPF_XF) {
+#pragma unroll
+      for (int q = 0; q < P; q++) {
+        // a coordinate that is not finite spreads through the zeros of the
+        // 6x6 product, as in the reference: the wave then takes the product
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(is_lost(r[q])) != 0 && (h->flags & F_R2), 0))
+          r[q] = mul_r_v(r[q], pool + h->r2);
+        else
+          roll(r[q], c[OM_XF + 6], c[OM_XF + 7]);
+        r[q].x += c[OM_XF + 8];
+        r[q].px += c[OM_XF + 9];
+        r[q].y += c[OM_XF + 10];
+        r[q].py += c[OM_XF + 11];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) lose(q, is_lost(r[q]), cur.last);
+  }
+  for (e = max(e, ops[o1].first); e < e1; e++) by_header(e, false);
+  if (REFS) copy_refs(I.nelem);
+#pragma unroll
+  for (int q = 0; q < P; q++) S.l[q] = Lane{r[q], fl[q]};
+  return S;
+}
 
 // P particles per lane, lane-major: lane l of a workgroup holds its slots
 // l*P .. l*P+P-1. live_begin (repacked turn blocks after the first; NULL
@@ -1540,8 +1963,8 @@ __device__ __forceinline__ R6 lost_state() { return R6{__builtin_nan(""), 0.0, 0
 // survive), so that the live workgroups of all instances are the leading
 // ones of the grid and the hardware spreads them evenly over the CUs; the
 // other workgroups end at once.
-template <bool EXT, int P, int U>
-__global__ void __launch_bounds__(512) track_kernel(const Instance* __restrict__ insts_g, int ninst,
+template <bool REFS, int P, int U>
+__global__ void __launch_bounds__(512, P == 1 ? 4 : 2) track_kernel(const Instance* __restrict__ insts_g, int ninst,
                                                     int nblocks, int xcd_order,
                                                     const int32_t* __restrict__ live_begin) {
   static_assert(P == 1 || P == 2, "one or two particles per lane");
@@ -1600,33 +2023,28 @@ __global__ void __launch_bounds__(512) track_kernel(const Instance* __restrict__
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (wave >= nw) return;
 
-  cDevElem* elems = (cDevElem*)I.elems;
-  cdouble* pool = (cdouble*)I.pool;
-  cint* slots = (cint*)I.slots;
-  const int64_t cs = I.cstride;
   const int losses = I.losses;
   int p[P];
-  bool has[P], lost[P];
-  R6 r[P];
+  // Of each slot: whether it holds a particle (L_HAS), whether the
+  // particle's state is in the lane's registers (L_ALIVE), and whether its
+  // loss has been recorded (L_LOST). A particle whose x is NaN is skipped by
+  // every element (at.c:142-161, *Pass.c): its state goes to memory for good
+  // when it is found (at the loss test, or at the first element for a NaN
+  // input) and the lane tracks the origin from then on, so that no element
+  // needs to mask lanes or keep their old state.
+  Lane L[P];
 #pragma unroll
   for (int q = 0; q < P; q++) {
     const int sl = tid * P + q;
-    has[q] = sl < held;  // this slot holds a particle
-    p[q] = has[q] ? (idx ? idx[first + sl] : first + sl) : 0;
-    r[q] = lost_state();
-    if (has[q]) {
-      const double* rp = I.r + (int64_t)p[q] * I.pstride;
-      r[q].x = rp[0];
-      r[q].px = rp[cs];
-      r[q].y = rp[2 * cs];
-      r[q].py = rp[3 * cs];
-      r[q].dp = rp[4 * cs];
-      r[q].ct = rp[5 * cs];
-    }
-    lost[q] = !has[q];  // slots without a particle never record a loss
-    if (has[q]) {
+    const bool has = sl < held;
+    p[q] = has ? (idx ? idx[first + sl] : first + sl) : 0;
+    L[q].r = idle_state();
+    L[q].flags = L_LOST;  // a slot without a particle never records a loss
+    if (has) {
+      L[q].r = load_state(I, p[q]);
+      L[q].flags = L_HAS | L_ALIVE;
       if (losses == 2) {
-        lost[q] = I.lost_flag[p[q]] != 0;  // recorded by an earlier call
+        if (I.lost_flag[p[q]] != 0) L[q].flags |= L_LOST;  // recorded by an earlier call
       } else if (losses) {
         I.lost_flag[p[q]] = 0;
         I.lost_turn[p[q]] = 0;
@@ -1636,37 +2054,29 @@ __global__ void __launch_bounds__(512) track_kernel(const Instance* __restrict__
     }
   }
 
-  const int nelem = I.nelem;
   const bool check = !I.elempass;
-  double* rout = I.rout;
-  const int64_t np6 = 6 * (int64_t)npart;
   const int nturns = I.nturns;
-  const bool refs = (I.n_first | I.n_std) != 0;  // uniform: skip the slot reads without refpts
   // Lost particles are dropped at turn boundaries and the survivors packed
   // into the leading lanes: with one particle per lane when packing frees a
   // wave (the waves left without particles end and free their SIMD slots),
   // with several whenever one was lost (a lane steps its particles together
   // only while none of them is lost). Not with refpts: lost particles still
   // fill their refpt copies, as in at.c.
-  const bool compact = check && !refs && nturns > 1;
+  const bool compact = check && !REFS && nturns > 1;
   double* s_r = lds;
   int* s_p = (int*)(lds + 6 * G);
   int* s_cnt = s_p + G;
   for (int t = 0; t < nturns; t++) {
     if (compact && t > 0) {
-      // A particle whose x is NaN is lost for good (elements skip it and the
-      // loss check leaves it as it is): store its final state now.
+      // drop the particles whose final state is stored
       int mine = 0, below = 0;
       int within[P];
 #pragma unroll
       for (int q = 0; q < P; q++) {
-        if (has[q] && __builtin_isnan(r[q].x)) {
-          store_state(I, p[q], r[q]);
-          has[q] = false;
-        }
-        const uint64_t m = __ballot(has[q]);
+        const bool on = (L[q].flags & L_ALIVE) != 0;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(on);
         within[q] = mine;
-        mine += has[q] ? 1 : 0;
+        mine += on ? 1 : 0;
         below += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                            __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
       }
@@ -1687,35 +2097,33 @@ __global__ void __launch_bounds__(512) track_kernel(const Instance* __restrict__
       if (need < nw || (P > 1 && total < held)) {  // uniform
 #pragma unroll
         for (int q = 0; q < P; q++) {
-          if (has[q]) {
+          if (L[q].flags & L_ALIVE) {
             const int j = off + below + within[q];
-            s_r[j] = r[q].x;
-            s_r[G + j] = r[q].px;
-            s_r[2 * G + j] = r[q].y;
-            s_r[3 * G + j] = r[q].py;
-            s_r[4 * G + j] = r[q].dp;
-            s_r[5 * G + j] = r[q].ct;
-            s_p[j] = p[q] | (lost[q] ? (int)0x80000000u : 0);
+            s_r[j] = L[q].r.x;
+            s_r[G + j] = L[q].r.px;
+            s_r[2 * G + j] = L[q].r.y;
+            s_r[3 * G + j] = L[q].r.py;
+            s_r[4 * G + j] = L[q].r.dp;
+            s_r[5 * G + j] = L[q].r.ct;
+            s_p[j] = p[q] | ((L[q].flags & L_LOST) ? (int)0x80000000u : 0);
           }
         }
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < P; q++) {
           const int j = tid * P + q;
-          has[q] = j < total;
-          if (has[q]) {
-            r[q].x = s_r[j];
-            r[q].px = s_r[G + j];
-            r[q].y = s_r[2 * G + j];
-            r[q].py = s_r[3 * G + j];
-            r[q].dp = s_r[4 * G + j];
-            r[q].ct = s_r[5 * G + j];
+          if (j < total) {
+            L[q].r.x = s_r[j];
+            L[q].r.px = s_r[G + j];
+            L[q].r.y = s_r[2 * G + j];
+            L[q].r.py = s_r[3 * G + j];
+            L[q].r.dp = s_r[4 * G + j];
+            L[q].r.ct = s_r[5 * G + j];
             const int v = s_p[j];
             p[q] = v & 0x7fffffff;
-            lost[q] = v < 0;
+            L[q].flags = L_HAS | L_ALIVE | (v < 0 ? L_LOST : 0);
           } else {
-            r[q] = lost_state();
-            lost[q] = true;
+            L[q].flags = L_LOST;
           }
         }
         held = total;
@@ -1723,126 +2131,19 @@ __global__ void __launch_bounds__(512) track_kernel(const Instance* __restrict__
         if (wave >= nw) return;  // this wave holds no particle any more
       }
     }
-    const int nturn = I.turn0 + t;
-    const int e0 = (t == 0) ? I.start_elem : 0;
-    cint* slot = slots + ((t == 0) ? 0 : nelem + 1);
-    const int64_t base = (t == 0) ? 0 : (int64_t)I.n_first + (int64_t)(t - 1) * I.n_std;
-    const int e1 = I.end_elem;
-    for (int e = e0; e < e1; e++) {
-      if (refs) {
-        const int sl = slot[e];
 #pragma unroll
-        for (int q = 0; q < P; q++)
-          if (has[q] && sl >= 0) store6(rout + (base + sl) * np6 + 6 * (int64_t)p[q], 1, r[q]);
-      }
-      cDevElem& h = elems[e];
-      bool unchanged = false;  // no coordinate changed: the loss check would repeat the last
-      if (h.kind == K_DRIFT && h.flags == 0) {
-        // A drift without misalignment or apertures (DriftPass.c:16-48), half
-        // the elements of a ring: tested first, from the header's first two
-        // words, and stepped without the element dispatch. Every element
-        // skips a particle whose x is NaN (at.c:142-161).
-        const double len = drift_length(h);
+    for (int q = 0; q < P; q++)
+      if (!(L[q].flags & L_ALIVE)) L[q].r = idle_state();
+    Slots<P> S;
 #pragma unroll
-        for (int q = 0; q < P; q++) {
-#if ATX_STRICT
-          if (!__builtin_isnan(r[q].x)) drift6(r[q], len);
-#else
-          // the fast build skips a NaN-x lane by a zero step instead of
-          // selecting its old coordinates: x stays NaN and a finite y, ct
-          // stay as they are (a lost particle's are zero). The operations
-          // and their rounding are drift6's in this build.
-          const double pn = fast_rcp(1.0 + r[q].dp);
-          const double nl = __builtin_isnan(r[q].x) ? 0.0 : len * pn;
-          r[q].x = __builtin_fma(nl, r[q].px, r[q].x);
-          r[q].y = __builtin_fma(nl, r[q].py, r[q].y);
-          const double p2 = __builtin_fma(r[q].px, r[q].px, r[q].py * r[q].py);
-          const double dct = (pn * nl) * p2;
-          const double hct = dct * 0.5;
-          r[q].ct = r[q].ct + hct;
-#endif
-        }
-      } else if (h.kind == K_IDENTITY && h.flags == 0) {
-        // A marker or monitor without misalignment or apertures
-        // (IdentityPass.c:20-43) changes no coordinate, so its loss check
-        // would repeat the one after the element before it: only the first
-        // element of the call checks.
-        unchanged = t > 0 || e > e0;
-      } else if (P == 1) {
-        if (!__builtin_isnan(r[0].x)) element_lane<EXT, 1, U>(r, h, pool, nturn);
-      } else {
-        // A lane steps its particles together. Every element skips a
-        // particle whose x is NaN (at.c:142-161, *Pass.c): in a wave that
-        // holds such a particle (a loss since the last compaction, or a NaN
-        // input), its state is kept in the lane's own LDS slots and put back
-        // after the element. Slots without a particle step too; they are
-        // never stored.
-        bool stale[P];
-        bool any = false;
+    for (int q = 0; q < P; q++) S.l[q] = L[q];
+    S = run_turn<REFS, P, U>(S, p[0], p[P - 1], insts_g + lo, t);
 #pragma unroll
-        for (int q = 0; q < P; q++) {
-          stale[q] = has[q] && __builtin_isnan(r[q].x);
-          any |= stale[q];
-        }
-        const bool keep = __ballot(any) != 0;  // uniform
-        if (keep) {
-#pragma unroll
-          for (int q = 0; q < P; q++) {
-            const int j = tid * P + q;
-            if (stale[q]) {
-              s_r[j] = r[q].x;
-              s_r[G + j] = r[q].px;
-              s_r[2 * G + j] = r[q].y;
-              s_r[3 * G + j] = r[q].py;
-              s_r[4 * G + j] = r[q].dp;
-              s_r[5 * G + j] = r[q].ct;
-            }
-          }
-        }
-        element_lane<EXT, P, U>(r, h, pool, nturn);
-        if (keep) {
-#pragma unroll
-          for (int q = 0; q < P; q++) {
-            const int j = tid * P + q;
-            if (stale[q]) {
-              r[q].x = s_r[j];
-              r[q].px = s_r[G + j];
-              r[q].y = s_r[2 * G + j];
-              r[q].py = s_r[3 * G + j];
-              r[q].dp = s_r[4 * G + j];
-              r[q].ct = s_r[5 * G + j];
-            }
-          }
-        }
-      }
-      if (check && !unchanged) {
-#pragma unroll
-        for (int q = 0; q < P; q++) {
-          if (losses) {
-            if (!lost[q] && is_lost(r[q])) {
-              lost[q] = true;
-              I.lost_flag[p[q]] = 1;
-              I.lost_turn[p[q]] = (uint32_t)nturn;
-              I.lost_elem[p[q]] = (uint32_t)e;
-              store6(I.lost_coord + 6 * (int64_t)p[q], 1, r[q]);
-              r[q] = lost_state();
-            }
-          } else if (has[q] && __builtin_isfinite(r[q].x) && is_lost(r[q])) {
-            r[q] = lost_state();  // at.c:142-161
-          }
-        }
-      }
-    }
-    if (refs) {
-      const int sl = slot[nelem];
-#pragma unroll
-      for (int q = 0; q < P; q++)
-        if (has[q] && sl >= 0) store6(rout + (base + sl) * np6 + 6 * (int64_t)p[q], 1, r[q]);
-    }
+    for (int q = 0; q < P; q++) L[q] = S.l[q];
   }
 #pragma unroll
   for (int q = 0; q < P; q++)
-    if (has[q]) store_state(I, p[q], r[q]);
+    if (L[q].flags & L_ALIVE) store_state(I, p[q], L[q].r);
 }
 
 }  // namespace ATX_NS
@@ -1851,13 +2152,13 @@ __global__ void __launch_bounds__(512) track_kernel(const Instance* __restrict__
 // The kernel of this object's launch shape: nblocks workgroups of `block`
 // lanes, block * ATX_PPT particle slots each.
 extern "C" hipError_t ATX_LAUNCH(const atx::Instance* d_insts, int ninst, int nblocks, int block,
-                                 int ext, int xcd_order, const int32_t* live_begin,
+                                 int refs, int xcd_order, const int32_t* live_begin,
                                  hipStream_t stream) {
   const size_t lds = atx::ATX_NS::compact_lds_bytes(block * ATX_PPT);
   // whole rounds of XCDs: the kernel's workgroup order needs the grid to
   // cover kXcds * ceil(n / kXcds) for every n <= nblocks
   const int grid = (nblocks + atx::kXcds - 1) / atx::kXcds * atx::kXcds;
-  if (ext)
+  if (refs)
     hipLaunchKernelGGL((atx::ATX_NS::track_kernel<true, ATX_PPT, ATX_UNROLL>), dim3(grid),
                        dim3(block), lds, stream, d_insts, ninst, nblocks, xcd_order, live_begin);
   else
@@ -1924,7 +2225,7 @@ __global__ void __launch_bounds__(1024) repack_kernel(const Instance* __restrict
       q = first_pass ? s : idx[s];
       alive = !__builtin_isnan(I.r[(int64_t)q * I.pstride]);
     }
-    const uint64_t m = __ballot(alive);
+    const uint64_t m = __builtin_amdgcn_ballot_w64(alive);
     const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
     if ((tid & 63) == 0) s_wave[wave] = __popcll(m);
