@@ -142,12 +142,25 @@ enum OpKind : int32_t {
   // ThinMPolePass without attributes: c[OT_*], c[OM_POLY...]
   OP_THIN2 = 10,
   OP_THIN3 = 11,
+  // the same multipoles with few coefficients that are not zero: B[order] only
+  // (L), that and B[0], A[0] (D), none (0)
+  OP_STR1L = 12,
+  OP_STR2L = 13,
+  OP_STR2D = 14,
+  OP_STR3L = 15,
+  OP_BND1L = 16,
+  OP_BND0 = 17,
+  OP_STRRAD1L = 18,
+  OP_BNDRAD1L = 19,
+  OP_BNDRAD0 = 20,
 };
 enum : int32_t {
   OPF_DRIFT = 1 << 8,  // a plain drift of length `len` before the element
   OPF_THICK = 2 << 8,  // corrector of non-zero length
   OPF_XF = 4 << 8,     // misaligned by transverse shifts and rolls: c[OM_XF...]
   OPF_EDGE = 8 << 8,   // a bend's edges by its header (not of constant strength)
+  OPF_MPOLE = 16 << 8, // a thick multipole
+  OPF_RAD = 32 << 8,   // a radiating one
 };
 // constants of OP_CORR, the thin and the thick multipoles
 enum OpSlot : int32_t {

@@ -670,6 +670,26 @@ void fill_op(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
     if (h.flags & F_R1) plain = plain && plain_roll(&pool[h.r1], &xf[4], &xf[5]);
     if (h.flags & F_R2) plain = plain && plain_roll(&pool[h.r2], &xf[6], &xf[7]);
     if (op == OP_GENERIC || !plain) return;
+    // the form of the field: which coefficients are not zero
+    const double* a = &pool[h.poly];
+    const double* b = a + h.order + 1;
+    bool lead = true;
+    for (int k = 1; k <= h.order; k++) lead = lead && a[k] == 0.0 && (k == h.order || b[k] == 0.0);
+    const bool dipole = a[0] != 0.0 || b[0] != 0.0;
+    if (lead && !dipole) {
+      switch (op) {
+        case OP_STR1: op = OP_STR1L; break;
+        case OP_STR2: op = OP_STR2L; break;
+        case OP_STR3: op = OP_STR3L; break;
+        case OP_STRRAD1: op = OP_STRRAD1L; break;
+        case OP_BND1: op = b[1] == 0.0 ? OP_BND0 : OP_BND1L; break;
+        case OP_BNDRAD1: op = b[1] == 0.0 ? OP_BNDRAD0 : OP_BNDRAD1L; break;
+      }
+    } else if (lead && op == OP_STR2) {
+      op = OP_STR2D;
+    }
+    op |= OPF_MPOLE;
+    if (h.kind == K_STRRAD || h.kind == K_BNDRAD) op |= OPF_RAD;
     if (h.flags & (F_T1 | F_T2 | F_R1 | F_R2)) op |= OPF_XF;
     if ((h.edge & 0xff) != E_CONST || ((h.edge >> 8) & 0xff) != E_CONST) op |= OPF_EDGE;
     r.op = drift | op;

@@ -536,6 +536,24 @@ __device__ __noinline__ R6 slices_ops(R6 r, cdouble* a, cdouble* b, int n, cdoub
 // instruction stream, and the magnet's scalar constants, loop control and
 // branches serve P particles. Per-particle maps that are rare or large stay
 // out of line and run once per particle.
+// The field of a magnet, by the coefficients that are not zero (chosen when the
+// lattice is compiled, atx_host.cpp fill_op). Quadrupoles, sextupoles and
+// octupoles have one coefficient and a bend often none, so the fast build
+// spells their kicks out instead of running Horner over zeros: 2 FP64
+// instructions instead of 6 per quadrupole kick, 5 instead of 10 per sextupole
+// kick, 8 instead of 14 per octupole kick, 20 instead of 26 per radiating
+// quadrupole kick, 26 instead of 42 per kick of a radiating bend without
+// gradient. The VALU issues on 83 % of the cycles of a full device, so time
+// follows the instruction count. The strict build evaluates all coefficients.
+// A particle whose result is not finite is recomputed with the general form
+// (run_turn): zeros times an infinity are NaN there, as in the reference.
+enum Form : int {
+  F_GENERAL = 0,  // Horner over all coefficients
+  F_LEAD = 1,     // B[N] only
+  F_LEAD0 = 2,    // B[N], B[0] and A[0] (a sextupole that is a corrector, too)
+  F_NOFIELD = 3   // none: a bend's own curvature
+};
+
 #if !ATX_STRICT
 // In-magnet drift of the fast build: nlh = nl / (2 (1+delta)) hoisted with
 // nl (delta is constant in a non-radiating magnet).
@@ -546,12 +564,102 @@ __device__ __forceinline__ void fastdrift_h(R6& r, double nl, double nlh) {
   r.ct = __builtin_fma(nlh, p2, r.ct);
 }
 
+// What a kick of length kl multiplies by, once per magnet. The rounding of
+// such a product is the same at every kick of every turn, so it would add up
+// over the turns instead of averaging out: its remainder is kept, too, and is
+// added where that costs nothing (radiating kicks) or once per magnet.
+struct Kick {
+  double kl, kli;         // length, length times curvature
+  double kb, kb2;         // kl B[N], twice that
+  double kb0, ka0;        // kl B[0], kl A[0]
+  double lo;              // remainder of kb (NOFIELD: of kli)
+  double rk;              // radiating: RAD_CONST gamma^3 kl (times the field's constant squared)
+};
+
+template <bool BEND, int N, int F>
+__device__ __forceinline__ Kick kick_of(cdouble* a, cdouble* b, double kl, double irho, double radk) {
+  Kick k;
+  k.kl = kl;
+  k.kli = BEND ? kl * irho : 0.0;
+  k.kb = k.kb2 = k.kb0 = k.ka0 = k.lo = 0.0;
+  if (F == F_LEAD || F == F_LEAD0) {
+    k.kb = kl * b[N];
+    k.kb2 = 2.0 * k.kb;
+    k.lo = __builtin_fma(kl, b[N], -k.kb);
+  }
+  if (F == F_NOFIELD) k.lo = __builtin_fma(kl, irho, -k.kli);
+  if (F == F_LEAD0) {
+    k.kb0 = kl * b[0];
+    k.ka0 = kl * a[0];
+  }
+  k.rk = radk;
+  if (F == F_LEAD && !BEND) k.rk = radk * (b[N] * b[N]);
+  if (F == F_NOFIELD) k.rk = radk * (irho * irho);
+  return k;
+}
+
+// The remainders of a whole magnet's kicks in one, c = their sum.
+template <bool BEND, int N, int F>
+__device__ __forceinline__ void kick_rest(R6& r, double c, double irho) {
+  if (F == F_NOFIELD) {
+    r.px = __builtin_fma(c, __builtin_fma(-r.x, irho, r.dp), r.px);
+  } else if (N == 1) {
+    r.px = __builtin_fma(-c, r.x, r.px);
+    r.py = __builtin_fma(c, r.y, r.py);
+  } else if (N == 2) {
+    r.px = __builtin_fma(-c, __builtin_fma(r.x, r.x, -(r.y * r.y)), r.px);
+    r.py = __builtin_fma(2.0 * c, r.x * r.y, r.py);
+  }
+}
+
+// driftkick.c:51-115 by form.
+template <bool BEND, int N, int F>
+__device__ __forceinline__ void kick(R6& r, const Kick& k, cdouble* a, cdouble* b, int n, double blo,
+                                     double alo, double irho) {
+  if (F == F_GENERAL) {
+    if (BEND) bnd_kick<N>(r, a, b, n, blo, alo, k.kl, irho, k.kli);
+    else str_kick<N>(r, a, b, n, blo, alo, k.kl);
+    return;
+  }
+  static_assert(F == F_GENERAL || N == 1 || !BEND, "bends: order 1");
+  if (BEND) {
+    // kl (re - (delta - x h) h) = kb x - kl h (delta - x h)
+    const double u = __builtin_fma(-r.x, irho, r.dp);
+    double px = r.px;
+    if (F == F_LEAD) {
+      px = __builtin_fma(-k.kb, r.x, px);
+      r.py = __builtin_fma(k.kb, r.y, r.py);
+    }
+    r.px = __builtin_fma(k.kli, u, px);
+    r.ct = __builtin_fma(k.kli, r.x, r.ct);
+    return;
+  }
+  double px = r.px, py = r.py;
+  if (F == F_LEAD0) {
+    px = px - k.kb0;
+    py = py + k.ka0;
+  }
+  if (N == 1) {
+    px = __builtin_fma(-k.kb, r.x, px);
+    py = __builtin_fma(k.kb, r.y, py);
+  } else if (N == 2) {  // z^2 = (x^2 - y^2) + i 2 x y
+    px = __builtin_fma(-k.kb, __builtin_fma(r.x, r.x, -(r.y * r.y)), px);
+    py = __builtin_fma(k.kb2, r.x * r.y, py);
+  } else {  // z^3 = x (x^2 - 3 y^2) + i y (3 x^2 - y^2)
+    const double x2 = r.x * r.x, y2 = r.y * r.y;
+    px = __builtin_fma(-k.kb, r.x * __builtin_fma(-3.0, y2, x2), px);
+    py = __builtin_fma(k.kb, r.y * __builtin_fma(3.0, x2, -y2), py);
+  }
+  r.px = px;
+  r.py = py;
+}
+
 // Radiating magnets of the fast build carry the transverse momenta as
 // angles x' = px/(1+delta), y' = py/(1+delta) from entry to exit: a drift is
 // then x += L x', ct += (L/2)(x'^2 + y'^2), its x'^2 + y'^2 is the kick's
 // s2 (the kick that follows a drift sees the same angles), and a kick turns
 // px = x'(1+delta') - kl Re, the reference's update, into
-// x' <- x' - kl Re / (1+delta'). pn = 1/(1+delta) as in rad_str_kick.
+// x' <- x' - kl Re / (1+delta'). pn = 1/(1+delta).
 struct Ang {
   double xp, yp, s2, pn;
 };
@@ -574,74 +682,94 @@ __device__ __forceinline__ void rad_drift_ang(R6& r, Ang& g, double len, double 
   r.ct = __builtin_fma(hlen, g.s2, r.ct);
 }
 
-// diff_str_kick.c:19-83 (bdiff == NULL) in angle form; radk = RAD_CONST
-// gamma^3 kl. The radiated factor (1+s2/2)/(1+s2) is the series of
-// rad_str_kick (relative error s2^4/2; a wave with s2 > 1e-4 divides).
-template <int N>
-__device__ __forceinline__ void rad_str_kick_ang(R6& r, Ang& g, cdouble* a, cdouble* b, int n,
-                                                 double blo, double alo, double kl, double radk) {
-  double re, im;
-  field<N>(r, a, b, n, blo, alo, re, im);
-  const double s2 = g.s2;
-  const double opd = 1.0 + r.dp;
-  const double cr = __builtin_fma(im, g.yp, -re * g.xp);
-  const double b2 = __builtin_fma(cr, cr, __builtin_fma(re, re, im * im));
-  // 1 - (s2/2)(1 - s2 + s2^2) by Horner in s2
-  const double f = __builtin_fma(s2, __builtin_fma(s2, __builtin_fma(-0.5, s2, 0.5), -0.5), 1.0);
-  const double oo = opd * opd;
-  const double d0 = r.dp;
-  double dp = __builtin_fma(-radk, (b2 * f) * oo, d0);
-  double opd2 = 1.0 + dp;
-  double e = __builtin_fma(-opd2, g.pn, 1.0);
-  double pn = __builtin_fma(g.pn, __builtin_fma(e, e, e), g.pn);
-  // one vote for both exceptions of the wave: a wide angle (the factor by
-  // division) and a large radiated fraction (the reciprocal from fast_rcp)
-  const bool wide = s2 > 1e-4;
-  if (__builtin_expect(__builtin_amdgcn_ballot_w64(wide || __builtin_fabs(e) > 2e-6) != 0, 0)) {
-    const double fw = __builtin_fma(0.5, s2, 1.0) * rcp1(1.0 + s2);
-    const double dpw = __builtin_fma(-radk, (b2 * fw) * oo, d0);
-    const double opw = 1.0 + dpw;
-    const double ew = __builtin_fma(-opw, g.pn, 1.0);
-    const double pw = __builtin_fma(g.pn, __builtin_fma(ew, ew, ew), g.pn);
-    dp = wide ? dpw : dp;
-    opd2 = wide ? opw : opd2;
-    e = wide ? ew : e;
-    pn = wide ? pw : pn;
-    pn = __builtin_fabs(e) > 2e-6 ? fast_rcp(opd2) : pn;
-  }
-  r.dp = dp;
-  const double klpn = kl * pn;
-  g.xp = __builtin_fma(-re, klpn, g.xp);
-  g.yp = __builtin_fma(im, klpn, g.yp);
-  g.pn = pn;
-}
-
-// diff_bnd_kick.c:85-174 (bdiff == NULL) in angle form.
-template <int N>
-__device__ __forceinline__ void rad_bnd_kick_ang(R6& r, Ang& g, cdouble* a, cdouble* b, int n,
-                                                 double blo, double alo, double kl, double irho,
-                                                 double kli, double radk) {
-  double re, im;
-  field<N>(r, a, b, n, blo, alo, re, im);
-  const double x = r.x;
+// diff_str_kick.c:19-83 and diff_bnd_kick.c:85-174 (bdiff == NULL) in angle
+// form. w is the radiated fraction, radk b2p factor (1+delta): delta falls by
+// w (1+delta), and 1/(1+delta) becomes pn/(1-w) = pn (1 + w + w^2) to a
+// relative w^3, below 1e-17 for |w| <= 2e-6. The last kick of a slice (REFRESH)
+// takes 1 - (1+delta') pn in the place of w: that holds the rounding errors of
+// pn as well, which would otherwise add up over the magnet.
+// Straight magnets: the factor (1+s2/2)/(1+s2) is 1 - (s2/2)(1 - s2 + s2^2),
+// relative error s2^4/2, below 1e-16 for s2 <= 1e-4 (angles up to 10 mrad).
+// CHECKED: lanes outside either range divide instead, under a vote per kick.
+// Otherwise `bad` collects them for the whole magnet, which is then run again
+// with the checks (run_turn): no branch in the slices. All other lanes get the
+// same bits either way.
+template <bool BEND, int N, int F, bool CHECKED, bool REFRESH>
+__device__ __forceinline__ void rad_kick_ang(R6& r, Ang& g, const Kick& k, cdouble* a, cdouble* b,
+                                             int n, double blo, double alo, double irho,
+                                             uint64_t& bad) {
+  const double x = r.x, y = r.y;
   const double s2 = g.s2;
   const double d0 = r.dp;
   const double opd = 1.0 + d0;
-  const double by = re + irho;
-  const double hx = __builtin_fma(x, irho, 1.0);
-  const double byh = by * hx;
-  const double bxh = im * hx;
-  const double cr = __builtin_fma(im, g.yp, -by * g.xp);
-  const double b2 = __builtin_fma(cr, cr, __builtin_fma(byh, byh, bxh * bxh));
-  const double f = __builtin_fma(0.5, s2, hx) * rcp1(__builtin_fma(hx, hx, s2));
-  r.dp = __builtin_fma(-radk, (b2 * f) * (opd * opd), d0);
-  const double pn = rcp_after_kick(1.0 + r.dp, g.pn);
-  const double u = __builtin_fma(-x, irho, d0);
-  const double v = __builtin_fma(-u, irho, re);
-  const double klpn = kl * pn;
-  g.xp = __builtin_fma(-v, klpn, g.xp);
-  g.yp = __builtin_fma(im, klpn, g.yp);
-  r.ct = __builtin_fma(kli, x, r.ct);
+  const double ro = k.rk * opd;
+  double re = 0.0, im = 0.0;
+  if (F == F_GENERAL) field<N>(r, a, b, n, blo, alo, re, im);
+  if (BEND && F == F_LEAD) {
+    re = b[1] * x;
+    im = b[1] * y;
+  }
+  double w;
+  bool odd = false;
+  if (BEND) {
+    const double hx = __builtin_fma(x, irho, 1.0);
+    double b2;  // squared field across the velocity, times its length squared
+    if (F == F_NOFIELD) {
+      b2 = __builtin_fma(g.xp, g.xp, hx * hx);
+    } else {
+      const double by = re + irho;
+      const double byh = by * hx;
+      const double bxh = im * hx;
+      const double cr = __builtin_fma(im, g.yp, -by * g.xp);
+      b2 = __builtin_fma(cr, cr, __builtin_fma(byh, byh, bxh * bxh));
+    }
+    const double f = __builtin_fma(0.5, s2, hx) * rcp1(__builtin_fma(hx, hx, s2));
+    w = (b2 * ro) * f;  // the reciprocal in f comes last
+  } else {
+    double b2;
+    if (F == F_LEAD) {  // |B|^2 over B[1]^2
+      const double cr = __builtin_fma(y, g.yp, -x * g.xp);
+      b2 = __builtin_fma(cr, cr, __builtin_fma(x, x, y * y));
+    } else {
+      const double cr = __builtin_fma(im, g.yp, -re * g.xp);
+      b2 = __builtin_fma(cr, cr, __builtin_fma(re, re, im * im));
+    }
+    const double f = __builtin_fma(s2, __builtin_fma(s2, __builtin_fma(-0.5, s2, 0.5), -0.5), 1.0);
+    w = b2 * (f * ro);  // f does not wait for x
+    odd = s2 > 1e-4;
+    if (CHECKED && __builtin_amdgcn_ballot_w64(odd) != 0) {
+      const double fw = __builtin_fma(0.5, s2, 1.0) * rcp1(1.0 + s2);
+      w = odd ? b2 * (fw * ro) : w;
+    }
+  }
+  r.dp = __builtin_fma(-w, opd, d0);
+  const double e = REFRESH ? __builtin_fma(-(1.0 + r.dp), g.pn, 1.0) : w;
+  double pn = __builtin_fma(g.pn, __builtin_fma(e, e, e), g.pn);
+  const bool far = __builtin_fabs(w) > 2e-6;
+  if (CHECKED) {
+    if (__builtin_amdgcn_ballot_w64(far) != 0) pn = far ? fast_rcp(1.0 + r.dp) : pn;
+  } else {
+    bad |= __builtin_amdgcn_ballot_w64(odd | far);
+  }
+  if (!BEND && F == F_LEAD) {
+    const double kn = __builtin_fma(k.kb, pn, k.lo);  // lo pn, to a relative delta
+    g.xp = __builtin_fma(-x, kn, g.xp);
+    g.yp = __builtin_fma(y, kn, g.yp);
+  } else if (BEND && F == F_NOFIELD) {
+    const double u = __builtin_fma(-x, irho, d0);
+    g.xp = __builtin_fma(u, __builtin_fma(k.kli, pn, k.lo), g.xp);
+    r.ct = __builtin_fma(k.kli, x, r.ct);
+  } else {
+    const double kn = k.kl * pn;
+    double v = re;
+    if (BEND) {
+      const double u = __builtin_fma(-x, irho, d0);
+      v = __builtin_fma(-u, irho, re);
+      r.ct = __builtin_fma(k.kli, x, r.ct);
+    }
+    g.xp = __builtin_fma(-v, kn, g.xp);
+    g.yp = __builtin_fma(im, kn, g.yp);
+  }
   g.pn = pn;
 }
 #endif
@@ -689,14 +817,19 @@ __device__ __forceinline__ void mpole_exit(R6& r, cDevElem& h, cdouble* pool, cd
 // Slices of StrMPoleSymplectic4Pass.c:79-93 and BndMPoleSymplectic4Pass.c:97-111
 // for the P particles of a lane; U slices per loop iteration. pn = 1/(1+delta)
 // at the entry, nl1, nl2 = the drift lengths times it.
-template <bool BEND, int N, int P, int U>
+// The fast build joins the last drift of a slice and the first of the next
+// (delta and the momenta are the same in both): three drifts per slice
+// instead of four. The path length is still added drift by drift: the terms of
+// a magnet's slices are nearly equal and round alike against a ct a million
+// times larger, so known answers of the reference hold that rounding.
+template <bool BEND, int N, int F, int P, int U>
 __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int n, int nslice,
                                              const double* nl1, const double* nl2, double k1,
                                              double k2, double irho) {
-  const double ki1 = k1 * irho, ki2 = k2 * irho;
   double blo, alo;
   horner_addends<N>(a, b, n, blo, alo);
 #if ATX_STRICT
+  const double ki1 = k1 * irho, ki2 = k2 * irho;
   // U slices per iteration: a constant-count inner loop, fully unrolled
   // (the slices may hold wave-wide votes, which a runtime-count unroll
   // cannot duplicate), then the remaining slices one by one
@@ -729,57 +862,73 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
   }
   for (; m < nslice; m++) slice();
 #else
-  double nh1[P], nh2[P];  // delta is constant through the slices
+  if (nslice <= 0) return;
+  const Kick c1 = kick_of<BEND, N, F>(a, b, k1, irho, 0.0);
+  const Kick c2 = kick_of<BEND, N, F>(a, b, k2, irho, 0.0);
+  double nh1[P], nh2[P], nl12[P];  // delta is constant through the slices
 #pragma unroll
   for (int q = 0; q < P; q++) {
     const double h2 = 0.5 * fast_rcp(1.0 + r[q].dp);
     nh1[q] = nl1[q] * h2;
     nh2[q] = nl2[q] * h2;
+    nl12[q] = 2.0 * nl1[q];
   }
-  // U slices per iteration: a constant-count inner loop, fully unrolled
-  // (the slices may hold wave-wide votes, which a runtime-count unroll
-  // cannot duplicate), then the remaining slices one by one
-  auto slice = [&]() {
+  auto drift = [&](const double* nl, const double* nh) {
 #pragma unroll
-    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl1[q], nh1[q]);
-#pragma unroll
-    for (int q = 0; q < P; q++) {
-      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
-    }
-#pragma unroll
-    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl2[q], nh2[q]);
-#pragma unroll
-    for (int q = 0; q < P; q++) {
-      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2); else str_kick<N>(r[q], a, b, n, blo, alo, k2);
-    }
-#pragma unroll
-    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl2[q], nh2[q]);
-#pragma unroll
-    for (int q = 0; q < P; q++) {
-      if (BEND) bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1); else str_kick<N>(r[q], a, b, n, blo, alo, k1);
-    }
-#pragma unroll
-    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl1[q], nh1[q]);
+    for (int q = 0; q < P; q++) fastdrift_h(r[q], nl[q], nh[q]);
   };
-  int m = 0;
+  auto drift2 = [&]() {  // the last drift of a slice and the first of the next
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      fastdrift_h(r[q], nl12[q], nh1[q]);
+      r[q].ct = __builtin_fma(nh1[q], __builtin_fma(r[q].px, r[q].px, r[q].py * r[q].py), r[q].ct);
+    }
+  };
+  auto kicks = [&](const Kick& c) {
+#pragma unroll
+    for (int q = 0; q < P; q++) kick<BEND, N, F>(r[q], c, a, b, n, blo, alo, irho);
+  };
+  auto body = [&]() {  // a slice without its outer drifts
+    kicks(c1);
+    drift(nl2, nh2);
+    kicks(c2);
+    drift(nl2, nh2);
+    kicks(c1);
+  };
+  drift(nl1, nh1);
+  int m = 1;
   for (; m + U <= nslice; m += U) {
 #pragma unroll
-    for (int u = 0; u < U; u++) slice();
+    for (int u = 0; u < U; u++) {
+      body();
+      drift2();
+    }
   }
-  for (; m < nslice; m++) slice();
+  for (; m < nslice; m++) {
+    body();
+    drift2();
+  }
+  body();
+  drift(nl1, nh1);
+  if (F != F_GENERAL) {
+    const double rest = (2.0 * c1.lo + c2.lo) * (double)nslice;
+#pragma unroll
+    for (int q = 0; q < P; q++) kick_rest<BEND, N, F>(r[q], rest, irho);
+  }
 #endif
 }
 
 // Slices of StrMPoleSymplectic4RadPass.c:83-99 and
-// BndMPoleSymplectic4RadPass.c:98-112, likewise.
-template <bool BEND, int N, int P, int U>
+// BndMPoleSymplectic4RadPass.c:98-112, likewise. CHECKED, bad: rad_kick_ang.
+template <bool BEND, int N, int F, int P, int U, bool CHECKED>
 __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, int n, int nslice,
                                                  double l1, double l2, double k1, double k2,
-                                                 double irho, double radc, double rk1, double rk2) {
-  const double ki1 = k1 * irho, ki2 = k2 * irho;
+                                                 double irho, double radc, double rk1, double rk2,
+                                                 uint64_t& bad) {
   double blo, alo;
   horner_addends<N>(a, b, n, blo, alo);
 #if ATX_STRICT
+  const double ki1 = k1 * irho, ki2 = k2 * irho;
   double pn = 0.0;  // unused: the strict steps divide as the reference does
   // U slices per iteration: a constant-count inner loop, fully unrolled
   // (the slices may hold wave-wide votes, which a runtime-count unroll
@@ -816,44 +965,53 @@ __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, 
   }
   for (; m < nslice; m++) slice();
 #else
-  const double hl1 = 0.5 * l1, hl2 = 0.5 * l2;
+  if (nslice <= 0) return;
+  const Kick c1 = kick_of<BEND, N, F>(a, b, k1, irho, rk1);
+  const Kick c2 = kick_of<BEND, N, F>(a, b, k2, irho, rk2);
+  const double hl1 = 0.5 * l1, hl2 = 0.5 * l2, l12 = 2.0 * l1;
   Ang g[P];
 #pragma unroll
   for (int q = 0; q < P; q++) g[q] = to_angles(r[q]);  // one reciprocal per magnet
-  // U slices per iteration: a constant-count inner loop, fully unrolled
-  // (the slices may hold wave-wide votes, which a runtime-count unroll
-  // cannot duplicate), then the remaining slices one by one
-  auto slice = [&]() {
+  auto drift = [&](double len, double hlen) {
 #pragma unroll
-    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l1, hl1);
-#pragma unroll
-    for (int q = 0; q < P; q++) {
-      if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, irho, ki1, rk1);
-      else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, rk1);
-    }
-#pragma unroll
-    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l2, hl2);
-#pragma unroll
-    for (int q = 0; q < P; q++) {
-      if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k2, irho, ki2, rk2);
-      else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k2, rk2);
-    }
-#pragma unroll
-    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l2, hl2);
-#pragma unroll
-    for (int q = 0; q < P; q++) {
-      if (BEND) rad_bnd_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, irho, ki1, rk1);
-      else rad_str_kick_ang<N>(r[q], g[q], a, b, n, blo, alo, k1, rk1);
-    }
-#pragma unroll
-    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], l1, hl1);
+    for (int q = 0; q < P; q++) rad_drift_ang(r[q], g[q], len, hlen);
   };
-  int m = 0;
+  auto drift2 = [&]() {  // the last drift of a slice and the first of the next
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      rad_drift_ang(r[q], g[q], l12, hl1);
+      r[q].ct = __builtin_fma(hl1, g[q].s2, r[q].ct);
+    }
+  };
+  auto kicks = [&](const Kick& c) {
+#pragma unroll
+    for (int q = 0; q < P; q++)
+      rad_kick_ang<BEND, N, F, CHECKED, false>(r[q], g[q], c, a, b, n, blo, alo, irho, bad);
+  };
+  auto body = [&]() {  // a slice without its outer drifts
+    kicks(c1);
+    drift(l2, hl2);
+    kicks(c2);
+    drift(l2, hl2);
+#pragma unroll
+    for (int q = 0; q < P; q++)
+      rad_kick_ang<BEND, N, F, CHECKED, true>(r[q], g[q], c1, a, b, n, blo, alo, irho, bad);
+  };
+  drift(l1, hl1);
+  int m = 1;
   for (; m + U <= nslice; m += U) {
 #pragma unroll
-    for (int u = 0; u < U; u++) slice();
+    for (int u = 0; u < U; u++) {
+      body();
+      drift2();
+    }
   }
-  for (; m < nslice; m++) slice();
+  for (; m < nslice; m++) {
+    body();
+    drift2();
+  }
+  body();
+  drift(l1, hl1);
 #pragma unroll
   for (int q = 0; q < P; q++) from_angles(r[q], g[q]);
 #endif
@@ -886,7 +1044,7 @@ __device__ __forceinline__ void mpole(R6* r, cDevElem& h, cdouble* pool) {
     for (int q = 0; q < P; q++)
       r[q] = slices_ops<BEND, false>(r[q], a, b, n, pool + h.ops, h.nslice, pn[q], irho, 0.0);
   } else {
-    mpole_slices<BEND, N, P, U>(r, a, b, n, h.nslice, nl1, nl2, s[S_K1], s[S_K2], irho);
+    mpole_slices<BEND, N, F_GENERAL, P, U>(r, a, b, n, h.nslice, nl1, nl2, s[S_K1], s[S_K2], irho);
   }
 #pragma unroll
   for (int q = 0; q < P; q++) mpole_exit<BEND, LEAN>(r[q], h, pool, s);
@@ -912,8 +1070,9 @@ __device__ __forceinline__ void mpole_rad(R6* r, cDevElem& h, cdouble* pool) {
     for (int q = 0; q < P; q++)
       r[q] = slices_ops<BEND, true>(r[q], a, b, n, pool + h.ops, h.nslice, 0.0, irho, radc);
   } else {
-    mpole_rad_slices<BEND, N, P, U>(r, a, b, n, h.nslice, s[S_L1], s[S_L2], s[S_K1], s[S_K2], irho,
-                                    radc, s[S_RK1], s[S_RK2]);
+    uint64_t bad = 0;
+    mpole_rad_slices<BEND, N, F_GENERAL, P, U, true>(r, a, b, n, h.nslice, s[S_L1], s[S_L2], s[S_K1],
+                                                     s[S_K2], irho, radc, s[S_RK1], s[S_RK2], bad);
   }
 #pragma unroll
   for (int q = 0; q < P; q++) mpole_exit<BEND, LEAN>(r[q], h, pool, s);
@@ -1544,6 +1703,23 @@ __device__ __forceinline__ R6 generic_element(const R6& r, cDevElem& h, cdouble*
   }
 }
 
+// at.c:115-139 predicate: any coordinate not finite, or |r_n| > 1 for n < 5.
+// Without short circuits: six compares and mask logic, no branch.
+__device__ __forceinline__ bool is_lost(const R6& r) {
+  const bool ok = (__builtin_fabs(r.x) <= 1.0) & (__builtin_fabs(r.px) <= 1.0) &
+                  (__builtin_fabs(r.y) <= 1.0) & (__builtin_fabs(r.py) <= 1.0) &
+                  (__builtin_fabs(r.dp) <= 1.0) & (__builtin_fabs(r.ct) < __builtin_inf());
+  return !ok;
+}
+
+// The same after a drift of a particle that passed the test before it:
+// px, py and delta are unchanged.
+__device__ __forceinline__ bool is_lost_drift(const R6& r) {
+  const bool ok = (__builtin_fabs(r.x) <= 1.0) & (__builtin_fabs(r.y) <= 1.0) &
+                  (__builtin_fabs(r.ct) < __builtin_inf());
+  return !ok;
+}
+
 // An edge of a bend by its header.
 __device__ __noinline__ R6 edge_call(R6 r, cDevElem* hp, cdouble* poolp, int exit) {
   cDevElem& h = *uniform(hp);
@@ -1558,10 +1734,10 @@ __device__ __noinline__ R6 edge_call(R6 r, cDevElem* hp, cdouble* poolp, int exi
 }
 
 // A thick multipole by its record; the misalignment is applied around it by
-// the caller.
-template <bool BEND, bool RAD, int N, int P, int U>
+// the caller. CHECKED, bad: rad_kick_ang.
+template <bool BEND, bool RAD, int N, int F, int P, int U, bool CHECKED>
 __device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flags, cDevElem* h,
-                                         cdouble* pool) {
+                                         cdouble* pool, uint64_t& bad) {
   cdouble* a = c + OM_POLY;
   cdouble* b = a + N + 1;
   const double irho = BEND ? c[OM_IRHO] : 0.0;
@@ -1577,8 +1753,9 @@ __device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flag
     }
   }
   if (RAD) {
-    mpole_rad_slices<BEND, N, P, U>(r, a, b, N, nslice, c[OM_L1], c[OM_L2], c[OM_K1], c[OM_K2],
-                                    irho, c[OM_RADC], c[OM_RK1], c[OM_RK2]);
+    mpole_rad_slices<BEND, N, F, P, U, CHECKED>(r, a, b, N, nslice, c[OM_L1], c[OM_L2], c[OM_K1],
+                                                c[OM_K2], irho, c[OM_RADC], c[OM_RK1], c[OM_RK2],
+                                                bad);
   } else {
     double nl1[P], nl2[P];
 #pragma unroll
@@ -1587,7 +1764,7 @@ __device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flag
       nl1[q] = c[OM_L1] * pn;
       nl2[q] = c[OM_L2] * pn;
     }
-    mpole_slices<BEND, N, P, U>(r, a, b, N, nslice, nl1, nl2, c[OM_K1], c[OM_K2], irho);
+    mpole_slices<BEND, N, F, P, U>(r, a, b, N, nslice, nl1, nl2, c[OM_K1], c[OM_K2], irho);
   }
   if (BEND) {
 #pragma unroll
@@ -1614,29 +1791,154 @@ __device__ __forceinline__ void thin_op(R6& r, cdouble* c) {
   r.ct -= bax * r.x - bay * r.y;
 }
 
+__device__ __forceinline__ bool is_finite(const R6& r) {
+  const double inf = __builtin_inf();
+  return (__builtin_fabs(r.x) < inf) & (__builtin_fabs(r.px) < inf) & (__builtin_fabs(r.y) < inf) &
+         (__builtin_fabs(r.py) < inf) & (__builtin_fabs(r.dp) < inf) & (__builtin_fabs(r.ct) < inf);
+}
+
+// Roll of both planes by the angle of (c, s): the 6x6 product of mul_r
+// without its zeros, in its order of summation.
+__device__ __forceinline__ void roll(R6& r, double c, double s) {
+  const double x = r.x, px = r.px;
+#if ATX_STRICT
+  r.x = c * x + s * r.y;
+  r.px = c * px + s * r.py;
+  r.y = -s * x + c * r.y;
+  r.py = -s * px + c * r.py;
+#else
+  r.x = __builtin_fma(s, r.y, c * x);
+  r.px = __builtin_fma(s, r.py, c * px);
+  r.y = __builtin_fma(c, r.y, -s * x);
+  r.py = __builtin_fma(c, r.py, -s * px);
+#endif
+}
+
+// The element of a record other than its markers and drift, for the P
+// particles of a lane. CHECKED, bad: rad_kick_ang.
+template <int P, int U, bool CHECKED>
+__device__ __forceinline__ void run_op(R6* r, int op, cLatOp* rec, cDevElem* h, cdouble* pool,
+                                       int nturn, uint64_t& bad) {
+  cdouble* c = rec->c;
+  if (op & OPF_XF) {
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      r[q].x += c[OM_XF];
+      r[q].px += c[OM_XF + 1];
+      r[q].y += c[OM_XF + 2];
+      r[q].py += c[OM_XF + 3];
+      roll(r[q], c[OM_XF + 4], c[OM_XF + 5]);
+    }
+  }
+  const int nslice = rec->nslice;
+#define ATX_MPOLE(BEND, RAD, N, F) \
+  mpole_op<BEND, RAD, N, F, P, U, CHECKED>(r, c, nslice, op, h, pool, bad)
+  switch (op & 0xff) {
+#if ATX_STRICT  // all coefficients, whatever the form
+    case OP_STR1: case OP_STR1L: ATX_MPOLE(false, false, 1, F_GENERAL); break;
+    case OP_STR2: case OP_STR2L: case OP_STR2D: ATX_MPOLE(false, false, 2, F_GENERAL); break;
+    case OP_STR3: case OP_STR3L: ATX_MPOLE(false, false, 3, F_GENERAL); break;
+    case OP_BND1: case OP_BND1L: case OP_BND0: ATX_MPOLE(true, false, 1, F_GENERAL); break;
+    case OP_STRRAD1: case OP_STRRAD1L: ATX_MPOLE(false, true, 1, F_GENERAL); break;
+    case OP_BNDRAD1: case OP_BNDRAD1L: case OP_BNDRAD0: ATX_MPOLE(true, true, 1, F_GENERAL); break;
+#else
+    case OP_STR1: ATX_MPOLE(false, false, 1, F_GENERAL); break;
+    case OP_STR1L: ATX_MPOLE(false, false, 1, F_LEAD); break;
+    case OP_STR2: ATX_MPOLE(false, false, 2, F_GENERAL); break;
+    case OP_STR2L: ATX_MPOLE(false, false, 2, F_LEAD); break;
+    case OP_STR2D: ATX_MPOLE(false, false, 2, F_LEAD0); break;
+    case OP_STR3: ATX_MPOLE(false, false, 3, F_GENERAL); break;
+    case OP_STR3L: ATX_MPOLE(false, false, 3, F_LEAD); break;
+    case OP_BND1: ATX_MPOLE(true, false, 1, F_GENERAL); break;
+    case OP_BND1L: ATX_MPOLE(true, false, 1, F_LEAD); break;
+    case OP_BND0: ATX_MPOLE(true, false, 1, F_NOFIELD); break;
+    case OP_STRRAD1: ATX_MPOLE(false, true, 1, F_GENERAL); break;
+    case OP_STRRAD1L: ATX_MPOLE(false, true, 1, F_LEAD); break;
+    case OP_BNDRAD1: ATX_MPOLE(true, true, 1, F_GENERAL); break;
+    case OP_BNDRAD1L: ATX_MPOLE(true, true, 1, F_LEAD); break;
+    case OP_BNDRAD0: ATX_MPOLE(true, true, 1, F_NOFIELD); break;
+#endif
+    case OP_THIN2:
+#pragma unroll
+      for (int q = 0; q < P; q++) thin_op<2>(r[q], c);
+      break;
+    case OP_THIN3:
+#pragma unroll
+      for (int q = 0; q < P; q++) thin_op<3>(r[q], c);
+      break;
+    case OP_APERTURE:  // AperturePass.c:9-26
+#pragma unroll
+      for (int q = 0; q < P; q++) rect_ap(r[q], c);
+      break;
+    case OP_CORR:
+#pragma unroll
+      for (int q = 0; q < P; q++) {
+        if (op & OPF_THICK) {
+          const double pn = rcp_opd(r[q]);
+          corrector_map(r[q], c[OC_XK], c[OC_YK], c[OC_Q0], c[OC_LEN] * pn, pn);
+        } else {
+          r[q].px += c[OC_XK];
+          r[q].py += c[OC_YK];
+        }
+      }
+      break;
+    default:
+#pragma unroll
+      for (int q = 0; q < P; q++) r[q] = generic_element<U>(r[q], *h, pool, nturn);
+      break;
+  }
+#undef ATX_MPOLE
+  if (op & OPF_XF) {
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+#if ATX_STRICT
+      // a coordinate that is not finite spreads through the zeros of the
+      // 6x6 product, as in the reference: the wave then takes the product
+      // (the fast build runs the whole element again, op_call)
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(is_lost(r[q])) != 0 && (h->flags & F_R2), 0))
+        r[q] = mul_r_v(r[q], pool + h->r2);
+      else
+#endif
+        roll(r[q], c[OM_XF + 6], c[OM_XF + 7]);
+      r[q].x += c[OM_XF + 8];
+      r[q].px += c[OM_XF + 9];
+      r[q].y += c[OM_XF + 10];
+      r[q].py += c[OM_XF + 11];
+    }
+  }
+}
+
+#if !ATX_STRICT
+// The same out of line for one particle, with the checks in the kicks. A
+// result that is not finite is computed again from the header: there a
+// coordinate that is not finite spreads through the zeros of the misalignment
+// matrices and of the multipole coefficients, as in the reference.
+template <int U>
+__device__ __noinline__ R6 op_call(R6 r, const LatOp* recp, cDevElem* hp, cdouble* poolp, int nturnp) {
+  cLatOp* rec = uniform((cLatOp*)recp);
+  cDevElem* h = uniform(hp);
+  cdouble* pool = uniform(poolp);
+  const int nturn = __builtin_amdgcn_readfirstlane(nturnp);
+  R6 v = r;
+  uint64_t bad = 0;
+  run_op<1, 1, true>(&v, rec->op, rec, h, pool, nturn, bad);
+  if (rec->op & OPF_MPOLE) {
+    const bool inf = !is_finite(v);
+    if (__builtin_amdgcn_ballot_w64(inf) != 0) {
+      const R6 g = generic_element<U>(r, *h, pool, nturn);
+      v = inf ? g : v;
+    }
+  }
+  return v;
+}
+#endif
+
 // The same out of line, for the few elements of a call that are not run by
 // records.
 template <int U>
 __device__ __noinline__ R6 header_call(R6 r, cDevElem* hp, cdouble* poolp, int nturnp) {
   return generic_element<U>(r, *uniform(hp), uniform(poolp),
                             __builtin_amdgcn_readfirstlane(nturnp));
-}
-
-// at.c:115-139 predicate: any coordinate not finite, or |r_n| > 1 for n < 5.
-// Without short circuits: six compares and mask logic, no branch.
-__device__ __forceinline__ bool is_lost(const R6& r) {
-  const bool ok = (__builtin_fabs(r.x) <= 1.0) & (__builtin_fabs(r.px) <= 1.0) &
-                  (__builtin_fabs(r.y) <= 1.0) & (__builtin_fabs(r.py) <= 1.0) &
-                  (__builtin_fabs(r.dp) <= 1.0) & (__builtin_fabs(r.ct) < __builtin_inf());
-  return !ok;
-}
-
-// The same after a drift of a particle that passed the test before it:
-// px, py and delta are unchanged.
-__device__ __forceinline__ bool is_lost_drift(const R6& r) {
-  const bool ok = (__builtin_fabs(r.x) <= 1.0) & (__builtin_fabs(r.y) <= 1.0) &
-                  (__builtin_fabs(r.ct) < __builtin_inf());
-  return !ok;
 }
 
 __device__ __forceinline__ void store6(double* base, int64_t cs, const R6& r) {
@@ -1692,23 +1994,6 @@ struct OpHead {
 
 __device__ __forceinline__ OpHead op_head(cLatOp* p) {
   return OpHead{p->op, p->last, p->len, ((cint*)p)[16], ((cint*)p)[32]};
-}
-
-// Roll of both planes by the angle of (c, s): the 6x6 product of mul_r
-// without its zeros, in its order of summation.
-__device__ __forceinline__ void roll(R6& r, double c, double s) {
-  const double x = r.x, px = r.px;
-#if ATX_STRICT
-  r.x = c * x + s * r.y;
-  r.px = c * px + s * r.py;
-  r.y = -s * x + c * r.y;
-  r.py = -s * px + c * r.py;
-#else
-  r.x = __builtin_fma(s, r.y, c * x);
-  r.px = __builtin_fma(s, r.py, c * px);
-  r.y = __builtin_fma(c, r.y, -s * x);
-  r.py = __builtin_fma(c, r.py, -s * px);
-#endif
 }
 
 // A particle with its lane's state: what the loss handling changes.
@@ -1788,6 +2073,7 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   cDevElem* elems = (cDevElem*)I.elems;
   cdouble* pool = (cdouble*)I.pool;
   cLatOp* ops = (cLatOp*)I.ops;
+  cint* opof = (cint*)I.opof;
   const int p[2] = {p0, p1};
   R6 r[P];
   int fl[P];
@@ -1817,8 +2103,7 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   uint64_t alive[P];
 #pragma unroll
   for (int q = 0; q < P; q++) alive[q] = __builtin_amdgcn_ballot_w64((fl[q] & L_ALIVE) != 0);
-  auto lose = [&](int q, bool lost, int e) {
-    const uint64_t bad = __builtin_amdgcn_ballot_w64(lost) & alive[q];
+  auto lose_mask = [&](int q, uint64_t bad, int e) {
     if (__builtin_expect(bad != 0, 0)) {
       Lane l{r[q], fl[q]};
       loss_call(&l, inst, p[q], (int)((bad >> (threadIdx.x & 63)) & 1), nturn, e);
@@ -1827,14 +2112,24 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
       alive[q] = __builtin_amdgcn_ballot_w64((fl[q] & L_ALIVE) != 0);
     }
   };
-  // One element by its header, with its refpt copy and loss test. A NaN
-  // input is skipped by the first element and lost at its test.
+  auto lose = [&](int q, bool lost, int e) {
+    lose_mask(q, __builtin_amdgcn_ballot_w64(lost) & alive[q], e);
+  };
+  // One element outside the loop over the records, with its refpt copy and loss
+  // test. A NaN input is skipped by the first element and lost at its test.
   auto by_header = [&](int e, bool entry) {
     if (REFS) copy_refs(e);
 #pragma unroll
     for (int q = 0; q < P; q++) {
       if (entry) lose(q, __builtin_isnan(r[q].x), e);
-      r[q] = header_call<U>(r[q], &elems[e], pool, nturn);
+#if !ATX_STRICT
+      // in the record's form, so that a turn split into calls rounds alike
+      cLatOp* rec = ops + opof[e];
+      if (rec->last == e && (rec->op & OPF_MPOLE))
+        r[q] = op_call<U>(r[q], (const LatOp*)rec, &elems[e], pool, nturn);
+      else
+#endif
+        r[q] = header_call<U>(r[q], &elems[e], pool, nturn);
       if (check) lose(q, is_lost(r[q]), e);
     }
   };
@@ -1852,7 +2147,6 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   // (whose input has not passed a loss test yet) and the elements of a
   // record that a partial turn starts or ends in run by their headers,
   // before and after the records.
-  cint* opof = (cint*)I.opof;
   const int o1 = opof[e1];
   int o0 = e0 < e1 ? 0 : o1;
   int e = e0;
@@ -1860,6 +2154,11 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
     o0 = opof[e0] + 1;
     for (const int stop = min(ops[o0].first, e1); e < stop; e++) by_header(e, e == e0);
   }
+#if !ATX_STRICT
+  // once a radiating magnet had to be run again with the checks in its kicks,
+  // the wave runs them with the checks for the rest of the turn
+  bool slow = false;
+#endif
   cLatOp* rec = ops + o0;
   cLatOp* const end = ops + max(o0, o1);
   OpHead nxt = op_head(rec);
@@ -1882,71 +2181,32 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
     }
     if (kind == OP_NONE) continue;
     if (REFS) copy_refs(cur.last);
-    cdouble* c = rec->c;
     cDevElem* h = &elems[cur.last];
-    if (cur.op & OPF_XF) {
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        r[q].x += c[OM_XF];
-        r[q].px += c[OM_XF + 1];
-        r[q].y += c[OM_XF + 2];
-        r[q].py += c[OM_XF + 3];
-        roll(r[q], c[OM_XF + 4], c[OM_XF + 5]);
-      }
-    }
-    switch (kind) {
-      case OP_STR1: mpole_op<false, false, 1, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
-      case OP_STR2: mpole_op<false, false, 2, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
-      case OP_STR3: mpole_op<false, false, 3, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
-      case OP_BND1: mpole_op<true, false, 1, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
-      case OP_STRRAD1: mpole_op<false, true, 1, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
-      case OP_BNDRAD1: mpole_op<true, true, 1, P, U>(r, c, rec->nslice, cur.op, h, pool); break;
-      case OP_THIN2:
-#pragma unroll
-        for (int q = 0; q < P; q++) thin_op<2>(r[q], c);
-        break;
-      case OP_THIN3:
-#pragma unroll
-        for (int q = 0; q < P; q++) thin_op<3>(r[q], c);
-        break;
-      case OP_APERTURE:  // AperturePass.c:9-26
-#pragma unroll
-        for (int q = 0; q < P; q++) rect_ap(r[q], c);
-        break;
-      case OP_CORR:
-#pragma unroll
-        for (int q = 0; q < P; q++) {
-          if (cur.op & OPF_THICK) {
-            const double pn = rcp_opd(r[q]);
-            corrector_map(r[q], c[OC_XK], c[OC_YK], c[OC_Q0], c[OC_LEN] * pn, pn);
-          } else {
-            r[q].px += c[OC_XK];
-            r[q].py += c[OC_YK];
-          }
-        }
-        break;
-      default:
-#pragma unroll
-        for (int q = 0; q < P; q++) r[q] = generic_element<U>(r[q], *h, pool, nturn);
-        break;
-    }
-    if (cur.op & OPF_XF) {
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        // a coordinate that is not finite spreads through the zeros of the
-        // 6x6 product, as in the reference: the wave then takes the product
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(is_lost(r[q])) != 0 && (h->flags & F_R2), 0))
-          r[q] = mul_r_v(r[q], pool + h->r2);
-        else
-          roll(r[q], c[OM_XF + 6], c[OM_XF + 7]);
-        r[q].x += c[OM_XF + 8];
-        r[q].px += c[OM_XF + 9];
-        r[q].y += c[OM_XF + 10];
-        r[q].py += c[OM_XF + 11];
-      }
-    }
+    uint64_t bad = 0;
+#if ATX_STRICT
+    run_op<P, U, true>(r, cur.op, rec, h, pool, nturn, bad);
 #pragma unroll
     for (int q = 0; q < P; q++) lose(q, is_lost(r[q]), cur.last);
+#else
+    bool again = slow && (cur.op & OPF_RAD);
+    R6 r0[P];
+#pragma unroll
+    for (int q = 0; q < P; q++) r0[q] = r[q];
+    if (__builtin_expect(!again, 1)) {
+      run_op<P, U, false>(r, cur.op, rec, h, pool, nturn, bad);
+      again = bad != 0;
+      slow |= again;
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+      bad = __builtin_amdgcn_ballot_w64(is_lost(r[q])) & alive[q];
+      if (__builtin_expect(again || (bad != 0 && (cur.op & OPF_MPOLE)), 0)) {
+        r[q] = op_call<U>(r0[q], (const LatOp*)rec, h, pool, nturn);
+        bad = __builtin_amdgcn_ballot_w64(is_lost(r[q])) & alive[q];
+      }
+      lose_mask(q, bad, cur.last);
+    }
+#endif
   }
   for (e = max(e, ops[o1].first); e < e1; e++) by_header(e, false);
   if (REFS) copy_refs(I.nelem);
