@@ -814,6 +814,15 @@ __device__ __forceinline__ void mpole_exit(R6& r, cDevElem& h, cdouble* pool, cd
   }
 }
 
+// Called once all constants of an element have been asked for (its arguments,
+// held here so that they have arrived): the loop over the records then asks for
+// the next record (run_turn).
+struct NotAhead {
+  template <class... T>
+  __device__ __forceinline__ void operator()(T...) const {}
+};
+__device__ __forceinline__ void hold(double v) { asm volatile("" ::"s"(v)); }
+
 // Slices of StrMPoleSymplectic4Pass.c:79-93 and BndMPoleSymplectic4Pass.c:97-111
 // for the P particles of a lane; U slices per loop iteration. pn = 1/(1+delta)
 // at the entry, nl1, nl2 = the drift lengths times it.
@@ -822,12 +831,18 @@ __device__ __forceinline__ void mpole_exit(R6& r, cDevElem& h, cdouble* pool, cd
 // instead of four. The path length is still added drift by drift: the terms of
 // a magnet's slices are nearly equal and round alike against a ct a million
 // times larger, so known answers of the reference hold that rounding.
-template <bool BEND, int N, int F, int P, int U>
+template <bool BEND, int N, int F, int P, int U, class Ahead>
 __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int n, int nslice,
                                              const double* nl1, const double* nl2, double k1,
-                                             double k2, double irho) {
+                                             double k2, double irho, const Ahead& ahead) {
   double blo, alo;
   horner_addends<N>(a, b, n, blo, alo);
+  if (F == F_GENERAL && N == 3) ahead(k1, k2, a[3], b[3], a[2], b[2], a[1], b[1], a[0], b[0]);
+  else if (F == F_GENERAL && N == 2) ahead(k1, k2, a[2], b[2], a[1], b[1], a[0], b[0]);
+  else if (F == F_GENERAL && N == 1) ahead(k1, k2, a[1], b[1], a[0], b[0]);
+  else if (F == F_LEAD0) ahead(k1, k2, b[N], a[0], b[0]);
+  else if (F == F_LEAD) ahead(k1, k2, b[N]);
+  else ahead(k1, k2);
 #if ATX_STRICT
   const double ki1 = k1 * irho, ki2 = k2 * irho;
   // U slices per iteration: a constant-count inner loop, fully unrolled
@@ -920,13 +935,17 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
 
 // Slices of StrMPoleSymplectic4RadPass.c:83-99 and
 // BndMPoleSymplectic4RadPass.c:98-112, likewise. CHECKED, bad: rad_kick_ang.
-template <bool BEND, int N, int F, int P, int U, bool CHECKED>
+template <bool BEND, int N, int F, int P, int U, bool CHECKED, class Ahead>
 __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, int n, int nslice,
                                                  double l1, double l2, double k1, double k2,
                                                  double irho, double radc, double rk1, double rk2,
-                                                 uint64_t& bad) {
+                                                 uint64_t& bad, const Ahead& ahead) {
   double blo, alo;
   horner_addends<N>(a, b, n, blo, alo);
+  const double rk = ATX_STRICT ? radc : rk1;
+  if (F == F_GENERAL && N == 1) ahead(l1, l2, k1, k2, rk, rk2, a[1], b[1], a[0], b[0]);
+  else if (F == F_LEAD) ahead(l1, l2, k1, k2, rk, rk2, b[N]);
+  else ahead(l1, l2, k1, k2, rk, rk2);
 #if ATX_STRICT
   const double ki1 = k1 * irho, ki2 = k2 * irho;
   double pn = 0.0;  // unused: the strict steps divide as the reference does
@@ -1044,7 +1063,8 @@ __device__ __forceinline__ void mpole(R6* r, cDevElem& h, cdouble* pool) {
     for (int q = 0; q < P; q++)
       r[q] = slices_ops<BEND, false>(r[q], a, b, n, pool + h.ops, h.nslice, pn[q], irho, 0.0);
   } else {
-    mpole_slices<BEND, N, F_GENERAL, P, U>(r, a, b, n, h.nslice, nl1, nl2, s[S_K1], s[S_K2], irho);
+    mpole_slices<BEND, N, F_GENERAL, P, U>(r, a, b, n, h.nslice, nl1, nl2, s[S_K1], s[S_K2], irho,
+                                          NotAhead());
   }
 #pragma unroll
   for (int q = 0; q < P; q++) mpole_exit<BEND, LEAN>(r[q], h, pool, s);
@@ -1072,7 +1092,8 @@ __device__ __forceinline__ void mpole_rad(R6* r, cDevElem& h, cdouble* pool) {
   } else {
     uint64_t bad = 0;
     mpole_rad_slices<BEND, N, F_GENERAL, P, U, true>(r, a, b, n, h.nslice, s[S_L1], s[S_L2], s[S_K1],
-                                                     s[S_K2], irho, radc, s[S_RK1], s[S_RK2], bad);
+                                                     s[S_K2], irho, radc, s[S_RK1], s[S_RK2], bad,
+                                                     NotAhead());
   }
 #pragma unroll
   for (int q = 0; q < P; q++) mpole_exit<BEND, LEAN>(r[q], h, pool, s);
@@ -1735,9 +1756,9 @@ __device__ __noinline__ R6 edge_call(R6 r, cDevElem* hp, cdouble* poolp, int exi
 
 // A thick multipole by its record; the misalignment is applied around it by
 // the caller. CHECKED, bad: rad_kick_ang.
-template <bool BEND, bool RAD, int N, int F, int P, int U, bool CHECKED>
+template <bool BEND, bool RAD, int N, int F, int P, int U, bool CHECKED, class Ahead>
 __device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flags, cDevElem* h,
-                                         cdouble* pool, uint64_t& bad) {
+                                         cdouble* pool, uint64_t& bad, const Ahead& ahead) {
   cdouble* a = c + OM_POLY;
   cdouble* b = a + N + 1;
   const double irho = BEND ? c[OM_IRHO] : 0.0;
@@ -1755,7 +1776,7 @@ __device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flag
   if (RAD) {
     mpole_rad_slices<BEND, N, F, P, U, CHECKED>(r, a, b, N, nslice, c[OM_L1], c[OM_L2], c[OM_K1],
                                                 c[OM_K2], irho, c[OM_RADC], c[OM_RK1], c[OM_RK2],
-                                                bad);
+                                                bad, ahead);
   } else {
     double nl1[P], nl2[P];
 #pragma unroll
@@ -1764,7 +1785,7 @@ __device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flag
       nl1[q] = c[OM_L1] * pn;
       nl2[q] = c[OM_L2] * pn;
     }
-    mpole_slices<BEND, N, F, P, U>(r, a, b, N, nslice, nl1, nl2, c[OM_K1], c[OM_K2], irho);
+    mpole_slices<BEND, N, F, P, U>(r, a, b, N, nslice, nl1, nl2, c[OM_K1], c[OM_K2], irho, ahead);
   }
   if (BEND) {
 #pragma unroll
@@ -1815,10 +1836,10 @@ __device__ __forceinline__ void roll(R6& r, double c, double s) {
 }
 
 // The element of a record other than its markers and drift, for the P
-// particles of a lane. CHECKED, bad: rad_kick_ang.
-template <int P, int U, bool CHECKED>
+// particles of a lane. CHECKED, bad: rad_kick_ang; ahead: NotAhead.
+template <int P, int U, bool CHECKED, class Ahead>
 __device__ __forceinline__ void run_op(R6* r, int op, cLatOp* rec, cDevElem* h, cdouble* pool,
-                                       int nturn, uint64_t& bad) {
+                                       int nturn, uint64_t& bad, const Ahead& ahead) {
   cdouble* c = rec->c;
   if (op & OPF_XF) {
 #pragma unroll
@@ -1832,7 +1853,7 @@ __device__ __forceinline__ void run_op(R6* r, int op, cLatOp* rec, cDevElem* h, 
   }
   const int nslice = rec->nslice;
 #define ATX_MPOLE(BEND, RAD, N, F) \
-  mpole_op<BEND, RAD, N, F, P, U, CHECKED>(r, c, nslice, op, h, pool, bad)
+  mpole_op<BEND, RAD, N, F, P, U, CHECKED>(r, c, nslice, op, h, pool, bad, ahead)
   switch (op & 0xff) {
 #if ATX_STRICT  // all coefficients, whatever the form
     case OP_STR1: case OP_STR1L: ATX_MPOLE(false, false, 1, F_GENERAL); break;
@@ -1861,16 +1882,20 @@ __device__ __forceinline__ void run_op(R6* r, int op, cLatOp* rec, cDevElem* h, 
     case OP_THIN2:
 #pragma unroll
       for (int q = 0; q < P; q++) thin_op<2>(r[q], c);
+      ahead();
       break;
     case OP_THIN3:
 #pragma unroll
       for (int q = 0; q < P; q++) thin_op<3>(r[q], c);
+      ahead();
       break;
     case OP_APERTURE:  // AperturePass.c:9-26
 #pragma unroll
       for (int q = 0; q < P; q++) rect_ap(r[q], c);
+      ahead();
       break;
     case OP_CORR:
+      ahead(c[OC_XK], c[OC_YK], c[OC_LEN], c[OC_Q0]);
 #pragma unroll
       for (int q = 0; q < P; q++) {
         if (op & OPF_THICK) {
@@ -1883,6 +1908,7 @@ __device__ __forceinline__ void run_op(R6* r, int op, cLatOp* rec, cDevElem* h, 
       }
       break;
     default:
+      ahead();
 #pragma unroll
       for (int q = 0; q < P; q++) r[q] = generic_element<U>(r[q], *h, pool, nturn);
       break;
@@ -1921,7 +1947,7 @@ __device__ __noinline__ R6 op_call(R6 r, const LatOp* recp, cDevElem* hp, cdoubl
   const int nturn = __builtin_amdgcn_readfirstlane(nturnp);
   R6 v = r;
   uint64_t bad = 0;
-  run_op<1, 1, true>(&v, rec->op, rec, h, pool, nturn, bad);
+  run_op<1, 1, true>(&v, rec->op, rec, h, pool, nturn, bad, NotAhead());
   if (rec->op & OPF_MPOLE) {
     const bool inf = !is_finite(v);
     if (__builtin_amdgcn_ballot_w64(inf) != 0) {
@@ -2165,7 +2191,15 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   for (; rec != end; rec++) {
     const OpHead cur = nxt;
     asm volatile("" ::"s"(cur.line1), "s"(cur.line2));
-    nxt = op_head(rec + 1);
+    // The next record's head, asked for when this record's constants have
+    // arrived: scalar loads return in any order, so that waiting for one waits
+    // for all, and a constant asked for after the head would wait for the L2.
+    auto ahead = [&](auto... c) {
+      (hold(c), ...);
+      cLatOp* p = rec + 1;
+      asm volatile("" : "+s"(p));
+      nxt = op_head(p);
+    };
     const int kind = cur.op & 0xff;
     if (REFS) {  // markers change nothing: only their copies
       const int ndo = (kind != OP_NONE ? 1 : 0) + ((cur.op & OPF_DRIFT) ? 1 : 0);
@@ -2179,12 +2213,15 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
 #pragma unroll
       for (int q = 0; q < P; q++) lose(q, is_lost_drift(r[q]), at);
     }
-    if (kind == OP_NONE) continue;
+    if (kind == OP_NONE) {
+      ahead();
+      continue;
+    }
     if (REFS) copy_refs(cur.last);
     cDevElem* h = &elems[cur.last];
     uint64_t bad = 0;
 #if ATX_STRICT
-    run_op<P, U, true>(r, cur.op, rec, h, pool, nturn, bad);
+    run_op<P, U, true>(r, cur.op, rec, h, pool, nturn, bad, ahead);
 #pragma unroll
     for (int q = 0; q < P; q++) lose(q, is_lost(r[q]), cur.last);
 #else
@@ -2192,8 +2229,10 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
     R6 r0[P];
 #pragma unroll
     for (int q = 0; q < P; q++) r0[q] = r[q];
-    if (__builtin_expect(!again, 1)) {
-      run_op<P, U, false>(r, cur.op, rec, h, pool, nturn, bad);
+    if (__builtin_expect(again, 0)) {
+      ahead();
+    } else {
+      run_op<P, U, false>(r, cur.op, rec, h, pool, nturn, bad, ahead);
       again = bad != 0;
       slow |= again;
     }
