@@ -191,7 +191,7 @@ struct Instance {
   const double* pool;
   const LatOp* ops;         // program records
   const int32_t* opof;      // record of each element
-  const int32_t* slots;     // 2*(nelem+1): refpt copy rank per element, first turn then later turns
+  const int32_t* slots;     // 2*(nelem/32+1): a bit per element with a copy, first turn then later turns
   double* r;                // particle state, updated in place
   double* rout;             // refpt copies (6, N, R, T) F-order
   uint8_t* lost_flag;

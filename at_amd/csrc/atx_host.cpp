@@ -776,6 +776,18 @@ int turn_slots(const uint32_t* refpts, int nref, int start, int end, int nelem, 
   return k;
 }
 
+// The copies of the two tables of ranks (first turn, later turns) as the kernel
+// reads them: one bit per element, nelem/32 + 1 words per table.
+size_t ref_words(int nelem) { return 2 * ((size_t)nelem / 32 + 1); }
+void ref_bits(const int32_t* slot, int nelem, int32_t* words) {
+  const size_t half = ref_words(nelem) / 2;
+  std::memset(words, 0, 2 * half * sizeof(int32_t));
+  for (int k = 0; k < 2; k++)
+    for (int e = 0; e <= nelem; e++)
+      if (slot[k * (size_t)(nelem + 1) + e] >= 0)
+        words[k * half + e / 32] |= (int32_t)(1u << (e % 32));
+}
+
 #define HIPCHK(x)                                                                         \
   do {                                                                                    \
     hipError_t e_ = (x);                                                                  \
@@ -1153,10 +1165,12 @@ int launch_repacked(std::vector<Instance>& insts, const std::vector<const std::v
 int single_instance(atx_lattice* lat, double* d_r, int64_t pstride, int64_t cstride, uint32_t np,
                     int nturns, const uint32_t* refpts, uint32_t nref, int turn0, int start, int end,
                     double* d_rout, uint8_t* d_lf, uint32_t* d_lt, uint32_t* d_le, double* d_lc,
-                    int losses, bool elempass, int32_t* slots, Instance& inst) {
+                    int losses, bool elempass, int32_t* bits, Instance& inst) {
   const int nelem = (int)lat->elems.size();
-  const int n_first = turn_slots(refpts, (int)nref, start, end, nelem, slots);
-  const int n_std = turn_slots(refpts, (int)nref, 0, end, nelem, slots + nelem + 1);
+  std::vector<int32_t> ranks(2 * (size_t)(nelem + 1));
+  const int n_first = turn_slots(refpts, (int)nref, start, end, nelem, ranks.data());
+  const int n_std = turn_slots(refpts, (int)nref, 0, end, nelem, ranks.data() + nelem + 1);
+  ref_bits(ranks.data(), nelem, bits);
   if ((n_first > 0 || n_std > 0) && !d_rout) return fail(ATX_E_VALUE, "r_out is NULL but refpts request copies");
   if (losses && (!d_lf || !d_lt || !d_le || !d_lc)) return fail(ATX_E_VALUE, "loss arrays are NULL");
   std::memset(&inst, 0, sizeof(inst));
@@ -1192,7 +1206,7 @@ int track_device(atx_lattice* lat, double* d_r, int64_t pstride, int64_t cstride
                  double* d_rout, uint8_t* d_lf, uint32_t* d_lt, uint32_t* d_le, double* d_lc,
                  int losses, bool elempass, hipStream_t stream, bool strict, bool repack = false) {
   const int nelem = (int)lat->elems.size();
-  std::vector<std::vector<int32_t>> slots(1, std::vector<int32_t>(2 * (size_t)(nelem + 1)));
+  std::vector<std::vector<int32_t>> slots(1, std::vector<int32_t>(ref_words(nelem)));
   std::vector<Instance> insts(1);
   int rc = single_instance(lat, d_r, pstride, cstride, np, nturns, refpts, nref, turn0, start, end,
                            d_rout, d_lf, d_lt, d_le, d_lc, losses, elempass, slots[0].data(), insts[0]);
@@ -1565,7 +1579,7 @@ int atx_track_batch(const atx_batch_item* items, int32_t nitems, int32_t nturns,
     in.losses = losses ? ((flags & ATX_CONTINUE_LOSSES) ? 2 : 1) : 0;
     if (in.nturns == 0) continue;
     insts.push_back(in);
-    auto ins = empty_slots.emplace(nelem, std::vector<int32_t>(2 * (size_t)(nelem + 1), -1));
+    auto ins = empty_slots.emplace(nelem, std::vector<int32_t>(ref_words(nelem), 0));
     slots.push_back(&ins.first->second);
   }
   if (insts.empty()) return ATX_OK;
@@ -1918,7 +1932,7 @@ int atx_element_matrices(atx_lattice* lat, const double* orbits, double step, do
   double* d_m = dev ? m66 : d_r + nr + no;
   // One instance per element: its 12 probes through that element alone
   // (at_elempass: no loss check), one 64-lane workgroup each.
-  std::vector<int32_t> slots(2 * (size_t)(nelem + 1));
+  std::vector<int32_t> slots(ref_words(nelem));
   std::vector<Instance> insts(nelem);
   rc = single_instance(lat, d_r, 6, 1, 12, 1, nullptr, 0, 0, 0, 1, nullptr, nullptr, nullptr,
                        nullptr, nullptr, 0, true, slots.data(), insts[0]);
