@@ -240,6 +240,19 @@ struct DiffArgs {
   int32_t pad;
 };
 
+// Element matrices by central differences (one wave per element).
+struct ElemMatArgs {
+  const DevElem* elems;
+  const double* pool;
+  const LatOp* ops;
+  const int32_t* opof;
+  const double* orbits;  // (6, nelem): orbit at the entrance of each element
+  double* m66;           // nelem x 36, column-major 6x6 per element
+  double step;
+  int32_t nelem;
+  int32_t pad;
+};
+
 // One block of turns of the adjoint sweep (gridDim.y indexes the items).
 struct AdjItem {
   const double* states;  // (nturns+1) blocks of (6, N): turn-start states, then the end state

@@ -36,8 +36,8 @@ ATX_TRACK_DECL(atx_launch_track_fast_p2_u1)
 ATX_TRACK_DECL(atx_launch_track_fast_p2_u2)
 #undef ATX_TRACK_DECL
 extern "C" hipError_t atx_launch_diffusion(const atx::DiffArgs*, hipStream_t);
-extern "C" hipError_t atx_launch_element_probes(const double*, double, double*, int, hipStream_t);
-extern "C" hipError_t atx_launch_element_diffs(const double*, double, double*, int, hipStream_t);
+extern "C" hipError_t atx_launch_element_matrices_strict(const atx::ElemMatArgs*, hipStream_t);
+extern "C" hipError_t atx_launch_element_matrices_fast(const atx::ElemMatArgs*, hipStream_t);
 extern "C" hipError_t atx_launch_repack(const atx::Instance*, int, int, hipStream_t);
 extern "C" hipError_t atx_launch_live_map(const atx::Instance*, int, int, int, int, int32_t*,
                                           hipStream_t);
@@ -192,24 +192,31 @@ bool integrator_scheme(int type, Scheme* s) {
 }  // namespace
 }  // namespace atx
 
+// Device copy of a compiled lattice, valid for (energy, rest).
+struct DeviceCopy {
+  bool valid = false;
+  double energy = -1.0, rest = -1.0;
+  int device = -1;
+  char* lat = nullptr;  // one allocation: program records, elements, pool, records of elements
+  atx::LatOp* ops = nullptr;
+  atx::DevElem* elems = nullptr;
+  double* pool = nullptr;
+  int32_t* opof = nullptr;
+  // host copies of per-element compile results used by the adjoint
+  std::vector<int32_t> r1inv, r2inv, order, kind;
+  std::vector<std::string> adjerr;
+};
+
 struct atx_lattice {
   std::vector<atx::HostElem> elems;
-  // device copy of the compiled lattice, valid for (energy, rest, elempass)
-  bool dev_valid = false;
-  double dev_energy = -1.0, dev_rest = -1.0;
-  bool dev_elempass = false;
-  int dev_device = -1;
-  char* d_lat = nullptr;  // one allocation: program records, elements, pool, records of elements
-  atx::LatOp* d_ops = nullptr;
-  atx::DevElem* d_elems = nullptr;
-  double* d_pool = nullptr;
-  int32_t* d_opof = nullptr;
+  // [0] for tracking, [1] for single elements: the revolution time of a cavity
+  // is the ring's in one and 0 in the other, and a program that alternates
+  // between them (element and diffusion matrices) would recompile at each call
+  DeviceCopy dev[2];
+  void invalidate() { dev[0].valid = dev[1].valid = false; }
   int64_t turn_counter = 0;
   int integrator = 4;
   atx_launch_shape shape{0, 0, 0, 0};  // atx_track / atx_elempass launches (0: default)
-  // host copies of per-element compile results used by the adjoint
-  std::vector<int32_t> h_r1inv, h_r2inv, h_order, h_kind;
-  std::vector<std::string> h_adjerr;
   std::mutex mu;
 };
 
@@ -798,15 +805,14 @@ void ref_bits(const int32_t* slot, int nelem, int32_t* words) {
 int ensure_device_lattice(atx_lattice* lat, double energy, double rest, bool elempass) {
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
-  if (lat->dev_valid && lat->dev_energy == energy && lat->dev_rest == rest &&
-      lat->dev_elempass == elempass && lat->dev_device == dev)
-    return ATX_OK;
+  DeviceCopy& d = lat->dev[elempass ? 1 : 0];
+  if (d.valid && d.energy == energy && d.rest == rest && d.device == dev) return ATX_OK;
   Compiled c;
   int rc = compile_lattice(lat, energy, rest, elempass, c);
   if (rc) return rc;
-  if (lat->d_lat) (void)hipFree(lat->d_lat);
-  lat->d_lat = nullptr;
-  lat->dev_valid = false;
+  if (d.lat) (void)hipFree(d.lat);
+  d.lat = nullptr;
+  d.valid = false;
   // one allocation and one copy; every part starts on a 64-byte line
   const size_t part[4] = {c.ops.size() * sizeof(LatOp), c.elems.size() * sizeof(DevElem),
                           c.pool.size() * sizeof(double), c.opof.size() * sizeof(int32_t)};
@@ -816,26 +822,25 @@ int ensure_device_lattice(atx_lattice* lat, double energy, double rest, bool ele
   std::vector<char> host(off[4]);
   for (int k = 0; k < 4; k++)
     if (part[k]) std::memcpy(host.data() + off[k], src[k], part[k]);
-  HIPCHK(hipMalloc((void**)&lat->d_lat, host.size()));
-  HIPCHK(hipMemcpy(lat->d_lat, host.data(), host.size(), hipMemcpyHostToDevice));
-  lat->d_ops = (LatOp*)(lat->d_lat + off[0]);
-  lat->d_elems = (DevElem*)(lat->d_lat + off[1]);
-  lat->d_pool = (double*)(lat->d_lat + off[2]);
-  lat->d_opof = (int32_t*)(lat->d_lat + off[3]);
-  lat->h_r1inv = c.r1inv;
-  lat->h_r2inv = c.r2inv;
-  lat->h_adjerr = c.adjerr;
-  lat->h_order.clear();
-  lat->h_kind.clear();
+  HIPCHK(hipMalloc((void**)&d.lat, host.size()));
+  HIPCHK(hipMemcpy(d.lat, host.data(), host.size(), hipMemcpyHostToDevice));
+  d.ops = (LatOp*)(d.lat + off[0]);
+  d.elems = (DevElem*)(d.lat + off[1]);
+  d.pool = (double*)(d.lat + off[2]);
+  d.opof = (int32_t*)(d.lat + off[3]);
+  d.r1inv = c.r1inv;
+  d.r2inv = c.r2inv;
+  d.adjerr = c.adjerr;
+  d.order.clear();
+  d.kind.clear();
   for (const auto& h : c.elems) {
-    lat->h_order.push_back(h.order);
-    lat->h_kind.push_back(h.kind);
+    d.order.push_back(h.order);
+    d.kind.push_back(h.kind);
   }
-  lat->dev_valid = true;
-  lat->dev_energy = energy;
-  lat->dev_rest = rest;
-  lat->dev_elempass = elempass;
-  lat->dev_device = dev;
+  d.valid = true;
+  d.energy = energy;
+  d.rest = rest;
+  d.device = dev;
   return ATX_OK;
 }
 
@@ -1174,10 +1179,11 @@ int single_instance(atx_lattice* lat, double* d_r, int64_t pstride, int64_t cstr
   if ((n_first > 0 || n_std > 0) && !d_rout) return fail(ATX_E_VALUE, "r_out is NULL but refpts request copies");
   if (losses && (!d_lf || !d_lt || !d_le || !d_lc)) return fail(ATX_E_VALUE, "loss arrays are NULL");
   std::memset(&inst, 0, sizeof(inst));
-  inst.elems = lat->d_elems;
-  inst.pool = lat->d_pool;
-  inst.ops = lat->d_ops;
-  inst.opof = lat->d_opof;
+  const DeviceCopy& d = lat->dev[elempass ? 1 : 0];
+  inst.elems = d.elems;
+  inst.pool = d.pool;
+  inst.ops = d.ops;
+  inst.opof = d.opof;
   inst.r = d_r;
   inst.rout = d_rout;
   inst.lost_flag = d_lf;
@@ -1315,7 +1321,8 @@ int atx_lattice_create(atx_lattice** out) {
 
 int atx_lattice_destroy(atx_lattice* lat) {
   if (!lat) return ATX_OK;
-  if (lat->d_lat) (void)hipFree(lat->d_lat);
+  for (auto& d : lat->dev)
+    if (d.lat) (void)hipFree(d.lat);
   delete lat;
   return ATX_OK;
 }
@@ -1330,7 +1337,7 @@ int atx_lattice_add_element(atx_lattice* lat, const char* pass_method, const cha
       e.fam = fam_name ? fam_name : "";
       e.kind = p.kind;
       lat->elems.push_back(std::move(e));
-      lat->dev_valid = false;
+      lat->invalidate();
       return (int)ATX_OK;
     }
   }
@@ -1348,7 +1355,7 @@ static int set_attr(atx_lattice* lat, const char* name, const double* v, int64_t
   a.v.assign(v, v + n);
   a.is_int = is_int;
   lat->elems.back().attrs[name] = std::move(a);
-  lat->dev_valid = false;
+  lat->invalidate();
   return ATX_OK;
 }
 
@@ -1375,7 +1382,7 @@ int atx_lattice_set_integrator(atx_lattice* lat, int32_t type) {
   std::lock_guard<std::mutex> g(lat->mu);
   if (lat->integrator != type) {
     lat->integrator = type;
-    lat->dev_valid = false;  // recompiled, as atgpu recreates its lattice (PyInterface.cpp:259-266)
+    lat->invalidate();  // recompiled, as atgpu recreates its lattice (PyInterface.cpp:259-266)
   }
   return ATX_OK;
 }
@@ -1559,10 +1566,10 @@ int atx_track_batch(const atx_batch_item* items, int32_t nitems, int32_t nturns,
     const int nelem = (int)it.lattice->elems.size();
     Instance in;
     std::memset(&in, 0, sizeof(in));
-    in.elems = it.lattice->d_elems;
-    in.pool = it.lattice->d_pool;
-    in.ops = it.lattice->d_ops;
-    in.opof = it.lattice->d_opof;
+    in.elems = it.lattice->dev[0].elems;
+    in.pool = it.lattice->dev[0].pool;
+    in.ops = it.lattice->dev[0].ops;
+    in.opof = it.lattice->dev[0].opof;
     in.r = it.r;
     in.lost_flag = it.lost_flag;
     in.lost_turn = it.lost_turn;
@@ -1656,8 +1663,8 @@ int atx_track_batch_noalloc(const atx_batch_item* items, int32_t nitems, int32_t
     atx_lattice* lat = it.lattice;
     // compiling or uploading a lattice allocates: it must already be on
     // this device for this energy
-    if (!(lat->dev_valid && lat->dev_energy == energy && lat->dev_rest == rest_energy &&
-          !lat->dev_elempass && lat->dev_device == dev))
+    const DeviceCopy& copy = lat->dev[0];
+    if (!(copy.valid && copy.energy == energy && copy.rest == rest_energy && copy.device == dev))
       return fail(ATX_E_VALUE, "item " + std::to_string(i) +
                                    ": lattice not on this device for this energy (track it once "
                                    "with atx_track or atx_track_batch first)");
@@ -1666,10 +1673,10 @@ int atx_track_batch_noalloc(const atx_batch_item* items, int32_t nitems, int32_t
     Instance& in = tab[n];
     std::memset(&in, 0, sizeof(in));
     const int nelem = (int)lat->elems.size();
-    in.elems = lat->d_elems;
-    in.pool = lat->d_pool;
-    in.ops = lat->d_ops;
-    in.opof = lat->d_opof;
+    in.elems = copy.elems;
+    in.pool = copy.pool;
+    in.ops = copy.ops;
+    in.opof = copy.opof;
     in.slots = nullptr;  // no refpts: the kernel reads no slot table
     in.r = it.r;
     in.lost_flag = it.lost_flag;
@@ -1739,7 +1746,7 @@ int atx_element_set_array_at(atx_lattice* lat, int32_t index, const char* name, 
   Attr a;
   a.v.assign(data, data + n);
   lat->elems[index].attrs[name] = std::move(a);
-  lat->dev_valid = false;
+  lat->invalidate();
   return ATX_OK;
 }
 
@@ -1754,23 +1761,23 @@ static int adjoint_launch(atx_lattice* lat, const std::vector<AdjItem>& items, d
   if (rc) return rc;
   std::vector<AdjElem> ae(nelem > 0 ? nelem : 1);
   for (int e = 0; e < nelem; e++) {
-    if (!lat->h_adjerr[e].empty())
+    if (!lat->dev[0].adjerr[e].empty())
       return fail(ATX_E_RUNTIME, "adjoint not available for element #" + std::to_string(e) + " " +
-                                     lat->elems[e].fam + " (" + lat->elems[e].pass + "): " + lat->h_adjerr[e]);
+                                     lat->elems[e].fam + " (" + lat->elems[e].pass + "): " + lat->dev[0].adjerr[e]);
     const int slot = grad_slot ? grad_slot[e] : -1;
     const int coeff = grad_coeff ? grad_coeff[e] : 0;
     if (slot >= 0) {
-      const int k = lat->h_kind[e];
+      const int k = lat->dev[0].kind[e];
       if (k != K_STR && k != K_BND && k != K_THIN)
         return fail(ATX_E_VALUE, "element #" + std::to_string(e) + " has no PolynomB to differentiate");
       if (slot >= num_params || !have_grad) return fail(ATX_E_VALUE, "gradient slot out of range");
-      if (coeff < 0 || coeff > lat->h_order[e])
+      if (coeff < 0 || coeff > lat->dev[0].order[e])
         return fail(ATX_E_VALUE, "element #" + std::to_string(e) + ": PolynomB index above MaxOrder");
     }
     ae[e].slot = slot;
     ae[e].coeff = coeff;
-    ae[e].r1inv = lat->h_r1inv[e];
-    ae[e].r2inv = lat->h_r2inv[e];
+    ae[e].r1inv = lat->dev[0].r1inv[e];
+    ae[e].r2inv = lat->dev[0].r2inv[e];
   }
   std::vector<AdjItem> run;
   int32_t max_np = 0;
@@ -1793,8 +1800,8 @@ static int adjoint_launch(atx_lattice* lat, const std::vector<AdjItem>& items, d
   hipError_t le = hipSuccess;
   if (ce == hipSuccess) {
     AdjArgs a;
-    a.elems = lat->d_elems;
-    a.pool = lat->d_pool;
+    a.elems = lat->dev[0].elems;
+    a.pool = lat->dev[0].pool;
     a.adj = (const AdjElem*)d_buf;
     a.items = (const AdjItem*)(d_buf + ae_pad);
     a.nelem = nelem;
@@ -1888,8 +1895,8 @@ int atx_diffusion_matrices(atx_lattice* lat, const double* orbits, double* bdiff
     }
   }
   DiffArgs a;
-  a.elems = lat->d_elems;
-  a.pool = lat->d_pool;
+  a.elems = lat->dev[0].elems;
+  a.pool = lat->dev[0].pool;
   a.orbits = d_o;
   a.bdiff = d_b;
   a.nelem = nelem;
@@ -1924,44 +1931,23 @@ int atx_element_matrices(atx_lattice* lat, const double* orbits, double step, do
   hipStream_t stream = (hipStream_t)stream_;
   const bool dev = (flags & ATX_DEVICE_POINTERS) != 0;
   const bool strict = (flags & ATX_STRICT) != 0;
-  // probes (6, 12 nelem), then (host arrays) the orbits and the matrices
-  const size_t nr = 72 * (size_t)nelem, no = 6 * (size_t)nelem, nm = 36 * (size_t)nelem;
-  double* d_r = nullptr;
-  HIPCHK(hipMallocAsync((void**)&d_r, (nr + (dev ? 0 : no + nm)) * sizeof(double), stream));
-  const double* d_o = dev ? orbits : d_r + nr;
-  double* d_m = dev ? m66 : d_r + nr + no;
-  // One instance per element: its 12 probes through that element alone
-  // (at_elempass: no loss check), one 64-lane workgroup each.
-  std::vector<int32_t> slots(ref_words(nelem));
-  std::vector<Instance> insts(nelem);
-  rc = single_instance(lat, d_r, 6, 1, 12, 1, nullptr, 0, 0, 0, 1, nullptr, nullptr, nullptr,
-                       nullptr, nullptr, 0, true, slots.data(), insts[0]);
-  if (rc) {
-    (void)hipFreeAsync(d_r, stream);
-    return rc;
-  }
-  for (int e = 1; e < nelem; e++) {
-    insts[e] = insts[0];
-    insts[e].r = d_r + 72 * (size_t)e;
-    insts[e].start_elem = e;
-    insts[e].end_elem = e + 1;
-  }
-  const atx_launch_shape in{64, 1, 0, 0};
-  atx_launch_shape shape;
-  rc = resolve_shape(&in, shape, strict);
+  // host arrays: the orbits, then the matrices
+  const size_t no = 6 * (size_t)nelem, nm = 36 * (size_t)nelem;
+  double* d_buf = nullptr;
   hipError_t e = hipSuccess;
-  if (!dev) e = hipMemcpyAsync(const_cast<double*>(d_o), orbits, no * sizeof(double),
-                               hipMemcpyHostToDevice, stream);
-  if (!rc && e == hipSuccess) e = atx_launch_element_probes(d_o, step, d_r, nelem, stream);
-  if (!rc && e == hipSuccess)
-    rc = launch_instances(insts, std::vector<const std::vector<int32_t>*>(nelem, &slots), shape,
-                          stream, strict);
-  if (!rc && e == hipSuccess) e = atx_launch_element_diffs(d_r, step, d_m, nelem, stream);
-  if (!rc && e == hipSuccess && !dev)
-    e = hipMemcpyAsync(m66, d_m, nm * sizeof(double), hipMemcpyDeviceToHost, stream);
-  hipError_t fe = hipFreeAsync(d_r, stream);
+  if (!dev) {
+    HIPCHK(hipMallocAsync((void**)&d_buf, (no + nm) * sizeof(double), stream));
+    e = hipMemcpyAsync(d_buf, orbits, no * sizeof(double), hipMemcpyHostToDevice, stream);
+  }
+  const DeviceCopy& d = lat->dev[1];
+  const ElemMatArgs a{d.elems, d.pool, d.ops, d.opof, dev ? orbits : d_buf, dev ? m66 : d_buf + no,
+                      step, nelem, 0};
+  if (e == hipSuccess)
+    e = (strict ? atx_launch_element_matrices_strict : atx_launch_element_matrices_fast)(&a, stream);
+  if (e == hipSuccess && !dev)
+    e = hipMemcpyAsync(m66, a.m66, nm * sizeof(double), hipMemcpyDeviceToHost, stream);
+  hipError_t fe = dev ? hipSuccess : hipFreeAsync(d_buf, stream);
   hipError_t se = dev ? hipSuccess : hipStreamSynchronize(stream);
-  if (rc) return rc;
   if (e != hipSuccess) return fail(ATX_E_RUNTIME, std::string("element matrices: ") + hipGetErrorString(e));
   if (fe != hipSuccess) return fail(ATX_E_RUNTIME, std::string("hipFreeAsync: ") + hipGetErrorString(fe));
   if (se != hipSuccess) return fail(ATX_E_RUNTIME, std::string("hipStreamSynchronize: ") + hipGetErrorString(se));

@@ -2487,39 +2487,68 @@ extern "C" hipError_t ATX_LAUNCH(const atx::Instance* d_insts, int ninst, int nb
   return hipGetLastError();
 }
 
+#if ATX_PPT == 1 && ATX_UNROLL == (ATX_STRICT ? 1 : 2)
+namespace atx {
+namespace ATX_NS {
+// Element matrices (matrix.py:195-202): lane c of element e's wave tracks its
+// entrance orbit plus column c of [D, -D], D = diag(step/2), through element e
+// alone (at.c at_elempass: no loss test, a NaN input stays as it is); the zeros
+// of -D are -0.0, as numpy adds them. m[i][j] = (probe j+ - probe j-)_i / step,
+// column-major, each column written by its lane.
+// One kernel from orbits to matrices: as a batch of single-element launches
+// this took a 448 KB instance table from the host and two kernels around the
+// tracking one. A wave per element keeps the element's constants scalar; the
+// idle lanes cost nothing, the launch (2,241 elements of a large ring: 2.2
+// waves per SIMD) is as long as the chain of one magnet. The bounds are those of
+// the tracking kernel, whose functions it calls.
+__global__ void __launch_bounds__(512, 4) element_matrix_kernel(ElemMatArgs args) {
+  const int e = (int)blockIdx.x;
+  const int c = (int)threadIdx.x;
+  const double h = 0.5 * args.step;
+  const double* o = args.orbits + 6 * (int64_t)e;
+  const double d = (c < 6) ? h : -h;
+  const double z = (c < 6) ? 0.0 : -0.0;
+  const int k = c % 6;
+  R6 r = {o[0] + (k == 0 ? d : z), o[1] + (k == 1 ? d : z), o[2] + (k == 2 ? d : z),
+          o[3] + (k == 3 ? d : z), o[4] + (k == 4 ? d : z), o[5] + (k == 5 ? d : z)};
+  const R6 in = r;
+  const bool skip = __builtin_isnan(r.x);
+  if (skip || c >= 12) r = idle_state();
+  cDevElem* h_e = (cDevElem*)args.elems + e;
+#if !ATX_STRICT
+  cLatOp* rec = (cLatOp*)args.ops + ((cint*)args.opof)[e];
+  if (rec->last == e && (rec->op & OPF_MPOLE))
+    r = op_call<ATX_UNROLL>(r, (const LatOp*)rec, h_e, (cdouble*)args.pool, 1);
+  else
+#endif
+    r = header_call<ATX_UNROLL>(r, h_e, (cdouble*)args.pool, 1);
+  if (skip) r = in;
+  const double v[6] = {r.x, r.px, r.y, r.py, r.dp, r.ct};
+  double* m = args.m66 + 36 * (int64_t)e + 6 * c;
+#pragma unroll
+  for (int i = 0; i < 6; i++) {
+    const double minus = __shfl_down(v[i], 6, 64);
+    if (c < 6) m[i] = (v[i] - minus) / args.step;
+  }
+}
+}  // namespace ATX_NS
+}  // namespace atx
+
+#if ATX_STRICT
+#define ATX_LAUNCH_ELEM atx_launch_element_matrices_strict
+#else
+#define ATX_LAUNCH_ELEM atx_launch_element_matrices_fast
+#endif
+extern "C" hipError_t ATX_LAUNCH_ELEM(const atx::ElemMatArgs* args, hipStream_t stream) {
+  if (args->nelem <= 0) return hipSuccess;
+  hipLaunchKernelGGL(atx::ATX_NS::element_matrix_kernel, dim3((unsigned)args->nelem), dim3(64), 0,
+                     stream, *args);
+  return hipGetLastError();
+}
+#endif
+
 #if ATX_AUX
 namespace atx {
-// Probes of atx_element_matrices (matrix.py:195-200): particle 12 e + c is
-// the entrance orbit of element e plus column c of [D, -D], D = diag(step/2):
-// +step/2 on coordinate c (c < 6), -step/2 on coordinate c - 6 (c >= 6), and
-// +0.0 (c < 6) or -0.0 (c >= 6) elsewhere, as numpy adds them; (6, 12 nelem)
-// F-order.
-__global__ void __launch_bounds__(256) element_probe_kernel(const double* __restrict__ orbits,
-                                                            double step, double* __restrict__ r,
-                                                            int nelem) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 12 * (int64_t)nelem) return;
-  const int64_t e = i / 12;
-  const int c = (int)(i % 12);
-  const double d = (c < 6) ? 0.5 * step : -(0.5 * step);
-  const double z = (c < 6) ? 0.0 : -0.0;
-#pragma unroll
-  for (int k = 0; k < 6; k++) r[6 * i + k] = orbits[6 * e + k] + ((k == c % 6) ? d : z);
-}
-
-// m[i][j] = (probe j+ - probe j-)_i / step (matrix.py:201-202), column-major
-// 6x6 per element ([i][j] at 36 e + i + 6 j).
-__global__ void __launch_bounds__(256) element_diff_kernel(const double* __restrict__ r,
-                                                           double step, double* __restrict__ m66,
-                                                           int nelem) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 36 * (int64_t)nelem) return;
-  const int64_t e = t / 36;
-  const int i = (int)(t % 6), j = (int)((t % 36) / 6);
-  const double* p = r + 72 * e;
-  m66[t] = (p[6 * j + i] - p[6 * (6 + j) + i]) / step;
-}
-
 // Repack between the turn blocks of a batched launch: one workgroup per
 // instance lists, in order, the particles still alive (x not NaN: a lost
 // particle is set to NaN, at.c:142-161) in idx[0..*nlive). The first pass
@@ -2644,24 +2673,6 @@ extern "C" hipError_t atx_launch_live_map(const atx::Instance* d_insts, int nins
   if (ninst <= 0) return hipSuccess;
   hipLaunchKernelGGL(atx::live_map_kernel, dim3(1), dim3(1024), 0, stream, d_insts, ninst, block,
                      fine, fine_limit, live_begin);
-  return hipGetLastError();
-}
-
-extern "C" hipError_t atx_launch_element_probes(const double* orbits, double step, double* r,
-                                                int nelem, hipStream_t stream) {
-  const int64_t n = 12 * (int64_t)nelem;
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(atx::element_probe_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                     stream, orbits, step, r, nelem);
-  return hipGetLastError();
-}
-
-extern "C" hipError_t atx_launch_element_diffs(const double* r, double step, double* m66,
-                                               int nelem, hipStream_t stream) {
-  const int64_t n = 36 * (int64_t)nelem;
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(atx::element_diff_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                     stream, r, step, m66, nelem);
   return hipGetLastError();
 }
 
