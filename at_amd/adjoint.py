@@ -7,7 +7,9 @@ backward is the hand-written adjoint kernel (atx_adjoint):
 
 * forward keeps one checkpoint of the particle state every ``checkpoint``
   turns (8 by default);
-* backward first recomputes every block forward from its checkpoint, all
+* the states at the start of each turn of the last block, where backward
+  begins, are kept as forward passes them;
+* backward first recomputes every other block forward from its checkpoint, all
   blocks together: turn j of every block is one batched launch
   (atx_track_batch, one instance per block with its own turn number), and
   the state at the start of each turn is kept; the blocks' arithmetic is
@@ -26,7 +28,8 @@ backward is the hand-written adjoint kernel (atx_adjoint):
   blocks (their turn-start states are recorded), g chosen by a cost model
   (sweep_plan).
 
-Memory: checkpoints (nturns/checkpoint + 1) x N x 48 B plus the turn-start
+Memory: checkpoints (nturns/checkpoint + 1) x N x 48 B and, from forward to
+backward, the last block's turn-start states; backward holds the turn-start
 states of all blocks, (nturns + nblocks) x N x 48 B (12.6 MB for 4,096
 particles and 64 turns); the parallel sweep adds (S - 1) x N x 288 B of
 sub-block matrices for S sub-blocks.
@@ -229,14 +232,32 @@ class TrackingLoss:
                 # ring's 8-turn block of 4,096 particles: 19.0 ms, against
                 # 20.3 ms in 256-thread workgroups)
                 small = n <= 64 * _device_simds(r.device)
-                while t < nturns:
-                    nt = min(cp, nturns - t)
-                    ckpts.append((t, nt, r.clone()))
+
+                def track(nt):
                     engine.track_batch([{"lattice": problem.dl, "r": r.data_ptr(), "n": n,
                                          "nturns": nt, "turn": t}], 0, energy=problem.energy,
                                        rest_energy=problem.rest, losses=False,
                                        block_size=64 if small else 0, stream=stream)
-                    t += nt
+
+                ctx.kept = None
+                while t < nturns:
+                    nt = min(cp, nturns - t)
+                    if t + nt < nturns or not ctx.needs_input_grad[0]:
+                        ckpts.append((t, nt, r.clone()))
+                        track(nt)
+                        t += nt
+                        continue
+                    # the block that backward starts with: turn by turn, its
+                    # turn-start states kept instead of recomputed (the large
+                    # ring, 4,096 particles, 8 turns: 10.9 of 44 ms)
+                    kept = torch.empty((nt + 1, n, 6), dtype=torch.float64, device=r.device)
+                    ckpts.append((t, nt, kept[0]))
+                    for j in range(nt):
+                        kept[j].copy_(r)
+                        track(1)
+                        t += 1
+                    kept[nt].copy_(r)
+                    ctx.kept = kept
                 loss, lam = _loss_and_seed(r)
                 ctx.ckpts = ckpts
                 ctx.strengths = strengths_np
@@ -258,20 +279,23 @@ class TrackingLoss:
                 # the lattice is shared: another forward may have set other
                 # strengths since this one; recompute and sweep with this one's
                 problem.set_strengths(ctx.strengths)
+                again = blocks if ctx.kept is None else blocks[:-1]
                 states = [torch.empty((nt + 1, n, 6), dtype=torch.float64,
-                                      device=particles.device) for _, nt, _ in blocks]
-                cur = [ck.clone() for _, _, ck in blocks]
-                for j in range(max(nt for _, nt, _ in blocks)):
+                                      device=particles.device) for _, nt, _ in again]
+                cur = [ck.clone() for _, _, ck in again]
+                for j in range(max((nt for _, nt, _ in again), default=0)):
                     items = []
-                    for k, (t0, nt, _) in enumerate(blocks):
+                    for k, (t0, nt, _) in enumerate(again):
                         if j < nt:
                             states[k][j].copy_(cur[k])
                             items.append({"lattice": problem.dl, "r": cur[k].data_ptr(), "n": n,
                                           "nturns": 1, "turn": t0 + j})
                     engine.track_batch(items, 0, energy=problem.energy,
                                        rest_energy=problem.rest, losses=False, stream=stream)
-                for k, (_, nt, _) in enumerate(blocks):
+                for k, (_, nt, _) in enumerate(again):
                     states[k][nt].copy_(cur[k])
+                if ctx.kept is not None:
+                    states.append(ctx.kept)
                 g = problem.sub_block
                 if g is None:
                     g = sweep_plan(n, [nt for _, nt, _ in blocks], _device_simds(particles.device))

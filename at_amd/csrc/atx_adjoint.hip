@@ -25,10 +25,20 @@ typedef __attribute__((address_space(4))) const double cdouble;
 typedef __attribute__((address_space(4))) const DevElem cDevElem;
 typedef __attribute__((address_space(4))) const AdjElem cAdjElem;
 typedef __attribute__((address_space(4))) const AdjItem cAdjItem;
+typedef __attribute__((address_space(4))) const LatOp cLatOp;
+typedef __attribute__((address_space(4))) const AdjRec cAdjRec;
+typedef __attribute__((address_space(4))) const int32_t cint;
 
 struct V6 {
   double x, px, y, py, dp, ct;
 };
+
+// 1/d within an ulp: the hardware estimate and two Newton steps.
+__device__ __forceinline__ double rcp(double d) {
+  double q = __builtin_amdgcn_rcp(d);
+  q = __builtin_fma(q, __builtin_fma(-d, q, 1.0), q);
+  return __builtin_fma(q, __builtin_fma(-d, q, 1.0), q);
+}
 
 // polynomial value and complex derivative: sum (B_k + i A_k) z^k, z = x + i y
 template <int N>
@@ -64,7 +74,7 @@ __device__ __forceinline__ void zpow(double x, double y, int j, double& zr, doub
 // Reverse of an in-magnet drift x' = x + nl px, ct' = ct + nl (px^2+py^2) u/2
 // with nl = L u, u = 1/(1+dp).
 __device__ __forceinline__ void drift_rev(V6& r, V6& l, double len) {
-  const double u = 1.0 / (1.0 + r.dp);
+  const double u = rcp(1.0 + r.dp);
   const double nl = len * u;
   const double p2 = r.px * r.px + r.py * r.py;
   r.x -= nl * r.px;
@@ -103,15 +113,27 @@ __device__ __forceinline__ void kick_rev(V6& r, V6& l, cdouble* a, cdouble* b, i
   r.py -= k * im;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+// v plus the v of the lane that the DPP control names (0 where there is none):
+// moves between lanes inside the VALU, where a shuffle goes through the LDS unit
+// and its latency.
+template <int CTRL>
+__device__ __forceinline__ double plus_dpp(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+  return v + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+// Sum of the wave in lane 63: within rows of 16 lanes (shifts right by 1, 2, 4,
+// 8), then each row's last lane to the next row, then to the upper half.
 __device__ __forceinline__ void grad_flush(double g, int slot, double* grad) {
-  const double s = wave_sum(g);
-  if ((threadIdx.x & 63) == 0) atomicAdd(grad + slot, s);
+  g = plus_dpp<0x111>(g);
+  g = plus_dpp<0x112>(g);
+  g = plus_dpp<0x114>(g);
+  g = plus_dpp<0x118>(g);
+  g = plus_dpp<0x142>(g);
+  g = plus_dpp<0x143>(g);
+  if ((threadIdx.x & 63) == 63) atomicAdd(grad + slot, g);
 }
 
 // misalignment: state r <- Minv r, adjoint l <- M^T l
@@ -287,10 +309,169 @@ __device__ __forceinline__ void element_rev(V6& r, V6& l, cDevElem& h, cAdjElem&
   }
 }
 
+// --- Elements by their records -----------------------------------------------
+// Reverse of the ops that a ring without radiation is made of. In a magnet
+// delta and lambda_ct are constant, so the reciprocal 1/(1+delta) and every
+// product of a drift's length with them are taken once per magnet: a drift is
+// 13 FP64 instructions instead of 35 (a division among them), two drifts in a
+// row are one, and the kicks are spelled out for the form of the field (7
+// instead of about 20 for a quadrupole). One wave of the large ring: 5.2 ->
+// 2.1 ms per turn.
+struct RevDrift {
+  double nl, nlu;     // L u, L u^2 with u = 1/(1+delta)
+  double hh;          // L u^2 / 2
+  double d, c;        // L u^2 lambda_ct, L u^3 lambda_ct
+};
+
+__device__ __forceinline__ RevDrift rev_drift(double len, double u, double lct) {
+  RevDrift k;
+  k.nl = len * u;
+  k.nlu = k.nl * u;
+  k.hh = 0.5 * k.nlu;
+  k.d = k.nlu * lct;
+  k.c = k.d * u;
+  return k;
+}
+
+__device__ __forceinline__ void drift_rev(V6& r, V6& l, const RevDrift& k) {
+  const double p2 = __builtin_fma(r.px, r.px, r.py * r.py);
+  const double t = __builtin_fma(r.px, l.x, r.py * l.y);
+  r.x = __builtin_fma(-k.nl, r.px, r.x);
+  r.y = __builtin_fma(-k.nl, r.py, r.y);
+  r.ct = __builtin_fma(-k.hh, p2, r.ct);
+  l.dp = __builtin_fma(-k.nlu, t, __builtin_fma(-k.c, p2, l.dp));
+  l.px = __builtin_fma(k.nl, l.x, __builtin_fma(k.d, r.px, l.px));
+  l.py = __builtin_fma(k.nl, l.y, __builtin_fma(k.d, r.py, l.py));
+}
+
+struct RevKick {
+  double kl, kb, kb2;    // length, length times B[N], twice that
+  double kh, khh, khl;   // bends: length times curvature, its square, lambda_ct
+};
+
+// Kick of length kl of a field B[N] z^N (LEAD) or none, in a straight or curved
+// frame; GRAD: g += d lambda / d B[N].
+template <bool BEND, int N, bool LEAD, bool GRAD>
+__device__ __forceinline__ void kick_rev(V6& r, V6& l, const RevKick& k, double irho, double& g) {
+  const double x = r.x, y = r.y, lx = l.px, ly = l.py;
+  if (BEND) {
+    r.px = __builtin_fma(-k.kh, __builtin_fma(-x, irho, r.dp), r.px);
+    r.ct = __builtin_fma(-k.kh, x, r.ct);
+    l.x = __builtin_fma(-k.khh, lx, l.x + k.khl);
+    l.dp = __builtin_fma(k.kh, lx, l.dp);
+  }
+  if (!LEAD) return;
+  // s + i t = z (l_py' ...): the products shared by the Jacobian and the gradient
+  const double s = __builtin_fma(y, ly, -x * lx);  // y l_py - x l_px
+  if (N == 1) {
+    r.px = __builtin_fma(k.kb, x, r.px);
+    r.py = __builtin_fma(-k.kb, y, r.py);
+    l.x = __builtin_fma(-k.kb, lx, l.x);
+    l.y = __builtin_fma(k.kb, ly, l.y);
+    if (GRAD) g = __builtin_fma(k.kl, s, g);
+  } else {
+    const double t = __builtin_fma(y, lx, x * ly);  // y l_px + x l_py
+    const double zr = __builtin_fma(x, x, -(y * y)), zi = 2.0 * x * y;
+    if (N == 2) {
+      r.px = __builtin_fma(k.kb, zr, r.px);
+      r.py = __builtin_fma(-k.kb, zi, r.py);
+      l.x = __builtin_fma(k.kb2, s, l.x);
+      l.y = __builtin_fma(k.kb2, t, l.y);
+      if (GRAD) g = __builtin_fma(k.kl, __builtin_fma(zi, ly, -zr * lx), g);
+    } else {  // z^3 = zr x - zi y + i (zr y + zi x); derivative 3 z^2
+      const double cr = __builtin_fma(zr, x, -zi * y), ci = __builtin_fma(zr, y, zi * x);
+      const double k3 = 3.0 * k.kb;
+      r.px = __builtin_fma(k.kb, cr, r.px);
+      r.py = __builtin_fma(-k.kb, ci, r.py);
+      l.x = __builtin_fma(k3, __builtin_fma(zi, ly, -zr * lx), l.x);
+      l.y = __builtin_fma(k3, __builtin_fma(zi, lx, zr * ly), l.y);
+      if (GRAD) g = __builtin_fma(k.kl, __builtin_fma(ci, ly, -cr * lx), g);
+    }
+  }
+}
+
+__device__ __forceinline__ void hold(double v) { asm volatile("" ::"s"(v)); }
+
+// ahead: asks for the next record, called when this one's constants have
+// arrived (scalar loads return in any order: a wait for one waits for all).
+template <bool BEND, int N, bool LEAD, bool GRAD, class Ahead>
+__device__ __forceinline__ double mpole_rev_op(V6& r, V6& l, cdouble* c, int nslice,
+                                               const Ahead& ahead) {
+  const double bn = LEAD ? c[OM_POLY + 2 * N + 1] : 0.0;
+  hold(c[OM_L1]);
+  hold(c[OM_L2]);
+  hold(c[OM_K1]);
+  hold(c[OM_K2]);
+  if (LEAD) hold(bn);
+  if (BEND) hold(c[OM_FX_OUT]);
+  ahead();
+  const double irho = BEND ? c[OM_IRHO] : 0.0;
+  const double u = rcp(1.0 + r.dp);
+  const RevDrift d1 = rev_drift(c[OM_L1], u, l.ct), d2 = rev_drift(c[OM_L2], u, l.ct);
+  const RevDrift d11 = {2.0 * d1.nl, 2.0 * d1.nlu, 2.0 * d1.hh, 2.0 * d1.d, 2.0 * d1.c};
+  RevKick k[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    k[i].kl = c[OM_K1 + i];
+    k[i].kb = k[i].kl * bn;
+    k[i].kb2 = 2.0 * k[i].kb;
+    k[i].kh = k[i].kl * irho;
+    k[i].khh = k[i].kh * irho;
+    k[i].khl = k[i].kh * l.ct;
+  }
+  double g = 0.0;
+  if (BEND) {
+    const double fx = c[OM_FX_OUT], fy = c[OM_FY_OUT];
+    l.x = __builtin_fma(fx, l.px, l.x);
+    l.y = __builtin_fma(-fy, l.py, l.y);
+    r.px = __builtin_fma(-r.x, fx, r.px);
+    r.py = __builtin_fma(r.y, fy, r.py);
+  }
+  auto body = [&]() {
+    kick_rev<BEND, N, LEAD, GRAD>(r, l, k[0], irho, g);
+    drift_rev(r, l, d2);
+    kick_rev<BEND, N, LEAD, GRAD>(r, l, k[1], irho, g);
+    drift_rev(r, l, d2);
+    kick_rev<BEND, N, LEAD, GRAD>(r, l, k[0], irho, g);
+  };
+  if (nslice > 0) {
+    drift_rev(r, l, d1);
+    for (int m = 1; m < nslice; m++) {
+      body();
+      drift_rev(r, l, d11);
+    }
+    body();
+    drift_rev(r, l, d1);
+  }
+  if (BEND) {
+    const double fx = c[OM_FX_IN], fy = c[OM_FY_IN];
+    l.x = __builtin_fma(fx, l.px, l.x);
+    l.y = __builtin_fma(-fy, l.py, l.y);
+    r.px = __builtin_fma(-r.x, fx, r.px);
+    r.py = __builtin_fma(r.y, fy, r.py);
+  }
+  return g;
+}
+
+template <bool BEND, int N, bool LEAD, class Ahead>
+__device__ __forceinline__ void mpole_rev_rec(V6& r, V6& l, cdouble* c, int nslice, int slot,
+                                              double* grad, const Ahead& ahead) {
+  if (LEAD && slot >= 0 && grad)
+    grad_flush(mpole_rev_op<BEND, N, LEAD, true>(r, l, c, nslice, ahead), slot, grad);
+  else
+    mpole_rev_op<BEND, N, LEAD, false>(r, l, c, nslice, ahead);
+}
+
+// By its header, out of line: the loop over the records keeps its registers.
+__device__ __noinline__ void element_rev_call(V6* rp, V6* lp, cDevElem* h, cAdjElem* ae,
+                                              cdouble* pool, double* grad, int nturn) {
+  element_rev(*rp, *lp, *h, *ae, pool, grad, nturn);
+}
+
 // grid: x over the particles of the largest item, y over the items; lanes
 // beyond an item's particle count idle with zero adjoint (a workgroup with
 // none of its particles returns at once: the kernel has no barrier)
-__global__ void __launch_bounds__(256) adjoint_kernel(AdjArgs args) {
+__global__ void __launch_bounds__(64, 4) adjoint_kernel(AdjArgs args) {
   cAdjItem& it = ((cAdjItem*)args.items)[blockIdx.y];
   const int npart = it.npart;
   if ((int)(blockIdx.x * blockDim.x) >= npart) return;
@@ -316,7 +497,57 @@ __global__ void __launch_bounds__(256) adjoint_kernel(AdjArgs args) {
     V6 r = {0, 0, 0, 0, 0, 0};
     if (live) r = V6{sp[0], sp[1], sp[2], sp[3], sp[4], sp[5]};
     const int nturn = it.turn0 + t;
-    for (int e = args.nelem - 1; e >= 0; e--) element_rev(r, l, elems[e], aes[e], pool, grad, nturn);
+    // the records backwards: their element, then their drift; markers change
+    // nothing
+    cLatOp* rec = (cLatOp*)args.ops + (args.nops - 1);
+    cAdjRec* ar = (cAdjRec*)args.recs + (args.nops - 1);
+    struct Head {
+      int op, last;
+      double len;
+      int nslice, slot, coeff, line1;
+    };
+    auto head = [](cLatOp* p, cAdjRec* q) {
+      return Head{p->op, p->last, p->len, p->nslice, q->slot, q->coeff, ((cint*)p)[16]};
+    };
+    Head nxt{0, 0, 0.0, 0, -1, 0, 0};
+    if (args.nops > 0) nxt = head(rec, ar);
+    for (int i = args.nops - 1; i >= 0; i--, rec--, ar--) {
+      const Head cur = nxt;
+      asm volatile("" ::"s"(cur.line1));
+      const int kind = cur.op & 0xff, sl = cur.slot;
+      cdouble* c = rec->c;
+      auto ahead = [&]() {
+        if (i == 0) return;
+        cLatOp* p = rec - 1;
+        asm volatile("" : "+s"(p));
+        nxt = head(p, ar - 1);
+      };
+      // the record's form, unless its gradient is of another coefficient or its
+      // edges or its alignment are in the header
+      const int order = kind == OP_STR2L ? 2 : kind == OP_STR3L ? 3 : 1;
+      const bool plain = !(cur.op & (OPF_XF | OPF_EDGE)) &&
+                         (sl < 0 || (cur.coeff == order && kind != OP_BND0));
+      switch (plain ? kind : (kind == OP_NONE ? OP_NONE : OP_GENERIC)) {
+        case OP_NONE:
+        case OP_APERTURE: ahead(); break;
+        case OP_STR1L: mpole_rev_rec<false, 1, true>(r, l, c, cur.nslice, sl, grad, ahead); break;
+        case OP_STR2L: mpole_rev_rec<false, 2, true>(r, l, c, cur.nslice, sl, grad, ahead); break;
+        case OP_STR3L: mpole_rev_rec<false, 3, true>(r, l, c, cur.nslice, sl, grad, ahead); break;
+        case OP_BND1L: mpole_rev_rec<true, 1, true>(r, l, c, cur.nslice, sl, grad, ahead); break;
+        case OP_BND0: mpole_rev_rec<true, 1, false>(r, l, c, cur.nslice, sl, grad, ahead); break;
+        default: {
+          ahead();
+          V6 r1 = r, l1 = l;
+          element_rev_call(&r1, &l1, &elems[cur.last], &aes[cur.last], pool, grad, nturn);
+          r = r1;
+          l = l1;
+        }
+      }
+      if (cur.op & OPF_DRIFT) {
+        const double u = rcp(1.0 + r.dp);
+        drift_rev(r, l, rev_drift(cur.len, u, l.ct));
+      }
+    }
   }
   if (active) {
     double* lp = it.lam + 6 * (int64_t)p;
@@ -336,7 +567,9 @@ __global__ void __launch_bounds__(256) adjoint_kernel(AdjArgs args) {
 // device item table); nitems <= 65535 (grid y limit)
 extern "C" hipError_t atx_launch_adjoint(const atx::AdjArgs* args, int32_t max_npart,
                                          hipStream_t stream) {
-  const int block = 256;
+  // single waves: the launches of a parallel sweep have one to three waves per
+  // SIMD, which the dispatcher spreads more evenly one by one
+  const int block = 64;
   const int nblocks = (max_npart + block - 1) / block;
   if (nblocks == 0 || args->nitems <= 0) return hipSuccess;
   hipLaunchKernelGGL(atx::adj::adjoint_kernel, dim3(nblocks, args->nitems), dim3(block), 0, stream,

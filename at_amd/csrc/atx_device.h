@@ -229,6 +229,12 @@ struct AdjElem {
   int32_t r2inv;
 };
 
+// The same of a record's element, beside the record.
+struct AdjRec {
+  int32_t slot;
+  int32_t coeff;
+};
+
 // Diffusion matrices (one lane per element): B of each radiating element
 // from its entrance orbit.
 struct DiffArgs {
@@ -268,8 +274,10 @@ struct AdjArgs {
   const DevElem* elems;
   const double* pool;
   const AdjElem* adj;
+  const LatOp* ops;
+  const AdjRec* recs;
   const AdjItem* items;
-  int32_t nelem;
+  int32_t nops;
   int32_t nitems;
 };
 

@@ -204,6 +204,7 @@ struct DeviceCopy {
   int32_t* opof = nullptr;
   // host copies of per-element compile results used by the adjoint
   std::vector<int32_t> r1inv, r2inv, order, kind;
+  std::vector<int32_t> last;  // last element of each program record (not of the terminal one)
   std::vector<std::string> adjerr;
 };
 
@@ -831,6 +832,8 @@ int ensure_device_lattice(atx_lattice* lat, double energy, double rest, bool ele
   d.r1inv = c.r1inv;
   d.r2inv = c.r2inv;
   d.adjerr = c.adjerr;
+  d.last.clear();
+  for (size_t k = 0; k + 1 < c.ops.size(); k++) d.last.push_back(c.ops[k].last);
   d.order.clear();
   d.kind.clear();
   for (const auto& h : c.elems) {
@@ -1787,11 +1790,17 @@ static int adjoint_launch(atx_lattice* lat, const std::vector<AdjItem>& items, d
       max_np = std::max(max_np, it.npart);
     }
   if (run.empty()) return ATX_OK;
-  // one buffer: the element table, then the items (both 8-byte aligned)
+  const std::vector<int32_t>& last = lat->dev[0].last;
+  std::vector<AdjRec> recs;
+  for (int32_t e : last) recs.push_back(AdjRec{ae[e].slot, ae[e].coeff});
+  // one buffer: the element table, the records', the items (all 8-byte aligned)
   const size_t ae_bytes = ae.size() * sizeof(AdjElem);
-  const size_t ae_pad = (ae_bytes + 255) & ~(size_t)255;
+  const size_t rec_bytes = recs.size() * sizeof(AdjRec);
+  const size_t rec_at = (ae_bytes + 255) & ~(size_t)255;
+  const size_t ae_pad = (rec_at + rec_bytes + 255) & ~(size_t)255;
   std::vector<unsigned char> host(ae_pad + run.size() * sizeof(AdjItem));
   std::memcpy(host.data(), ae.data(), ae_bytes);
+  std::memcpy(host.data() + rec_at, recs.data(), rec_bytes);
   std::memcpy(host.data() + ae_pad, run.data(), run.size() * sizeof(AdjItem));
   hipStream_t stream = (hipStream_t)stream_;
   unsigned char* d_buf = nullptr;
@@ -1803,8 +1812,10 @@ static int adjoint_launch(atx_lattice* lat, const std::vector<AdjItem>& items, d
     a.elems = lat->dev[0].elems;
     a.pool = lat->dev[0].pool;
     a.adj = (const AdjElem*)d_buf;
+    a.ops = lat->dev[0].ops;
+    a.recs = (const AdjRec*)(d_buf + rec_at);
     a.items = (const AdjItem*)(d_buf + ae_pad);
-    a.nelem = nelem;
+    a.nops = (int32_t)recs.size();
     a.nitems = (int32_t)run.size();
     le = atx_launch_adjoint(&a, max_np, stream);
   }

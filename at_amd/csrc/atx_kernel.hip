@@ -2212,6 +2212,13 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   for (; rec != end; rec++) {
     const OpHead cur = nxt;
     asm volatile("" ::"s"(cur.line1), "s"(cur.line2));
+#if ATX_STRICT
+    // The strict build's divisions take long enough for the head to come, and
+    // it is 6 % faster with the head asked for here (large ring, 32,003
+    // particles: 7.07 against 7.55 ms per turn).
+    nxt = op_head(rec + 1);
+    const NotAhead ahead;
+#else
     // The next record's head, asked for when this record's constants have
     // arrived: scalar loads return in any order, so that waiting for one waits
     // for all, and a constant asked for after the head would wait for the L2.
@@ -2221,6 +2228,7 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
       asm volatile("" : "+s"(p));
       nxt = op_head(p);
     };
+#endif
     const int kind = cur.op & 0xff;
     if (REFS) {  // markers change nothing: only their copies
       const int ndo = (kind != OP_NONE ? 1 : 0) + ((cur.op & OPF_DRIFT) ? 1 : 0);
