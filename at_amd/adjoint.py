@@ -95,10 +95,10 @@ def _sweep_cost(lanes: int, simds: int) -> float:
     """Time per turn of one adjoint launch over `lanes` particles, in units
     of a launch with at most one wave per SIMD: below that the dependent FP64
     chain of each lane sets the time; above it the time grows as
-    0.536 + 0.533 w with w waves per SIMD (fitted to launches over the large
-    ring of 4,096-particle items: 1.57 at w = 1.9, 1.97 at w = 2.7, 6.77 at
-    w = 11.7; it orders 1-, 2- and 4-turn sub-blocks as measured)."""
-    return max(1.0, 0.536 + 0.533 * lanes / (64.0 * simds))
+    0.55 + 0.76 w with w waves per SIMD (fitted to launches over the large
+    ring: 1.25 at w = 1, 2.9 at w = 2.7, 8.6 at w = 10.8; it orders 1-, 2- and
+    4-turn sub-blocks of 1,000 to 16,384 particles as measured)."""
+    return max(1.0, 0.55 + 0.76 * lanes / (64.0 * simds))
 
 
 def sweep_plan(npart: int, block_turns, simds: int) -> int:

@@ -471,7 +471,7 @@ __device__ __noinline__ void element_rev_call(V6* rp, V6* lp, cDevElem* h, cAdjE
 // grid: x over the particles of the largest item, y over the items; lanes
 // beyond an item's particle count idle with zero adjoint (a workgroup with
 // none of its particles returns at once: the kernel has no barrier)
-__global__ void __launch_bounds__(64, 4) adjoint_kernel(AdjArgs args) {
+__global__ void __launch_bounds__(256, 2) adjoint_kernel(AdjArgs args) {
   cAdjItem& it = ((cAdjItem*)args.items)[blockIdx.y];
   const int npart = it.npart;
   if ((int)(blockIdx.x * blockDim.x) >= npart) return;
@@ -567,9 +567,14 @@ __global__ void __launch_bounds__(64, 4) adjoint_kernel(AdjArgs args) {
 // device item table); nitems <= 65535 (grid y limit)
 extern "C" hipError_t atx_launch_adjoint(const atx::AdjArgs* args, int32_t max_npart,
                                          hipStream_t stream) {
-  // single waves: the launches of a parallel sweep have one to three waves per
-  // SIMD, which the dispatcher spreads more evenly one by one
-  const int block = 64;
+  // Few waves run one to a workgroup, each on a CU that it shares with as few as
+  // possible (4,096 particles: 2.29 ms per turn, 2.51 in workgroups of four);
+  // from about two per CU on, a workgroup of four puts one on each SIMD of a
+  // CU, where single ones pile up (65,536 particles: 2.8 ms, 3.6 one by one).
+  // Two waves per SIMD suffice: with registers for four the sweep is 3 to 5 %
+  // slower at every size from 64 to 11,000 waves.
+  const int64_t waves = (int64_t)((max_npart + 63) / 64) * args->nitems;
+  const int block = waves <= 512 ? 64 : 256;
   const int nblocks = (max_npart + block - 1) / block;
   if (nblocks == 0 || args->nitems <= 0) return hipSuccess;
   hipLaunchKernelGGL(atx::adj::adjoint_kernel, dim3(nblocks, args->nitems), dim3(block), 0, stream,
