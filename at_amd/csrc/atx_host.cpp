@@ -102,11 +102,22 @@ struct HostElem {
   std::string pass;
   std::string fam;
   int kind = 0;
-  std::map<std::string, Attr> attrs;
+  // about ten per element, looked up by their names some thirty times in a
+  // compilation: a search through a row of them, without a key to build
+  std::vector<std::pair<std::string, Attr>> attrs;
 
   const Attr* get(const char* n) const {
-    auto it = attrs.find(n);
-    return it == attrs.end() ? nullptr : &it->second;
+    for (const auto& a : attrs)
+      if (a.first == n) return &a.second;
+    return nullptr;
+  }
+  void set(const char* n, Attr&& v) {
+    for (auto& a : attrs)
+      if (a.first == n) {
+        a.second = std::move(v);
+        return;
+      }
+    attrs.emplace_back(n, std::move(v));
   }
 };
 
@@ -1330,25 +1341,72 @@ int atx_lattice_destroy(atx_lattice* lat) {
   return ATX_OK;
 }
 
-int atx_lattice_add_element(atx_lattice* lat, const char* pass_method, const char* fam_name) {
-  if (!lat || !pass_method) return fail(ATX_E_VALUE, "NULL argument");
-  for (const auto& p : kPasses) {
-    if (std::strcmp(p.name, pass_method) == 0) {
-      std::lock_guard<std::mutex> g(lat->mu);
-      HostElem e;
-      e.pass = pass_method;
-      e.fam = fam_name ? fam_name : "";
-      e.kind = p.kind;
-      lat->elems.push_back(std::move(e));
-      lat->invalidate();
-      return (int)ATX_OK;
-    }
-  }
+// Kind of a pass method, -1 when there is none of that name.
+static int pass_kind(const char* pass_method) {
+  for (const auto& p : kPasses)
+    if (std::strcmp(p.name, pass_method) == 0) return p.kind;
+  return -1;
+}
+
+static int unknown_pass(const atx_lattice* lat, const char* pass_method, const char* fam_name) {
   return fail(ATX_E_RUNTIME, std::string("Not implemented PassMethod: ") + pass_method +
                                  " in element #" + std::to_string(lat->elems.size()) + " (" +
                                  (fam_name ? fam_name : "") + ")");
 }
 
+int atx_lattice_add_element(atx_lattice* lat, const char* pass_method, const char* fam_name) {
+  if (!lat || !pass_method) return fail(ATX_E_VALUE, "NULL argument");
+  const int kind = pass_kind(pass_method);
+  if (kind < 0) return unknown_pass(lat, pass_method, fam_name);
+  std::lock_guard<std::mutex> g(lat->mu);
+  HostElem e;
+  e.pass = pass_method;
+  e.fam = fam_name ? fam_name : "";
+  e.kind = kind;
+  lat->elems.push_back(std::move(e));
+  lat->invalidate();
+  return (int)ATX_OK;
+}
+
+int atx_lattice_add_elements(atx_lattice* lat, int32_t n, const char* const* strings,
+                             int32_t nstrings, const int32_t* elems, const int32_t* attrs,
+                             int64_t nattrs, const double* values, int64_t nvalues) {
+  g_err.clear();
+  if (!lat) return fail(ATX_E_VALUE, "NULL lattice");
+  if (n < 0 || nstrings < 0 || nattrs < 0 || nvalues < 0) return fail(ATX_E_VALUE, "negative count");
+  if (n == 0) return ATX_OK;
+  if (!strings || !elems || (nattrs > 0 && !attrs) || (nvalues > 0 && !values))
+    return fail(ATX_E_VALUE, "NULL argument");
+  std::lock_guard<std::mutex> g(lat->mu);
+  std::vector<int> kinds(nstrings, -2);  // of the strings that are pass methods
+  int64_t at = 0, v = 0;
+  lat->elems.reserve(lat->elems.size() + n);
+  lat->invalidate();
+  for (int32_t i = 0; i < n; i++) {
+    const int32_t ps = elems[3 * i], fs = elems[3 * i + 1], count = elems[3 * i + 2];
+    if (ps < 0 || ps >= nstrings || fs < 0 || fs >= nstrings || count < 0 || count > nattrs - at)
+      return fail(ATX_E_VALUE, "element table out of range");
+    if (kinds[ps] == -2) kinds[ps] = pass_kind(strings[ps]);
+    if (kinds[ps] < 0) return unknown_pass(lat, strings[ps], strings[fs]);
+    HostElem e;
+    e.pass = strings[ps];
+    e.fam = strings[fs];
+    e.kind = kinds[ps];
+    e.attrs.reserve(count);
+    for (int32_t k = 0; k < count; k++, at++) {
+      const int32_t name = attrs[2 * at] >> 1, len = attrs[2 * at + 1];
+      if (name < 0 || name >= nstrings || len < 0 || len > nvalues - v)
+        return fail(ATX_E_VALUE, "attribute table out of range");
+      Attr a;
+      a.v.assign(values + v, values + v + len);
+      a.is_int = (attrs[2 * at] & 1) != 0;
+      v += len;
+      e.set(strings[name], std::move(a));
+    }
+    lat->elems.push_back(std::move(e));
+  }
+  return ATX_OK;
+}
 static int set_attr(atx_lattice* lat, const char* name, const double* v, int64_t n, bool is_int) {
   if (!lat || !name) return fail(ATX_E_VALUE, "NULL argument");
   if (lat->elems.empty()) return fail(ATX_E_VALUE, "no element to set an attribute on");
@@ -1357,7 +1415,7 @@ static int set_attr(atx_lattice* lat, const char* name, const double* v, int64_t
   Attr a;
   a.v.assign(v, v + n);
   a.is_int = is_int;
-  lat->elems.back().attrs[name] = std::move(a);
+  lat->elems.back().set(name, std::move(a));
   lat->invalidate();
   return ATX_OK;
 }
@@ -1748,7 +1806,7 @@ int atx_element_set_array_at(atx_lattice* lat, int32_t index, const char* name, 
   if (index < 0 || index >= (int32_t)lat->elems.size()) return fail(ATX_E_VALUE, "element index out of range");
   Attr a;
   a.v.assign(data, data + n);
-  lat->elems[index].attrs[name] = std::move(a);
+  lat->elems[index].set(name, std::move(a));
   lat->invalidate();
   return ATX_OK;
 }

@@ -8,6 +8,7 @@ only compute path: importing this module raises when it is missing.
 
 from __future__ import annotations
 
+import array
 import atexit
 import ctypes as C
 import os
@@ -36,6 +37,7 @@ ATX_REPACK = 0x20
 # Exported symbols, as declared in include/atx.h.
 EXPORTS = (
     "atx_last_error", "atx_lattice_create", "atx_lattice_destroy", "atx_lattice_add_element",
+    "atx_lattice_add_elements",
     "atx_element_set_double", "atx_element_set_int", "atx_element_set_array",
     "atx_lattice_num_elements", "atx_lattice_check", "atx_track", "atx_elempass",
     "atx_track_batch", "atx_lattice_turn_counter", "atx_device_count", "atx_device_info",
@@ -131,6 +133,9 @@ def load_library(path: str | None = None) -> C.CDLL:
         lib.atx_lattice_create.argtypes = [C.POINTER(C.c_void_p)]
         lib.atx_lattice_destroy.argtypes = [C.c_void_p]
         lib.atx_lattice_add_element.argtypes = [C.c_void_p, C.c_char_p, C.c_char_p]
+        lib.atx_lattice_add_elements.argtypes = [C.c_void_p, C.c_int32, C.POINTER(C.c_char_p),
+                                                 C.c_int32, C.c_void_p, C.c_void_p, C.c_int64,
+                                                 C.c_void_p, C.c_int64]
         lib.atx_element_set_double.argtypes = [C.c_void_p, C.c_char_p, C.c_double]
         lib.atx_element_set_int.argtypes = [C.c_void_p, C.c_char_p, C.c_int64]
         lib.atx_element_set_array.argtypes = [C.c_void_p, C.c_char_p, _dp, C.c_int64]
@@ -213,24 +218,76 @@ def _check(rc: int, lib) -> None:
 _SKIP = {"FamName", "PassMethod", "Class"}
 
 
-def _send_attribute(lib, h, name: str, value) -> None:
-    if name in _SKIP or name.startswith("_"):
-        return
-    bname = name.encode()
-    if isinstance(value, (bool, np.bool_)):
-        _check(lib.atx_element_set_int(h, bname, int(value)), lib)
-    elif isinstance(value, (int, np.integer)):
-        _check(lib.atx_element_set_int(h, bname, int(value)), lib)
-    elif isinstance(value, (float, np.floating)):
-        _check(lib.atx_element_set_double(h, bname, float(value)), lib)
-    elif isinstance(value, np.ndarray) and value.dtype.kind in "fiub":
-        a = np.asarray(value, dtype=np.float64)
-        a = np.ascontiguousarray(a.ravel(order="F"))
-        _check(lib.atx_element_set_array(h, bname, a.ctypes.data_as(_dp), a.size), lib)
-    elif isinstance(value, (list, tuple)) and all(isinstance(v, (int, float)) for v in value):
-        a = np.ascontiguousarray(np.asarray(value, dtype=np.float64))
-        _check(lib.atx_element_set_array(h, bname, a.ctypes.data_as(_dp), a.size), lib)
-    # other attribute types (strings, objects) carry no pass-method parameter
+def _number_or_array(value):
+    """(is an integer, values) of an attribute that carries a pass-method
+    parameter, None for strings and objects."""
+    if isinstance(value, (bool, np.bool_, int, np.integer)):
+        v = int(value)
+        if not -(1 << 63) <= v < 1 << 63:
+            v = (v + (1 << 63)) % (1 << 64) - (1 << 63)
+        return 1, [float(v)]
+    if isinstance(value, (float, np.floating)):
+        return 0, [float(value)]
+    if isinstance(value, np.ndarray) and value.dtype.kind in "fiub":
+        return 0, np.asarray(value, dtype=np.float64).ravel(order="F").tolist()
+    if isinstance(value, (list, tuple)) and all(isinstance(v, (int, float)) for v in value):
+        return 0, np.asarray(value, dtype=np.float64).tolist()
+    return None
+
+
+class _Packed:
+    """The tables of atx_lattice_add_elements for a sequence of elements."""
+
+    def __init__(self):
+        self.strings: dict[str, int] = {}
+        self.elems: list[int] = []
+        self.attrs: list[int] = []
+        self.values: list[float] = []
+
+    def add(self, elements) -> None:
+        strings, attrs, values = self.strings, self.attrs, self.values
+        string = lambda t: strings.setdefault(t, len(strings))  # noqa: E731
+        names: dict[str, int] = {}  # attribute name -> string, -1: never sent
+        f64, ndarray = np.dtype(np.float64), np.ndarray
+        for index, e in enumerate(elements):
+            pm = getattr(e, "PassMethod", None)
+            if pm is None:
+                raise AttributeError(f"Element #{index} has no PassMethod")
+            if type(pm) is not str:
+                pm = pm.encode().decode()
+            first = len(attrs)
+            for name, value in vars(e).items():
+                k = names.get(name)
+                if k is None:
+                    skip = name in _SKIP or name.startswith("_")
+                    k = names[name] = -1 if skip else 2 * string(name)
+                if k < 0:
+                    continue
+                kind = type(value)
+                if kind is float:
+                    values.append(value)
+                    attrs += k, 1
+                elif kind is ndarray and value.dtype is f64 and value.ndim == 1:
+                    v = value.tolist()
+                    values += v
+                    attrs += k, len(v)
+                else:
+                    got = _number_or_array(value)
+                    if got is not None:
+                        values += got[1]
+                        attrs += k + got[0], len(got[1])
+            self.elems += (string(pm), string(str(getattr(e, "FamName", ""))),
+                           (len(attrs) - first) // 2)
+
+    def send(self, lib, h) -> int:
+        texts = (C.c_char_p * len(self.strings))(*[t.encode() for t in self.strings])
+        elems, attrs = array.array("i", self.elems), array.array("i", self.attrs)
+        values = array.array("d", self.values)
+        n = len(elems) // 3
+        _check(lib.atx_lattice_add_elements(h, n, texts, len(texts), elems.buffer_info()[0],
+                                            attrs.buffer_info()[0], len(attrs) // 2,
+                                            values.buffer_info()[0], len(values)), lib)
+        return n
 
 
 class DeviceLattice:
@@ -244,17 +301,14 @@ class DeviceLattice:
         self.nelem = 0
         self.integrator = 4
         try:
-            for i, e in enumerate(elements):
-                pm = getattr(e, "PassMethod", None)
-                if pm is None:
-                    raise AttributeError(f"Element #{i} has no PassMethod")
-                fam = str(getattr(e, "FamName", ""))
-                rc = self.lib.atx_lattice_add_element(h, pm.encode(), fam.encode())
-                if rc != ATX_OK:
-                    _raise(rc, self.lib)
-                for name, value in vars(e).items():
-                    _send_attribute(self.lib, h, name, value)
-                self.nelem += 1
+            # one call for all elements: an attribute sent by itself costs about
+            # 0.8 us, and a ring has thousands (2,241 elements: 10.5 ms, 2.6 in one)
+            packed = _Packed()
+            try:
+                packed.add(elements)
+            finally:
+                # an element that cannot be packed: those before it are checked first
+                self.nelem = packed.send(self.lib, h)
         except Exception:
             self.close()
             raise

@@ -67,6 +67,15 @@ const char *atx_last_error(void);
 int atx_lattice_create(atx_lattice **out);
 int atx_lattice_destroy(atx_lattice *lat);
 int atx_lattice_add_element(atx_lattice *lat, const char *pass_method, const char *fam_name);
+/* Many elements and their attributes in one call (a ring of 2,241 elements has
+ * 13,000). strings: a table of texts; elems: three entries per element, the
+ * strings of its pass method and family name and its number of attributes;
+ * attrs: two per attribute, in the elements' order, 2 x the string of its name
+ * (+ 1: an integer) and its number of values; values: theirs, in that order.
+ * An unknown pass method ends the call; the elements before it are added. */
+int atx_lattice_add_elements(atx_lattice *lat, int32_t n, const char *const *strings,
+                             int32_t nstrings, const int32_t *elems, const int32_t *attrs,
+                             int64_t nattrs, const double *values, int64_t nvalues);
 int atx_element_set_double(atx_lattice *lat, const char *name, double value);
 int atx_element_set_int(atx_lattice *lat, const char *name, int64_t value);
 int atx_element_set_array(atx_lattice *lat, const char *name, const double *data, int64_t n);
