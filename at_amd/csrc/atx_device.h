@@ -125,7 +125,7 @@ static_assert(sizeof(DevElem) == 64, "DevElem must stay 64 bytes (dword fields: 
 // index of the last of them. The constants an op needs are in the record
 // itself, at fixed offsets, so that no address depends on an earlier load. A
 // terminal record follows the last one: the kernel reads the head (the first
-// 16 bytes) one record ahead.
+// 32 bytes) one record ahead.
 enum OpKind : int32_t {
   OP_NONE = 0,      // no element after the markers and the drift
   OP_GENERIC = 1,   // the element by its DevElem header
@@ -178,8 +178,8 @@ struct LatOp {
   int32_t last;    // index of the record's last element
   double len;      // the drift's length
   int32_t first;   // index of its first element (the next record's: one past its last)
-  int32_t nslice;
-  int32_t pad[2];
+  int32_t nslice;  // at least 1 (thick multipoles)
+  double lead;     // their B[order]
   double c[kOpConsts];
 };
 static_assert(sizeof(LatOp) == 256, "LatOp: four 64-byte lines");

@@ -668,7 +668,7 @@ void fill_op(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
     r.c[OT_BAY] = sc[S_BAY];
     for (int k = 0; k < 2 * (h.order + 1); k++) r.c[OM_POLY + k] = pool[h.poly + k];
   } else if ((h.kind == K_STR || h.kind == K_BND || h.kind == K_STRRAD || h.kind == K_BNDRAD) &&
-             !(h.flags & (F_RAP | F_EAP | F_SCALE)) && h.fringe == 0 && h.ops < 0) {
+             !(h.flags & (F_RAP | F_EAP | F_SCALE)) && h.fringe == 0 && h.ops < 0 && h.nslice > 0) {
     int op = OP_GENERIC;
     if (h.kind == K_STR && h.order >= 1 && h.order <= 3) op = OP_STR1 + (h.order - 1);
     if (h.order == 1) {
@@ -713,6 +713,7 @@ void fill_op(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
     if ((h.edge & 0xff) != E_CONST || ((h.edge >> 8) & 0xff) != E_CONST) op |= OPF_EDGE;
     r.op = drift | op;
     r.nslice = h.nslice;
+    r.lead = b[h.order];
     static const int from[8] = {S_L1, S_L2, S_K1, S_K2, S_IRHO, S_RADC, S_RK1, S_RK2};
     for (int k = 0; k < 8; k++) r.c[k] = sc[from[k]];
     for (int k = 0; k < 2 * (h.order + 1); k++) r.c[OM_POLY + k] = pool[h.poly + k];

@@ -106,7 +106,8 @@ __device__ __forceinline__ void change_pref(R6& r, double s) { r = change_pref_v
 
 // Apertures are decisions: evaluated without contraction in both builds so
 // that the loss element is the reference's (atlalib.c:164-190).
-__device__ __forceinline__ void rect_ap(R6& r, cdouble* lim) {
+template <class L>
+__device__ __forceinline__ void rect_ap(R6& r, const L& lim) {
 #pragma clang fp contract(off)
   const bool out = (r.x < lim[0]) | (r.x > lim[1]) | (r.y < lim[2]) | (r.y > lim[3]);
   r.ct = out ? __builtin_inf() : r.ct;
@@ -570,6 +571,7 @@ __device__ __forceinline__ void fastdrift_h(R6& r, double nl, double nlh) {
 // added where that costs nothing (radiating kicks) or once per magnet.
 struct Kick {
   double kl, kli;         // length, length times curvature
+  double bn;              // B[N]
   double kb, kb2;         // kl B[N], twice that
   double kb0, ka0;        // kl B[0], kl A[0]
   double lo;              // remainder of kb (NOFIELD: of kli)
@@ -577,15 +579,16 @@ struct Kick {
 };
 
 template <bool BEND, int N, int F>
-__device__ __forceinline__ Kick kick_of(cdouble* a, cdouble* b, double kl, double irho, double radk) {
+__device__ __forceinline__ Kick kick_of(cdouble* a, cdouble* b, double lead, double kl, double irho,
+                                        double radk) {
   Kick k;
   k.kl = kl;
   k.kli = BEND ? kl * irho : 0.0;
   k.kb = k.kb2 = k.kb0 = k.ka0 = k.lo = 0.0;
   if (F == F_LEAD || F == F_LEAD0) {
-    k.kb = kl * b[N];
+    k.kb = kl * lead;
     k.kb2 = 2.0 * k.kb;
-    k.lo = __builtin_fma(kl, b[N], -k.kb);
+    k.lo = __builtin_fma(kl, lead, -k.kb);
   }
   if (F == F_NOFIELD) k.lo = __builtin_fma(kl, irho, -k.kli);
   if (F == F_LEAD0) {
@@ -593,7 +596,8 @@ __device__ __forceinline__ Kick kick_of(cdouble* a, cdouble* b, double kl, doubl
     k.ka0 = kl * a[0];
   }
   k.rk = radk;
-  if (F == F_LEAD && !BEND) k.rk = radk * (b[N] * b[N]);
+  k.bn = lead;
+  if (F == F_LEAD && !BEND) k.rk = radk * (lead * lead);
   if (F == F_NOFIELD) k.rk = radk * (irho * irho);
   return k;
 }
@@ -706,8 +710,8 @@ __device__ __forceinline__ void rad_kick_ang(R6& r, Ang& g, const Kick& k, cdoub
   double re = 0.0, im = 0.0;
   if (F == F_GENERAL) field<N>(r, a, b, n, blo, alo, re, im);
   if (BEND && F == F_LEAD) {
-    re = b[1] * x;
-    im = b[1] * y;
+    re = k.bn * x;
+    im = k.bn * y;
   }
   double w;
   bool odd = false;
@@ -749,7 +753,9 @@ __device__ __forceinline__ void rad_kick_ang(R6& r, Ang& g, const Kick& k, cdoub
   if (CHECKED) {
     if (__builtin_amdgcn_ballot_w64(far) != 0) pn = far ? fast_rcp(1.0 + r.dp) : pn;
   } else {
-    bad |= __builtin_amdgcn_ballot_w64(odd | far);
+    // (a ballot each: of their union the compiler makes two more instructions)
+    if (!BEND) bad |= __builtin_amdgcn_ballot_w64(odd);
+    bad |= __builtin_amdgcn_ballot_w64(far);
   }
   if (!BEND && F == F_LEAD) {
     const double kn = __builtin_fma(k.kb, pn, k.lo);  // lo pn, to a relative delta
@@ -833,15 +839,15 @@ __device__ __forceinline__ void hold(double v) { asm volatile("" ::"s"(v)); }
 // times larger, so known answers of the reference hold that rounding.
 template <bool BEND, int N, int F, int P, int U, class Ahead>
 __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int n, int nslice,
-                                             const double* nl1, const double* nl2, double k1,
-                                             double k2, double irho, const Ahead& ahead) {
+                                             double lead, const double* nl1, const double* nl2,
+                                             double k1, double k2, double irho,
+                                             const Ahead& ahead) {
   double blo, alo;
   horner_addends<N>(a, b, n, blo, alo);
   if (F == F_GENERAL && N == 3) ahead(k1, k2, a[3], b[3], a[2], b[2], a[1], b[1], a[0], b[0]);
   else if (F == F_GENERAL && N == 2) ahead(k1, k2, a[2], b[2], a[1], b[1], a[0], b[0]);
   else if (F == F_GENERAL && N == 1) ahead(k1, k2, a[1], b[1], a[0], b[0]);
-  else if (F == F_LEAD0) ahead(k1, k2, b[N], a[0], b[0]);
-  else if (F == F_LEAD) ahead(k1, k2, b[N]);
+  else if (F == F_LEAD0) ahead(k1, k2, a[0], b[0]);
   else ahead(k1, k2);
 #if ATX_STRICT
   const double ki1 = k1 * irho, ki2 = k2 * irho;
@@ -877,9 +883,8 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
   }
   for (; m < nslice; m++) slice();
 #else
-  if (nslice <= 0) return;
-  const Kick c1 = kick_of<BEND, N, F>(a, b, k1, irho, 0.0);
-  const Kick c2 = kick_of<BEND, N, F>(a, b, k2, irho, 0.0);
+  const Kick c1 = kick_of<BEND, N, F>(a, b, lead, k1, irho, 0.0);
+  const Kick c2 = kick_of<BEND, N, F>(a, b, lead, k2, irho, 0.0);
   double nh1[P], nh2[P], nl12[P];  // delta is constant through the slices
 #pragma unroll
   for (int q = 0; q < P; q++) {
@@ -937,14 +942,13 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
 // BndMPoleSymplectic4RadPass.c:98-112, likewise. CHECKED, bad: rad_kick_ang.
 template <bool BEND, int N, int F, int P, int U, bool CHECKED, class Ahead>
 __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, int n, int nslice,
-                                                 double l1, double l2, double k1, double k2,
-                                                 double irho, double radc, double rk1, double rk2,
+                                                 double lead, double l1, double l2, double k1,
+                                                 double k2, double irho, double radc, double rk1, double rk2,
                                                  uint64_t& bad, const Ahead& ahead) {
   double blo, alo;
   horner_addends<N>(a, b, n, blo, alo);
   const double rk = ATX_STRICT ? radc : rk1;
   if (F == F_GENERAL && N == 1) ahead(l1, l2, k1, k2, rk, rk2, a[1], b[1], a[0], b[0]);
-  else if (F == F_LEAD) ahead(l1, l2, k1, k2, rk, rk2, b[N]);
   else ahead(l1, l2, k1, k2, rk, rk2);
 #if ATX_STRICT
   const double ki1 = k1 * irho, ki2 = k2 * irho;
@@ -984,9 +988,8 @@ __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, 
   }
   for (; m < nslice; m++) slice();
 #else
-  if (nslice <= 0) return;
-  const Kick c1 = kick_of<BEND, N, F>(a, b, k1, irho, rk1);
-  const Kick c2 = kick_of<BEND, N, F>(a, b, k2, irho, rk2);
+  const Kick c1 = kick_of<BEND, N, F>(a, b, lead, k1, irho, rk1);
+  const Kick c2 = kick_of<BEND, N, F>(a, b, lead, k2, irho, rk2);
   const double hl1 = 0.5 * l1, hl2 = 0.5 * l2, l12 = 2.0 * l1;
   Ang g[P];
 #pragma unroll
@@ -1062,8 +1065,8 @@ __device__ __forceinline__ void mpole(R6* r, cDevElem& h, cdouble* pool) {
 #pragma unroll
     for (int q = 0; q < P; q++)
       r[q] = slices_ops<BEND, false>(r[q], a, b, n, pool + h.ops, h.nslice, pn[q], irho, 0.0);
-  } else {
-    mpole_slices<BEND, N, F_GENERAL, P, U>(r, a, b, n, h.nslice, nl1, nl2, s[S_K1], s[S_K2], irho,
+  } else if (h.nslice > 0) {
+    mpole_slices<BEND, N, F_GENERAL, P, U>(r, a, b, n, h.nslice, 0.0, nl1, nl2, s[S_K1], s[S_K2], irho,
                                           NotAhead());
   }
 #pragma unroll
@@ -1089,9 +1092,9 @@ __device__ __forceinline__ void mpole_rad(R6* r, cDevElem& h, cdouble* pool) {
 #pragma unroll
     for (int q = 0; q < P; q++)
       r[q] = slices_ops<BEND, true>(r[q], a, b, n, pool + h.ops, h.nslice, 0.0, irho, radc);
-  } else {
+  } else if (h.nslice > 0) {
     uint64_t bad = 0;
-    mpole_rad_slices<BEND, N, F_GENERAL, P, U, true>(r, a, b, n, h.nslice, s[S_L1], s[S_L2], s[S_K1],
+    mpole_rad_slices<BEND, N, F_GENERAL, P, U, true>(r, a, b, n, h.nslice, 0.0, s[S_L1], s[S_L2], s[S_K1],
                                                      s[S_K2], irho, radc, s[S_RK1], s[S_RK2], bad,
                                                      NotAhead());
   }
@@ -1724,21 +1727,20 @@ __device__ __forceinline__ R6 generic_element(const R6& r, cDevElem& h, cdouble*
   }
 }
 
-// at.c:115-139 predicate: any coordinate not finite, or |r_n| > 1 for n < 5.
-// Without short circuits: six compares and mask logic, no branch.
-__device__ __forceinline__ bool is_lost(const R6& r) {
-  const bool ok = (__builtin_fabs(r.x) <= 1.0) & (__builtin_fabs(r.px) <= 1.0) &
-                  (__builtin_fabs(r.y) <= 1.0) & (__builtin_fabs(r.py) <= 1.0) &
-                  (__builtin_fabs(r.dp) <= 1.0) & (__builtin_fabs(r.ct) < __builtin_inf());
-  return !ok;
+// at.c:115-139 predicate: any coordinate not finite, or |r_n| > 1 for n < 5, as
+// the lanes of the wave that fail it: a ballot per compare is one instruction, a
+// ballot of their union takes two more. After a drift of a particle that passed
+// the test before it, px, py and delta are unchanged.
+__device__ __forceinline__ uint64_t lost_lanes_drift(const R6& r) {
+  return __builtin_amdgcn_ballot_w64(!(__builtin_fabs(r.x) <= 1.0)) |
+         __builtin_amdgcn_ballot_w64(!(__builtin_fabs(r.y) <= 1.0)) |
+         __builtin_amdgcn_ballot_w64(!(__builtin_fabs(r.ct) < __builtin_inf()));
 }
 
-// The same after a drift of a particle that passed the test before it:
-// px, py and delta are unchanged.
-__device__ __forceinline__ bool is_lost_drift(const R6& r) {
-  const bool ok = (__builtin_fabs(r.x) <= 1.0) & (__builtin_fabs(r.y) <= 1.0) &
-                  (__builtin_fabs(r.ct) < __builtin_inf());
-  return !ok;
+__device__ __forceinline__ uint64_t lost_lanes(const R6& r) {
+  return lost_lanes_drift(r) | __builtin_amdgcn_ballot_w64(!(__builtin_fabs(r.px) <= 1.0)) |
+         __builtin_amdgcn_ballot_w64(!(__builtin_fabs(r.py) <= 1.0)) |
+         __builtin_amdgcn_ballot_w64(!(__builtin_fabs(r.dp) <= 1.0));
 }
 
 // An edge of a bend by its header.
@@ -1754,14 +1756,45 @@ __device__ __noinline__ R6 edge_call(R6 r, cDevElem* hp, cdouble* poolp, int exi
   return r;
 }
 
+// Head of a program record, read one record ahead: its flags and op, the
+// index of its last element, its drift's length, its number of slices and
+// leading coefficient, its first constants. It holds a word of the record's next
+// two lines, too: reading them brings the lines into the scalar cache.
+struct OpConsts {
+  double v[8];
+};
+struct OpHead {
+  int op, last;
+  double len;
+  int first, nslice;
+  double lead;
+  OpConsts k;
+  int line1, line2;
+};
+
+__device__ __forceinline__ OpConsts op_consts(cLatOp* p) {
+  OpConsts k;
+#pragma unroll
+  for (int i = 0; i < 8; i++) k.v[i] = p->c[i];
+  return k;
+}
+
+__device__ __forceinline__ OpHead op_head(cLatOp* p) {
+  return OpHead{p->op, p->last, p->len, p->first, p->nslice, p->lead, op_consts(p),
+                ((cint*)p)[16], ((cint*)p)[32]};
+}
+
 // A thick multipole by its record; the misalignment is applied around it by
 // the caller. CHECKED, bad: rad_kick_ang.
 template <bool BEND, bool RAD, int N, int F, int P, int U, bool CHECKED, class Ahead>
-__device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flags, cDevElem* h,
-                                         cdouble* pool, uint64_t& bad, const Ahead& ahead) {
+__device__ __forceinline__ void mpole_op(R6* r, const OpHead& o, cdouble* c, cDevElem* h,
+                                         cdouble* pool, uint64_t& bad,
+                                         const Ahead& ahead) {
   cdouble* a = c + OM_POLY;
   cdouble* b = a + N + 1;
-  const double irho = BEND ? c[OM_IRHO] : 0.0;
+  const int nslice = o.nslice, flags = o.op;
+  const OpConsts& k = o.k;
+  const double irho = BEND ? k.v[OM_IRHO] : 0.0;
   if (BEND) {
 #pragma unroll
     for (int q = 0; q < P; q++) {
@@ -1774,18 +1807,19 @@ __device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flag
     }
   }
   if (RAD) {
-    mpole_rad_slices<BEND, N, F, P, U, CHECKED>(r, a, b, N, nslice, c[OM_L1], c[OM_L2], c[OM_K1],
-                                                c[OM_K2], irho, c[OM_RADC], c[OM_RK1], c[OM_RK2],
-                                                bad, ahead);
+    mpole_rad_slices<BEND, N, F, P, U, CHECKED>(r, a, b, N, nslice, o.lead, k.v[OM_L1], k.v[OM_L2],
+                                                k.v[OM_K1], k.v[OM_K2], irho, k.v[OM_RADC],
+                                                k.v[OM_RK1], k.v[OM_RK2], bad, ahead);
   } else {
     double nl1[P], nl2[P];
 #pragma unroll
     for (int q = 0; q < P; q++) {
       const double pn = rcp_opd(r[q]);
-      nl1[q] = c[OM_L1] * pn;
-      nl2[q] = c[OM_L2] * pn;
+      nl1[q] = k.v[OM_L1] * pn;
+      nl2[q] = k.v[OM_L2] * pn;
     }
-    mpole_slices<BEND, N, F, P, U>(r, a, b, N, nslice, nl1, nl2, c[OM_K1], c[OM_K2], irho, ahead);
+    mpole_slices<BEND, N, F, P, U>(r, a, b, N, nslice, o.lead, nl1, nl2, k.v[OM_K1], k.v[OM_K2], irho,
+                                   ahead);
   }
   if (BEND) {
 #pragma unroll
@@ -1802,11 +1836,11 @@ __device__ __forceinline__ void mpole_op(R6* r, cdouble* c, int nslice, int flag
 
 // ThinMPolePass.c:42-63 by its record.
 template <int N>
-__device__ __forceinline__ void thin_op(R6& r, cdouble* c) {
+__device__ __forceinline__ void thin_op(R6& r, const OpConsts& k, cdouble* c) {
   cdouble* a = c + OM_POLY;
   cdouble* b = a + N + 1;
   str_kick<N>(r, a, b, N, b[N - 1], a[N - 1], 1.0);
-  const double bax = c[OT_BAX], bay = c[OT_BAY];
+  const double bax = k.v[OT_BAX], bay = k.v[OT_BAY];
   r.px += bax * r.dp;
   r.py -= bay * r.dp;
   r.ct -= bax * r.x - bay * r.y;
@@ -1838,9 +1872,12 @@ __device__ __forceinline__ void roll(R6& r, double c, double s) {
 // The element of a record other than its markers and drift, for the P
 // particles of a lane. CHECKED, bad: rad_kick_ang; ahead: NotAhead.
 template <int P, int U, bool CHECKED, class Ahead>
-__device__ __forceinline__ void run_op(R6* r, int op, cLatOp* rec, cDevElem* h, cdouble* pool,
-                                       int nturn, uint64_t& bad, const Ahead& ahead) {
+__device__ __forceinline__ void run_op(R6* r, const OpHead& o, cLatOp* rec, cDevElem* h,
+                                       cdouble* pool, int nturn, uint64_t& bad,
+                                       const Ahead& ahead) {
   cdouble* c = rec->c;
+  const OpConsts& k = o.k;
+  const int op = o.op;
   if (op & OPF_XF) {
 #pragma unroll
     for (int q = 0; q < P; q++) {
@@ -1851,67 +1888,84 @@ __device__ __forceinline__ void run_op(R6* r, int op, cLatOp* rec, cDevElem* h, 
       roll(r[q], c[OM_XF + 4], c[OM_XF + 5]);
     }
   }
-  const int nslice = rec->nslice;
 #define ATX_MPOLE(BEND, RAD, N, F) \
-  mpole_op<BEND, RAD, N, F, P, U, CHECKED>(r, c, nslice, op, h, pool, bad, ahead)
-  switch (op & 0xff) {
-#if ATX_STRICT  // all coefficients, whatever the form
-    case OP_STR1: case OP_STR1L: ATX_MPOLE(false, false, 1, F_GENERAL); break;
-    case OP_STR2: case OP_STR2L: case OP_STR2D: ATX_MPOLE(false, false, 2, F_GENERAL); break;
-    case OP_STR3: case OP_STR3L: ATX_MPOLE(false, false, 3, F_GENERAL); break;
-    case OP_BND1: case OP_BND1L: case OP_BND0: ATX_MPOLE(true, false, 1, F_GENERAL); break;
-    case OP_STRRAD1: case OP_STRRAD1L: ATX_MPOLE(false, true, 1, F_GENERAL); break;
-    case OP_BNDRAD1: case OP_BNDRAD1L: case OP_BNDRAD0: ATX_MPOLE(true, true, 1, F_GENERAL); break;
+  mpole_op<BEND, RAD, N, F, P, U, CHECKED>(r, o, c, h, pool, bad, ahead)
+  // One bit per kind, tested in groups and in the order of how common they are:
+  // a test that fails falls through, where a switch becomes a tree of five
+  // levels with a taken branch at most of them. (The shift is opaque, as the
+  // tests would be turned into that switch.)
+  uint32_t sel;
+  asm("s_lshl_b32 %0, 1, %1" : "=s"(sel) : "s"(op & 0xff) : "scc");
+  auto is = [&](auto... k) { return (sel & ((1u << k) | ...)) != 0; };
+#if ATX_STRICT
+  constexpr int kGen = F_GENERAL;  // all coefficients, whatever the form
+  if (is(OP_STRRAD1, OP_STRRAD1L, OP_BNDRAD1, OP_BNDRAD1L, OP_BNDRAD0)) {
+    if (is(OP_STRRAD1, OP_STRRAD1L)) ATX_MPOLE(false, true, 1, kGen);
+    else ATX_MPOLE(true, true, 1, kGen);
+  } else if (is(OP_STR1, OP_STR1L, OP_BND1, OP_BND1L, OP_BND0)) {
+    if (is(OP_STR1, OP_STR1L)) ATX_MPOLE(false, false, 1, kGen);
+    else ATX_MPOLE(true, false, 1, kGen);
+  } else if (is(OP_STR2, OP_STR2L, OP_STR2D)) {
+    ATX_MPOLE(false, false, 2, kGen);
+  } else if (is(OP_STR3, OP_STR3L)) {
+    ATX_MPOLE(false, false, 3, kGen);
 #else
-    case OP_STR1: ATX_MPOLE(false, false, 1, F_GENERAL); break;
-    case OP_STR1L: ATX_MPOLE(false, false, 1, F_LEAD); break;
-    case OP_STR2: ATX_MPOLE(false, false, 2, F_GENERAL); break;
-    case OP_STR2L: ATX_MPOLE(false, false, 2, F_LEAD); break;
-    case OP_STR2D: ATX_MPOLE(false, false, 2, F_LEAD0); break;
-    case OP_STR3: ATX_MPOLE(false, false, 3, F_GENERAL); break;
-    case OP_STR3L: ATX_MPOLE(false, false, 3, F_LEAD); break;
-    case OP_BND1: ATX_MPOLE(true, false, 1, F_GENERAL); break;
-    case OP_BND1L: ATX_MPOLE(true, false, 1, F_LEAD); break;
-    case OP_BND0: ATX_MPOLE(true, false, 1, F_NOFIELD); break;
-    case OP_STRRAD1: ATX_MPOLE(false, true, 1, F_GENERAL); break;
-    case OP_STRRAD1L: ATX_MPOLE(false, true, 1, F_LEAD); break;
-    case OP_BNDRAD1: ATX_MPOLE(true, true, 1, F_GENERAL); break;
-    case OP_BNDRAD1L: ATX_MPOLE(true, true, 1, F_LEAD); break;
-    case OP_BNDRAD0: ATX_MPOLE(true, true, 1, F_NOFIELD); break;
+  if (is(OP_STRRAD1L, OP_BNDRAD0, OP_BNDRAD1L)) {
+    if (is(OP_STRRAD1L)) ATX_MPOLE(false, true, 1, F_LEAD);
+    else if (is(OP_BNDRAD0)) ATX_MPOLE(true, true, 1, F_NOFIELD);
+    else ATX_MPOLE(true, true, 1, F_LEAD);
+  } else if (is(OP_STR1L, OP_STR2L, OP_STR2D, OP_STR3L)) {
+    if (is(OP_STR1L)) ATX_MPOLE(false, false, 1, F_LEAD);
+    else if (is(OP_STR2L)) ATX_MPOLE(false, false, 2, F_LEAD);
+    else if (is(OP_STR2D)) ATX_MPOLE(false, false, 2, F_LEAD0);
+    else ATX_MPOLE(false, false, 3, F_LEAD);
+  } else if (is(OP_BND0)) {
+    ATX_MPOLE(true, false, 1, F_NOFIELD);
+  } else if (is(OP_BND1L)) {
+    ATX_MPOLE(true, false, 1, F_LEAD);
 #endif
-    case OP_THIN2:
+  } else if (is(OP_THIN2)) {
 #pragma unroll
-      for (int q = 0; q < P; q++) thin_op<2>(r[q], c);
-      ahead();
-      break;
-    case OP_THIN3:
+    for (int q = 0; q < P; q++) thin_op<2>(r[q], k, c);
+    ahead();
+  } else if (is(OP_CORR)) {
+    ahead(k.v[OC_XK], k.v[OC_YK], k.v[OC_LEN], k.v[OC_Q0]);
 #pragma unroll
-      for (int q = 0; q < P; q++) thin_op<3>(r[q], c);
-      ahead();
-      break;
-    case OP_APERTURE:  // AperturePass.c:9-26
-#pragma unroll
-      for (int q = 0; q < P; q++) rect_ap(r[q], c);
-      ahead();
-      break;
-    case OP_CORR:
-      ahead(c[OC_XK], c[OC_YK], c[OC_LEN], c[OC_Q0]);
-#pragma unroll
-      for (int q = 0; q < P; q++) {
-        if (op & OPF_THICK) {
-          const double pn = rcp_opd(r[q]);
-          corrector_map(r[q], c[OC_XK], c[OC_YK], c[OC_Q0], c[OC_LEN] * pn, pn);
-        } else {
-          r[q].px += c[OC_XK];
-          r[q].py += c[OC_YK];
-        }
+    for (int q = 0; q < P; q++) {
+      if (op & OPF_THICK) {
+        const double pn = rcp_opd(r[q]);
+        corrector_map(r[q], k.v[OC_XK], k.v[OC_YK], k.v[OC_Q0], k.v[OC_LEN] * pn, pn);
+      } else {
+        r[q].px += k.v[OC_XK];
+        r[q].py += k.v[OC_YK];
       }
-      break;
-    default:
-      ahead();
+    }
+  } else if (is(OP_APERTURE)) {  // AperturePass.c:9-26
 #pragma unroll
-      for (int q = 0; q < P; q++) r[q] = generic_element<U>(r[q], *h, pool, nturn);
-      break;
+    for (int q = 0; q < P; q++) rect_ap(r[q], k.v);
+    ahead();
+#if !ATX_STRICT
+  } else if (is(OP_STRRAD1)) {
+    ATX_MPOLE(false, true, 1, F_GENERAL);
+  } else if (is(OP_STR1)) {
+    ATX_MPOLE(false, false, 1, F_GENERAL);
+  } else if (is(OP_STR2)) {
+    ATX_MPOLE(false, false, 2, F_GENERAL);
+  } else if (is(OP_STR3)) {
+    ATX_MPOLE(false, false, 3, F_GENERAL);
+  } else if (is(OP_BNDRAD1)) {
+    ATX_MPOLE(true, true, 1, F_GENERAL);
+  } else if (is(OP_BND1)) {
+    ATX_MPOLE(true, false, 1, F_GENERAL);
+#endif
+  } else if (is(OP_THIN3)) {
+#pragma unroll
+    for (int q = 0; q < P; q++) thin_op<3>(r[q], k, c);
+    ahead();
+  } else {
+    ahead();
+#pragma unroll
+    for (int q = 0; q < P; q++) r[q] = generic_element<U>(r[q], *h, pool, nturn);
   }
 #undef ATX_MPOLE
   if (op & OPF_XF) {
@@ -1921,7 +1975,7 @@ __device__ __forceinline__ void run_op(R6* r, int op, cLatOp* rec, cDevElem* h, 
       // a coordinate that is not finite spreads through the zeros of the
       // 6x6 product, as in the reference: the wave then takes the product
       // (the fast build runs the whole element again, op_call)
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(is_lost(r[q])) != 0 && (h->flags & F_R2), 0))
+      if (__builtin_expect(lost_lanes(r[q]) != 0 && (h->flags & F_R2), 0))
         r[q] = mul_r_v(r[q], pool + h->r2);
       else
 #endif
@@ -1947,7 +2001,7 @@ __device__ __noinline__ R6 op_call(R6 r, const LatOp* recp, cDevElem* hp, cdoubl
   const int nturn = __builtin_amdgcn_readfirstlane(nturnp);
   R6 v = r;
   uint64_t bad = 0;
-  run_op<1, 1, true>(&v, rec->op, rec, h, pool, nturn, bad, NotAhead());
+  run_op<1, 1, true>(&v, op_head(rec), rec, h, pool, nturn, bad, NotAhead());
   if (rec->op & OPF_MPOLE) {
     const bool inf = !is_finite(v);
     if (__builtin_amdgcn_ballot_w64(inf) != 0) {
@@ -2006,21 +2060,6 @@ __device__ __forceinline__ R6 lost_state() { return R6{__builtin_nan(""), 0.0, 0
 
 // What a lane without a live particle tracks: the origin.
 __device__ __forceinline__ R6 idle_state() { return R6{0.0, 0.0, 0.0, 0.0, 0.0, 0.0}; }
-
-// Head of a program record, read one record ahead: its flags and op, the
-// index of its last element, its drift's length.
-// It holds a word of each of the record's other lines, too: reading them
-// brings the lines into the scalar cache before the op asks for its
-// constants.
-struct OpHead {
-  int op, last;
-  double len;
-  int line1, line2;
-};
-
-__device__ __forceinline__ OpHead op_head(cLatOp* p) {
-  return OpHead{p->op, p->last, p->len, ((cint*)p)[16], ((cint*)p)[32]};
-}
 
 // A particle with its lane's state: what the loss handling changes.
 struct Lane {
@@ -2159,16 +2198,13 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
       alive[q] = __builtin_amdgcn_ballot_w64((fl[q] & L_ALIVE) != 0);
     }
   };
-  auto lose = [&](int q, bool lost, int e) {
-    lose_mask(q, __builtin_amdgcn_ballot_w64(lost) & alive[q], e);
-  };
   // One element outside the loop over the records, with its refpt copy and loss
   // test. A NaN input is skipped by the first element and lost at its test.
   auto by_header = [&](int e, bool entry) {
     if (REFS) copy_refs(e);
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      if (entry) lose(q, __builtin_isnan(r[q].x), e);
+      if (entry) lose_mask(q, __builtin_amdgcn_ballot_w64(__builtin_isnan(r[q].x)) & alive[q], e);
 #if !ATX_STRICT
       // in the record's form, so that a turn split into calls rounds alike
       cLatOp* rec = ops + opof[e];
@@ -2177,7 +2213,7 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
       else
 #endif
         r[q] = header_call<U>(r[q], &elems[e], pool, nturn);
-      if (check) lose(q, is_lost(r[q]), e);
+      if (check) lose_mask(q, lost_lanes(r[q]) & alive[q], e);
     }
   };
   // The loop over the records. With few waves per SIMD it is bound by the
@@ -2204,14 +2240,19 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
 #if !ATX_STRICT
   // once a radiating magnet had to be run again with the checks in its kicks,
   // the wave runs them with the checks for the rest of the turn
-  bool slow = false;
+  int slow = 0;  // OPF_RAD then
 #endif
   cLatOp* rec = ops + o0;
   cLatOp* const end = ops + max(o0, o1);
   OpHead nxt = op_head(rec);
   for (; rec != end; rec++) {
-    const OpHead cur = nxt;
+    OpHead cur = nxt;
     asm volatile("" ::"s"(cur.line1), "s"(cur.line2));
+    // With copies the constants come with the head: a load of the op's own
+    // would wait beside the copies' words (8,191 particles, a copy at every
+    // element: 2.53 against 3.00 ms per turn). Without, 16 scalar registers
+    // less are worth more (24,001 particles: 2.02 against 2.05 ms).
+    if (!REFS) cur.k = op_consts(rec);
 #if ATX_STRICT
     // The strict build's divisions take long enough for the head to come, and
     // it is 6 % faster with the head asked for here (large ring, 32,003
@@ -2232,47 +2273,66 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
     const int kind = cur.op & 0xff;
     if (REFS) {  // markers change nothing: only their copies
       const int ndo = (kind != OP_NONE ? 1 : 0) + ((cur.op & OPF_DRIFT) ? 1 : 0);
-      for (int k = rec->first; k <= cur.last - ndo; k++) copy_refs(k);
+      for (int k = cur.first; k <= cur.last - ndo; k++) copy_refs(k);
     }
+    const int at = cur.last - (kind != OP_NONE ? 1 : 0);  // the drift
+    // In the fast build without copies the particles that the drift lost are
+    // handled with those that the element lost, the rest of the wave then takes
+    // the element again: one branch to a rare path per record.
+    constexpr bool kLater = !ATX_STRICT && !REFS;
+    uint64_t gone[P] = {};
     if (cur.op & OPF_DRIFT) {
-      const int at = cur.last - (kind != OP_NONE ? 1 : 0);
       if (REFS) copy_refs(at);
 #pragma unroll
       for (int q = 0; q < P; q++) drift6(r[q], cur.len);
 #pragma unroll
-      for (int q = 0; q < P; q++) lose(q, is_lost_drift(r[q]), at);
+      for (int q = 0; q < P; q++) {
+        gone[q] = lost_lanes_drift(r[q]) & alive[q];
+        if (!kLater) lose_mask(q, gone[q], at);
+      }
     }
     if (kind == OP_NONE) {
       ahead();
+      if (kLater)
+#pragma unroll
+        for (int q = 0; q < P; q++) lose_mask(q, gone[q], at);
       continue;
     }
     if (REFS) copy_refs(cur.last);
     cDevElem* h = &elems[cur.last];
     uint64_t bad = 0;
 #if ATX_STRICT
-    run_op<P, U, true>(r, cur.op, rec, h, pool, nturn, bad, ahead);
+    run_op<P, U, true>(r, cur, rec, h, pool, nturn, bad, ahead);
 #pragma unroll
-    for (int q = 0; q < P; q++) lose(q, is_lost(r[q]), cur.last);
+    for (int q = 0; q < P; q++) lose_mask(q, lost_lanes(r[q]) & alive[q], cur.last);
 #else
-    bool again = slow && (cur.op & OPF_RAD);
+    bool again = (cur.op & slow) != 0;
     R6 r0[P];
 #pragma unroll
     for (int q = 0; q < P; q++) r0[q] = r[q];
     if (__builtin_expect(again, 0)) {
       ahead();
     } else {
-      run_op<P, U, false>(r, cur.op, rec, h, pool, nturn, bad, ahead);
+      run_op<P, U, false>(r, cur, rec, h, pool, nturn, bad, ahead);
       again = bad != 0;
-      slow |= again;
+      slow |= again ? OPF_RAD : 0;
     }
+    uint64_t rare = 0;
 #pragma unroll
-    for (int q = 0; q < P; q++) {
-      bad = __builtin_amdgcn_ballot_w64(is_lost(r[q])) & alive[q];
-      if (__builtin_expect(again || (bad != 0 && (cur.op & OPF_MPOLE)), 0)) {
-        r[q] = op_call<U>(r0[q], (const LatOp*)rec, h, pool, nturn);
-        bad = __builtin_amdgcn_ballot_w64(is_lost(r[q])) & alive[q];
+    for (int q = 0; q < P; q++) rare |= (lost_lanes(r[q]) & alive[q]) | (kLater ? gone[q] : 0);
+    if (__builtin_expect(again || rare != 0, 0)) {
+#pragma unroll
+      for (int q = 0; q < P; q++) {
+        const bool first = kLater && gone[q] != 0;
+        if (first) {
+          r[q] = r0[q];
+          lose_mask(q, gone[q], at);
+          r0[q] = r[q];
+        }
+        if (first || again || (cur.op & OPF_MPOLE))
+          r[q] = op_call<U>(r0[q], (const LatOp*)rec, h, pool, nturn);
+        lose_mask(q, lost_lanes(r[q]) & alive[q], cur.last);
       }
-      lose_mask(q, bad, cur.last);
     }
 #endif
   }
