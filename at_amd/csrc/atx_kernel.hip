@@ -20,6 +20,8 @@
 //     delta is constant; agreement with the reference is to rounding.
 #include <hip/hip_runtime.h>
 
+#include <limits.h>
+
 #include "atx_device.h"
 #include "atx_libm.h"
 
@@ -695,13 +697,28 @@ __device__ __forceinline__ void rad_drift_ang(R6& r, Ang& g, double len, double 
 // Straight magnets: the factor (1+s2/2)/(1+s2) is 1 - (s2/2)(1 - s2 + s2^2),
 // relative error s2^4/2, below 1e-16 for s2 <= 1e-4 (angles up to 10 mrad).
 // CHECKED: lanes outside either range divide instead, under a vote per kick.
-// Otherwise `bad` collects them for the whole magnet, which is then run again
-// with the checks (run_turn): no branch in the slices. All other lanes get the
-// same bits either way.
+// Otherwise the largest s2 and |w| of the magnet are kept, and a magnet in which
+// one was outside is run again with the checks (run_turn): no branch and no
+// compare in the slices. All other lanes get the same bits either way. The
+// largest are kept by their high words, two of them with one v_max3_i32; of
+// the kicks of length K1 and K2, whose w have opposite signs, each for itself
+// (of negative numbers, too, the high word grows with the magnitude).
+struct Largest {
+  int s2, w[2];
+};
+__device__ __forceinline__ int high_word(double v) {
+  return (int)(uint32_t)(__builtin_bit_cast(uint64_t, v) >> 32);
+}
+__device__ __forceinline__ uint64_t outside(const Largest& m) {
+  constexpr int kS2 = 0x3F1A36E2, kW = 0x3EC0C6F7;  // of 1e-4 and 2e-6
+  return __builtin_amdgcn_ballot_w64(m.s2 >= kS2) |
+         __builtin_amdgcn_ballot_w64((m.w[0] & 0x7fffffff) >= kW) |
+         __builtin_amdgcn_ballot_w64((m.w[1] & 0x7fffffff) >= kW);
+}
 template <bool BEND, int N, int F, bool CHECKED, bool REFRESH>
 __device__ __forceinline__ void rad_kick_ang(R6& r, Ang& g, const Kick& k, cdouble* a, cdouble* b,
                                              int n, double blo, double alo, double irho,
-                                             uint64_t& bad) {
+                                             int& most_s2, int& most_w) {
   const double x = r.x, y = r.y;
   const double s2 = g.s2;
   const double d0 = r.dp;
@@ -740,7 +757,10 @@ __device__ __forceinline__ void rad_kick_ang(R6& r, Ang& g, const Kick& k, cdoub
     }
     const double f = __builtin_fma(s2, __builtin_fma(s2, __builtin_fma(-0.5, s2, 0.5), -0.5), 1.0);
     w = b2 * (f * ro);  // f does not wait for x
-    odd = s2 > 1e-4;
+    if (CHECKED)
+      odd = s2 > 1e-4;
+    else
+      most_s2 = max(most_s2, high_word(s2));
     if (CHECKED && __builtin_amdgcn_ballot_w64(odd) != 0) {
       const double fw = __builtin_fma(0.5, s2, 1.0) * rcp1(1.0 + s2);
       w = odd ? b2 * (fw * ro) : w;
@@ -749,13 +769,11 @@ __device__ __forceinline__ void rad_kick_ang(R6& r, Ang& g, const Kick& k, cdoub
   r.dp = __builtin_fma(-w, opd, d0);
   const double e = REFRESH ? __builtin_fma(-(1.0 + r.dp), g.pn, 1.0) : w;
   double pn = __builtin_fma(g.pn, __builtin_fma(e, e, e), g.pn);
-  const bool far = __builtin_fabs(w) > 2e-6;
   if (CHECKED) {
+    const bool far = __builtin_fabs(w) > 2e-6;
     if (__builtin_amdgcn_ballot_w64(far) != 0) pn = far ? fast_rcp(1.0 + r.dp) : pn;
   } else {
-    // (a ballot each: of their union the compiler makes two more instructions)
-    if (!BEND) bad |= __builtin_amdgcn_ballot_w64(odd);
-    bad |= __builtin_amdgcn_ballot_w64(far);
+    most_w = max(most_w, high_word(w));
   }
   if (!BEND && F == F_LEAD) {
     const double kn = __builtin_fma(k.kb, pn, k.lo);  // lo pn, to a relative delta
@@ -1005,30 +1023,31 @@ __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, 
       r[q].ct = __builtin_fma(hl1, g[q].s2, r[q].ct);
     }
   };
-  auto kicks = [&](const Kick& c) {
+  Largest m = {0, {INT_MIN, INT_MIN}};
+  auto kicks = [&](const Kick& c, int& most_w) {
 #pragma unroll
     for (int q = 0; q < P; q++)
-      rad_kick_ang<BEND, N, F, CHECKED, false>(r[q], g[q], c, a, b, n, blo, alo, irho, bad);
+      rad_kick_ang<BEND, N, F, CHECKED, false>(r[q], g[q], c, a, b, n, blo, alo, irho, m.s2, most_w);
   };
   auto body = [&]() {  // a slice without its outer drifts
-    kicks(c1);
+    kicks(c1, m.w[0]);
     drift(l2, hl2);
-    kicks(c2);
+    kicks(c2, m.w[1]);
     drift(l2, hl2);
 #pragma unroll
     for (int q = 0; q < P; q++)
-      rad_kick_ang<BEND, N, F, CHECKED, true>(r[q], g[q], c1, a, b, n, blo, alo, irho, bad);
+      rad_kick_ang<BEND, N, F, CHECKED, true>(r[q], g[q], c1, a, b, n, blo, alo, irho, m.s2, m.w[0]);
   };
   drift(l1, hl1);
-  int m = 1;
-  for (; m + U <= nslice; m += U) {
+  int k = 1;
+  for (; k + U <= nslice; k += U) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
       body();
       drift2();
     }
   }
-  for (; m < nslice; m++) {
+  for (; k < nslice; k++) {
     body();
     drift2();
   }
@@ -1036,6 +1055,7 @@ __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, 
   drift(l1, hl1);
 #pragma unroll
   for (int q = 0; q < P; q++) from_angles(r[q], g[q]);
+  if (!CHECKED) bad |= outside(m);
 #endif
 }
 
