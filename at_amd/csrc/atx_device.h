@@ -243,7 +243,7 @@ struct DiffArgs {
   const double* orbits;  // (6, nelem): orbit at the entrance of each element
   double* bdiff;         // nelem x 36, column-major 6x6 per element
   int32_t nelem;
-  int32_t pad;
+  int32_t row_major;     // [i][j] at j+6i
 };
 
 // Element matrices by central differences (one wave per element).
@@ -256,7 +256,7 @@ struct ElemMatArgs {
   double* m66;           // nelem x 36, column-major 6x6 per element
   double step;
   int32_t nelem;
-  int32_t pad;
+  int32_t row_major;     // [i][j] at j+6i
 };
 
 // One block of turns of the adjoint sweep (gridDim.y indexes the items).

@@ -1970,7 +1970,7 @@ int atx_diffusion_matrices(atx_lattice* lat, const double* orbits, double* bdiff
   a.orbits = d_o;
   a.bdiff = d_b;
   a.nelem = nelem;
-  a.pad = 0;
+  a.row_major = (flags & ATX_ROW_MAJOR) ? 1 : 0;
   hipError_t le = atx_launch_diffusion(&a, stream);
   if (dev) {
     if (le != hipSuccess) return fail(ATX_E_RUNTIME, std::string("diffusion launch: ") + hipGetErrorString(le));
@@ -2011,7 +2011,7 @@ int atx_element_matrices(atx_lattice* lat, const double* orbits, double step, do
   }
   const DeviceCopy& d = lat->dev[1];
   const ElemMatArgs a{d.elems, d.pool, d.ops, d.opof, dev ? orbits : d_buf, dev ? m66 : d_buf + no,
-                      step, nelem, 0};
+                      step, nelem, (flags & ATX_ROW_MAJOR) ? 1 : 0};
   if (e == hipSuccess)
     e = (strict ? atx_launch_element_matrices_strict : atx_launch_element_matrices_fast)(&a, stream);
   if (e == hipSuccess && !dev)

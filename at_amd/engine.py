@@ -29,6 +29,7 @@ ATX_E_NODEVICE = 4
 
 ATX_DEVICE_POINTERS = 0x1
 ATX_STRICT = 0x2
+ATX_ROW_MAJOR = 0x40
 ATX_KEEP_COUNTER = 0x4
 ATX_SOA = 0x8
 ATX_CONTINUE_LOSSES = 0x10
@@ -381,11 +382,11 @@ class DeviceLattice:
         o = np.asfortranarray(orbits, dtype=np.float64)
         if o.shape != (6, self.nelem):
             raise ValueError("orbits must have shape (6, number of elements)")
-        b = np.zeros(36 * self.nelem, dtype=np.float64)
+        b = np.empty((self.nelem, 6, 6), dtype=np.float64)
         _check(self.lib.atx_diffusion_matrices(self.h, o.ctypes.data, b.ctypes.data,
-                                               float(energy), float(rest_energy), None, 0),
-               self.lib)
-        return b.reshape(self.nelem, 6, 6).transpose(0, 2, 1).copy()
+                                               float(energy), float(rest_energy), None,
+                                               ATX_ROW_MAJOR), self.lib)
+        return b
 
     def element_matrices(self, orbits: np.ndarray, step: float, energy: float,
                          rest_energy: float, strict: bool = False) -> np.ndarray:
@@ -395,11 +396,12 @@ class DeviceLattice:
         o = np.asfortranarray(orbits, dtype=np.float64)
         if o.shape != (6, self.nelem):
             raise ValueError("orbits must have shape (6, number of elements)")
-        m = np.zeros(36 * self.nelem, dtype=np.float64)
+        m = np.empty((self.nelem, 6, 6), dtype=np.float64)
         _check(self.lib.atx_element_matrices(self.h, o.ctypes.data, float(step), m.ctypes.data,
                                              float(energy), float(rest_energy), None,
-                                             ATX_STRICT if strict else 0), self.lib)
-        return m.reshape(self.nelem, 6, 6).transpose(0, 2, 1).copy()
+                                             ATX_ROW_MAJOR | (ATX_STRICT if strict else 0)),
+               self.lib)
+        return m
 
     def check(self, energy: float, rest_energy: float) -> None:
         _check(self.lib.atx_lattice_check(self.h, float(energy), float(rest_energy)), self.lib)

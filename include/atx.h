@@ -50,6 +50,8 @@ extern "C" {
                                   * slots and the workgroups that hold them, over all
                                   * instances, at the front of the grid; the blocks run as one
                                   * hipGraph. Results are identical to a plain launch. */
+#define ATX_ROW_MAJOR 0x40u      /* atx_element_matrices, atx_diffusion_matrices: row-major 6x6
+                                    blocks ([i][j] at j+6i) */
 
 typedef struct atx_lattice atx_lattice;
 
@@ -255,7 +257,7 @@ int atx_diffusion_matrices(atx_lattice *lat, const double *orbits, double *bdiff
  * around the orbit at its entrance. Probe j+ / j- is the orbit with +step/2
  * / -step/2 added to coordinate j (matrix.py:195-199), passed through that
  * element alone (no loss check); m[i][j] = (probe j+ - probe j-)_i / step.
- * One tracking launch over all elements (one instance each).
+ * One launch, a wave per element.
  *   orbits  (6, nelem) F-order: orbit at the entrance of each element
  *   m66     nelem blocks of 36 doubles, column-major 6x6 ([i][j] at i+6j)
  *   step    the reference's XYStep (nonzero)

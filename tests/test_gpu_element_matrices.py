@@ -112,3 +112,30 @@ def test_device_pointers_and_argument_errors(ring):
         d_m.close()
     finally:
         dl.close()
+
+
+@pytest.mark.parametrize("nelem", [1, 63, 64, 65])
+def test_row_major_is_the_transpose(nelem):
+    """Both layouts of the C ABI, around a wave of diffusion lanes, with an
+    orbit that is not finite among them (all products are taken for it)."""
+    from at_amd.lattice import Dipole, Quadrupole
+
+    rad = ("StrMPoleSymplectic4RadPass", "BndMPoleSymplectic4RadPass")
+    elems = [Quadrupole("Q", 0.4, 1.2, PassMethod=rad[0]) if k % 2 else
+             Dipole("B", 1.0, 0.05, 0.2, PassMethod=rad[1]) for k in range(nelem)]
+    dl = engine.DeviceLattice(elems)
+    orbits = np.asfortranarray(np.random.default_rng(2).standard_normal((6, nelem)) * 1e-4)
+    orbits[3, nelem // 2] = np.inf
+    energy, rest = 6.0e9, 510998.95
+    for name, call in (("m66", dl.lib.atx_element_matrices), ("bdiff", dl.lib.atx_diffusion_matrices)):
+        out = []
+        for flags in (0, engine.ATX_ROW_MAJOR):
+            m = np.full((nelem, 6, 6), 7.0)
+            step = (3e-8,) if name == "m66" else ()
+            args = (dl.h, orbits.ctypes.data, *step, m.ctypes.data, energy, rest, None, flags)
+            assert call(*args) == 0, engine.load_library().atx_last_error()
+            out.append(m)
+        np.testing.assert_array_equal(out[0].transpose(0, 2, 1), out[1], err_msg=name)
+        ok = np.arange(nelem) != nelem // 2
+        assert np.isfinite(out[1][ok]).all() and (nelem == 1 or np.abs(out[1][ok]).max() > 0)
+    dl.close()
