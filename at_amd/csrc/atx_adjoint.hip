@@ -315,8 +315,8 @@ __device__ __forceinline__ void element_rev(V6& r, V6& l, cDevElem& h, cAdjElem&
 // product of a drift's length with them are taken once per magnet: a drift is
 // 13 FP64 instructions instead of 35 (a division among them), two drifts in a
 // row are one, and the kicks are spelled out for the form of the field (7
-// instead of about 20 for a quadrupole). One wave of the large ring: 5.2 ->
-// 2.1 ms per turn.
+// instead of about 20 for a quadrupole). 4,096 particles and 8 turns of the large
+// ring: the two sweeps 21.0 -> 9.6 ms.
 struct RevDrift {
   double nl, nlu;     // L u, L u^2 with u = 1/(1+delta)
   double hh;          // L u^2 / 2
@@ -361,7 +361,6 @@ __device__ __forceinline__ void kick_rev(V6& r, V6& l, const RevKick& k, double 
     l.dp = __builtin_fma(k.kh, lx, l.dp);
   }
   if (!LEAD) return;
-  // s + i t = z (l_py' ...): the products shared by the Jacobian and the gradient
   const double s = __builtin_fma(y, ly, -x * lx);  // y l_py - x l_px
   if (N == 1) {
     r.px = __builtin_fma(k.kb, x, r.px);

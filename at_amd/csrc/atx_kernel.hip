@@ -15,7 +15,7 @@
 //     atintegrators/*.c, with the same divisions, so results agree bit for
 //     bit with the CPU reference except where a device transcendental (sin in
 //     RFCavityPass, tan in per-particle edge fringes) enters;
-//   ATX_STRICT=0, -ffp-contract=fast: the same maps with FMA contraction,
+//   ATX_STRICT=0, -ffp-contract=on: the same maps with FMA contraction,
 //     hand-fused Horner steps and the 1/(1+delta) reciprocals hoisted where
 //     delta is constant; agreement with the reference is to rounding.
 #include <hip/hip_runtime.h>
@@ -544,8 +544,8 @@ __device__ __noinline__ R6 slices_ops(R6 r, cdouble* a, cdouble* b, int n, cdoub
 // octupoles have one coefficient and a bend often none, so the fast build
 // spells their kicks out instead of running Horner over zeros: 2 FP64
 // instructions instead of 6 per quadrupole kick, 5 instead of 10 per sextupole
-// kick, 8 instead of 14 per octupole kick, 20 instead of 26 per radiating
-// quadrupole kick, 26 instead of 42 per kick of a radiating bend without
+// kick, 8 instead of 14 per octupole kick, 19 instead of 23 per radiating
+// quadrupole kick, 20 instead of 33 per kick of a radiating bend without
 // gradient. The VALU issues on 83 % of the cycles of a full device, so time
 // follows the instruction count. The strict build evaluates all coefficients.
 // A particle whose result is not finite is recomputed with the general form
@@ -2276,16 +2276,18 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
       if (check) lose_mask(q, lost_lanes(r[q]) & alive[q], e);
     }
   };
-  // The loop over the records. With few waves per SIMD it is bound by the
+  // The loop over the records. With few waves per SIMD it was bound by the
   // time around an element's arithmetic: scalar loads waited for one after
   // the other (kind, then flags, then pool offsets, then constants), a tree of
   // branches over 147 KB of code, and the state copied for lanes that skip
-  // an element. One record per drift-and-element pair, its head read one
-  // record ahead, its constants at fixed offsets, no skipping lanes and 35
-  // KB of code brought the large ring (10 slices per magnet) from 3.35 to
-  // 2.56 ms per turn for one wave, from 3.54 to 2.70 for 24,001 particles and
-  // from 8.32 to 7.70 for 262,144; without the slices (extrapolated from 4
-  // and 10 per magnet) one wave went from 1.33 to 0.58 ms.
+  // an element. One record per drift-and-element pair with its constants at
+  // fixed offsets, its head read one record ahead, no skipping lanes, tests of
+  // one bit, one rare path per record, and kicks by form: the large ring (10
+  // slices per magnet) from 3.35 to 1.85 ms per turn for one wave, from 3.54 to
+  // 1.92 for 24,001 particles, from 8.32 to 6.25 for 262,144; the FODO ring (320
+  // elements) for one wave from 354 to 162 us. What bounds it now: one wave
+  // issues an FP64 instruction in 4.6 to 7.5 cycles, depending on how many of
+  // its chains are independent, and four waves share the VALU's 4 cycles.
   // A turn runs the records o0..o1-1 whole. The first element of a call
   // (whose input has not passed a loss test yet) and the elements of a
   // record that a partial turn starts or ends in run by their headers,
