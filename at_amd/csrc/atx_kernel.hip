@@ -254,8 +254,7 @@ __device__ __forceinline__ void bnd_kick(R6& r, cdouble* a, cdouble* b, int n, d
 }
 
 // Radiating drift (diff_drift.c:30-43).
-__device__ __forceinline__ void rad_drift(R6& r, double len) {
-  const double pn = 1.0 / (1.0 + r.dp);
+__device__ __forceinline__ void rad_drift(R6& r, double len, double pn) {
   const double nl = len * pn;
   r.x += nl * r.px;
   r.y += nl * r.py;
@@ -298,9 +297,8 @@ __device__ __forceinline__ void rad_drift_pn(R6& r, double len, double pn) {
 #endif
 
 // Radiating straight kick (diff_str_kick.c:19-83, bdiff == NULL).
-// radc = RAD_CONST*gamma^3 (strict); radk = radc*kl (fast). The fast build
-// takes pn = 1/(1+delta) at entry and returns it updated to the radiated
-// delta.
+// radc = RAD_CONST*gamma^3 (strict); radk = radc*kl (fast). Takes pn =
+// 1/(1+delta) at entry and returns it for the radiated delta.
 template <int N>
 __device__ __forceinline__ void rad_str_kick(R6& r, cdouble* a, cdouble* b, int n, double blo,
                                              double alo, double kl, double radc, double radk,
@@ -308,9 +306,8 @@ __device__ __forceinline__ void rad_str_kick(R6& r, cdouble* a, cdouble* b, int 
   double re, im;
   field<N>(r, a, b, n, blo, alo, re, im);
 #if ATX_STRICT
-  (void)pn_io;
   (void)radk;
-  double pn = 1.0 / (1.0 + r.dp);
+  double pn = pn_io;
   const double xpr = r.px * pn;
   const double ypr = r.py * pn;
   const double vn2 = 1.0 / (1.0 + xpr * xpr + ypr * ypr);
@@ -323,6 +320,7 @@ __device__ __forceinline__ void rad_str_kick(R6& r, cdouble* a, cdouble* b, int 
   r.py = ypr / pn;
   r.px -= kl * re;
   r.py += kl * im;
+  pn_io = pn;
 #else
   (void)radc;
   const double pn_in = pn_io;
@@ -355,9 +353,8 @@ __device__ __forceinline__ void rad_bnd_kick(R6& r, cdouble* a, cdouble* b, int 
   double re, im;
   field<N>(r, a, b, n, blo, alo, re, im);
 #if ATX_STRICT
-  (void)pn_io;
   (void)radk;
-  double pn = 1.0 / (1.0 + r.dp);
+  double pn = pn_io;
   const double x = r.x;
   const double xpr = r.px * pn;
   const double ypr = r.py * pn;
@@ -378,6 +375,7 @@ __device__ __forceinline__ void rad_bnd_kick(R6& r, cdouble* a, cdouble* b, int 
   r.px -= kl * (re - (d0 - r.x * irho) * irho);
   r.py += kl * im;
   r.ct += kli * r.x;
+  pn_io = pn;
 #else
   (void)radc;
   const double pn_in = pn_io;
@@ -518,7 +516,7 @@ __device__ __noinline__ R6 slices_ops(R6 r, cdouble* a, cdouble* b, int n, cdoub
     for (int j = 0; j < nop; j++) {
       const double len = op[2 + 2 * j];
       if (op[1 + 2 * j] == 0.0) {
-        if (RAD) rad_drift(r, len); else fastdrift(r, len * pn0, h2);
+        if (RAD) rad_drift(r, len, 1.0 / (1.0 + r.dp)); else fastdrift(r, len * pn0, h2);
       } else {
         if (RAD) {
           double pn = 1.0 / (1.0 + r.dp);
@@ -970,34 +968,38 @@ __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, 
   else ahead(l1, l2, k1, k2, rk, rk2);
 #if ATX_STRICT
   const double ki1 = k1 * irho, ki2 = k2 * irho;
-  double pn = 0.0;  // unused: the strict steps divide as the reference does
+  // 1/(1+delta), divided as the reference does; delta changes in the kicks only,
+  // so the quotient of one kick is that of the drifts and the kick after it
+  double pn[P];
+#pragma unroll
+  for (int q = 0; q < P; q++) pn[q] = 1.0 / (1.0 + r[q].dp);
   // U slices per iteration: a constant-count inner loop, fully unrolled
   // (the slices may hold wave-wide votes, which a runtime-count unroll
   // cannot duplicate), then the remaining slices one by one
   auto slice = [&]() {
 #pragma unroll
-    for (int q = 0; q < P; q++) rad_drift(r[q], l1);
+    for (int q = 0; q < P; q++) rad_drift(r[q], l1, pn[q]);
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1, radc, 0.0, pn);
-      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k1, radc, 0.0, pn);
+      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1, radc, 0.0, pn[q]);
+      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k1, radc, 0.0, pn[q]);
     }
 #pragma unroll
-    for (int q = 0; q < P; q++) rad_drift(r[q], l2);
+    for (int q = 0; q < P; q++) rad_drift(r[q], l2, pn[q]);
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2, radc, 0.0, pn);
-      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k2, radc, 0.0, pn);
+      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k2, irho, ki2, radc, 0.0, pn[q]);
+      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k2, radc, 0.0, pn[q]);
     }
 #pragma unroll
-    for (int q = 0; q < P; q++) rad_drift(r[q], l2);
+    for (int q = 0; q < P; q++) rad_drift(r[q], l2, pn[q]);
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1, radc, 0.0, pn);
-      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k1, radc, 0.0, pn);
+      if (BEND) rad_bnd_kick<N>(r[q], a, b, n, blo, alo, k1, irho, ki1, radc, 0.0, pn[q]);
+      else rad_str_kick<N>(r[q], a, b, n, blo, alo, k1, radc, 0.0, pn[q]);
     }
 #pragma unroll
-    for (int q = 0; q < P; q++) rad_drift(r[q], l1);
+    for (int q = 0; q < P; q++) rad_drift(r[q], l1, pn[q]);
   };
   int m = 0;
   for (; m + U <= nslice; m += U) {
