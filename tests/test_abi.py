@@ -212,3 +212,42 @@ def test_element_matrices_argument_errors():
     with pytest.raises(ValueError):
         lat.element_matrices(np.zeros((6, 2)), 1e-8, 3e9, 0.0)
 
+
+
+def test_elements_in_one_call():
+    """atx_lattice_add_elements: errors in the order of the elements, the value
+    types that carry parameters, and tables that do not fit."""
+    import types
+
+    bare = types.SimpleNamespace(FamName="x")
+    with pytest.raises(RuntimeError, match=r"UnknownPass in element #1"):
+        engine.DeviceLattice([Drift("d", 1.0), Drift("d", 1.0, PassMethod="UnknownPass"), bare])
+    with pytest.raises(AttributeError, match="Element #1 has no PassMethod"):
+        engine.DeviceLattice([Drift("d", 1.0), bare])
+    q = Quadrupole("q", 0.5, 1.0)
+    q.Length = np.float32(0.5)
+    q.NumIntSteps = np.int64(3)
+    q.PolynomA = [0, 0]
+    q.PolynomB = np.array([0, 1], dtype=np.int32)
+    q.R1 = np.asfortranarray(np.eye(6))
+    q.Comment, q._private, q.Extra = "text", 1.0, [1.0, "x"]
+    lat = engine.DeviceLattice([q, Marker("m")])
+    lat.check(0.0, 0.0)
+    assert lat.nelem == lat.lib.atx_lattice_num_elements(lat.h) == 2
+    lat.close()
+    lib = engine.load_library()
+    h = C.c_void_p()
+    assert lib.atx_lattice_create(C.byref(h)) == 0
+    texts = (C.c_char_p * 3)(b"DriftPass", b"fam", b"Length")
+    one = (C.c_double * 1)(1.0)
+
+    def add(elem, attr, nvalues=1):
+        e, a = (C.c_int32 * 3)(*elem), (C.c_int32 * 2)(*attr)
+        return lib.atx_lattice_add_elements(h, 1, texts, 3, e, a, 1, one, nvalues)
+
+    assert add((0, 1, 1), (4, 1)) == 0
+    for elem, attr in (((3, 1, 1), (4, 1)), ((0, -1, 1), (4, 1)), ((0, 1, 2), (4, 1)),
+                       ((0, 1, 1), (6, 1)), ((0, 1, 1), (4, 2)), ((0, 1, 1), (4, -1))):
+        assert add(elem, attr) == engine.ATX_E_VALUE, (elem, attr)
+    assert lib.atx_lattice_num_elements(h) == 1
+    assert lib.atx_lattice_destroy(h) == 0
