@@ -161,6 +161,8 @@ enum : int32_t {
   OPF_EDGE = 8 << 8,   // a bend's edges by its header (not of constant strength)
   OPF_MPOLE = 16 << 8, // a thick multipole
   OPF_RAD = 32 << 8,   // a radiating one
+  OPF_R1 = 64 << 8,    // misaligned with a roll at the entry, at the exit
+  OPF_R2 = 128 << 8,
 };
 // constants of OP_CORR, the thin and the thick multipoles
 enum OpSlot : int32_t {

@@ -676,13 +676,17 @@ void fill_op(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
       if (h.kind == K_STRRAD) op = OP_STRRAD1;
       if (h.kind == K_BNDRAD) op = OP_BNDRAD1;
     }
-    // a missing transform is the identity: + 0 and (1, 0) leave a coordinate as it is
+    // A missing transform leaves a coordinate as it is: + -0.0, and no roll in
+    // the strict build (in the fast one (1, 0), which does so for finite ones).
+    // The sums of a rolled coordinate start from 0.0, so one that is zero is
+    // +0.0: with a roll the zeros of a shift are +0.0, before it and after it.
     double* xf = r.c + OM_XF;
     const double* t1 = (h.flags & F_T1) ? &pool[h.t1] : nullptr;
     const double* t2 = (h.flags & F_T2) ? &pool[h.t2] : nullptr;
+    const double zero1 = (h.flags & F_R1) ? 0.0 : -0.0, zero2 = (h.flags & F_R2) ? 0.0 : -0.0;
     for (int k = 0; k < 4; k++) {
-      xf[k] = t1 ? t1[k] : 0.0;
-      xf[8 + k] = t2 ? t2[k] : 0.0;
+      xf[k] = (t1 ? t1[k] : -0.0) + zero1;
+      xf[8 + k] = (t2 ? t2[k] : -0.0) + zero2;
     }
     xf[4] = xf[6] = 1.0;
     bool plain = (!t1 || plain_shift(t1)) && (!t2 || plain_shift(t2));
@@ -710,6 +714,8 @@ void fill_op(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
     op |= OPF_MPOLE;
     if (h.kind == K_STRRAD || h.kind == K_BNDRAD) op |= OPF_RAD;
     if (h.flags & (F_T1 | F_T2 | F_R1 | F_R2)) op |= OPF_XF;
+    if (h.flags & F_R1) op |= OPF_R1;
+    if (h.flags & F_R2) op |= OPF_R2;
     if ((h.edge & 0xff) != E_CONST || ((h.edge >> 8) & 0xff) != E_CONST) op |= OPF_EDGE;
     r.op = drift | op;
     r.nslice = h.nslice;

@@ -1915,7 +1915,8 @@ __device__ __forceinline__ bool is_finite(const R6& r) {
 }
 
 // Roll of both planes by the angle of (c, s): the 6x6 product of mul_r
-// without its zeros, in its order of summation.
+// without its zeros, in its order of summation (that it starts from 0.0 shows
+// in the sign of a zero only: fill_op).
 __device__ __forceinline__ void roll(R6& r, double c, double s) {
   const double x = r.x, px = r.px;
 #if ATX_STRICT
@@ -1931,6 +1932,26 @@ __device__ __forceinline__ void roll(R6& r, double c, double s) {
 #endif
 }
 
+__device__ __forceinline__ void shift(R6& r, cdouble* t) {
+  r.x += t[0];
+  r.px += t[1];
+  r.y += t[2];
+  r.py += t[3];
+}
+
+#if ATX_STRICT
+// A coordinate that is not finite spreads through the zeros of the 6x6
+// product, as in the reference: a wave with one takes the product. (An infinite
+// x of a particle without loss record enters a magnet; others come out of one.
+// The fast build runs the whole element again, op_call.)
+__device__ __forceinline__ void strict_roll(R6& r, cdouble* cs, cdouble* m) {
+  if (__builtin_expect(lost_lanes(r) != 0, 0))
+    r = mul_r_v(r, m);
+  else
+    roll(r, cs[0], cs[1]);
+}
+#endif
+
 // The element of a record other than its markers and drift, for the P
 // particles of a lane. CHECKED, bad: rad_kick_ang; ahead: NotAhead.
 template <int P, int U, bool CHECKED, class Ahead>
@@ -1943,11 +1964,13 @@ __device__ __forceinline__ void run_op(R6* r, const OpHead& o, cLatOp* rec, cDev
   if (op & OPF_XF) {
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      r[q].x += c[OM_XF];
-      r[q].px += c[OM_XF + 1];
-      r[q].y += c[OM_XF + 2];
-      r[q].py += c[OM_XF + 3];
+#if ATX_STRICT
+      shift(r[q], c + OM_XF);
+      if (op & OPF_R1) strict_roll(r[q], c + OM_XF + 4, pool + h->r1);
+#else
+      shift(r[q], c + OM_XF);
       roll(r[q], c[OM_XF + 4], c[OM_XF + 5]);
+#endif
     }
   }
 #define ATX_MPOLE(BEND, RAD, N, F) \
@@ -2034,18 +2057,12 @@ __device__ __forceinline__ void run_op(R6* r, const OpHead& o, cLatOp* rec, cDev
 #pragma unroll
     for (int q = 0; q < P; q++) {
 #if ATX_STRICT
-      // a coordinate that is not finite spreads through the zeros of the
-      // 6x6 product, as in the reference: the wave then takes the product
-      // (the fast build runs the whole element again, op_call)
-      if (__builtin_expect(lost_lanes(r[q]) != 0 && (h->flags & F_R2), 0))
-        r[q] = mul_r_v(r[q], pool + h->r2);
-      else
+      if (op & OPF_R2) strict_roll(r[q], c + OM_XF + 6, pool + h->r2);
+      shift(r[q], c + OM_XF + 8);
+#else
+      roll(r[q], c[OM_XF + 6], c[OM_XF + 7]);
+      shift(r[q], c + OM_XF + 8);
 #endif
-        roll(r[q], c[OM_XF + 6], c[OM_XF + 7]);
-      r[q].x += c[OM_XF + 8];
-      r[q].px += c[OM_XF + 9];
-      r[q].y += c[OM_XF + 10];
-      r[q].py += c[OM_XF + 11];
     }
   }
 }
