@@ -572,8 +572,8 @@ __device__ __forceinline__ void fastdrift_h(R6& r, double nl, double nlh) {
 struct Kick {
   double kl, kli;         // length, length times curvature
   double bn;              // B[N]
-  double kb, kb2;         // kl B[N], twice that
-  double kb0, ka0;        // kl B[0], kl A[0]
+  double kb, kb2;         // kl B[N], twice that (LEAD0: 2 B[N])
+  double b0, a0;          // B[0], A[0]
   double lo;              // remainder of kb (NOFIELD: of kli)
   double rk;              // radiating: RAD_CONST gamma^3 kl (times the field's constant squared)
 };
@@ -584,16 +584,19 @@ __device__ __forceinline__ Kick kick_of(cdouble* a, cdouble* b, double lead, dou
   Kick k;
   k.kl = kl;
   k.kli = BEND ? kl * irho : 0.0;
-  k.kb = k.kb2 = k.kb0 = k.ka0 = k.lo = 0.0;
-  if (F == F_LEAD || F == F_LEAD0) {
+  k.kb = k.kb2 = k.b0 = k.a0 = k.lo = 0.0;
+  if (F == F_LEAD) {
     k.kb = kl * lead;
     k.kb2 = 2.0 * k.kb;
     k.lo = __builtin_fma(kl, lead, -k.kb);
   }
   if (F == F_NOFIELD) k.lo = __builtin_fma(kl, irho, -k.kli);
   if (F == F_LEAD0) {
-    k.kb0 = kl * b[0];
-    k.ka0 = kl * a[0];
+    k.kb2 = 2.0 * lead;
+    k.b0 = b[0];
+    k.a0 = a[0];
+    asm("" : "=v"(k.b0) : "0"(k.b0));  // an FMA reads one scalar: horner_addends
+    asm("" : "=v"(k.a0) : "0"(k.a0));
   }
   k.rk = radk;
   k.bn = lead;
@@ -640,10 +643,14 @@ __device__ __forceinline__ void kick(R6& r, const Kick& k, cdouble* a, cdouble* 
   }
   double px = r.px, py = r.py;
   if (F == F_LEAD0) {
-    px = px - k.kb0;
-    py = py + k.ka0;
-  }
-  if (N == 1) {
+    // the dipole with the rest of the field: kl B[0] added by itself would round
+    // alike at every kick (30 kicks: twice to four times the error)
+    static_assert(F != F_LEAD0 || N == 2, "a sextupole");
+    const double re = __builtin_fma(k.bn, __builtin_fma(r.x, r.x, -(r.y * r.y)), k.b0);
+    const double im = __builtin_fma(k.kb2, r.x * r.y, k.a0);
+    px = __builtin_fma(-k.kl, re, px);
+    py = __builtin_fma(k.kl, im, py);
+  } else if (N == 1) {
     px = __builtin_fma(-k.kb, r.x, px);
     py = __builtin_fma(k.kb, r.y, py);
   } else if (N == 2) {  // z^2 = (x^2 - y^2) + i 2 x y
@@ -946,7 +953,7 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
   }
   body();
   drift(nl1, nh1);
-  if (F != F_GENERAL) {
+  if (F == F_LEAD || F == F_NOFIELD) {
     const double rest = (2.0 * c1.lo + c2.lo) * (double)nslice;
 #pragma unroll
     for (int q = 0; q < P; q++) kick_rest<BEND, N, F>(r[q], rest, irho);

@@ -1,0 +1,73 @@
+"""GPU: rounding of the fast build's kicks against extended precision, by the
+form of the field. A magnet of 10 slices kicks a particle 30 times; each kick
+rounds px and py once, so the error of a particle is a random walk of 30 steps
+of rms 0.29 units in the last place: 1.6 units. A product that is rounded alike at
+every kick adds up instead, to 30 x 0.25 units on average. Bound: 2.4 units
+(half as much again for the coordinates that the kick is computed from)."""
+
+import numpy as np
+import pytest
+
+from at_amd import engine
+from at_amd.lattice import Lattice, Particle, Sextupole
+from oracle import pyoracle as po
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(np.finfo(np.longdouble).eps > 2e-19,
+                                 reason="no extended precision on this machine")]
+
+N, SLICES = 20000, 10
+# the engine's Forest-Ruth coefficients (doubles)
+DRIFT = (0.6756035959798286638, -0.1756035959798286639)
+KICK = (1.351207191959657328, -1.702414383919314656)
+
+
+def _exact(m, beam):
+    """The magnet's slices in extended precision, from the same double constants."""
+    ld = np.longdouble
+    x, px, y, py, dp, ct = beam.astype(ld)
+    a, b = [ld(v) for v in m.PolynomA], [ld(v) for v in m.PolynomB]
+    step = m.Length / m.NumIntSteps
+    irho = ld(getattr(m, "BendingAngle", 0.0) / m.Length)
+    d1, d2, k1, k2 = (ld(step * v) for v in DRIFT + KICK)
+    p = 1 / (1 + dp)
+    for _ in range(m.NumIntSteps):
+        for d, k in ((d1, k1), (d2, k2), (d2, k1), (d1, None)):
+            x, y = x + d * p * px, y + d * p * py
+            ct = ct + d * p * p * (px * px + py * py) / 2
+            if k is None:
+                continue
+            re, im = b[-1], a[-1]
+            for i in range(len(a) - 2, -1, -1):
+                re, im = re * x - im * y + b[i], im * x + re * y + a[i]
+            px, py = px - k * (re - (dp - x * irho) * irho), py + k * im
+            ct = ct + k * irho * x
+    return np.array([x, px, y, py, dp, ct])
+
+
+def _pass(m, beam):
+    ring = Lattice([m], energy=3.0e9, particle=Particle("electron"), name="one")
+    dl = engine.DeviceLattice(ring)
+    try:
+        got = beam.copy(order="F")
+        dl.track(got, 1, None, energy=ring.energy, rest_energy=ring.particle.rest_energy)
+    finally:
+        dl.close()
+    return got
+
+
+def _beam(scale):
+    return np.asfortranarray(np.random.default_rng(21).uniform(-1.0, 1.0, (6, N))
+                             * np.array(scale)[:, None])
+
+
+@pytest.mark.parametrize("s", [0.55, 0.8, 1.1, 1.45])
+def test_sextupole_with_steerer(s):
+    m = Sextupole("S", 0.2, 120.0 * s, PolynomB=[1e-5 * s, 0.0, 120.0 * s],
+                  PolynomA=[-2e-5 * s, 0.0, 0.0], NumIntSteps=SLICES)
+    beam = _beam([1e-3, 1e-4, 1e-3, 1e-4, 1e-3, 1e-3])
+    exact, got = _exact(m, beam), _pass(m, beam)
+    for k in (1, 3):
+        units = (got[k] - exact[k]).astype(float) / np.spacing(np.abs(got[k]))
+        units = units[np.abs(got[k]) > 2e-5]  # a coordinate that passes zero keeps larger roundings
+        assert np.sqrt(np.mean(units * units)) < 2.4
