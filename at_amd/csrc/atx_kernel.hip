@@ -605,7 +605,9 @@ __device__ __forceinline__ Kick kick_of(cdouble* a, cdouble* b, double lead, dou
   return k;
 }
 
-// The remainders of a whole magnet's kicks in one, c = their sum.
+// The remainders of a whole magnet's kicks in one, c = their sum. Taken at the
+// first kick: a particle that overflows in a strong multipole leaves it with
+// coordinates whose powers are far above its kicks.
 template <bool BEND, int N, int F>
 __device__ __forceinline__ void kick_rest(R6& r, double c, double irho) {
   if (F == F_NOFIELD) {
@@ -939,6 +941,11 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
     kicks(c1);
   };
   drift(nl1, nh1);
+  if (F == F_LEAD || F == F_NOFIELD) {
+    const double rest = (2.0 * c1.lo + c2.lo) * (double)nslice;
+#pragma unroll
+    for (int q = 0; q < P; q++) kick_rest<BEND, N, F>(r[q], rest, irho);
+  }
   int m = 1;
   for (; m + U <= nslice; m += U) {
 #pragma unroll
@@ -953,11 +960,6 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
   }
   body();
   drift(nl1, nh1);
-  if (F == F_LEAD || F == F_NOFIELD) {
-    const double rest = (2.0 * c1.lo + c2.lo) * (double)nslice;
-#pragma unroll
-    for (int q = 0; q < P; q++) kick_rest<BEND, N, F>(r[q], rest, irho);
-  }
 #endif
 }
 

@@ -10,16 +10,16 @@ import pytest
 
 from at_amd import engine
 from at_amd.lattice import Lattice, Particle, Sextupole
-from oracle import pyoracle as po
 
 pytestmark = [pytest.mark.gpu,
               pytest.mark.skipif(np.finfo(np.longdouble).eps > 2e-19,
                                  reason="no extended precision on this machine")]
 
 N, SLICES = 20000, 10
-# the engine's Forest-Ruth coefficients (doubles)
-DRIFT = (0.6756035959798286638, -0.1756035959798286639)
-KICK = (1.351207191959657328, -1.702414383919314656)
+# the engine's Forest-Ruth coefficients, with their roundings
+CBRT2 = 1.25992104989487316477
+DRIFT = (1.0 / (2.0 * (2.0 - CBRT2)), 0.5 - (1.0 / (2.0 * (2.0 - CBRT2))))
+KICK = (1.0 / (2.0 - CBRT2), 1.0 - 2.0 / (2.0 - CBRT2))
 
 
 def _exact(m, beam):

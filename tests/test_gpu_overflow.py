@@ -100,6 +100,25 @@ def test_loss_coordinates(kind, slices, how):
     np.testing.assert_allclose(got, ref, rtol=1e-8, atol=1e-8)
 
 
+@pytest.mark.parametrize("kind,slices", [("sext", 2), ("steerer", 2), ("oct", 1)])
+def test_finite_loss_coordinates(kind, slices):
+    """Particles that a strong multipole throws far out, but not to infinity: each kick raises the
+    relative error to its power at most, as above, in the fast build as well."""
+    n = 2000
+    rng = np.random.default_rng(14)
+    beam = np.asfortranarray(1e-3 * rng.standard_normal((6, n)))
+    beam[0], beam[2] = rng.uniform(0.2, 0.99, n), rng.uniform(0.0, 0.9, n)
+    ring = _ring(_magnet(kind, slices))
+    ref = beam.copy(order="F")
+    _, want = po.atpass(ring, ref, 1, losses=True)
+    assert np.abs(want["coord"][0]).max() > 1e20 and np.isfinite(want["coord"]).all()
+    for strict in (True, False):
+        got, have = _track(ring, beam, strict)
+        for k in ("islost", "turn", "elem"):
+            np.testing.assert_array_equal(have[k], want[k], err_msg=k)
+        np.testing.assert_allclose(have["coord"], want["coord"], rtol=0 if strict else 1e-8, atol=0)
+
+
 @pytest.mark.parametrize("how", MOVES)
 @pytest.mark.parametrize("kind,slices", [("sext", 2), ("oct", 2), ("quad", 2)])
 def test_infinite_input_without_loss_records(kind, slices, how):
