@@ -568,7 +568,9 @@ __device__ __forceinline__ void fastdrift_h(R6& r, double nl, double nlh) {
 // What a kick of length kl multiplies by, once per magnet. The rounding of
 // such a product is the same at every kick of every turn, so it would add up
 // over the turns instead of averaging out: its remainder is kept, too, and is
-// added where that costs nothing (radiating kicks) or once per magnet.
+// added where that costs nothing (radiating kicks) or once per magnet
+// (kick_rest). Constants that are only added (a dipole in a sextupole) are the
+// addends of the field, which kl then multiplies at each kick.
 struct Kick {
   double kl, kli;         // length, length times curvature
   double bn;              // B[N]
@@ -605,26 +607,49 @@ __device__ __forceinline__ Kick kick_of(cdouble* a, cdouble* b, double lead, dou
   return k;
 }
 
-// The remainders of a whole magnet's kicks in one, c = their sum. Taken at the
-// first kick: a particle that overflows in a strong multipole leaves it with
-// coordinates whose powers are far above its kicks.
+// A non-radiating bend with a gradient: kl (re - (delta - x h) h) is
+// kl (c x - d) with c = B[1] + h^2 for the magnet and d = h delta for the
+// particle, and their remainders.
+struct BendGrad {
+  double c, c_lo;
+  double d, d_lo;
+};
+
+__device__ __forceinline__ BendGrad bend_grad(double lead, double irho, double dp) {
+  BendGrad g;
+  g.c = __builtin_fma(irho, irho, lead);
+  g.c_lo = __builtin_fma(irho, irho, lead - g.c);
+  g.d = irho * dp;
+  g.d_lo = __builtin_fma(irho, dp, -g.d);
+  return g;
+}
+
+// The remainders of a whole magnet's kicks in one: lo = the sum of theirs, kl =
+// of their lengths. Taken at the first kick: a particle that overflows in a strong
+// multipole leaves it with coordinates whose powers are far above its kicks.
 template <bool BEND, int N, int F>
-__device__ __forceinline__ void kick_rest(R6& r, double c, double irho) {
-  if (F == F_NOFIELD) {
-    r.px = __builtin_fma(c, __builtin_fma(-r.x, irho, r.dp), r.px);
+__device__ __forceinline__ void kick_rest(R6& r, double lo, double kl, double irho,
+                                          const BendGrad& g) {
+  if (BEND) {
+    r.px = __builtin_fma(-kl, __builtin_fma(g.c_lo, r.x, -g.d_lo), r.px);
+    if (F == F_LEAD) r.py = __builtin_fma(lo, r.y, r.py);
   } else if (N == 1) {
-    r.px = __builtin_fma(-c, r.x, r.px);
-    r.py = __builtin_fma(c, r.y, r.py);
+    r.px = __builtin_fma(-lo, r.x, r.px);
+    r.py = __builtin_fma(lo, r.y, r.py);
   } else if (N == 2) {
-    r.px = __builtin_fma(-c, __builtin_fma(r.x, r.x, -(r.y * r.y)), r.px);
-    r.py = __builtin_fma(2.0 * c, r.x * r.y, r.py);
+    r.px = __builtin_fma(-lo, __builtin_fma(r.x, r.x, -(r.y * r.y)), r.px);
+    r.py = __builtin_fma(2.0 * lo, r.x * r.y, r.py);
+  } else {
+    const double x2 = r.x * r.x, y2 = r.y * r.y;
+    r.px = __builtin_fma(-lo, r.x * __builtin_fma(-3.0, y2, x2), r.px);
+    r.py = __builtin_fma(lo, r.y * __builtin_fma(3.0, x2, -y2), r.py);
   }
 }
 
 // driftkick.c:51-115 by form.
 template <bool BEND, int N, int F>
 __device__ __forceinline__ void kick(R6& r, const Kick& k, cdouble* a, cdouble* b, int n, double blo,
-                                     double alo, double irho) {
+                                     double alo, double irho, const BendGrad& g) {
   if (F == F_GENERAL) {
     if (BEND) bnd_kick<N>(r, a, b, n, blo, alo, k.kl, irho, k.kli);
     else str_kick<N>(r, a, b, n, blo, alo, k.kl);
@@ -632,14 +657,8 @@ __device__ __forceinline__ void kick(R6& r, const Kick& k, cdouble* a, cdouble* 
   }
   static_assert(F == F_GENERAL || N == 1 || !BEND, "bends: order 1");
   if (BEND) {
-    // kl (re - (delta - x h) h) = kb x - kl h (delta - x h)
-    const double u = __builtin_fma(-r.x, irho, r.dp);
-    double px = r.px;
-    if (F == F_LEAD) {
-      px = __builtin_fma(-k.kb, r.x, px);
-      r.py = __builtin_fma(k.kb, r.y, r.py);
-    }
-    r.px = __builtin_fma(k.kli, u, px);
+    r.px = __builtin_fma(-k.kl, __builtin_fma(g.c, r.x, -g.d), r.px);
+    if (F == F_LEAD) r.py = __builtin_fma(k.kb, r.y, r.py);
     r.ct = __builtin_fma(k.kli, r.x, r.ct);
     return;
   }
@@ -911,8 +930,10 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
   const Kick c1 = kick_of<BEND, N, F>(a, b, lead, k1, irho, 0.0);
   const Kick c2 = kick_of<BEND, N, F>(a, b, lead, k2, irho, 0.0);
   double nh1[P], nh2[P], nl12[P];  // delta is constant through the slices
+  BendGrad bg[P] = {};
 #pragma unroll
   for (int q = 0; q < P; q++) {
+    if (BEND && F != F_GENERAL) bg[q] = bend_grad(F == F_LEAD ? lead : 0.0, irho, r[q].dp);
     const double h2 = 0.5 * fast_rcp(1.0 + r[q].dp);
     nh1[q] = nl1[q] * h2;
     nh2[q] = nl2[q] * h2;
@@ -931,7 +952,7 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
   };
   auto kicks = [&](const Kick& c) {
 #pragma unroll
-    for (int q = 0; q < P; q++) kick<BEND, N, F>(r[q], c, a, b, n, blo, alo, irho);
+    for (int q = 0; q < P; q++) kick<BEND, N, F>(r[q], c, a, b, n, blo, alo, irho, bg[q]);
   };
   auto body = [&]() {  // a slice without its outer drifts
     kicks(c1);
@@ -942,9 +963,10 @@ __device__ __forceinline__ void mpole_slices(R6* r, cdouble* a, cdouble* b, int 
   };
   drift(nl1, nh1);
   if (F == F_LEAD || F == F_NOFIELD) {
-    const double rest = (2.0 * c1.lo + c2.lo) * (double)nslice;
+    const double lo = (2.0 * c1.lo + c2.lo) * (double)nslice;
+    const double kl = (2.0 * k1 + k2) * (double)nslice;
 #pragma unroll
-    for (int q = 0; q < P; q++) kick_rest<BEND, N, F>(r[q], rest, irho);
+    for (int q = 0; q < P; q++) kick_rest<BEND, N, F>(r[q], lo, kl, irho, bg[q]);
   }
   int m = 1;
   for (; m + U <= nslice; m += U) {

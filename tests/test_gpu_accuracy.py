@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from at_amd import engine
-from at_amd.lattice import Lattice, Particle, Sextupole
+from at_amd.lattice import Dipole, Lattice, Octupole, Particle, Sextupole
 
 pytestmark = [pytest.mark.gpu,
               pytest.mark.skipif(np.finfo(np.longdouble).eps > 2e-19,
@@ -61,6 +61,12 @@ def _beam(scale):
                              * np.array(scale)[:, None])
 
 
+def _rms_units(got, exact):
+    units = (got - exact).astype(float) / np.spacing(np.abs(got))
+    units = units[np.abs(got) > 2e-5]  # a coordinate that passes zero keeps larger roundings
+    return np.sqrt(np.mean(units * units))
+
+
 @pytest.mark.parametrize("s", [0.55, 0.8, 1.1, 1.45])
 def test_sextupole_with_steerer(s):
     m = Sextupole("S", 0.2, 120.0 * s, PolynomB=[1e-5 * s, 0.0, 120.0 * s],
@@ -68,6 +74,30 @@ def test_sextupole_with_steerer(s):
     beam = _beam([1e-3, 1e-4, 1e-3, 1e-4, 1e-3, 1e-3])
     exact, got = _exact(m, beam), _pass(m, beam)
     for k in (1, 3):
-        units = (got[k] - exact[k]).astype(float) / np.spacing(np.abs(got[k]))
-        units = units[np.abs(got[k]) > 2e-5]  # a coordinate that passes zero keeps larger roundings
-        assert np.sqrt(np.mean(units * units)) < 2.4
+        assert _rms_units(got[k], exact[k]) < 2.4
+
+
+@pytest.mark.parametrize("s", [0.55, 0.8, 1.1, 1.25])
+def test_octupole_strength(s):
+    """The part of the error that is proportional to the kick, as a relative error of the
+    strength. The remainder of the product is added once, at the first kick: a coordinate that
+    changes by less than 0.4 leaves 0.4 x 1.1e-16, and the roundings of 20,000 particles
+    2e-17 (5 sigma). Without the remainder: up to 1.1e-16 and the sum of two of them."""
+    m = Octupole("O", 0.05, [0, 0, 0, 0], [0, 0, 0, 60000.0 * s], NumIntSteps=SLICES)
+    beam = _beam([8e-3, 1e-5, 8e-3, 1e-5, 1e-3, 1e-3])
+    exact, got = _exact(m, beam), _pass(m, beam)
+    for k in (1, 3):
+        kick = (exact[k] - beam[k]).astype(float)
+        err = (got[k] - exact[k]).astype(float)
+        assert abs(np.sum(err * kick) / np.sum(kick * kick)) < np.finfo(float).eps / 3
+
+
+@pytest.mark.parametrize("s", [0.55, 0.8, 1.1, 1.45])
+def test_bend_with_gradient(s):
+    """One rounding per kick: 1.58 units, and a hundredth of that for 20,000 particles (the
+    curvature and the gradient kicked one after the other make two, the second on a smaller
+    coordinate: 1.8)."""
+    m = Dipole("B", 1.0, 0.02 * s, -0.6 * s, NumIntSteps=SLICES)
+    beam = _beam([8e-3, 1e-4, 4e-3, 1e-4, 1e-3, 1e-3])
+    exact, got = _exact(m, beam), _pass(m, beam)
+    assert _rms_units(got[1], exact[1]) < 1.65
