@@ -173,8 +173,9 @@ enum OpSlot : int32_t {
   OM_FX_IN = 12, OM_FY_IN = 13, OM_FX_OUT = 14, OM_FY_OUT = 15,  // bends (order 1)
   // entry: x, px, y, py shifts, then cos and sin of the roll; exit: cos, sin, shifts
   OM_XF = 16,
+  OM_INV = 28,  // cos and sin of the inverse rolls (adjoint): entry, exit
 };
-constexpr int kOpConsts = 28;
+constexpr int kOpConsts = 36;
 struct LatOp {
   int32_t op;      // OpKind | OPF_*
   int32_t last;    // index of the record's last element
@@ -184,7 +185,7 @@ struct LatOp {
   double lead;     // their B[order]
   double c[kOpConsts];
 };
-static_assert(sizeof(LatOp) == 256, "LatOp: four 64-byte lines");
+static_assert(sizeof(LatOp) == 320, "LatOp: five 64-byte lines");
 
 // One tracked lattice instance inside a launch. A single-lattice call has one
 // instance; batched error realisations have one per lattice.

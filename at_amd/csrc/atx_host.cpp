@@ -693,6 +693,11 @@ void fill_op(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
     if (h.flags & F_R1) plain = plain && plain_roll(&pool[h.r1], &xf[4], &xf[5]);
     if (h.flags & F_R2) plain = plain && plain_roll(&pool[h.r2], &xf[6], &xf[7]);
     if (op == OP_GENERIC || !plain) return;
+    for (int side = 0; side < 2; side++) {  // the inverse of [c s; -s c] has c, -s over c^2 + s^2
+      const long double c = xf[4 + 2 * side], s = xf[5 + 2 * side];
+      r.c[OM_INV + 2 * side] = (double)(c / (c * c + s * s));
+      r.c[OM_INV + 2 * side + 1] = (double)(s / (c * c + s * s));
+    }
     // the form of the field: which coefficients are not zero
     const double* a = &pool[h.poly];
     const double* b = a + h.order + 1;
