@@ -558,14 +558,14 @@ __global__ void __launch_bounds__(256, 2) adjoint_kernel(AdjArgs args) {
       // the record's form, unless its gradient is of another coefficient or its
       // edges are in the header
       const int order = kind == OP_STR2L || kind == OP_STR2D ? 2 : kind == OP_STR3L ? 3 : 1;
-      const bool form = kind >= OP_STR1L && kind <= OP_BND0 && !(cur.op & OPF_EDGE) &&
+      const bool form = kind >= OP_STR1L && kind <= OP_BND0 && !(cur.op & (OPF_ENDS | OPF_HXF)) &&
                         (sl < 0 || (cur.coeff == order && kind != OP_BND0));
       const bool moved = form && (cur.op & OPF_XF);
       if (moved) {
         shift_rev(r, c + OM_XF + 8);
         roll_rev(r, l, c[OM_XF + 6], c[OM_XF + 7], c[OM_INV + 2], c[OM_INV + 3]);
       }
-      switch (form ? kind : (kind == OP_NONE || kind == OP_APERTURE ? OP_NONE : OP_GENERIC)) {
+      switch (form ? kind : (kind == OP_NONE || kind == OP_APERTURE || kind == OP_MARK ? OP_NONE : OP_GENERIC)) {
 #define ATX_REV(BEND, N, LEAD, DIPOLE) \
   mpole_rev_rec<BEND, N, LEAD, DIPOLE>(r, l, c, cur.nslice, rec->lead, sl, grad, ahead)
         case OP_NONE: ahead(); break;

@@ -124,26 +124,26 @@ static_assert(sizeof(DevElem) == 64, "DevElem must stay 64 bytes (dword fields: 
 // (flag OPF_DRIFT), the element of `op` (other than OP_NONE); `last` is the
 // index of the last of them. The constants an op needs are in the record
 // itself, at fixed offsets, so that no address depends on an earlier load. A
-// terminal record follows the last one: the kernel reads the head (the first
-// 32 bytes) one record ahead.
+// terminal record follows the last one, whole like the others: the kernel reads
+// a record's head and a word of each of its next two lines (up to byte 132) one
+// record ahead.
 enum OpKind : int32_t {
   OP_NONE = 0,      // no element after the markers and the drift
   OP_GENERIC = 1,   // the element by its DevElem header
   OP_APERTURE = 2,  // AperturePass: c[0..3] = limits
-  OP_CORR = 3,      // CorrectorPass without attributes: c[OC_*]
-  // thick multipoles without FieldScaling, quadrupole fringes, apertures and
-  // op table, of the orders that rings are made of: c[OM_*]
+  OP_CORR = 3,      // CorrectorPass: c[OC_*]
+  // thick multipoles with all coefficients (of order 0: as of order 1): c[OM_*]
   OP_STR1 = 4,
   OP_STR2 = 5,
   OP_STR3 = 6,
   OP_BND1 = 7,
   OP_STRRAD1 = 8,
   OP_BNDRAD1 = 9,
-  // ThinMPolePass without attributes: c[OT_*], c[OM_POLY...]
+  // ThinMPolePass: c[OT_*], c[OM_POLY...]
   OP_THIN2 = 10,
   OP_THIN3 = 11,
-  // the same multipoles with few coefficients that are not zero: B[order] only
-  // (L), that and B[0], A[0] (D), none (0)
+  // those of any order up to 3 with few coefficients that are not zero: one B only (L, its
+  // index), B[2], B[0] and A[0] (D), none (0)
   OP_STR1L = 12,
   OP_STR2L = 13,
   OP_STR2D = 14,
@@ -153,39 +153,73 @@ enum OpKind : int32_t {
   OP_STRRAD1L = 18,
   OP_BNDRAD1L = 19,
   OP_BNDRAD0 = 20,
+  OP_STRRAD2 = 21,
+  OP_STRRAD3 = 22,
+  OP_BND2 = 23,
+  OP_BND3 = 24,
+  OP_BNDRAD2 = 25,
+  OP_BNDRAD3 = 26,
+  OP_MARK = 27,     // IdentityPass with apertures
+  OP_DRIFT = 28,    // DriftPass with apertures: c[0] = length
+};
+// The strict build evaluates all coefficients: its kinds, in the highest byte of
+// `op`, are the four kinds of multipole plus MaxOrder. OP_NONE to OP_CORR keep
+// their numbers.
+enum StrictKind : int32_t {
+  SK_THIN2 = 4,
+  SK_THIN3 = 5,
+  SK_MARK = 6,
+  SK_DRIFT = 7,
+  SK_STR = 8,
+  SK_BND = 12,
+  SK_STRRAD = 16,
+  SK_BNDRAD = 20,
 };
 enum : int32_t {
   OPF_DRIFT = 1 << 8,  // a plain drift of length `len` before the element
   OPF_THICK = 2 << 8,  // corrector of non-zero length
   OPF_XF = 4 << 8,     // misaligned by transverse shifts and rolls: c[OM_XF...]
-  OPF_EDGE = 8 << 8,   // a bend's edges by its header (not of constant strength)
+  OPF_ENDS = 8 << 8,   // a bend's edges by its header (not of constant strength, or with
+                       // quadrupole fringes)
   OPF_MPOLE = 16 << 8, // a thick multipole
   OPF_RAD = 32 << 8,   // a radiating one
   OPF_R1 = 64 << 8,    // misaligned with a roll at the entry, at the exit
   OPF_R2 = 128 << 8,
+  OPF_FRINGE = 1 << 16,  // a straight magnet's quadrupole fringes, by the header
+  OPF_HXF = 2 << 16,     // misaligned otherwise: by the header
+  OPF_RAP = 4 << 16,     // rectangular aperture at entry and exit: c[OM_RAP...]
+  OPF_EAP = 8 << 16,     // elliptical one: c[OM_EAP...]
+  OPF_SCALE = 16 << 16,  // FieldScaling: c[OM_SCALE...]
+  OPF_FULL = 32 << 16,   // rare, run by the kernel's full loop only (fast build, strict build)
+  OPF_FULL_STRICT = 64 << 16,
+  OPF_AROUND = OPF_XF | OPF_HXF | OPF_RAP | OPF_EAP | OPF_SCALE | OPF_FRINGE,
 };
+constexpr int kStrictShift = 24;
 // constants of OP_CORR, the thin and the thick multipoles
 enum OpSlot : int32_t {
   OC_XK = 0, OC_YK = 1, OC_LEN = 2, OC_Q0 = 3,
   OT_BAX = 0, OT_BAY = 1,
   OM_L1 = 0, OM_L2 = 1, OM_K1 = 2, OM_K2 = 3, OM_IRHO = 4, OM_RADC = 5, OM_RK1 = 6, OM_RK2 = 7,
-  OM_POLY = 8,  // A[0..order], then B[0..order]
-  OM_FX_IN = 12, OM_FY_IN = 13, OM_FX_OUT = 14, OM_FY_OUT = 15,  // bends (order 1)
+  OM_POLY = 8,  // A[0..order], then B[0..order] (of order 0: as of order 1)
+  OM_FX_IN = 12, OM_FY_IN = 13, OM_FX_OUT = 14, OM_FY_OUT = 15,  // bends
   // entry: x, px, y, py shifts, then cos and sin of the roll; exit: cos, sin, shifts
   OM_XF = 16,
-  OM_INV = 28,  // cos and sin of the inverse rolls (adjoint): entry, exit
+  OM_INV = 28,    // cos and sin of the inverse rolls (adjoint): entry, exit
+  OM_POLY2 = 32,  // A and B of bends of order 2 and 3, in the place of OM_POLY
+  OM_RAP = 40, OM_EAP = 44,
+  OM_SCALE = 46,  // FieldScaling and its reciprocal
 };
-constexpr int kOpConsts = 36;
+constexpr int kOpConsts = 52;
 struct LatOp {
-  int32_t op;      // OpKind | OPF_*
+  int32_t op;      // OpKind | OPF_* | StrictKind << kStrictShift
   int32_t last;    // index of the record's last element
   double len;      // the drift's length
   int32_t first;   // index of its first element (the next record's: one past its last)
   int32_t nslice;  // at least 1 (thick multipoles)
-  double lead;     // their B[order]
+  double lead;     // their highest coefficient that is not zero (B)
   double c[kOpConsts];
 };
-static_assert(sizeof(LatOp) == 320, "LatOp: five 64-byte lines");
+static_assert(sizeof(LatOp) == 448, "LatOp: seven 64-byte lines");
 
 // One tracked lattice instance inside a launch. A single-lattice call has one
 // instance; batched error realisations have one per lattice.
@@ -215,7 +249,7 @@ struct Instance {
   int32_t losses;           // 1: record the loss map (at.c checkiflost); 0: setlost only;
                             // 2: as 1, continuing the map of an earlier call
   int32_t elempass;         // 1: single element pass, no loss check (at.c at_elempass)
-  int32_t pad;
+  int32_t full;             // the lattice has records with OPF_FULL (OPF_FULL_STRICT)
   // Repacked launches: lanes take particles idx[0..*nlive) instead of
   // 0..npart (both written by repack_kernel); NULL for plain launches.
   const int32_t* idx;

@@ -213,6 +213,7 @@ struct DeviceCopy {
   atx::DevElem* elems = nullptr;
   double* pool = nullptr;
   int32_t* opof = nullptr;
+  bool full = false, full_strict = false;  // records that only the full loop runs
   // host copies of per-element compile results used by the adjoint
   std::vector<int32_t> r1inv, r2inv, order, kind;
   std::vector<int32_t> last;  // last element of each program record (not of the terminal one)
@@ -648,87 +649,139 @@ bool plain_roll(const double* m, double* c, double* s) {
   return true;
 }
 
+// The maps around an element that its record holds: FieldScaling, apertures and
+// misalignments, those that are neither shifts nor rolls by the element's header
+// (flags of the result; -1: not representable). The kernel takes 1/(1+delta) after
+// them, the reference before T1 and R1, so these have to leave delta alone.
+int32_t fill_around(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
+  int32_t op = 0;
+  if (h.flags & F_SCALE) {
+    op |= OPF_SCALE | OPF_FULL | OPF_FULL_STRICT;
+    r.c[OM_SCALE] = pool[h.sc + S_SCALE];
+    r.c[OM_SCALE + 1] = pool[h.sc + S_INVSCALE];
+  }
+  if (h.flags & F_RAP) {
+    op |= OPF_RAP;
+    for (int k = 0; k < 4; k++) r.c[OM_RAP + k] = pool[h.rap + k];
+  }
+  if (h.flags & F_EAP) {
+    op |= OPF_EAP | OPF_FULL | OPF_FULL_STRICT;
+    for (int k = 0; k < 2; k++) r.c[OM_EAP + k] = pool[h.eap + k];
+  }
+  if (!(h.flags & (F_T1 | F_T2 | F_R1 | F_R2))) return op;
+  // A missing transform leaves a coordinate as it is: + -0.0, and no roll in
+  // the strict build (in the fast one (1, 0), which does so for finite ones).
+  // The sums of a rolled coordinate start from 0.0, so one that is zero is
+  // +0.0: with a roll the zeros of a shift are +0.0, before it and after it.
+  double* xf = r.c + OM_XF;
+  const double* t1 = (h.flags & F_T1) ? &pool[h.t1] : nullptr;
+  const double* t2 = (h.flags & F_T2) ? &pool[h.t2] : nullptr;
+  const double zero1 = (h.flags & F_R1) ? 0.0 : -0.0, zero2 = (h.flags & F_R2) ? 0.0 : -0.0;
+  for (int k = 0; k < 4; k++) {
+    xf[k] = (t1 ? t1[k] : -0.0) + zero1;
+    xf[8 + k] = (t2 ? t2[k] : -0.0) + zero2;
+  }
+  xf[4] = xf[6] = 1.0;
+  bool plain = (!t1 || plain_shift(t1)) && (!t2 || plain_shift(t2));
+  if (h.flags & F_R1) plain = plain_roll(&pool[h.r1], &xf[4], &xf[5]) && plain;
+  if (h.flags & F_R2) plain = plain_roll(&pool[h.r2], &xf[6], &xf[7]) && plain;
+  if (!plain) {
+    if (t1 && t1[4] != 0.0) return -1;
+    for (int k = 0; k < 6 && (h.flags & F_R1); k++)
+      if (pool[h.r1 + 4 + 6 * k] != (k == 4 ? 1.0 : 0.0)) return -1;
+    return op | OPF_HXF | OPF_FULL | OPF_FULL_STRICT;
+  }
+  for (int side = 0; side < 2; side++) {  // the inverse of [c s; -s c] has c, -s over c^2 + s^2
+    const long double c = xf[4 + 2 * side], s = xf[5 + 2 * side];
+    r.c[OM_INV + 2 * side] = (double)(c / (c * c + s * s));
+    r.c[OM_INV + 2 * side + 1] = (double)(s / (c * c + s * s));
+  }
+  return op | OPF_XF | ((h.flags & F_R1) ? OPF_R1 : 0) | ((h.flags & F_R2) ? OPF_R2 : 0);
+}
+
+// The form of a thick multipole's field: its kind by its highest coefficient that
+// is not zero, `lead` that coefficient if it is a B and the only one.
+int32_t field_form(const DevElem& h, const double* a, const double* b, double* lead) {
+  const bool bend = h.kind == K_BND || h.kind == K_BNDRAD;
+  const bool rad = h.kind == K_STRRAD || h.kind == K_BNDRAD;
+  int n = h.order;
+  while (n > 0 && a[n] == 0.0 && b[n] == 0.0) n--;
+  bool only = a[n] == 0.0;  // B[n] and no other from 1 on
+  for (int k = 1; k < n; k++) only = only && a[k] == 0.0 && b[k] == 0.0;
+  const bool dipole = a[0] != 0.0 || b[0] != 0.0;
+  *lead = b[h.order];
+  if (only && !dipole) {
+    *lead = n > 0 ? b[n] : 0.0;
+    if (bend && n == 0) return rad ? OP_BNDRAD0 : OP_BND0;
+    if (n <= 1) return bend ? (rad ? OP_BNDRAD1L : OP_BND1L) : (rad ? OP_STRRAD1L : OP_STR1L);
+    if (!bend && !rad) return n == 2 ? OP_STR2L : OP_STR3L;
+    *lead = b[h.order];
+  }
+  if (only && n == 2 && h.order == 2 && h.kind == K_STR) return OP_STR2D;
+  static const int32_t general[4][3] = {{OP_STR1, OP_STR2, OP_STR3},
+                                        {OP_BND1, OP_BND2, OP_BND3},
+                                        {OP_STRRAD1, OP_STRRAD2, OP_STRRAD3},
+                                        {OP_BNDRAD1, OP_BNDRAD2, OP_BNDRAD3}};
+  return general[(bend ? 1 : 0) + (rad ? 2 : 0)][std::max(h.order, 1) - 1];
+}
+
 // The op of an element with constants in its record, or OP_GENERIC.
 void fill_op(const DevElem& h, const std::vector<double>& pool, LatOp& r) {
   const double* sc = &pool[h.sc];
   const int32_t drift = r.op;  // the flags so far
-  r.op = drift | OP_GENERIC;
+  r.op = drift | OP_GENERIC | (OP_GENERIC << kStrictShift);
+  auto set = [&](int32_t op, int32_t strict) { r.op = drift | op | (strict << kStrictShift); };
   if (h.kind == K_APERTURE) {
-    r.op = drift | OP_APERTURE;
+    set(OP_APERTURE, OP_APERTURE);
     for (int k = 0; k < 4; k++) r.c[k] = pool[h.rap + k];
-  } else if (h.kind == K_CORR && (h.flags & ~(uint32_t)F_THICK) == 0) {
-    r.op = drift | OP_CORR | ((h.flags & F_THICK) ? OPF_THICK : 0);
+    return;
+  }
+  const bool straight = !(h.flags & (F_T1 | F_T2 | F_R1 | F_R2 | F_SCALE));
+  if (h.kind == K_IDENTITY && straight) {
+    set(OP_MARK | fill_around(h, pool, r), SK_MARK);
+  } else if (h.kind == K_DRIFT && straight) {
+    set(OP_DRIFT | fill_around(h, pool, r), SK_DRIFT);
+    r.c[0] = sc[S_D_LEN];
+  } else if (h.kind == K_CORR && straight) {
+    set(OP_CORR | ((h.flags & F_THICK) ? OPF_THICK : 0) | fill_around(h, pool, r), OP_CORR);
     r.c[OC_XK] = sc[S_C_XK];
     r.c[OC_YK] = sc[S_C_YK];
     r.c[OC_LEN] = sc[S_C_LEN];
     r.c[OC_Q0] = sc[S_C_Q0];
-  } else if (h.kind == K_THIN && h.flags == 0 && (h.order == 2 || h.order == 3)) {
-    r.op = drift | (h.order == 2 ? OP_THIN2 : OP_THIN3);
+  } else if (h.kind == K_THIN && straight && (h.order == 2 || h.order == 3)) {
+    set((h.order == 2 ? OP_THIN2 : OP_THIN3) | fill_around(h, pool, r),
+        h.order == 2 ? SK_THIN2 : SK_THIN3);
     r.c[OT_BAX] = sc[S_BAX];
     r.c[OT_BAY] = sc[S_BAY];
     for (int k = 0; k < 2 * (h.order + 1); k++) r.c[OM_POLY + k] = pool[h.poly + k];
   } else if ((h.kind == K_STR || h.kind == K_BND || h.kind == K_STRRAD || h.kind == K_BNDRAD) &&
-             !(h.flags & (F_RAP | F_EAP | F_SCALE)) && h.fringe == 0 && h.ops < 0 && h.nslice > 0) {
-    int op = OP_GENERIC;
-    if (h.kind == K_STR && h.order >= 1 && h.order <= 3) op = OP_STR1 + (h.order - 1);
-    if (h.order == 1) {
-      if (h.kind == K_BND) op = OP_BND1;
-      if (h.kind == K_STRRAD) op = OP_STRRAD1;
-      if (h.kind == K_BNDRAD) op = OP_BNDRAD1;
-    }
-    // A missing transform leaves a coordinate as it is: + -0.0, and no roll in
-    // the strict build (in the fast one (1, 0), which does so for finite ones).
-    // The sums of a rolled coordinate start from 0.0, so one that is zero is
-    // +0.0: with a roll the zeros of a shift are +0.0, before it and after it.
-    double* xf = r.c + OM_XF;
-    const double* t1 = (h.flags & F_T1) ? &pool[h.t1] : nullptr;
-    const double* t2 = (h.flags & F_T2) ? &pool[h.t2] : nullptr;
-    const double zero1 = (h.flags & F_R1) ? 0.0 : -0.0, zero2 = (h.flags & F_R2) ? 0.0 : -0.0;
-    for (int k = 0; k < 4; k++) {
-      xf[k] = (t1 ? t1[k] : -0.0) + zero1;
-      xf[8 + k] = (t2 ? t2[k] : -0.0) + zero2;
-    }
-    xf[4] = xf[6] = 1.0;
-    bool plain = (!t1 || plain_shift(t1)) && (!t2 || plain_shift(t2));
-    if (h.flags & F_R1) plain = plain && plain_roll(&pool[h.r1], &xf[4], &xf[5]);
-    if (h.flags & F_R2) plain = plain && plain_roll(&pool[h.r2], &xf[6], &xf[7]);
-    if (op == OP_GENERIC || !plain) return;
-    for (int side = 0; side < 2; side++) {  // the inverse of [c s; -s c] has c, -s over c^2 + s^2
-      const long double c = xf[4 + 2 * side], s = xf[5 + 2 * side];
-      r.c[OM_INV + 2 * side] = (double)(c / (c * c + s * s));
-      r.c[OM_INV + 2 * side + 1] = (double)(s / (c * c + s * s));
-    }
-    // the form of the field: which coefficients are not zero
+             h.ops < 0 && h.nslice > 0 && h.order <= 3) {
+    const int32_t around = fill_around(h, pool, r);
+    if (around < 0) return;
+    const bool bend = h.kind == K_BND || h.kind == K_BNDRAD;
+    const bool rad = h.kind == K_STRRAD || h.kind == K_BNDRAD;
     const double* a = &pool[h.poly];
     const double* b = a + h.order + 1;
-    bool lead = true;
-    for (int k = 1; k <= h.order; k++) lead = lead && a[k] == 0.0 && (k == h.order || b[k] == 0.0);
-    const bool dipole = a[0] != 0.0 || b[0] != 0.0;
-    if (lead && !dipole) {
-      switch (op) {
-        case OP_STR1: op = OP_STR1L; break;
-        case OP_STR2: op = OP_STR2L; break;
-        case OP_STR3: op = OP_STR3L; break;
-        case OP_STRRAD1: op = OP_STRRAD1L; break;
-        case OP_BND1: op = b[1] == 0.0 ? OP_BND0 : OP_BND1L; break;
-        case OP_BNDRAD1: op = b[1] == 0.0 ? OP_BNDRAD0 : OP_BNDRAD1L; break;
-      }
-    } else if (lead && op == OP_STR2) {
-      op = OP_STR2D;
-    }
-    op |= OPF_MPOLE;
-    if (h.kind == K_STRRAD || h.kind == K_BNDRAD) op |= OPF_RAD;
-    if (h.flags & (F_T1 | F_T2 | F_R1 | F_R2)) op |= OPF_XF;
-    if (h.flags & F_R1) op |= OPF_R1;
-    if (h.flags & F_R2) op |= OPF_R2;
-    if ((h.edge & 0xff) != E_CONST || ((h.edge >> 8) & 0xff) != E_CONST) op |= OPF_EDGE;
-    r.op = drift | op;
+    int32_t op = field_form(h, a, b, &r.lead) | around | OPF_MPOLE;
+    if (rad) op |= OPF_RAD;
+    if (bend && (h.edge != (E_CONST | (E_CONST << 8)) || h.fringe != 0)) op |= OPF_ENDS;
+    if (!bend && h.fringe != 0) op |= OPF_FRINGE;
+    const int32_t kind = op & 0xff;
+    if (kind >= OP_STRRAD2 && kind <= OP_BNDRAD3) op |= OPF_FULL;
+    // the strict build has straight magnets of orders 1 to 3 (radiating: 1 and 2) and
+    // bends of orders 0 and 1 inline
+    if (bend ? h.order > 1 : h.order == 0 || (rad && h.order == 3)) op |= OPF_FULL_STRICT;
+    set(op, (bend ? (rad ? SK_BNDRAD : SK_BND) : (rad ? SK_STRRAD : SK_STR)) + h.order);
     r.nslice = h.nslice;
-    r.lead = b[h.order];
     static const int from[8] = {S_L1, S_L2, S_K1, S_K2, S_IRHO, S_RADC, S_RK1, S_RK2};
     for (int k = 0; k < 8; k++) r.c[k] = sc[from[k]];
-    for (int k = 0; k < 2 * (h.order + 1); k++) r.c[OM_POLY + k] = pool[h.poly + k];
-    if (h.kind == K_BND || h.kind == K_BNDRAD) {
+    const int rows = std::max(h.order, 1) + 1;
+    double* poly = r.c + (bend && h.order > 1 ? OM_POLY2 : OM_POLY);
+    for (int k = 0; k <= h.order; k++) {
+      poly[k] = a[k];
+      poly[rows + k] = b[k];
+    }
+    if (bend) {
       r.c[OM_FX_IN] = sc[S_FX_IN];
       r.c[OM_FY_IN] = sc[S_FY_IN];
       r.c[OM_FX_OUT] = sc[S_FX_OUT];
@@ -856,7 +909,12 @@ int ensure_device_lattice(atx_lattice* lat, double energy, double rest, bool ele
   d.r2inv = c.r2inv;
   d.adjerr = c.adjerr;
   d.last.clear();
-  for (size_t k = 0; k + 1 < c.ops.size(); k++) d.last.push_back(c.ops[k].last);
+  d.full = d.full_strict = false;
+  for (size_t k = 0; k + 1 < c.ops.size(); k++) {
+    d.last.push_back(c.ops[k].last);
+    d.full |= (c.ops[k].op & OPF_FULL) != 0;
+    d.full_strict |= (c.ops[k].op & OPF_FULL_STRICT) != 0;
+  }
   d.order.clear();
   d.kind.clear();
   for (const auto& h : c.elems) {
@@ -1196,7 +1254,7 @@ int launch_repacked(std::vector<Instance>& insts, const std::vector<const std::v
 int single_instance(atx_lattice* lat, double* d_r, int64_t pstride, int64_t cstride, uint32_t np,
                     int nturns, const uint32_t* refpts, uint32_t nref, int turn0, int start, int end,
                     double* d_rout, uint8_t* d_lf, uint32_t* d_lt, uint32_t* d_le, double* d_lc,
-                    int losses, bool elempass, int32_t* bits, Instance& inst) {
+                    int losses, bool elempass, bool strict, int32_t* bits, Instance& inst) {
   const int nelem = (int)lat->elems.size();
   std::vector<int32_t> ranks(2 * (size_t)(nelem + 1));
   const int n_first = turn_slots(refpts, (int)nref, start, end, nelem, ranks.data());
@@ -1229,6 +1287,7 @@ int single_instance(atx_lattice* lat, double* d_r, int64_t pstride, int64_t cstr
   inst.block_begin = 0;
   inst.losses = losses ? 1 : 0;
   inst.elempass = elempass ? 1 : 0;
+  inst.full = (strict ? d.full_strict : d.full) ? 1 : 0;
   return ATX_OK;
 }
 
@@ -1241,7 +1300,7 @@ int track_device(atx_lattice* lat, double* d_r, int64_t pstride, int64_t cstride
   std::vector<std::vector<int32_t>> slots(1, std::vector<int32_t>(ref_words(nelem)));
   std::vector<Instance> insts(1);
   int rc = single_instance(lat, d_r, pstride, cstride, np, nturns, refpts, nref, turn0, start, end,
-                           d_rout, d_lf, d_lt, d_le, d_lc, losses, elempass, slots[0].data(), insts[0]);
+                           d_rout, d_lf, d_lt, d_le, d_lc, losses, elempass, strict, slots[0].data(), insts[0]);
   if (rc) return rc;
   if (np == 0 || nturns <= 0) return ATX_OK;
   atx_launch_shape shape;
@@ -1643,6 +1702,7 @@ int atx_track_batch(const atx_batch_item* items, int32_t nitems, int32_t nturns,
     in.pool = it.lattice->dev[0].pool;
     in.ops = it.lattice->dev[0].ops;
     in.opof = it.lattice->dev[0].opof;
+    in.full = (strict ? it.lattice->dev[0].full_strict : it.lattice->dev[0].full) ? 1 : 0;
     in.r = it.r;
     in.lost_flag = it.lost_flag;
     in.lost_turn = it.lost_turn;
@@ -1750,6 +1810,7 @@ int atx_track_batch_noalloc(const atx_batch_item* items, int32_t nitems, int32_t
     in.pool = copy.pool;
     in.ops = copy.ops;
     in.opof = copy.opof;
+    in.full = (strict ? copy.full_strict : copy.full) ? 1 : 0;
     in.slots = nullptr;  // no refpts: the kernel reads no slot table
     in.r = it.r;
     in.lost_flag = it.lost_flag;

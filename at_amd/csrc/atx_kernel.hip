@@ -8,7 +8,8 @@
 // lane of a wave is at the same record, so its constants land in SGPRs and
 // its branches are scalar. The loop over the records has no divergent branch
 // (losses, the only ones, are handled in a function that the whole wave
-// calls), and keeps the common elements inline and all others in functions.
+// calls), and keeps the common elements inline and all others in functions;
+// lattices with rarer forms or maps (OPF_FULL) take a loop that has those, too.
 //
 // This file is compiled twice:
 //   ATX_STRICT=1, -ffp-contract=off: the reference operation order of
@@ -544,8 +545,8 @@ __device__ __noinline__ R6 slices_ops(R6 r, cdouble* a, cdouble* b, int n, cdoub
 // instructions instead of 6 per quadrupole kick, 5 instead of 10 per sextupole
 // kick, 8 instead of 14 per octupole kick, 19 instead of 23 per radiating
 // quadrupole kick, 20 instead of 33 per kick of a radiating bend without
-// gradient. The VALU issues on 83 % of the cycles of a full device, so time
-// follows the instruction count. The strict build evaluates all coefficients.
+// gradient. (The VALU issued on 83 % of the cycles of a full device before that,
+// so time follows the instruction count.) The strict build evaluates all coefficients.
 // A particle whose result is not finite is recomputed with the general form
 // (run_turn): zeros times an infinity are NaN there, as in the reference.
 enum Form : int {
@@ -655,7 +656,6 @@ __device__ __forceinline__ void kick(R6& r, const Kick& k, cdouble* a, cdouble* 
     else str_kick<N>(r, a, b, n, blo, alo, k.kl);
     return;
   }
-  static_assert(F == F_GENERAL || N == 1 || !BEND, "bends: order 1");
   if (BEND) {
     r.px = __builtin_fma(-k.kl, __builtin_fma(g.c, r.x, -g.d), r.px);
     if (F == F_LEAD) r.py = __builtin_fma(k.kb, r.y, r.py);
@@ -995,7 +995,11 @@ __device__ __forceinline__ void mpole_rad_slices(R6* r, cdouble* a, cdouble* b, 
   double blo, alo;
   horner_addends<N>(a, b, n, blo, alo);
   const double rk = ATX_STRICT ? radc : rk1;
-  if (F == F_GENERAL && N == 1) ahead(l1, l2, k1, k2, rk, rk2, a[1], b[1], a[0], b[0]);
+  if (F == F_GENERAL && N == 3)
+    ahead(l1, l2, k1, k2, rk, rk2, a[3], b[3], a[2], b[2], a[1], b[1], a[0], b[0]);
+  else if (F == F_GENERAL && N == 2)
+    ahead(l1, l2, k1, k2, rk, rk2, a[2], b[2], a[1], b[1], a[0], b[0]);
+  else if (F == F_GENERAL && N == 1) ahead(l1, l2, k1, k2, rk, rk2, a[1], b[1], a[0], b[0]);
   else ahead(l1, l2, k1, k2, rk, rk2);
 #if ATX_STRICT
   const double ki1 = k1 * irho, ki2 = k2 * irho;
@@ -1169,7 +1173,9 @@ __device__ __forceinline__ T uniform(T p) {
 // the loop over the records then keeps its registers (and its code, which
 // has to stay in the instruction cache) for the common ops. A call costs about
 // 0.4 us with one wave per SIMD (the callee saves the scalar registers it
-// uses), so what rings are made of runs inline.
+// uses), so what has a record runs inline: multipoles of orders above 3 and of
+// other integrators, misaligned elements of other kinds, cavities and the exact
+// passes are left.
 template <bool BEND, bool RAD, int N, int U, bool LEAN>
 __device__ __noinline__ R6 mpole_call(R6 r, cDevElem* hp, cdouble* poolp) {
   cDevElem& h = *uniform(hp);
@@ -1836,23 +1842,31 @@ __device__ __forceinline__ uint64_t lost_lanes(const R6& r) {
          __builtin_amdgcn_ballot_w64(!(__builtin_fabs(r.dp) <= 1.0));
 }
 
-// An edge of a bend by its header.
-__device__ __noinline__ R6 edge_call(R6 r, cDevElem* hp, cdouble* poolp, int exit) {
+// The ends of a magnet by its header: a bend's edge and the quadrupole fringe.
+__device__ __noinline__ R6 ends_call(R6 r, cDevElem* hp, cdouble* poolp, int exit) {
   cDevElem& h = *uniform(hp);
-  cdouble* s = uniform(poolp) + h.sc;
-  if (__builtin_amdgcn_readfirstlane(exit))
-    edge<false>(r, (h.edge >> 8) & 0xff, s[S_IRHO], s[S_FX_OUT], s[S_FY_OUT], s[S_EDGE_OUT],
-                s[S_CORR_OUT], -1.0);
-  else
-    edge<false>(r, h.edge & 0xff, s[S_IRHO], s[S_FX_IN], s[S_FY_IN], s[S_EDGE_IN], s[S_CORR_IN],
-                1.0);
+  cdouble* pool = uniform(poolp);
+  cdouble* s = pool + h.sc;
+  const bool bend = h.kind == K_BND || h.kind == K_BNDRAD;
+  if (__builtin_amdgcn_readfirstlane(exit)) {
+    if (h.fringe & 0xff00) quad_fringe_out(r, h, pool, s[S_B2]);
+    if (bend)
+      edge<false>(r, (h.edge >> 8) & 0xff, s[S_IRHO], s[S_FX_OUT], s[S_FY_OUT], s[S_EDGE_OUT],
+                  s[S_CORR_OUT], -1.0);
+  } else {
+    if (bend)
+      edge<false>(r, h.edge & 0xff, s[S_IRHO], s[S_FX_IN], s[S_FY_IN], s[S_EDGE_IN], s[S_CORR_IN],
+                  1.0);
+    if (h.fringe & 0xff) quad_fringe_in(r, h, pool, s[S_B2]);
+  }
   return r;
 }
 
 // Head of a program record, read one record ahead: its flags and op, the
 // index of its last element, its drift's length, its number of slices and
-// leading coefficient, its first constants. It holds a word of the record's next
-// two lines, too: reading them brings the lines into the scalar cache.
+// leading coefficient. It holds a word of the record's next two lines, too: reading
+// them brings the lines into the scalar cache. (Its first constants are read with
+// the record itself.)
 struct OpConsts {
   double v[8];
 };
@@ -1873,26 +1887,25 @@ __device__ __forceinline__ OpConsts op_consts(cLatOp* p) {
 }
 
 __device__ __forceinline__ OpHead op_head(cLatOp* p) {
-  return OpHead{p->op, p->last, p->len, p->first, p->nslice, p->lead, op_consts(p),
+  return OpHead{p->op, p->last, p->len, p->first, p->nslice, p->lead, OpConsts{},
                 ((cint*)p)[16], ((cint*)p)[32]};
 }
 
 // A thick multipole by its record; the misalignment is applied around it by
 // the caller. CHECKED, bad: rad_kick_ang.
-template <bool BEND, bool RAD, int N, int F, int P, int U, bool CHECKED, class Ahead>
-__device__ __forceinline__ void mpole_op(R6* r, const OpHead& o, cdouble* c, cDevElem* h,
-                                         cdouble* pool, uint64_t& bad,
-                                         const Ahead& ahead) {
-  cdouble* a = c + OM_POLY;
-  cdouble* b = a + N + 1;
+template <bool BEND, bool RAD, int N, int F, int P, int U, bool CHECKED, class Header, class Ahead>
+__device__ __forceinline__ void mpole_op(R6* r, const OpHead& o, cdouble* c, const Header& hdr,
+                                         uint64_t& bad, const Ahead& ahead) {
+  cdouble* a = c + (BEND && N > 1 ? OM_POLY2 : OM_POLY);
+  cdouble* b = a + (N == 0 ? 2 : N + 1);
   const int nslice = o.nslice, flags = o.op;
   const OpConsts& k = o.k;
   const double irho = BEND ? k.v[OM_IRHO] : 0.0;
   if (BEND) {
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      if (flags & OPF_EDGE) {
-        r[q] = edge_call(r[q], h, pool, 0);
+      if (flags & OPF_ENDS) {
+        r[q] = ends_call(r[q], hdr.elem(), hdr.pool(), 0);
       } else {
         r[q].px += r[q].x * c[OM_FX_IN];
         r[q].py -= r[q].y * c[OM_FY_IN];
@@ -1917,8 +1930,8 @@ __device__ __forceinline__ void mpole_op(R6* r, const OpHead& o, cdouble* c, cDe
   if (BEND) {
 #pragma unroll
     for (int q = 0; q < P; q++) {
-      if (flags & OPF_EDGE) {
-        r[q] = edge_call(r[q], h, pool, 1);
+      if (flags & OPF_ENDS) {
+        r[q] = ends_call(r[q], hdr.elem(), hdr.pool(), 1);
       } else {
         r[q].px += r[q].x * c[OM_FX_OUT];
         r[q].py -= r[q].y * c[OM_FY_OUT];
@@ -1975,57 +1988,133 @@ __device__ __forceinline__ void shift(R6& r, cdouble* t) {
 // product, as in the reference: a wave with one takes the product. (An infinite
 // x of a particle without loss record enters a magnet; others come out of one.
 // The fast build runs the whole element again, op_call.)
-__device__ __forceinline__ void strict_roll(R6& r, cdouble* cs, cdouble* m) {
+template <class Matrix>
+__device__ __forceinline__ void strict_roll(R6& r, cdouble* cs, const Matrix& m) {
   if (__builtin_expect(lost_lanes(r) != 0, 0))
-    r = mul_r_v(r, m);
+    r = mul_r_v(r, m());
   else
     roll(r, cs[0], cs[1]);
 }
 #endif
 
+// Where an element's header and the pool are: known, or looked up in the instance
+// when they are needed, so that the loop over the records does not keep them in
+// scalar registers for what is rare.
+struct KnownHeader {
+  cDevElem* e;
+  cdouble* p;
+  __device__ __forceinline__ cDevElem* elem() const { return e; }
+  __device__ __forceinline__ cdouble* pool() const { return p; }
+};
+struct LateHeader {
+  cInstance* inst;
+  int index;
+  __device__ __forceinline__ cInstance* late() const {
+    cInstance* p = inst;
+    asm volatile("" : "+s"(p));
+    return p;
+  }
+  __device__ __forceinline__ cDevElem* elem() const { return (cDevElem*)late()->elems + index; }
+  __device__ __forceinline__ cdouble* pool() const { return (cdouble*)late()->pool; }
+};
+
+// The maps before and after an element that its record holds. FULL: all of them,
+// otherwise those of elements without OPF_FULL. (One test for the last three first,
+// in the build without copies: 3.63 against 3.73 ms per turn for 131,072 particles of
+// a misaligned ring; with copies each by itself: 2.53 against 2.70 ms, 8,191.)
+template <bool FULL, bool REFS, class Header>
+__device__ __forceinline__ void around_entry(R6& r, int op, cdouble* c, const Header& hdr) {
+  if (FULL && (op & OPF_SCALE)) change_pref(r, c[OM_SCALE]);
+  if (op & OPF_XF) {
+    shift(r, c + OM_XF);
+#if ATX_STRICT
+    if (op & OPF_R1) strict_roll(r, c + OM_XF + 4, [&]() { return hdr.pool() + hdr.elem()->r1; });
+#else
+    roll(r, c[OM_XF + 4], c[OM_XF + 5]);
+#endif
+  }
+  if (FULL && (op & OPF_HXF)) {
+    cDevElem& h = *hdr.elem();
+    if (h.flags & F_T1) add_t(r, hdr.pool() + h.t1);
+    if (h.flags & F_R1) r = mul_r_inl(r, hdr.pool() + h.r1);
+  }
+  if (REFS || (op & (OPF_RAP | OPF_EAP | OPF_FRINGE))) {
+    if (op & OPF_RAP) rect_ap(r, c + OM_RAP);
+    if (FULL && (op & OPF_EAP)) ellip_ap(r, c + OM_EAP);
+    if (op & OPF_FRINGE) r = ends_call(r, hdr.elem(), hdr.pool(), 0);
+  }
+}
+
+template <bool FULL, bool REFS, class Header>
+__device__ __forceinline__ void around_exit(R6& r, int op, cdouble* c, const Header& hdr) {
+  if (REFS || (op & (OPF_RAP | OPF_EAP | OPF_FRINGE))) {
+    if (op & OPF_FRINGE) r = ends_call(r, hdr.elem(), hdr.pool(), 1);
+    // (an element without length has one aperture; the second changes nothing)
+    if (op & OPF_RAP) rect_ap(r, c + OM_RAP);
+    if (FULL && (op & OPF_EAP)) ellip_ap(r, c + OM_EAP);
+  }
+  if (FULL && (op & OPF_HXF)) {
+    cDevElem& h = *hdr.elem();
+    if (h.flags & F_R2) r = mul_r_inl(r, hdr.pool() + h.r2);
+    if (h.flags & F_T2) add_t(r, hdr.pool() + h.t2);
+  }
+  if (op & OPF_XF) {
+#if ATX_STRICT
+    if (op & OPF_R2) strict_roll(r, c + OM_XF + 6, [&]() { return hdr.pool() + hdr.elem()->r2; });
+#else
+    roll(r, c[OM_XF + 6], c[OM_XF + 7]);
+#endif
+    shift(r, c + OM_XF + 8);
+  }
+  if (FULL && (op & OPF_SCALE)) change_pref(r, c[OM_SCALE + 1]);
+}
+
 // The element of a record other than its markers and drift, for the P
-// particles of a lane. CHECKED, bad: rad_kick_ang; ahead: NotAhead.
-template <int P, int U, bool CHECKED, class Ahead>
-__device__ __forceinline__ void run_op(R6* r, const OpHead& o, cLatOp* rec, cDevElem* h,
-                                       cdouble* pool, int nturn, uint64_t& bad,
-                                       const Ahead& ahead) {
+// particles of a lane. CHECKED, bad: rad_kick_ang; ahead: NotAhead. FULL: with the
+// kinds that have OPF_FULL.
+template <int P, int U, bool CHECKED, bool FULL, bool REFS, class Header, class Turn, class Ahead>
+__device__ __forceinline__ void run_op(R6* r, const OpHead& o, cLatOp* rec, const Header& hdr,
+                                       const Turn& nturn, uint64_t& bad, const Ahead& ahead) {
   cdouble* c = rec->c;
   const OpConsts& k = o.k;
   const int op = o.op;
-  if (op & OPF_XF) {
+  if (op & OPF_AROUND) {
 #pragma unroll
-    for (int q = 0; q < P; q++) {
-#if ATX_STRICT
-      shift(r[q], c + OM_XF);
-      if (op & OPF_R1) strict_roll(r[q], c + OM_XF + 4, pool + h->r1);
-#else
-      shift(r[q], c + OM_XF);
-      roll(r[q], c[OM_XF + 4], c[OM_XF + 5]);
-#endif
-    }
+    for (int q = 0; q < P; q++) around_entry<FULL, REFS>(r[q], op, c, hdr);
   }
 #define ATX_MPOLE(BEND, RAD, N, F) \
-  mpole_op<BEND, RAD, N, F, P, U, CHECKED>(r, o, c, h, pool, bad, ahead)
+  mpole_op<BEND, RAD, N, F, P, U, CHECKED>(r, o, c, hdr, bad, ahead)
   // One bit per kind, tested in groups and in the order of how common they are:
   // a test that fails falls through, where a switch becomes a tree of five
   // levels with a taken branch at most of them. (The shift is opaque, as the
   // tests would be turned into that switch.)
   uint32_t sel;
-  asm("s_lshl_b32 %0, 1, %1" : "=s"(sel) : "s"(op & 0xff) : "scc");
+  asm("s_lshl_b32 %0, 1, %1" : "=s"(sel) : "s"(ATX_STRICT ? op >> kStrictShift : op & 0xff) : "scc");
   auto is = [&](auto... k) { return (sel & ((1u << k) | ...)) != 0; };
 #if ATX_STRICT
   constexpr int kGen = F_GENERAL;  // all coefficients, whatever the form
-  if (is(OP_STRRAD1, OP_STRRAD1L, OP_BNDRAD1, OP_BNDRAD1L, OP_BNDRAD0)) {
-    if (is(OP_STRRAD1, OP_STRRAD1L)) ATX_MPOLE(false, true, 1, kGen);
-    else ATX_MPOLE(true, true, 1, kGen);
-  } else if (is(OP_STR1, OP_STR1L, OP_BND1, OP_BND1L, OP_BND0)) {
-    if (is(OP_STR1, OP_STR1L)) ATX_MPOLE(false, false, 1, kGen);
-    else ATX_MPOLE(true, false, 1, kGen);
-  } else if (is(OP_STR2, OP_STR2L, OP_STR2D)) {
-    ATX_MPOLE(false, false, 2, kGen);
-  } else if (is(OP_STR3, OP_STR3L)) {
-    ATX_MPOLE(false, false, 3, kGen);
+  auto from = [&](auto k) { return (sel >> k) != 0; };
+  if (from(SK_STRRAD)) {
+    if (is(SK_STRRAD + 1)) ATX_MPOLE(false, true, 1, kGen);
+    else if (is(SK_BNDRAD + 1)) ATX_MPOLE(true, true, 1, kGen);
+    else if (is(SK_BNDRAD)) ATX_MPOLE(true, true, 0, kGen);
+    else if (!FULL || is(SK_STRRAD + 2)) ATX_MPOLE(false, true, 2, kGen);
+    else if (is(SK_BNDRAD + 2)) ATX_MPOLE(true, true, 2, kGen);
+    else if (is(SK_STRRAD + 3)) ATX_MPOLE(false, true, 3, kGen);
+    else if (is(SK_BNDRAD + 3)) ATX_MPOLE(true, true, 3, kGen);
+    else ATX_MPOLE(false, true, 0, kGen);
+  } else if (from(SK_STR)) {
+    if (is(SK_STR + 1)) ATX_MPOLE(false, false, 1, kGen);
+    else if (is(SK_STR + 2)) ATX_MPOLE(false, false, 2, kGen);
+    else if (is(SK_BND + 1)) ATX_MPOLE(true, false, 1, kGen);
+    else if (is(SK_STR + 3)) ATX_MPOLE(false, false, 3, kGen);
+    else if (!FULL || is(SK_BND)) ATX_MPOLE(true, false, 0, kGen);
+    else if (is(SK_STR)) ATX_MPOLE(false, false, 0, kGen);
+    else if (is(SK_BND + 2)) ATX_MPOLE(true, false, 2, kGen);
+    else ATX_MPOLE(true, false, 3, kGen);
+  } else if (is(SK_THIN2)) {
 #else
+  constexpr int SK_THIN3 = OP_THIN3, SK_DRIFT = OP_DRIFT, SK_MARK = OP_MARK;
   if (is(OP_STRRAD1L, OP_BNDRAD0, OP_BNDRAD1L)) {
     if (is(OP_STRRAD1L)) ATX_MPOLE(false, true, 1, F_LEAD);
     else if (is(OP_BNDRAD0)) ATX_MPOLE(true, true, 1, F_NOFIELD);
@@ -2039,8 +2128,8 @@ __device__ __forceinline__ void run_op(R6* r, const OpHead& o, cLatOp* rec, cDev
     ATX_MPOLE(true, false, 1, F_NOFIELD);
   } else if (is(OP_BND1L)) {
     ATX_MPOLE(true, false, 1, F_LEAD);
-#endif
   } else if (is(OP_THIN2)) {
+#endif
 #pragma unroll
     for (int q = 0; q < P; q++) thin_op<2>(r[q], k, c);
     ahead();
@@ -2060,6 +2149,10 @@ __device__ __forceinline__ void run_op(R6* r, const OpHead& o, cLatOp* rec, cDev
 #pragma unroll
     for (int q = 0; q < P; q++) rect_ap(r[q], k.v);
     ahead();
+  } else if (is(SK_DRIFT)) {
+    ahead(k.v[0]);
+#pragma unroll
+    for (int q = 0; q < P; q++) drift6(r[q], k.v[0]);
 #if !ATX_STRICT
   } else if (is(OP_STRRAD1)) {
     ATX_MPOLE(false, true, 1, F_GENERAL);
@@ -2073,28 +2166,31 @@ __device__ __forceinline__ void run_op(R6* r, const OpHead& o, cLatOp* rec, cDev
     ATX_MPOLE(true, true, 1, F_GENERAL);
   } else if (is(OP_BND1)) {
     ATX_MPOLE(true, false, 1, F_GENERAL);
+  } else if (FULL && is(OP_STRRAD2, OP_STRRAD3)) {
+    if (is(OP_STRRAD2)) ATX_MPOLE(false, true, 2, F_GENERAL);
+    else ATX_MPOLE(false, true, 3, F_GENERAL);
+  } else if (FULL && is(OP_BNDRAD2, OP_BNDRAD3)) {
+    if (is(OP_BNDRAD2)) ATX_MPOLE(true, true, 2, F_GENERAL);
+    else ATX_MPOLE(true, true, 3, F_GENERAL);
+  } else if (FULL && is(OP_BND2, OP_BND3)) {
+    if (is(OP_BND2)) ATX_MPOLE(true, false, 2, F_GENERAL);
+    else ATX_MPOLE(true, false, 3, F_GENERAL);
 #endif
-  } else if (is(OP_THIN3)) {
+  } else if (is(SK_THIN3)) {
 #pragma unroll
     for (int q = 0; q < P; q++) thin_op<3>(r[q], k, c);
     ahead();
   } else {
     ahead();
+    if (!is(SK_MARK)) {
 #pragma unroll
-    for (int q = 0; q < P; q++) r[q] = generic_element<U>(r[q], *h, pool, nturn);
+      for (int q = 0; q < P; q++) r[q] = generic_element<U>(r[q], *hdr.elem(), hdr.pool(), nturn());
+    }
   }
 #undef ATX_MPOLE
-  if (op & OPF_XF) {
+  if (op & OPF_AROUND) {
 #pragma unroll
-    for (int q = 0; q < P; q++) {
-#if ATX_STRICT
-      if (op & OPF_R2) strict_roll(r[q], c + OM_XF + 6, pool + h->r2);
-      shift(r[q], c + OM_XF + 8);
-#else
-      roll(r[q], c[OM_XF + 6], c[OM_XF + 7]);
-      shift(r[q], c + OM_XF + 8);
-#endif
-    }
+    for (int q = 0; q < P; q++) around_exit<FULL, REFS>(r[q], op, c, hdr);
   }
 }
 
@@ -2111,7 +2207,10 @@ __device__ __noinline__ R6 op_call(R6 r, const LatOp* recp, cDevElem* hp, cdoubl
   const int nturn = __builtin_amdgcn_readfirstlane(nturnp);
   R6 v = r;
   uint64_t bad = 0;
-  run_op<1, 1, true>(&v, op_head(rec), rec, h, pool, nturn, bad, NotAhead());
+  OpHead head = op_head(rec);
+  head.k = op_consts(rec);
+  run_op<1, 1, true, true, false>(&v, head, rec, KnownHeader{h, pool}, [&]() { return nturn; }, bad,
+                           NotAhead());
   if (rec->op & OPF_MPOLE) {
     const bool inf = !is_finite(v);
     if (__builtin_amdgcn_ballot_w64(inf) != 0) {
@@ -2240,15 +2339,24 @@ struct Slots {
   Lane l[P];
 };
 
-template <bool REFS, int P, int U>
+// FULL: with the kinds that have OPF_FULL, which cost the others registers.
+template <bool REFS, int P, int U, bool FULL>
 __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Instance* instp, int tp) {
   const Instance* inst = uniform(instp);
   cInstance& I = *(cInstance*)inst;
   const int t = __builtin_amdgcn_readfirstlane(tp);
-  cDevElem* elems = (cDevElem*)I.elems;
-  cdouble* pool = (cdouble*)I.pool;
   cLatOp* ops = (cLatOp*)I.ops;
-  cint* opof = (cint*)I.opof;
+  // What is needed rarely is read from the instance again, so that the fast
+  // build's loop does not keep it in scalar registers. (The strict build, whose
+  // loop is larger, is 2 % faster with it kept.)
+  auto late = [&]() -> cInstance& {
+    cInstance* i = (cInstance*)inst;
+#if !ATX_STRICT
+    asm volatile("" : "+s"(i));
+#endif
+    return *i;
+  };
+  auto opof = [&](int e) { return ((cint*)late().opof)[e]; };
   const int p[2] = {p0, p1};
   R6 r[P];
   int fl[P];
@@ -2258,7 +2366,7 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
     fl[q] = S.l[q].flags;
   }
   const bool check = !I.elempass;
-  const int nturn = I.turn0 + t;
+  auto nturn = [&]() { return late().turn0 + t; };
   const int e0 = (t == 0) ? I.start_elem : 0;
   const int e1 = I.end_elem;
   // Live particles that fail the loss test after element e: `lost` is the
@@ -2273,7 +2381,6 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   // up per element made each element wait for a scalar load, and the copy was a
   // call. One particle with a copy at each of 320 elements took 337 us per
   // turn that way, against 189 us without copies.
-  cint* bits = REFS ? (cint*)I.slots + ((t == 0) ? 0 : I.nelem / 32 + 1) : nullptr;
   const int64_t copy = 6 * (int64_t)I.npart;
   double* dst[P];
   int word = -1;
@@ -2286,7 +2393,8 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   auto copy_refs = [&](int e) {
     if ((e >> 5) != word) {
       word = e >> 5;
-      here = (uint32_t)bits[word];
+      cInstance& J = late();
+      here = (uint32_t)((cint*)J.slots)[((t == 0) ? 0 : J.nelem / 32 + 1) + word];
     }
     if (!((here >> (e & 31)) & 1)) return;
 #pragma unroll
@@ -2302,7 +2410,7 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   auto lose_mask = [&](int q, uint64_t bad, int e) {
     if (__builtin_expect(bad != 0, 0)) {
       Lane l{r[q], fl[q]};
-      loss_call(&l, inst, p[q], (int)((bad >> (threadIdx.x & 63)) & 1), nturn, e);
+      loss_call(&l, inst, p[q], (int)((bad >> (threadIdx.x & 63)) & 1), nturn(), e);
       r[q] = l.r;
       fl[q] = l.flags;
       alive[q] = __builtin_amdgcn_ballot_w64((fl[q] & L_ALIVE) != 0);
@@ -2312,17 +2420,18 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   // test. A NaN input is skipped by the first element and lost at its test.
   auto by_header = [&](int e, bool entry) {
     if (REFS) copy_refs(e);
+    const LateHeader hdr{&I, e};
 #pragma unroll
     for (int q = 0; q < P; q++) {
       if (entry) lose_mask(q, __builtin_amdgcn_ballot_w64(__builtin_isnan(r[q].x)) & alive[q], e);
 #if !ATX_STRICT
       // in the record's form, so that a turn split into calls rounds alike
-      cLatOp* rec = ops + opof[e];
+      cLatOp* rec = ops + opof(e);
       if (rec->last == e && (rec->op & OPF_MPOLE))
-        r[q] = op_call<U>(r[q], (const LatOp*)rec, &elems[e], pool, nturn);
+        r[q] = op_call<U>(r[q], (const LatOp*)rec, hdr.elem(), hdr.pool(), nturn());
       else
 #endif
-        r[q] = header_call<U>(r[q], &elems[e], pool, nturn);
+        r[q] = header_call<U>(r[q], hdr.elem(), hdr.pool(), nturn());
       if (check) lose_mask(q, lost_lanes(r[q]) & alive[q], e);
     }
   };
@@ -2342,29 +2451,26 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   // (whose input has not passed a loss test yet) and the elements of a
   // record that a partial turn starts or ends in run by their headers,
   // before and after the records.
-  const int o1 = opof[e1];
+  const int o1 = opof(e1);
   int o0 = e0 < e1 ? 0 : o1;
   int e = e0;
   if (t == 0 && e0 < e1) {
-    o0 = opof[e0] + 1;
+    o0 = opof(e0) + 1;
     for (const int stop = min(ops[o0].first, e1); e < stop; e++) by_header(e, e == e0);
   }
-#if !ATX_STRICT
   // once a radiating magnet had to be run again with the checks in its kicks,
   // the wave runs them with the checks for the rest of the turn
-  int slow = 0;  // OPF_RAD then
-#endif
+  [[maybe_unused]] int slow = 0;  // OPF_RAD then
   cLatOp* rec = ops + o0;
   cLatOp* const end = ops + max(o0, o1);
   OpHead nxt = op_head(rec);
   for (; rec != end; rec++) {
     OpHead cur = nxt;
     asm volatile("" ::"s"(cur.line1), "s"(cur.line2));
-    // With copies the constants come with the head: a load of the op's own
-    // would wait beside the copies' words (8,191 particles, a copy at every
-    // element: 2.53 against 3.00 ms per turn). Without, 16 scalar registers
-    // less are worth more (24,001 particles: 2.02 against 2.05 ms).
-    if (!REFS) cur.k = op_consts(rec);
+    // The first constants are asked for here and not with the head: 16 scalar
+    // registers less over the record before (24,001 particles: 2.02 against 2.05 ms
+    // per turn; with a copy at every element, 8,191 particles: 2.59 against 2.74).
+    cur.k = op_consts(rec);
 #if ATX_STRICT
     // The strict build's divisions take long enough for the head to come, and
     // it is 6 % faster with the head asked for here (large ring, 32,003
@@ -2411,21 +2517,21 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
       continue;
     }
     if (REFS) copy_refs(cur.last);
-    cDevElem* h = &elems[cur.last];
+    const LateHeader hdr{&I, cur.last};
     uint64_t bad = 0;
 #if ATX_STRICT
-    run_op<P, U, true>(r, cur, rec, h, pool, nturn, bad, ahead);
+    run_op<P, U, true, FULL, REFS>(r, cur, rec, hdr, nturn, bad, ahead);
 #pragma unroll
     for (int q = 0; q < P; q++) lose_mask(q, lost_lanes(r[q]) & alive[q], cur.last);
 #else
-    bool again = (cur.op & slow) != 0;
     R6 r0[P];
 #pragma unroll
     for (int q = 0; q < P; q++) r0[q] = r[q];
+    bool again = (cur.op & slow) != 0;
     if (__builtin_expect(again, 0)) {
       ahead();
     } else {
-      run_op<P, U, false>(r, cur, rec, h, pool, nturn, bad, ahead);
+      run_op<P, U, false, FULL, REFS>(r, cur, rec, hdr, nturn, bad, ahead);
       again = bad != 0;
       slow |= again ? OPF_RAD : 0;
     }
@@ -2442,13 +2548,14 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
           r0[q] = r[q];
         }
         if (first || again || (cur.op & OPF_MPOLE))
-          r[q] = op_call<U>(r0[q], (const LatOp*)rec, h, pool, nturn);
+          r[q] = op_call<U>(r0[q], (const LatOp*)rec, hdr.elem(), hdr.pool(), nturn());
         lose_mask(q, lost_lanes(r[q]) & alive[q], cur.last);
       }
     }
 #endif
   }
-  for (e = max(e, ops[o1].first); e < e1; e++) by_header(e, false);
+  const int stop = late().end_elem;
+  for (e = max(e, ((cLatOp*)late().ops)[opof(stop)].first); e < stop; e++) by_header(e, false);
   if (REFS) copy_refs(I.nelem);
 #pragma unroll
   for (int q = 0; q < P; q++) S.l[q] = Lane{r[q], fl[q]};
@@ -2637,7 +2744,10 @@ __global__ void __launch_bounds__(512, P == 1 ? 4 : 2) track_kernel(const Instan
     Slots<P> S;
 #pragma unroll
     for (int q = 0; q < P; q++) S.l[q] = L[q];
-    S = run_turn<REFS, P, U>(S, p[0], p[P - 1], insts_g + lo, t);
+    if (I.full)
+      S = run_turn<REFS, P, U, true>(S, p[0], p[P - 1], insts_g + lo, t);
+    else
+      S = run_turn<REFS, P, U, false>(S, p[0], p[P - 1], insts_g + lo, t);
 #pragma unroll
     for (int q = 0; q < P; q++) L[q] = S.l[q];
   }

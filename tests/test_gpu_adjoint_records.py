@@ -1,6 +1,6 @@
 """GPU: the adjoint of a magnet by its record (misaligned by shifts and rolls or not,
-by the form of its field) against the adjoint by its header, which an aperture on
-the magnet selects, and against central differences of the oracle. The two
+by the form of its field) against the adjoint by its header, which zero coefficients
+up to MaxOrder 4 select, and against central differences of the oracle. The two
 adjoints differ in rounding only: a few hundred operations on entries up to the
 matrix's largest, 1e-12 of it."""
 
@@ -98,7 +98,11 @@ def test_record_equals_header(kind, how):
     elems = [L.Drift("D", 0.3), m, L.Drift("D", 0.2)]
     rows, grad = _adjoint(elems, 1, coeff)
     by_header, _ = _magnet(kind, how)
-    by_header.RApertures = np.array([-1.0, 1.0, -1.0, 1.0])
+    for name in ("PolynomA", "PolynomB"):
+        poly = np.zeros(5)
+        poly[:len(getattr(m, name))] = getattr(m, name)
+        setattr(by_header, name, poly)
+    by_header.MaxOrder = 4
     rows_h, grad_h = _adjoint([L.Drift("D", 0.3), by_header, L.Drift("D", 0.2)], 1, coeff)
     np.testing.assert_allclose(rows, rows_h, rtol=0, atol=1e-12 * max(1.0, np.abs(rows_h).max()))
     np.testing.assert_allclose(grad, grad_h, rtol=0, atol=1e-12 * np.abs(grad_h).max())
