@@ -2337,10 +2337,13 @@ __device__ __noinline__ void copy_call(R6 r, const Instance* inst, double* dst, 
 template <int P>
 struct Slots {
   Lane l[P];
+  int at;  // record to go on from; kTurn: from the start, kDone: the turn is over
 };
+enum : int { kTurn = -1, kDone = -2 };
 
 // FULL: with the kinds that have OPF_FULL, which cost the others registers.
-template <bool REFS, int P, int U, bool FULL>
+// CHECKED: with the checks in the kicks of radiating magnets (fast build).
+template <bool REFS, int P, int U, bool FULL, bool CHECKED>
 __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Instance* instp, int tp) {
   const Instance* inst = uniform(instp);
   cInstance& I = *(cInstance*)inst;
@@ -2452,15 +2455,14 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
   // record that a partial turn starts or ends in run by their headers,
   // before and after the records.
   const int o1 = opof(e1);
-  int o0 = e0 < e1 ? 0 : o1;
+  const int from = __builtin_amdgcn_readfirstlane(S.at);
+  int o0 = from >= 0 ? from : e0 < e1 ? 0 : o1;
   int e = e0;
-  if (t == 0 && e0 < e1) {
+  if (t == 0 && e0 < e1 && from < 0) {
     o0 = opof(e0) + 1;
     for (const int stop = min(ops[o0].first, e1); e < stop; e++) by_header(e, e == e0);
   }
-  // once a radiating magnet had to be run again with the checks in its kicks,
-  // the wave runs them with the checks for the rest of the turn
-  [[maybe_unused]] int slow = 0;  // OPF_RAD then
+  [[maybe_unused]] int slow = 0;  // with copies: OPF_RAD once a radiating magnet had to be run again
   cLatOp* rec = ops + o0;
   cLatOp* const end = ops + max(o0, o1);
   OpHead nxt = op_head(rec);
@@ -2527,13 +2529,13 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
     R6 r0[P];
 #pragma unroll
     for (int q = 0; q < P; q++) r0[q] = r[q];
-    bool again = (cur.op & slow) != 0;
-    if (__builtin_expect(again, 0)) {
+    bool again = REFS && (cur.op & slow) != 0;
+    if (REFS && __builtin_expect(again, 0)) {
       ahead();
     } else {
-      run_op<P, U, false, FULL, REFS>(r, cur, rec, hdr, nturn, bad, ahead);
-      again = bad != 0;
-      slow |= again ? OPF_RAD : 0;
+      run_op<P, U, CHECKED, FULL, REFS>(r, cur, rec, hdr, nturn, bad, ahead);
+      again = (bad & (alive[0] | alive[P - 1])) != 0;
+      if (REFS) slow |= again ? OPF_RAD : 0;
     }
     uint64_t rare = 0;
 #pragma unroll
@@ -2551,8 +2553,25 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
           r[q] = op_call<U>(r0[q], (const LatOp*)rec, hdr.elem(), hdr.pool(), nturn());
         lose_mask(q, lost_lanes(r[q]) & alive[q], cur.last);
       }
+      // Once a radiating magnet had to be run again with the checks in its kicks, the
+      // wave takes the rest of the turn with the checks: a particle above 10 mrad or a
+      // ring that radiates more than 2e-6 in a kick seldom has one such magnet only
+      // (run again one by one, 262,144 particles of the large ring at 20 GeV took 11.7
+      // ms per turn, 9.5 this way). With copies they are run one by one: the way out
+      // of the loop costs it 4 %.
+      if (!CHECKED && !REFS && again) {
+        e = ~(int)(rec + 1 - (cLatOp*)late().ops);
+        break;
+      }
     }
 #endif
+  }
+#pragma unroll
+  for (int q = 0; q < P; q++) S.l[q] = Lane{r[q], fl[q]};
+  S.at = kDone;
+  if (!CHECKED && !REFS && e < 0) {
+    S.at = ~e;
+    return S;
   }
   const int stop = late().end_elem;
   for (e = max(e, ((cLatOp*)late().ops)[opof(stop)].first); e < stop; e++) by_header(e, false);
@@ -2744,10 +2763,13 @@ __global__ void __launch_bounds__(512, P == 1 ? 4 : 2) track_kernel(const Instan
     Slots<P> S;
 #pragma unroll
     for (int q = 0; q < P; q++) S.l[q] = L[q];
+    S.at = kTurn;
     if (I.full)
-      S = run_turn<REFS, P, U, true>(S, p[0], p[P - 1], insts_g + lo, t);
+      S = run_turn<REFS, P, U, true, ATX_STRICT>(S, p[0], p[P - 1], insts_g + lo, t);
     else
-      S = run_turn<REFS, P, U, false>(S, p[0], p[P - 1], insts_g + lo, t);
+      S = run_turn<REFS, P, U, false, ATX_STRICT>(S, p[0], p[P - 1], insts_g + lo, t);
+    if (!ATX_STRICT && !REFS && __builtin_amdgcn_readfirstlane(S.at) >= 0)
+      S = run_turn<REFS, P, U, true, true>(S, p[0], p[P - 1], insts_g + lo, t);
 #pragma unroll
     for (int q = 0; q < P; q++) L[q] = S.l[q];
   }
