@@ -216,6 +216,10 @@ class TrackingLoss:
     def apply(problem: Problem, strengths, particles, nturns: int):
         import torch
 
+        # inside forward gradients are always off, and needs_input_grad does not
+        # tell whether they were: without a backward to come nothing is kept
+        recording = torch.is_grad_enabled()
+
         class _F(torch.autograd.Function):
             @staticmethod
             def forward(ctx, theta):
@@ -242,7 +246,7 @@ class TrackingLoss:
                 ctx.kept = None
                 while t < nturns:
                     nt = min(cp, nturns - t)
-                    if t + nt < nturns or not ctx.needs_input_grad[0]:
+                    if t + nt < nturns or not (recording and ctx.needs_input_grad[0]):
                         ckpts.append((t, nt, r.clone()))
                         track(nt)
                         t += nt
