@@ -208,6 +208,7 @@ enum OpSlot : int32_t {
   OM_POLY2 = 32,  // A and B of bends of order 2 and 3, in the place of OM_POLY
   OM_RAP = 40, OM_EAP = 44,
   OM_SCALE = 46,  // FieldScaling and its reciprocal
+  OM_ZERO = 48,   // strict build: zeros that an OPF_XF adds to delta and ct at entry, exit
 };
 constexpr int kOpConsts = 52;
 struct LatOp {

@@ -681,6 +681,10 @@ int32_t fill_around(const DevElem& h, const std::vector<double>& pool, LatOp& r)
     xf[k] = (t1 ? t1[k] : -0.0) + zero1;
     xf[8 + k] = (t2 ? t2[k] : -0.0) + zero2;
   }
+  for (int k = 0; k < 2; k++) {
+    r.c[OM_ZERO + k] = (t1 ? t1[4 + k] : -0.0) + zero1;
+    r.c[OM_ZERO + 2 + k] = (t2 ? t2[4 + k] : -0.0) + zero2;
+  }
   xf[4] = xf[6] = 1.0;
   bool plain = (!t1 || plain_shift(t1)) && (!t2 || plain_shift(t2));
   if (h.flags & F_R1) plain = plain_roll(&pool[h.r1], &xf[4], &xf[5]) && plain;

@@ -2029,6 +2029,8 @@ __device__ __forceinline__ void around_entry(R6& r, int op, cdouble* c, const He
     shift(r, c + OM_XF);
 #if ATX_STRICT
     if (op & OPF_R1) strict_roll(r, c + OM_XF + 4, [&]() { return hdr.pool() + hdr.elem()->r1; });
+    r.dp += c[OM_ZERO];
+    r.ct += c[OM_ZERO + 1];
 #else
     roll(r, c[OM_XF + 4], c[OM_XF + 5]);
 #endif
@@ -2061,6 +2063,8 @@ __device__ __forceinline__ void around_exit(R6& r, int op, cdouble* c, const Hea
   if (op & OPF_XF) {
 #if ATX_STRICT
     if (op & OPF_R2) strict_roll(r, c + OM_XF + 6, [&]() { return hdr.pool() + hdr.elem()->r2; });
+    r.dp += c[OM_ZERO + 2];
+    r.ct += c[OM_ZERO + 3];
 #else
     roll(r, c[OM_XF + 6], c[OM_XF + 7]);
 #endif

@@ -134,3 +134,19 @@ def test_infinite_input_without_loss_records(kind, slices, how):
     np.testing.assert_array_equal(got, ref)
     got, _ = _track(ring, beam, False, losses=False)
     np.testing.assert_allclose(got, ref, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("how", MOVES)
+def test_signs_of_zero(how):
+    """Strict build: a particle at (signed) zeros passes a magnet without kicks as in the oracle."""
+    beam = np.zeros((6, 64), order="F")
+    beam[np.random.default_rng(13).integers(0, 2, (6, 64)) == 1] = -0.0
+    m = _move(Quadrupole("Q", 0.4, 0.0), how)
+    for t in ("T1", "T2"):
+        if how == "all":
+            setattr(m, t, np.array([0.0, -0.0, -0.0, 0.0, 0.0, 0.0]))
+    ring = _ring(m)
+    ref = beam.copy(order="F")
+    po.atpass(ring, ref, 1)
+    got, _ = _track(ring, beam, True, losses=False)
+    np.testing.assert_array_equal(np.signbit(got), np.signbit(ref))
