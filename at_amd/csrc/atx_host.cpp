@@ -1452,6 +1452,8 @@ int atx_lattice_add_elements(atx_lattice* lat, int32_t n, const char* const* str
   if (n == 0) return ATX_OK;
   if (!strings || !elems || (nattrs > 0 && !attrs) || (nvalues > 0 && !values))
     return fail(ATX_E_VALUE, "NULL argument");
+  for (int32_t k = 0; k < nstrings; k++)
+    if (!strings[k]) return fail(ATX_E_VALUE, "NULL string");
   std::lock_guard<std::mutex> g(lat->mu);
   std::vector<int> kinds(nstrings, -2);  // of the strings that are pass methods
   int64_t at = 0, v = 0;
@@ -1482,6 +1484,7 @@ int atx_lattice_add_elements(atx_lattice* lat, int32_t n, const char* const* str
   }
   return ATX_OK;
 }
+
 static int set_attr(atx_lattice* lat, const char* name, const double* v, int64_t n, bool is_int) {
   if (!lat || !name) return fail(ATX_E_VALUE, "NULL argument");
   if (lat->elems.empty()) return fail(ATX_E_VALUE, "no element to set an attribute on");
