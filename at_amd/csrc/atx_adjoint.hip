@@ -578,11 +578,16 @@ __global__ void __launch_bounds__(256, 2) adjoint_kernel(AdjArgs args) {
 #undef ATX_REV
         default: {
           ahead();
-          // inline: as a function it costs the loop its scalar registers (9.8
-          // against 8.9 ms for 8 turns of 4,096 particles of the large ring), and
+          // Inline: as a function it costs the loop its scalar registers (9.8
+          // against 8.8 ms for 8 turns of 4,096 particles of the large ring), and
           // with its pointers in vector registers the loads are one per lane (a
-          // corrected error realisation without forms for misalignment: 126 ms)
-          element_rev(r, l, elems[cur.last], aes[cur.last], pool, grad, nturn);
+          // corrected error realisation without forms for misalignment: 126 ms).
+          // On copies: the matrix products take the states by address, and the
+          // loop's own would live in memory (12.1 ms).
+          V6 r1 = r, l1 = l;
+          element_rev(r1, l1, elems[cur.last], aes[cur.last], pool, grad, nturn);
+          r = r1;
+          l = l1;
         }
       }
       if (moved) {
