@@ -85,8 +85,8 @@ enum Slot : int32_t {
   S_RK1 = 19, S_RK2 = 20,                   // S_RADC * S_K1, S_RADC * S_K2 (fast build)
   S_ELEN = 21,                              // Length (exact multipoles)
   S_DIFC = 22,                              // DIF_CONST * gamma^5 (diffusion matrices)
-  S_HL1 = 23, S_HL2 = 24,                   // S_L1 / 2, S_L2 / 2 (fast radiating drifts)
-  S_NSCALAR = 26,
+  S_NSCALAR = 23,
+  S_NSHORT = 8,                             // of elements that are no multipoles
   // RF cavity
   S_RF_HALF = 0, S_RF_NV = 1, S_RF_TWOPIF = 2, S_RF_LAG = 3, S_RF_PHILAG = 4, S_RF_HFT0 = 5,
   // corrector
@@ -105,11 +105,9 @@ struct DevElem {
   int32_t t1, r1;     // pool offsets (valid when the flag is set)
   int32_t r2, t2;
   int32_t rap, eap;   // RApertures (4) / Limits (4); EApertures (2)
-  int32_t edge;       // EdgeMode at entrance | (EdgeMode at exit << 8); DriftPass: low
-                      // word of the Length bits
+  int32_t edge;       // EdgeMode at entrance | (EdgeMode at exit << 8)
   int32_t ops;        // pool offset of the slice op table (integrators other than 4), -1: none
-  int32_t fringe;     // QuadFringe at entrance | (QuadFringe at exit << 8); DriftPass: high
-                      // word of the Length bits
+  int32_t fringe;     // QuadFringe at entrance | (QuadFringe at exit << 8)
   int32_t fq;         // pool offset of the elegant fringe matrices: in-P, in-M, out-M, out-P (8 each)
 };
 

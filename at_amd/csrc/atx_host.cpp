@@ -365,6 +365,7 @@ int compile_elem(const HostElem& e, int idx, double energy, double rest, double 
   std::vector<double>& pool = out.pool;
   double sc[S_NSCALAR];
   for (double& v : sc) v = 0.0;
+  int nsc = S_NSHORT;
 
   switch (e.kind) {
     case K_IDENTITY:
@@ -373,14 +374,6 @@ int compile_elem(const HostElem& e, int idx, double energy, double rest, double 
     case K_DRIFT:
     case K_EXDRIFT:  // DriftPass.c:50-80, ExactDriftPass.c:46-75
       sc[S_D_LEN] = rd.dbl("Length");
-      if (e.kind == K_DRIFT) {
-        // the tracking kernel reads a drift's length from its header (edge,
-        // fringe: unused by drifts), saving a dependent load per drift
-        uint64_t bits;
-        std::memcpy(&bits, &sc[S_D_LEN], sizeof(bits));
-        h.edge = (int32_t)(uint32_t)bits;
-        h.fringe = (int32_t)(uint32_t)(bits >> 32);
-      }
       transforms(rd, h, pool);
       break;
     case K_CAVITY: {  // CavityPass.c:62-88
@@ -444,6 +437,7 @@ int compile_elem(const HostElem& e, int idx, double energy, double rest, double 
       if (nv != 0.0) h.flags |= F_RFKICK;
     } break;
     default: {  // multipoles
+      nsc = S_NSCALAR;
       const bool thin = (e.kind == K_THIN);
       const bool bend = (e.kind == K_BND || e.kind == K_BNDRAD);
       const bool exact = (e.kind == K_EXMPOLE || e.kind == K_EXMPOLERAD);
@@ -505,8 +499,6 @@ int compile_elem(const HostElem& e, int idx, double energy, double rest, double 
       const double sl = len / (double)nslice;
       sc[S_L1] = sl * kDrift1;
       sc[S_L2] = sl * kDrift2;
-      sc[S_HL1] = 0.5 * sc[S_L1];
-      sc[S_HL2] = 0.5 * sc[S_L2];
       sc[S_K1] = sl * kKick1;
       sc[S_K2] = sl * kKick2;
       sc[S_ELEN] = len;
@@ -590,7 +582,7 @@ int compile_elem(const HostElem& e, int idx, double energy, double rest, double 
     } break;
   }
   if (rd.err) return rd.err;
-  h.sc = push(pool, sc, S_NSCALAR);
+  h.sc = push(pool, sc, nsc);
   if (h.kind == K_STR || h.kind == K_BND || h.kind == K_STRRAD || h.kind == K_BNDRAD) {
     auto flat = [](int m) { return m == E_CONST || m == E_DIVP || m == E_MULPN; };
     if (!(h.flags & F_SCALE) && h.fringe == 0 && h.ops < 0 && flat(h.edge & 0xff) &&
@@ -619,7 +611,7 @@ int compile_elem(const HostElem& e, int idx, double energy, double rest, double 
   if (h.kind == K_CAVITY || h.kind == K_EXDRIFT || h.kind == K_EXMPOLE || h.kind == K_EXMPOLERAD)
     aerr = "pass method without an adjoint";
   if (h.flags & F_SCALE) aerr = "FieldScaling != 1";
-  if (h.kind != K_DRIFT && h.fringe) aerr = "quadrupole fringe";  // a drift's holds its length
+  if (h.fringe) aerr = "quadrupole fringe";
   if (h.ops >= 0) aerr = "integrator other than 4";
   for (int side = 0; side < 2; side++) {
     const int m = (h.edge >> (8 * side)) & 0xff;

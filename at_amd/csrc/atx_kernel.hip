@@ -284,17 +284,6 @@ __device__ __forceinline__ double rcp_after_kick(double opd2, double pn) {
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) q = far ? fast_rcp(opd2) : q;
   return q;
 }
-
-// Fast build: inside a radiating magnet delta changes only in the kicks, so
-// pn = 1/(1+delta) is computed once at entry and then by each kick for the
-// radiated delta, and carried to the drifts.
-__device__ __forceinline__ void rad_drift_pn(R6& r, double len, double pn) {
-  const double nl = len * pn;
-  r.x = __builtin_fma(nl, r.px, r.x);
-  r.y = __builtin_fma(nl, r.py, r.y);
-  const double p2 = __builtin_fma(r.px, r.px, r.py * r.py);
-  r.ct = __builtin_fma(nl * pn * 0.5, p2, r.ct);
-}
 #endif
 
 // Radiating straight kick (diff_str_kick.c:19-83, bdiff == NULL).
