@@ -208,7 +208,7 @@ enum OpSlot : int32_t {
   OM_SCALE = 46,  // FieldScaling and its reciprocal
   OM_ZERO = 48,   // strict build: zeros that an OPF_XF adds to delta and ct at entry, exit
 };
-constexpr int kOpConsts = 52;
+constexpr int kOpConsts = 60;  // 52 and padding
 struct LatOp {
   int32_t op;      // OpKind | OPF_* | StrictKind << kStrictShift
   int32_t last;    // index of the record's last element
@@ -218,7 +218,9 @@ struct LatOp {
   double lead;     // their highest coefficient that is not zero (B)
   double c[kOpConsts];
 };
-static_assert(sizeof(LatOp) == 448, "LatOp: seven 64-byte lines");
+// Four lines of the L2: with 448 bytes, where every other record starts in the middle
+// of one, a turn of the large ring takes 1.92 ms instead of 1.88 (24,001 particles).
+static_assert(sizeof(LatOp) == 512, "LatOp: four 128-byte lines");
 
 // One tracked lattice instance inside a launch. A single-lattice call has one
 // instance; batched error realisations have one per lattice.
