@@ -867,6 +867,16 @@ void ref_bits(const int32_t* slot, int nelem, int32_t* words) {
         words[k * half + e / 32] |= (int32_t)(1u << (e % 32));
 }
 
+// Whether the copies of these tables are made elsewhere than at the end of a turn.
+bool inner_refs(const std::vector<int32_t>& words, int nelem) {
+  const size_t half = words.size() / 2;
+  for (size_t i = 0; i < words.size(); i++) {
+    const bool last = i % half == (size_t)nelem / 32;
+    if ((uint32_t)words[i] & ~(last ? 1u << (nelem % 32) : 0u)) return true;
+  }
+  return false;
+}
+
 #define HIPCHK(x)                                                                         \
   do {                                                                                    \
     hipError_t e_ = (x);                                                                  \
@@ -1034,9 +1044,14 @@ int launch_instances(std::vector<Instance>& insts, const std::vector<const std::
   const int block = shape.block;
   const int per_wg = block * shape.ppt;  // particle slots per workgroup
   int nblocks = 0;
-  bool refs = false;  // some instance has refpt copies: the kernel with them
-  for (auto& in : insts) {
-    refs |= (in.n_first | in.n_std) != 0;
+  // Some instance has refpt copies before the end of a turn: the kernel with them.
+  // (Those at the end only, what a tracking call asks for by default, cost it 10 %:
+  // 1,000 particles of the large ring 2.13 against 1.93 ms per turn, and a
+  // dynamic-aperture grid of 24,001 3.86 against 2.82.)
+  bool refs = false;
+  for (size_t i = 0; i < insts.size(); i++) {
+    Instance& in = insts[i];
+    refs |= (in.n_first | in.n_std) != 0 && inner_refs(*slots[i], in.nelem);
     in.block_begin = nblocks;
     nblocks += (int)((in.npart + per_wg - 1) / per_wg);
   }

@@ -2681,7 +2681,8 @@ __global__ void __launch_bounds__(512, P == 1 ? 4 : 2) track_kernel(const Instan
   // with several whenever one was lost (a lane steps its particles together
   // only while none of them is lost). Not with refpts: lost particles still
   // fill their refpt copies, as in at.c.
-  const bool compact = check && !REFS && nturns > 1;
+  const bool ends = !REFS && (I.n_first | I.n_std) != 0;  // copies at the end of a turn only
+  const bool compact = check && !REFS && !ends && nturns > 1;
   double* s_r = lds;
   int* s_p = (int*)(lds + 6 * G);
   int* s_cnt = s_p + G;
@@ -2765,6 +2766,16 @@ __global__ void __launch_bounds__(512, P == 1 ? 4 : 2) track_kernel(const Instan
       S = run_turn<REFS, P, U, true, true>(S, p[0], p[P - 1], insts_g + lo, t);
 #pragma unroll
     for (int q = 0; q < P; q++) L[q] = S.l[q];
+    if (ends) {
+      const int64_t base = (t == 0) ? 0 : (int64_t)I.n_first + (int64_t)(t - 1) * I.n_std;
+      double* out = I.rout + base * 6 * (int64_t)npart;
+#pragma unroll
+      for (int q = 0; q < P; q++) {
+        if (!(L[q].flags & L_HAS)) continue;
+        const bool alive = (L[q].flags & L_ALIVE) != 0;
+        store6(out + 6 * (int64_t)p[q], 1, alive ? L[q].r : load_state(I, p[q]));
+      }
+    }
   }
 #pragma unroll
   for (int q = 0; q < P; q++)
