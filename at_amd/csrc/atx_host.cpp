@@ -935,9 +935,13 @@ int ensure_device_lattice(atx_lattice* lat, double energy, double rest, bool ele
 
 constexpr int kBlock = 256;
 constexpr int kPpt = 1;
-// two slices per loop iteration in the fast build (120 VGPRs, four waves per
-// SIMD); one in the strict build, whose two-slice kernel needs 136 VGPRs and
-// would run three waves per SIMD
+// One particle per lane, two slices per loop iteration in the fast build and one
+// in the strict build. All shapes of one particle run four waves per SIMD. The large
+// ring, ms per turn by particles per lane / slices per iteration: 24,001 particles
+// 1.98 (1/1), 1.96 (1/2), 1.89 (1/4), 3.40 (2/2: half the waves); 262,144 6.60,
+// 6.59, 6.46, 6.43; 1,048,576 24.5, 24.2, 24.4, 24.0; strict, 32,003 6.45 (1/1),
+// 6.26 (1/2), 12.5 (2/2). Four slices, and two in the strict build, would be 2 to 4
+// % faster with few waves.
 constexpr int kUnrollFast = 2;
 constexpr int kUnrollStrict = 1;
 
@@ -1180,7 +1184,10 @@ int launch_repacked(std::vector<Instance>& insts, const std::vector<const std::v
   bytes += ninst * sizeof(int32_t);
   const size_t live_off = bytes;  // live workgroup map of the current block
   bytes += (ninst + 2) * sizeof(int32_t);
-  // survivors that fit in two waves per SIMD run one wave per workgroup
+  // Survivors that fit in two waves per SIMD run one wave per workgroup (up to half,
+  // one, two, four waves per SIMD, and never: 16 dynamic-aperture grids 73.1, 72.5,
+  // 71.5, 73.9, 72.8 ms, 8 grids 46.3, 45.7, 45.2, 45.5, 46.4, 8 served requests
+  // 63.8, 63.8, 67.0, 67.4, 63.5).
   int dev = 0, ncu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
