@@ -2313,6 +2313,17 @@ __device__ __noinline__ void loss_call(Lane* lp, const Instance* inst, int p, in
   *lp = l;
 }
 
+// Waits here for a state that a rare path has read from memory. The compiler
+// would wait at the next use that the common path shares, and there for the copies
+// of the record before, too (strict build, a copy at every element, 8,191
+// particles: 7.17 -> 6.72 ms per turn of the large ring, with the word of copies
+// waited for where it is read; no faster in the fast build).
+__device__ __forceinline__ void arrived(R6& r, int& flags) {
+#if ATX_STRICT
+  asm volatile("" : "+v"(r.x), "+v"(r.px), "+v"(r.y), "+v"(r.py), "+v"(r.dp), "+v"(r.ct), "+v"(flags));
+#endif
+}
+
 // Refpt copy: dst is the particle's six doubles in r_out; a particle whose
 // state is final is copied from memory.
 __device__ __noinline__ void copy_call(R6 r, const Instance* inst, double* dst, int p, int flags) {
@@ -2391,10 +2402,20 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
       word = e >> 5;
       cInstance& J = late();
       here = (uint32_t)((cint*)J.slots)[((t == 0) ? 0 : J.nelem / 32 + 1) + word];
+#if ATX_STRICT
+      asm volatile("" : "+s"(here));  // arrived()
+#endif
     }
     if (!((here >> (e & 31)) & 1)) return;
 #pragma unroll
     for (int q = 0; q < P; q++) {
+      // A whole wave of live particles is stored without looking at its lanes
+      // (8,191 particles of the large ring: 2.52 -> 2.46 ms per turn, 64: 2.32 -> 2.25).
+      if (alive[q] == ~(uint64_t)0) {
+        store6(dst[q], 1, r[q]);
+        dst[q] += copy;
+        continue;
+      }
       const bool has = (fl[q] & L_HAS) != 0;
       if (__builtin_expect((__builtin_amdgcn_ballot_w64(has) & ~alive[q]) != 0, 0))
         copy_call(r[q], inst, dst[q], p[q], fl[q]);
@@ -2409,6 +2430,7 @@ __device__ __noinline__ Slots<P> run_turn(Slots<P> S, int p0, int p1, const Inst
       loss_call(&l, inst, p[q], (int)((bad >> (threadIdx.x & 63)) & 1), nturn(), e);
       r[q] = l.r;
       fl[q] = l.flags;
+      if (REFS) arrived(r[q], fl[q]);
       alive[q] = __builtin_amdgcn_ballot_w64((fl[q] & L_ALIVE) != 0);
     }
   };
